@@ -107,7 +107,10 @@ def draw(rng):
             if batch * sum(a * b for a, b in zip(widths, widths[1:])) <= 1 << 29:      # above it the emitter keeps the layers apart
                 return {"kind": kind, "batch": batch, "widths": "-".join(map(str, widths))}
     if kind in ("cnn_f32", "qcnn"):
-        return {"kind": kind, "batch": _size(rng, 1, 1024 if kind == "cnn_f32" else 4096)}
+        while True:
+            batch = _size(rng, 1, 1024 if kind == "cnn_f32" else 4096)
+            if batch not in (64, 256, 4096):      # these are listed
+                return {"kind": kind, "batch": batch}
     if kind == "gemm_f32":
         M, N, K = _draw_gemm_sizes(rng, CONV_F32_FLOPS, 1, 4)
         return {"kind": kind, "M": M, "N": N, "K": K, "transA": rng.random() < 0.2, "transB": rng.random() < 0.5, "bias": rng.random() < 0.8,
