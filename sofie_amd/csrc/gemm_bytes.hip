@@ -40,9 +40,60 @@ __device__ __forceinline__ void tile_of_workgroup(int pid, int tiles_m, int tile
    tn = (pid % width) / gsize;
 }
 
-template <class Mma, int BK, int NSETS, int TI, int TJ, int OUT, bool B_KN, bool FULL>
+// How much k_gemm_bytes may assume about its operands.
+//   WHOLE_TILES  every tile lies inside the matrices, rows of whole 16-byte chunks
+//   CHUNK_ROWS   ragged tiles; K, leading dimensions and pointers multiples of 16
+//   DWORD_ROWS   ... multiples of 4 with K >= 16
+//   ANY_ROWS     nothing but K >= 16 (and N >= 4 with B [K,N])
+enum TileMode { WHOLE_TILES, CHUNK_ROWS, DWORD_ROWS, ANY_ROWS };
+
+// Bytes k .. k + 15 of a row of K >= 16 bytes that starts at any address, zero behind K. load_row_chunk requests the dwords
+// they lie in (loads from odd addresses are taken apart lane by lane: 256 x 1000 x 1001 in k_gemm_bytes_direct took 13.6 us
+// with them and 5.7 us with K = 1000), row_chunk puts them together once they are there. A chunk that would run over the
+// end of the row is requested so that it ends there and is moved down. No byte outside the aligned dwords of the row is
+// touched. SHIFTS: some row or K is no multiple of four bytes (without it the fifth dword is not requested).
+struct RowChunk {
+   v4i d;
+   int e;
+};
+template <bool SHIFTS>
+__device__ __forceinline__ void load_row_chunk(RowChunk &c, const unsigned char *row, int k, int K)
+{
+   const unsigned char *p = row + (k < K - 16 ? k : K - 16);
+   const int sh = (int)(reinterpret_cast<uintptr_t>(p) & 3u);
+   p -= sh;
+   __builtin_memcpy(&c.d, __builtin_assume_aligned(p, 4), 16);
+   if constexpr (SHIFTS) c.e = *reinterpret_cast<const int *>(p + (sh ? 16 : 12));
+}
+template <bool SHIFTS>
+__device__ __forceinline__ v4i row_chunk(const RowChunk &c, const unsigned char *row, int k, int K)
+{
+   v4i v = c.d;
+   if constexpr (SHIFTS) {
+      const unsigned sh = (unsigned)((reinterpret_cast<uintptr_t>(row) + (k < K - 16 ? k : K - 16)) & 3u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+         v[i] = (int)__builtin_amdgcn_alignbyte((unsigned)(i < 3 ? c.d[i + 1] : c.e), (unsigned)c.d[i], sh);
+   }
+   return v;
+}
+__device__ __forceinline__ v4i trim_row_chunk(v4i v, int k, int K)
+{
+   const int drop = k - (K - 16);      // bytes in front of k that load_row_chunk had to take along
+   if (drop <= 0) return v;
+   if (drop >= 16) return v4i{0, 0, 0, 0};
+   typedef unsigned long long u64;
+   const u64 lo = ((u64)(unsigned)v[1] << 32) | (unsigned)v[0], hi = ((u64)(unsigned)v[3] << 32) | (unsigned)v[2];
+   const int bits = drop * 8;
+   const u64 rl = bits < 64 ? (lo >> bits) | (hi << (64 - bits)) : hi >> (bits - 64);
+   const u64 rh = bits < 64 ? hi >> bits : 0;
+   return v4i{(int)(unsigned)rl, (int)(unsigned)(rl >> 32), (int)(unsigned)rh, (int)(unsigned)(rh >> 32)};
+}
+
+template <class Mma, int BK, int NSETS, int TI, int TJ, int OUT, bool B_KN, TileMode MODE>
 __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_gemm_bytes(GemmArgs g)
 {
+   constexpr bool FULL = MODE == WHOLE_TILES, ANY = MODE >= DWORD_ROWS, SHIFTS = MODE == ANY_ROWS;
    constexpr int BN = 2 * TI * 32, BM = 2 * TJ * 32;
    constexpr int LDK = BK + 16;
    constexpr int CPR = BK / 16;
@@ -101,6 +152,7 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    struct Staged {
       v4i a[A_CH];
       v4i b[B_CH];
+      int ae[SHIFTS ? A_CH : 1], be[SHIFTS ? B_CH : 1];      // the fifth dwords of chunks off a dword
    };
    const v4i zero4 = {0, 0, 0, 0};
 
@@ -118,6 +170,7 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    }
    const unsigned char *pb[B_PARTS];
    bool okb[B_PARTS];
+   [[maybe_unused]] int down[B_PARTS];
 #pragma unroll
    for (int i = 0; i < B_PARTS; ++i) {
       if constexpr (!B_KN) {
@@ -130,19 +183,54 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
          const int kg = u % CPR, ng = u / CPR;
          const int gn = n0 + ng * 4;
          okb[i] = (B_UNITS % 256 == 0 || u < B_UNITS) && (FULL || gn < g.N);
-         pb[i] = g.B + (size_t)(kg * 16) * g.ldb + (okb[i] ? gn : 0);
+         if constexpr (ANY) {
+            // the last columns: four that end with the row, moved down (what a dword holds behind column N is not stored)
+            const int col = okb[i] ? gn : 0, first = col < g.N - 4 ? col : g.N - 4;
+            pb[i] = g.B + first;
+            down[i] = (col - first) * 8;
+         } else {
+            pb[i] = g.B + (size_t)(kg * 16) * g.ldb + (okb[i] ? gn : 0);
+         }
       }
    }
-   const int kmax = g.K - 16;   // K is a multiple of 16 on this path
+   const int kmax = g.K - 16;   // the start of the last whole chunk of a row
 
    auto fetch_a = [&](Staged &G, int k0, int i) {
       const int kc = ((i * 256 + tid) % CPR) * 16;
+      if constexpr (ANY) {
+         // (rows behind M are copies of the last one and their results are not stored)
+         RowChunk c;
+         load_row_chunk<SHIFTS>(c, pa[i] - kc, k0 + kc, g.K);
+         G.a[i] = c.d;
+         if constexpr (SHIFTS) G.ae[i] = c.e;
+         return;
+      }
       const bool kin = FULL || k0 + kc <= kmax;
       const v4i v = *reinterpret_cast<const v4i *>(pa[i] + (kin ? k0 : kmax - kc));
       G.a[i] = (oka[i] && kin) ? v : zero4;
    };
    auto fetch_b = [&](Staged &G, int k0, int i) {
       const int kc = ((i * 256 + tid) % CPR) * 16;
+      if constexpr (ANY && !B_KN) {
+         RowChunk c;
+         load_row_chunk<SHIFTS>(c, pb[i] - kc, k0 + kc, g.K);
+         G.b[i] = c.d;
+         if constexpr (SHIFTS) G.be[i] = c.e;
+         return;
+      }
+      if constexpr (ANY && B_KN) {
+         // rows behind K are copies of the last one: A's zeros meet them
+#pragma unroll
+         for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+               const int k = k0 + kc + 4 * q + e;
+               unsigned d;
+               __builtin_memcpy(&d, pb[i] + (size_t)(k < g.K ? k : g.K - 1) * g.ldb, 4);
+               G.b[i * 4 + q][e] = (int)(d >> down[i]);
+            }
+         return;
+      }
       const bool kin = FULL || k0 + kc <= kmax;
       if constexpr (!B_KN) {
          const v4i v = *reinterpret_cast<const v4i *>(pb[i] + (kin ? k0 : kmax - kc));
@@ -160,15 +248,28 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
          }
       }
    };
-   auto stash_a = [&](const Staged &G, int stage, int i) {
+   // (k0: the K-step the set was requested for)
+   auto stash_a = [&](const Staged &G, int stage, int k0, int i) {
       const int c = i * 256 + tid;
-      *reinterpret_cast<v4i *>(sA + stage * BM * LDK + (c / CPR) * LDK + (c % CPR) * 16) = G.a[i];
+      v4i v = G.a[i];
+      if constexpr (ANY) {
+         const int kc = (c % CPR) * 16;
+         v = row_chunk<SHIFTS>(RowChunk{G.a[i], G.ae[SHIFTS ? i : 0]}, pa[i] - kc, k0 + kc, g.K);
+         if (k0 + BK > g.K) v = trim_row_chunk(v, k0 + kc, g.K);
+      }
+      *reinterpret_cast<v4i *>(sA + stage * BM * LDK + (c / CPR) * LDK + (c % CPR) * 16) = v;
    };
-   auto stash_b = [&](const Staged &G, int stage, int i) {
+   auto stash_b = [&](const Staged &G, int stage, int k0, int i) {
       unsigned char *b = sB + stage * BN * LDK;
       if constexpr (!B_KN) {
          const int c = i * 256 + tid;
-         *reinterpret_cast<v4i *>(b + (c / CPR) * LDK + (c % CPR) * 16) = G.b[i];
+         v4i v = G.b[i];
+         if constexpr (ANY) {
+            const int kc = (c % CPR) * 16;
+            v = row_chunk<SHIFTS>(RowChunk{G.b[i], G.be[SHIFTS ? i : 0]}, pb[i] - kc, k0 + kc, g.K);
+            if (k0 + BK > g.K) v = trim_row_chunk(v, k0 + kc, g.K);
+         }
+         *reinterpret_cast<v4i *>(b + (c / CPR) * LDK + (c % CPR) * 16) = v;
       } else {
          const int u = i * 256 + tid;
          const bool live = B_UNITS % 256 == 0 || u < B_UNITS;
@@ -197,15 +298,15 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    };
    // Pieces of a tile pair are numbered 0..A_CH+B_PARTS-1 and dealt round-robin to the MFMA
    // groups of a K-step; group `grp` of `ngrp` moves the pieces p with p % ngrp == grp.
-   auto move_pieces = [&](Staged &G, int stage, int k_next, int grp, int ngrp, bool do_stash, bool do_fetch) {
+   auto move_pieces = [&](Staged &G, int stage, int k_held, int k_next, int grp, int ngrp, bool do_stash, bool do_fetch) {
 #pragma unroll
       for (int p = 0; p < A_CH + B_PARTS; ++p) {
          if (p % ngrp != grp) continue;
          if (p < A_CH) {
-            if (do_stash) stash_a(G, stage, p);
+            if (do_stash) stash_a(G, stage, k_held, p);
             if (do_fetch) fetch_a(G, k_next, p);
          } else {
-            if (do_stash) stash_b(G, stage, p - A_CH);
+            if (do_stash) stash_b(G, stage, k_held, p - A_CH);
             if (do_fetch) fetch_b(G, k_next, p - A_CH);
          }
       }
@@ -247,7 +348,7 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    //   substep NSUB-1:     multiply while set 0 is refilled from the other stage.
    // The instruction order is pinned with scheduling barriers so that every group of TJ MFMAs
    // has memory instructions issued right behind it to overlap with.
-   auto kstep = [&](int stage, Staged &G, int k_next, bool more) {
+   auto kstep = [&](int stage, Staged &G, int k_held, int k_next, bool more) {
       constexpr int NGRP = (NSUB - 1) * TMAX;
 #pragma unroll
       for (int sub = 0; sub < NSUB - 1; ++sub) {
@@ -255,7 +356,7 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
          for (int i = 0; i < TMAX; ++i) {
             read_pair((sub + 1) & 1, stage, sub + 1, i);
             mma_row(sub & 1, i);
-            move_pieces(G, stage ^ 1, k_next, sub * TMAX + i, NGRP, more, true);
+            move_pieces(G, stage ^ 1, k_held, k_next, sub * TMAX + i, NGRP, more, true);
             __builtin_amdgcn_sched_barrier(0);
          }
       }
@@ -276,12 +377,12 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    // unconditional keeps the number of loads in flight identical on every path.
    Staged G[NSETS];
    if (nk > 0) {
-      move_pieces(G[0], 0, 0, 0, 1, false, true);               // tile 0
+      move_pieces(G[0], 0, 0, 0, 0, 1, false, true);               // tile 0
 #pragma unroll
-      for (int s = 1; s < NSETS; ++s) move_pieces(G[s], 0, kclamp(s), 0, 1, false, true);   // tiles 1 .. NSETS-1
+      for (int s = 1; s < NSETS; ++s) move_pieces(G[s], 0, 0, kclamp(s), 0, 1, false, true);   // tiles 1 .. NSETS-1
       // (the later tiles are requested before tile 0 is waited for: their way from memory runs under its)
-      move_pieces(G[0], 0, 0, 0, 1, true, false);               // tile 0 -> stage 0
-      move_pieces(G[0], 0, kclamp(NSETS), 0, 1, false, true);   // tile NSETS
+      move_pieces(G[0], 0, 0, 0, 0, 1, true, false);               // tile 0 -> stage 0
+      move_pieces(G[0], 0, 0, kclamp(NSETS), 0, 1, false, true);   // tile NSETS
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < TMAX; ++i) read_pair(0, 0, 0, i);
@@ -294,11 +395,11 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
    int kt = 0;
    for (; kt + UNR <= nk; kt += UNR) {
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) kstep(u & 1, G[(u + 1) % NSETS], kclamp(kt + u + 1 + NSETS), kt + u + 1 < nk);
+      for (int u = 0; u < UNR; ++u) kstep(u & 1, G[(u + 1) % NSETS], kclamp(kt + u + 1), kclamp(kt + u + 1 + NSETS), kt + u + 1 < nk);
    }
 #pragma unroll
    for (int u = 0; u < UNR - 1; ++u)
-      if (kt + u < nk) kstep(u & 1, G[(u + 1) % NSETS], klast, kt + u + 1 < nk);
+      if (kt + u < nk) kstep(u & 1, G[(u + 1) % NSETS], kclamp(kt + u + 1), klast, kt + u + 1 < nk);
    __syncthreads();
 
    tile_epilogue<Mma, TI, TJ, OUT, 4>(g, acc, smem, tid, m0 + wm * (TJ * 32), n0, wn, BN);
@@ -879,6 +980,16 @@ __global__ void __launch_bounds__(512, 2) k_gemm_dma16(GemmArgs g)
       tile_epilogue_wave16<NI, MJ, OUT, 0>(g, acc, stg, s_scale + wn * 128, s_bias + wn * 128, lane, m_wave, n_wave);
 }
 
+__device__ __forceinline__ void transpose_4x4_bytes(unsigned d0, unsigned d1, unsigned d2, unsigned d3, unsigned (&o)[4])
+{
+   const unsigned t0 = __builtin_amdgcn_perm(d1, d0, 0x05010400u), t1 = __builtin_amdgcn_perm(d1, d0, 0x07030602u);
+   const unsigned t2 = __builtin_amdgcn_perm(d3, d2, 0x05010400u), t3 = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
+   o[0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+   o[1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+   o[2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+   o[3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+}
+
 // Byte-matrix transpose src [R, C] (ld_src) -> dst [C, R] (ld_dst), R % 16 == 0, C % 4 == 0.
 // A thread takes 16 rows x 4 columns (16 dwords), transposes them in registers with
 // v_perm_b32 and writes four 16-byte row segments; eight neighbouring lanes write 128
@@ -897,14 +1008,10 @@ __global__ void __launch_bounds__(256) k_transpose_bytes(const unsigned char *__
    unsigned o[4][4];
 #pragma unroll
    for (int q = 0; q < 4; ++q) {
-      const unsigned t0 = __builtin_amdgcn_perm(d[4 * q + 1], d[4 * q + 0], 0x05010400u);
-      const unsigned t1 = __builtin_amdgcn_perm(d[4 * q + 1], d[4 * q + 0], 0x07030602u);
-      const unsigned t2 = __builtin_amdgcn_perm(d[4 * q + 3], d[4 * q + 2], 0x05010400u);
-      const unsigned t3 = __builtin_amdgcn_perm(d[4 * q + 3], d[4 * q + 2], 0x07030602u);
-      o[0][q] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-      o[1][q] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-      o[2][q] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-      o[3][q] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+      unsigned t[4];
+      transpose_4x4_bytes(d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3], t);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j][q] = t[j];
    }
 #pragma unroll
    for (int j = 0; j < 4; ++j) {
@@ -920,8 +1027,71 @@ int transpose_bytes(sofie_hip_ctx *ctx, const unsigned char *src, unsigned char 
    return check_launch(ctx, "k_transpose_bytes");
 }
 
-// Any shape, any alignment: one thread per output element. Correctness path for operands
-// the tiled kernel cannot take (K not a multiple of 16, unaligned rows).
+// One-byte operands in any storage -> rows of K bytes as the fast kernels read them: A [M][Kp] and B^T [N][Kp], Kp = K
+// rounded up to 16 with zeros behind K. One launch for both: the first `blocks_a` workgroups copy rows of A (none if A may
+// stay where it is), the rest copy rows of B [N,K] or, kn, transpose B [K,N]. Bound by HBM (each byte read and written
+// once); byte loads would cost a request per byte, so a thread of the copy takes 16 bytes from wherever they start and a
+// thread of the transpose four columns of 16 rows.
+struct CopyOperandsArgs {
+   const unsigned char *A, *B;
+   unsigned char *Ap, *Bp;
+   int M, N, K, lda, ldb, Kp, kn, blocks_a, groups_k;
+};
+
+__global__ void __launch_bounds__(256) k_copy_operands(CopyOperandsArgs g)
+{
+   const int b = blockIdx.x - g.blocks_a;
+   if (b < 0 || !g.kn) {
+      const bool is_a = b < 0;
+      const unsigned char *src = is_a ? g.A : g.B;
+      unsigned char *dst = is_a ? g.Ap : g.Bp;
+      const int rows = is_a ? g.M : g.N, ld = is_a ? g.lda : g.ldb;
+      const size_t chunks = (size_t)rows * (g.Kp >> 4);
+      const size_t c = (size_t)(is_a ? blockIdx.x : b) * 256 + threadIdx.x;
+      if (c >= chunks) return;
+      const int cpr = g.Kp >> 4;
+      const size_t r = c / cpr;
+      const int k = (int)(c - r * cpr) * 16;
+      const unsigned char *row = src + r * ld;
+      RowChunk q;
+      load_row_chunk<true>(q, row, k, g.K);
+      *reinterpret_cast<v4i *>(dst + c * 16) = trim_row_chunk(row_chunk<true>(q, row, k, g.K), k, g.K);
+      return;
+   }
+   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+   const int rg = (b % g.groups_k) * 8 + (lane & 7);                        // group of 16 rows of B (bytes of K)
+   const int cg = ((b / g.groups_k) * 4 + wave) * 8 + (lane >> 3);          // group of 4 columns
+   if (rg * 16 >= g.Kp || cg * 4 >= g.N) return;
+   unsigned o[4][4];
+#pragma unroll
+   for (int q = 0; q < 4; ++q) {
+      unsigned d[4], t[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+         const int k = rg * 16 + 4 * q + e;
+         const unsigned char *p = g.B + (size_t)(k < g.K ? k : 0) * g.ldb;
+         unsigned v = 0;
+         if (g.N >= 4) {
+            const int first = cg * 4 < g.N - 4 ? cg * 4 : g.N - 4;
+            __builtin_memcpy(&v, p + first, 4);
+            v >>= (cg * 4 - first) * 8;
+         } else {
+            for (int i = 0; i < g.N; ++i) v |= (unsigned)p[i] << (8 * i);
+         }
+         d[e] = k < g.K ? v : 0u;
+      }
+      transpose_4x4_bytes(d[0], d[1], d[2], d[3], t);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j][q] = t[j];
+   }
+#pragma unroll
+   for (int j = 0; j < 4; ++j)
+      if (cg * 4 + j < g.N)
+         *reinterpret_cast<v4i *>(g.Bp + (size_t)(cg * 4 + j) * g.Kp + rg * 16) = v4i{(int)o[j][0], (int)o[j][1], (int)o[j][2], (int)o[j][3]};
+}
+
+// Any shape, any alignment: one thread per output element. For products whose rows are shorter than the 16 bytes (or,
+// with B [K,N], the 4 columns) the tiled kernel loads at a time, an empty sum included.
 template <bool IS_INT, int OUT>
 __global__ void k_gemm_bytes_simple(GemmArgs g, int transB)
 {
@@ -950,60 +1120,6 @@ __global__ void k_gemm_bytes_simple(GemmArgs g, int transB)
    if constexpr (ESZ == 1) *out = (unsigned char)((int)fminf(__uint_as_float(r), 255.0f) - 128);
    else if constexpr (ESZ == 2) *reinterpret_cast<unsigned short *>(out) = (unsigned short)r;
    else *reinterpret_cast<unsigned *>(out) = r;
-}
-
-// int8 product with at most 16 output columns (the last layer of a classifier): B^T [N,K] is tiny and
-// stays in cache, the work is streaming A. 16 lanes share a row of A, each takes every 16th 16-byte
-// chunk of K and multiplies it into all N columns with v_dot4_i32_i8; the 16 partial sums of a column
-// are added with four butterfly steps inside the 16-lane group. Four rows per wavefront.
-template <int OUT, int NMAX>
-__global__ void __launch_bounds__(256) k_qgemm_skinny(GemmArgs g)
-{
-   const int lane16 = threadIdx.x & 15;
-   const int row = (int)(((size_t)blockIdx.x * 256 + threadIdx.x) >> 4);
-   const int m = row < g.M ? row : g.M - 1;
-   const uint8_t *a = g.A + (size_t)m * g.lda;
-   int acc[NMAX];
-#pragma unroll
-   for (int n = 0; n < NMAX; ++n) acc[n] = 0;
-   const int chunks = g.K >> 4;
-   for (int c = lane16; c < chunks; c += 16) {
-      const v4i av = *reinterpret_cast<const v4i *>(a + c * 16);
-#pragma unroll
-      for (int n = 0; n < NMAX; ++n) {
-         if (n < g.N) {
-            const v4i bv = *reinterpret_cast<const v4i *>(g.B + (size_t)n * g.ldb + c * 16);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[n] = __builtin_amdgcn_sdot4(av[e], bv[e], acc[n], false);
-         }
-      }
-   }
-#pragma unroll
-   for (int n = 0; n < NMAX; ++n) {
-#pragma unroll
-      for (int d = 1; d < 16; d <<= 1) acc[n] += __shfl_xor(acc[n], d, 16);
-   }
-   if (row >= g.M) return;
-   constexpr int ESZ = OutSize<OUT>::value;
-#pragma unroll
-   for (int n = 0; n < NMAX; ++n) {
-      if (n == lane16 && n < g.N) {
-         const unsigned r = epilogue_value<true, OUT>(g, g.scale ? g.scale[n] : 0.0f,
-                                                      g.bias ? static_cast<const int *>(g.bias)[n] : 0, acc[n], 0.0f);
-         unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)m * g.ldy + n) * ESZ;
-         if constexpr (ESZ == 1) *out = (unsigned char)((int)fminf(__uint_as_float(r), 255.0f) - 128);
-         else *reinterpret_cast<unsigned *>(out) = r;
-      }
-   }
-}
-
-template <int OUT>
-int launch_skinny(sofie_hip_ctx *ctx, GemmArgs &g)
-{
-   const dim3 grid((unsigned)(((size_t)g.M * 16 + 255) / 256)), block(256);
-   if (g.N <= 8) hipLaunchKernelGGL((k_qgemm_skinny<OUT, 8>), grid, block, 0, ctx->stream, g);
-   else hipLaunchKernelGGL((k_qgemm_skinny<OUT, 16>), grid, block, 0, ctx->stream, g);
-   return check_launch(ctx, "k_qgemm_skinny");
 }
 
 template <class Mma, int OUT> struct IS_SPLITTABLE {
@@ -1131,7 +1247,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish_pair(GemmArgs g1, const i
    }
 }
 
-template <class Mma, int BK, int NSETS, int TI, int TJ, int OUT, bool B_KN, bool FULL>
+template <class Mma, int BK, int NSETS, int TI, int TJ, int OUT, bool B_KN, TileMode MODE>
 int launch_tiled_impl(sofie_hip_ctx *ctx, GemmArgs &g)
 {
    constexpr int BN = 2 * TI * 32, BM = 2 * TJ * 32;
@@ -1142,7 +1258,7 @@ int launch_tiled_impl(sofie_hip_ctx *ctx, GemmArgs &g)
    static_assert(lds <= 160 * 1024, "tile does not fit the 160 KB LDS");
    g.tiles_m = cdiv(g.M, BM);
    g.tiles_n = cdiv(g.N, BN);
-   constexpr auto kern = k_gemm_bytes<Mma, BK, NSETS, TI, TJ, OUT, B_KN, FULL>;
+   constexpr auto kern = k_gemm_bytes<Mma, BK, NSETS, TI, TJ, OUT, B_KN, MODE>;
    SOFIE_LARGE_LDS(kern);
    const int splits = (IS_SPLITTABLE<Mma, OUT>::value && g.splits > 1) ? g.splits : 1;
    hipLaunchKernelGGL(kern, dim3(g.tiles_m * g.tiles_n * splits), dim3(256), lds, ctx->stream, g);
@@ -1154,8 +1270,8 @@ int launch_tiled(sofie_hip_ctx *ctx, GemmArgs &g)
 {
    constexpr int BN = 2 * TI * 32, BM = 2 * TJ * 32;
    if (g.M % BM == 0 && g.N % BN == 0 && g.K % BK == 0)
-      return launch_tiled_impl<Mma, BK, NSETS, TI, TJ, OUT, B_KN, true>(ctx, g);
-   return launch_tiled_impl<Mma, BK, NSETS, TI, TJ, OUT, B_KN, false>(ctx, g);
+      return launch_tiled_impl<Mma, BK, NSETS, TI, TJ, OUT, B_KN, WHOLE_TILES>(ctx, g);
+   return launch_tiled_impl<Mma, BK, NSETS, TI, TJ, OUT, B_KN, CHUNK_ROWS>(ctx, g);
 }
 
 template <class Mma, int BK, int NST, int OUT, bool B_KN = false>
@@ -1192,20 +1308,19 @@ int launch_dma(sofie_hip_ctx *ctx, GemmArgs &g)
    return check_launch(ctx, "k_gemm_dma");
 }
 
-// Few rows of A (M <= 32: a quantised layer on a small batch) with B [N][K]: the product is a pass over B, bound by
-// memory, and 64 x 64 tiles would give a handful of compute units all the work. A wavefront owns all rows of A (MT
-// tiles of 16 rows, v_mfma_i32_16x16x64_i8) and 64 columns; B goes from global memory straight into the matrix
+// Few rows of A (M <= 16: a quantised layer on a small batch) with B [N][K]: the product is a pass over B, bound by
+// memory, and 64 x 64 tiles would give a handful of compute units all the work. A wavefront owns all rows of A
+// (v_mfma_i32_16x16x64_i8) and 64 columns; B goes from global memory straight into the matrix
 // instruction's operand registers: lane (j = lane % 16, kq = lane / 16) loads bytes k0 + 16 kq .. + 15 of column 16 q + j,
 // which is its part of the operand of tile q as it stands, and the same bytes of its row of A. The grid is column
 // blocks x slices of K; a wavefront takes a quarter of the slice in chunks of 64 k (consecutive chunks: the two halves
 // of a 128-byte line are fetched one behind the other), three chunks of loads in flight while one is multiplied; the
 // four wavefronts' sums meet in LDS and go to the scratch buffer [slice][M][ldp] that k_splitk_finish adds up and
 // converts (integer sums: the result is that of the unsplit kernels bit for bit).
-template <int MT>
 __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial, int ldp, int kslice)
 {
    constexpr unsigned OUTSIDE = 0x80000000u;
-   __shared__ int red[2 * MT * 4 * 4 * 64];
+   __shared__ int red[2 * 4 * 4 * 64];
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int j = lane & 15, kq = lane >> 4;
    const int c0 = blockIdx.x * 64;
@@ -1216,28 +1331,23 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
       const_cast<uint8_t *>(g.A), 0, (int)((size_t)(g.M - 1) * g.lda + g.K), 0x00020000);
    const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t *>(g.B), 0, (int)((size_t)(g.N - 1) * g.ldb + g.K), 0x00020000);
-   unsigned a_off[MT], b_off[4];
-#pragma unroll
-   for (int t = 0; t < MT; ++t) a_off[t] = t * 16 + j < g.M ? (unsigned)((t * 16 + j) * g.lda + 16 * kq) : OUTSIDE;
+   const unsigned a_off = j < g.M ? (unsigned)(j * g.lda + 16 * kq) : OUTSIDE;
+   unsigned b_off[4];
 #pragma unroll
    for (int q = 0; q < 4; ++q) b_off[q] = c0 + 16 * q + j < g.N ? (unsigned)((c0 + 16 * q + j) * g.ldb + 16 * kq) : OUTSIDE;
    struct Chunk {
-      v4i a[MT], b[4];
+      v4i a, b[4];
    };
    auto load = [&](Chunk &c, int k0) {
       const bool in = k0 + 16 * kq < k_end;     // K and the wavefronts' shares are multiples of 16: a lane's bytes are in or out together
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-         c.a[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, in ? a_off[t] : OUTSIDE, k0, 0));
+      c.a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, in ? a_off : OUTSIDE, k0, 0));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
          c.b[q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(brs, in ? b_off[q] : OUTSIDE, k0, 0));
    };
-   v4i acc[MT][4];
+   v4i acc[4];
 #pragma unroll
-   for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[t][q] = v4i{0, 0, 0, 0};
+   for (int q = 0; q < 4; ++q) acc[q] = v4i{0, 0, 0, 0};
    Chunk c0_, c1_, c2_, c3_;
    int k0 = k_begin;
    load(c0_, k0);
@@ -1246,9 +1356,7 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    for (; k0 < k_end; k0 += 64) {
       load(c3_, k0 + 192);
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-         for (int t = 0; t < MT; ++t) acc[t][q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(c0_.a[t], c0_.b[q], acc[t][q], 0, 0, 0);
+      for (int q = 0; q < 4; ++q) acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(c0_.a, c0_.b[q], acc[q], 0, 0, 0);
       c0_ = c1_;
       c1_ = c2_;
       c2_ = c3_;
@@ -1256,21 +1364,17 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    // wavefronts 2 and 3 hand their sums to 0 and 1, then 1 hands its to 0
    auto put = [&](int *dst) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-         for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dst[((t * 4 + q) * 4 + r) * 64 + lane] = acc[t][q][r];
+         for (int r = 0; r < 4; ++r) dst[(q * 4 + r) * 64 + lane] = acc[q][r];
    };
    auto add = [&](const int *src) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-         for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][q][r] += src[((t * 4 + q) * 4 + r) * 64 + lane];
+         for (int r = 0; r < 4; ++r) acc[q][r] += src[(q * 4 + r) * 64 + lane];
    };
-   constexpr int BLOCK = MT * 4 * 4 * 64;
+   constexpr int BLOCK = 4 * 4 * 64;
    if (wave >= 2) put(red + (wave - 2) * BLOCK);
    __syncthreads();
    if (wave < 2) add(red + wave * BLOCK);
@@ -1279,20 +1383,18 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    __syncthreads();
    if (wave != 0) return;
    add(red);
-   // tile (t, q), register r: row t * 16 + kq * 4 + r, column c0 + 16 q + j
+   // tile q, register r: row kq * 4 + r, column c0 + 16 q + j
    int *const out = partial + (size_t)blockIdx.y * g.M * ldp;
 #pragma unroll
-   for (int t = 0; t < MT; ++t)
+   for (int r = 0; r < 4; ++r) {
+      const int m = kq * 4 + r;
+      if (m >= g.M) continue;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-         const int m = t * 16 + kq * 4 + r;
-         if (m >= g.M) continue;
-#pragma unroll
-         for (int q = 0; q < 4; ++q) {
-            const int n = c0 + 16 * q + j;
-            if (n < ldp) out[(size_t)m * ldp + n] = acc[t][q][r];
-         }
+      for (int q = 0; q < 4; ++q) {
+         const int n = c0 + 16 * q + j;
+         if (n < ldp) out[(size_t)m * ldp + n] = acc[q][r];
       }
+   }
 }
 
 // The same pass over B for at most 16 rows of A and enough columns to give every compute unit a workgroup without
@@ -1358,31 +1460,278 @@ __global__ void __launch_bounds__(512) k_qgemm_few_rows_whole(GemmArgs g, int kp
    }
 }
 
+struct Mma16I8 {
+   typedef v4i Acc;
+   static __device__ __forceinline__ Acc mma(v4i a0, v4i a1, v4i b0, v4i b1, Acc c)
+   {
+      c = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, c, 0, 0, 0);
+      return __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, c, 0, 0, 0);
+   }
+};
+struct Mma16F8 {
+   typedef v4f Acc;
+   static __device__ __forceinline__ Acc mma(v4i a0, v4i a1, v4i b0, v4i b1, Acc c)
+   {
+      const v8i a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]}, b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+      return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+   }
+};
+
+template <class Mma> struct SelectMma16 { typedef Mma16I8 type; };
+template <> struct SelectMma16<MmaF8> { typedef Mma16F8 type; };
+
+// Small products, A [M,K] and B^T [N,K] in rows that may start at any byte: a workgroup owns 16 MI rows x 16 NJ columns
+// and all of K. Its eight wavefronts take the chunks of 128 bytes of K in turn, with DEPTH chunks of loads in flight each,
+// straight from global memory into the operand registers: lane (row % 16, kq) loads the 32 bytes kq of its rows' chunks
+// (the order of K inside a chunk is the same for A and B and does not matter), no LDS and no barrier on the way. The
+// wavefronts' sums meet in LDS and every four of them leave as one store. A product this small is latency: one trip to
+// memory for everything, where the tiled kernel makes one per K-step (256 x 1000 x 1000: 5.4 us against 12.2 on 128 x 128
+// tiles, 6.2 on 64 x 64; 8 x 1001 x 1001: 5.3 / 11.5 / 6.7; 4096 x 16 x 12800: 14 / 70 / 38; all read at up to 43 bytes
+// per ns and compute unit, which is what a larger product pays for its smaller tiles).
+// Two workgroups per compute unit (128 registers) but for 32 x 32 tiles, whose operands would not fit them.
+template <class Mma, int OUT, int MI, int NJ, bool SHIFTS>
+__global__ void __launch_bounds__(512, MI * NJ == 4 ? 1 : 4) k_gemm_bytes_direct(GemmArgs g)
+{
+   constexpr bool IS_INT = __is_same(typename Mma::Acc, v4i);
+   constexpr int ESZ = OutSize<OUT>::value;
+   constexpr int DEPTH = MI * NJ == 2 ? 2 : 3;
+   constexpr int V = MI * NJ * 64;                     // quads of output columns of the tile
+   __shared__ __align__(16) typename Mma::Acc red[8][V];
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int r16 = lane & 15, kq = lane >> 4;
+   int tm, tn;
+   tile_of_workgroup(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
+   const int m0 = tm * 16 * MI, n0 = tn * 16 * NJ;
+   // the outputs this thread will finish: row om, columns on .. on + 3
+   const int om = m0 + (tid / (64 * NJ)) * 16 + (tid & 15), on = n0 + (tid / 64 % NJ) * 16 + ((tid >> 4) & 3) * 4;
+   float sc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+   int bi[4] = {0, 0, 0, 0};
+   if (tid < V) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+         if (on + e >= g.N) continue;
+         if (g.scale) sc[e] = g.scale[on + e];
+         if (g.bias) bi[e] = static_cast<const int *>(g.bias)[on + e];
+      }
+   }
+   const unsigned char *pa[MI], *pb[NJ];
+#pragma unroll
+   for (int i = 0; i < MI; ++i) {
+      const int m = m0 + i * 16 + r16;
+      pa[i] = g.A + (size_t)(m < g.M ? m : g.M - 1) * g.lda;
+   }
+#pragma unroll
+   for (int j = 0; j < NJ; ++j) {
+      const int n = n0 + j * 16 + r16;
+      pb[j] = g.B + (size_t)(n < g.N ? n : g.N - 1) * g.ldb;
+   }
+   struct Chunk {
+      RowChunk a[MI][2], b[NJ][2];
+   };
+   auto load = [&](Chunk &c, int k0) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+         const int k = k0 + kq * 32 + h * 16;
+#pragma unroll
+         for (int i = 0; i < MI; ++i) load_row_chunk<SHIFTS>(c.a[i][h], pa[i], k, g.K);
+#pragma unroll
+         for (int j = 0; j < NJ; ++j) load_row_chunk<SHIFTS>(c.b[j][h], pb[j], k, g.K);
+      }
+   };
+   typename Mma::Acc acc[MI][NJ];
+#pragma unroll
+   for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+         for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
+   auto multiply = [&](const Chunk &c, int k0) {
+      v4i a[MI][2], b[NJ][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+         const int k = k0 + kq * 32 + h * 16;
+#pragma unroll
+         for (int i = 0; i < MI; ++i) a[i][h] = row_chunk<SHIFTS>(c.a[i][h], pa[i], k, g.K);
+#pragma unroll
+         for (int j = 0; j < NJ; ++j) b[j][h] = row_chunk<SHIFTS>(c.b[j][h], pb[j], k, g.K);
+      }
+      if (k0 + 128 > g.K) {      // uniform: the last chunk
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            const int k = k0 + kq * 32 + h * 16;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) a[i][h] = trim_row_chunk(a[i][h], k, g.K);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) b[j][h] = trim_row_chunk(b[j][h], k, g.K);
+         }
+      }
+      // rows of the result are columns n (the B^T operand first): a lane ends up with four consecutive n of one m
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+         for (int j = 0; j < NJ; ++j) acc[i][j] = Mma::mma(b[j][0], b[j][1], a[i][0], a[i][1], acc[i][j]);
+   };
+   constexpr int STEP = 8 * 128;
+   Chunk c[DEPTH];
+   int k0 = wave * 128;
+#pragma unroll
+   for (int d = 0; d < DEPTH; ++d) load(c[d], k0 + d * STEP);
+   while (k0 < g.K) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+         if (k0 < g.K) multiply(c[d], k0);
+         if (k0 + DEPTH * STEP < g.K) load(c[d], k0 + DEPTH * STEP);
+         k0 += STEP;
+      }
+   }
+#pragma unroll
+   for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) red[wave][(i * NJ + j) * 64 + lane] = acc[i][j];
+   __syncthreads();
+   if (tid >= V || om >= g.M || on >= g.N) return;
+   typename Mma::Acc s = red[0][tid];
+#pragma unroll
+   for (int w = 1; w < 8; ++w)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += red[w][tid][e];
+   unsigned v[4];
+#pragma unroll
+   for (int e = 0; e < 4; ++e) {
+      if constexpr (IS_INT) v[e] = epilogue_value<true, OUT>(g, sc[e], bi[e], s[e], 0.0f);
+      else v[e] = epilogue_value<false, OUT>(g, 0.0f, bi[e], 0, s[e]);
+      if constexpr (ESZ == 1) v[e] = (unsigned)((int)fminf(__uint_as_float(v[e]), 255.0f) - 128) & 0xffu;
+   }
+   unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)om * g.ldy + on) * ESZ;
+   if (on + 4 <= g.N) {
+      if constexpr (ESZ == 1) {
+         const unsigned p = v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24);
+         __builtin_memcpy(out, &p, 4);
+      } else if constexpr (ESZ == 2) {
+         const v2i p = {(int)(v[0] | (v[1] << 16)), (int)(v[2] | (v[3] << 16))};
+         __builtin_memcpy(out, &p, 8);
+      } else {
+         const v4i p = {(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+         __builtin_memcpy(out, &p, 16);
+      }
+   } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+         if (on + e >= g.N) break;
+         if constexpr (ESZ == 1) out[e] = (unsigned char)v[e];
+         else if constexpr (ESZ == 2) reinterpret_cast<unsigned short *>(out)[e] = (unsigned short)v[e];
+         else reinterpret_cast<unsigned *>(out)[e] = v[e];
+      }
+   }
+}
+
+template <class Mma, int OUT, int MI, int NJ>
+int launch_direct_as(sofie_hip_ctx *ctx, GemmArgs &g, TileMode mode)
+{
+   typedef typename SelectMma16<Mma>::type Mma16;
+   g.tiles_m = cdiv(g.M, 16 * MI);
+   g.tiles_n = cdiv(g.N, 16 * NJ);
+   const dim3 grid(g.tiles_m * g.tiles_n);
+   if (mode == ANY_ROWS) hipLaunchKernelGGL((k_gemm_bytes_direct<Mma16, OUT, MI, NJ, true>), grid, dim3(512), 0, ctx->stream, g);
+   else hipLaunchKernelGGL((k_gemm_bytes_direct<Mma16, OUT, MI, NJ, false>), grid, dim3(512), 0, ctx->stream, g);
+   return check_launch(ctx, "k_gemm_bytes_direct");
+}
+
+// What the kernels may assume about rows of A and of B [N,K] (see TileMode).
+TileMode row_mode(const GemmArgs &g)
+{
+   const uintptr_t bits = reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.B) | (unsigned)g.lda | (unsigned)g.ldb | (unsigned)g.K;
+   return (bits & 15u) == 0 ? CHUNK_ROWS : (bits & 3u) == 0 ? DWORD_ROWS : ANY_ROWS;
+}
+
+// The kernel for a product of fewer than 128 tiles of 256 x 256, B [N,K], by an estimate of its time behind the launch.
+//   direct   a round of resident workgroups costs 1 us to start and meet, and a compute unit takes in 43 bytes per ns
+//            (28 where the chunks have to be put together from dwords)
+//   tiles    0.54 us per K-step of 128 bytes for 128 x 128 tiles, half of that for 64 x 64, 1.3 and 1.6 times as much where
+//            rows are no whole chunks or no whole dwords; 2.5 / 0.8 us for the epilogue; a compute unit takes its tiles in turn
+// Fitted to the times of every kernel on 35 sizes from 1 x 1024 x 1024 to 1166 x 2937 x 2491 and 8001 x 101 x 513 (4.5 to 40 us).
+struct SmallChoice {
+   int tile;          // 64 or 128: k_gemm_bytes on tiles of that size; 0: k_gemm_bytes_direct
+   int mi, nj;
+   float us;
+};
+SmallChoice small_choice(const sofie_hip_ctx *ctx, const GemmArgs &g, TileMode mode)
+{
+   const int cus = ctx->num_cus;
+   SmallChoice best = {0, 0, 0, 1e30f};
+   auto consider = [&](int tile, int mi, int nj, float us) {
+      if (us < best.us) best = {tile, mi, nj, us};
+   };
+   const float rate = mode == ANY_ROWS ? 28e3f : 43e3f;
+   for (int i = 0; i < 4; ++i) {
+      const int mi = 1 + (i >> 1), nj = 1 + (i & 1);
+      const long long wgs = (long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj), per_cu = (wgs + cus - 1) / cus;
+      const int resident = mi * nj == 4 ? 1 : 2;
+      consider(0, mi, nj, (float)((per_cu + resident - 1) / resident) + (float)per_cu * 16 * (mi + nj) * g.K / rate);
+   }
+   const float slower = mode == ANY_ROWS ? 1.6f : mode == DWORD_ROWS ? 1.3f : 1.0f;
+   for (int tile = 64; tile <= 128; tile *= 2) {
+      const long long wgs = (long long)cdiv(g.M, tile) * cdiv(g.N, tile), per_cu = (wgs + cus - 1) / cus;
+      const float step = slower * (tile == 64 ? 0.27f : 0.54f), epilogue = tile == 64 ? 0.8f : 2.5f;
+      consider(tile, 0, 0, (float)per_cu * (cdiv(g.K, 128) * step + epilogue));
+   }
+   return best;
+}
+
+// Scratch memory of a call behind the operand copies it may already hold there (g.scratch_used bytes, reserved together
+// with this by copy_operands, so that the buffer does not move under the copies).
+int call_scratch(sofie_hip_ctx *ctx, const GemmArgs &g, size_t bytes, void **ptr)
+{
+   if (int rc = workspace(ctx, g.scratch_used + bytes, ptr)) return rc;
+   *ptr = static_cast<unsigned char *>(*ptr) + g.scratch_used;
+   return SOFIE_HIP_OK;
+}
+
+// At most 16 rows on a B of some size, in one launch with K cut inside the workgroups only: enough columns for a
+// workgroup of 16 columns on at least every second compute unit, and a K of which everything is requested at once (at
+// 8 x 8192 x 8192 k_gemm_bytes_direct is ahead, 12.7 against 14.5 us; up to K = 4096 the two are equal: 16 x 4096 x 4096 5.9 / 6.1).
+bool few_rows_whole(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   return g.M <= 16 && cdiv(g.N, 16) * 2 >= ctx->num_cus && g.K >= 512 && g.K <= 4096 && (size_t)g.N * g.K >= ((size_t)2 << 20) &&
+          (size_t)g.N * g.ldb + g.K < (1u << 31);
+}
+// ... or with K in slices, for fewer columns and a long K: 4 x 64 x 65536 16.7 against 41.5 us in one launch
+// (k_gemm_bytes_direct), 16 x 1024 x 32768 18.3 / 29.9, 8 x 256 x 16384 10.0 / 13.3, 8 x 1024 x 8192 8.5 / 7.9. The second
+// launch costs what it gains at a B of 8 MB; of smaller ones those from 3 MB keep it (8 x 1536 x 2048: 7.7 / 4.7).
+bool few_rows_sliced(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   return g.M <= 16 && g.N >= 64 && cdiv(g.N, 16) * 2 < ctx->num_cus && g.K >= 512 && (size_t)g.N * g.K >= ((size_t)3 << 20) &&
+          (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);
+}
+
 // Slices of K so that about eight workgroups per compute unit exist, every wavefront with at least two chunks, and the
 // partial sums a fraction of B's bytes.
+int few_rows_splits(const sofie_hip_ctx *ctx, const GemmArgs &g, int *kslice)
+{
+   int splits = 8 * ctx->num_cus / cdiv(g.N, 64);
+   if (splits > g.K / 512) splits = g.K / 512;
+   if (splits > g.K / (16 * g.M)) splits = g.K / (16 * g.M);
+   if (splits < 1) splits = 1;
+   *kslice = cdiv(cdiv(g.K, splits), 256) * 256;
+   return cdiv(g.K, *kslice);
+}
+
 template <int OUT>
 int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g)
 {
-   // enough columns for a workgroup of 16 columns on at least every second compute unit: one launch, K cut inside the
-   // workgroups only (8 x 4096 x 4096: 5.7 against 9.3 us for the call; the second launch was a third of it)
-   if (g.M <= 16 && cdiv(g.N, 16) * 2 >= ctx->num_cus) {
+   if (few_rows_whole(ctx, g)) {
       const int kper = cdiv(cdiv(g.K, 8), 64) * 64;
       hipLaunchKernelGGL((k_qgemm_few_rows_whole<OUT>), dim3(cdiv(g.N, 16)), dim3(512), 0, ctx->stream, g, kper);
       return check_launch(ctx, "k_qgemm_few_rows_whole");
    }
    const int blocks = cdiv(g.N, 64);
-   int splits = 8 * ctx->num_cus / blocks;
-   if (splits > g.K / 512) splits = g.K / 512;
-   if (splits > g.K / (16 * g.M)) splits = g.K / (16 * g.M);
-   if (splits < 1) splits = 1;
-   const int kslice = cdiv(cdiv(g.K, splits), 256) * 256;
-   splits = cdiv(g.K, kslice);
+   int kslice = 0;
+   const int splits = few_rows_splits(ctx, g, &kslice);
    const int ldp = cdiv(g.N, 4) * 4;
    void *part = nullptr;
-   if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
+   if (int rc = call_scratch(ctx, g, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
    const dim3 grid(blocks, splits);
-   if (g.M <= 16) hipLaunchKernelGGL(k_qgemm_few_rows<1>, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
-   else hipLaunchKernelGGL(k_qgemm_few_rows<2>, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
+   hipLaunchKernelGGL(k_qgemm_few_rows, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
    if (int rc = check_launch(ctx, "k_qgemm_few_rows")) return rc;
    const size_t threads = (size_t)g.M * (ldp / 4);
    hipLaunchKernelGGL((k_splitk_finish<OUT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, g,
@@ -1398,7 +1747,7 @@ int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, int splits, int kslice, cons
 {
    const int ldp = cdiv(g.N, 4) * 4;
    void *part = nullptr;
-   if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
+   if (int rc = call_scratch(ctx, g, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
    GemmArgs p = g;
    p.Y = part;
    p.ldy = ldp;
@@ -1457,7 +1806,125 @@ bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, int &splits, int 
    if (splits > 16) splits = 16;
    kslice = cdiv(cdiv(g.K, splits), 128) * 128;
    splits = cdiv(g.K, kslice);
-   return splits > 1;
+   if (splits < 2) return false;
+   // against one launch of the small-product kernels: 4 us for the second launch and the epilogues, the steps of a slice,
+   // and the partial sums written and read at 8 TB/s (300 x 130 x 8464: 14.7 us in slices, 7.5 in one launch; 256 x 256 x 12800:
+   // 12.5 / 13.2; 128 x 128 x 32768: 15.4 / 29.4; 4096 x 256 x 12800: 23.7 / 32.5)
+   const float us = 4.0f + 0.54f * (kslice / 128) + 8.0f * splits * (float)g.M * g.N / 8e6f;
+   return us < small_choice(ctx, g, CHUNK_ROWS).us;
+}
+
+bool big_product(const GemmArgs &g) { return (size_t)g.M * g.N >= (size_t)256 * 256 * 128 && g.M >= 256 && g.N >= 256; }
+// Scratch bytes dispatch_nk needs for the partial sums of this product.
+template <class Mma>
+size_t nk_scratch_bytes(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   if constexpr (__is_same(typename Mma::Acc, v16i)) {
+      const size_t sums = (size_t)g.M * (cdiv(g.N, 4) * 4) * sizeof(int);
+      int splits = 1, kslice = 0;
+      if (few_rows_whole(ctx, g)) return 0;
+      if (few_rows_sliced(ctx, g)) return few_rows_splits(ctx, g, &kslice) * sums;
+      if (!big_product(g) && split_k_plan(ctx, g, splits, kslice)) return splits * sums;
+   }
+   return 0;
+}
+
+// Products of fewer than 128 tiles of 256 x 256, A [M,K] and B^T [N,K] with K >= 16 in rows that may start anywhere.
+template <class Mma, int OUT>
+int launch_small(sofie_hip_ctx *ctx, GemmArgs &g)
+{
+   constexpr int BK = 128;
+   constexpr int NSETS = __is_same(typename Mma::Acc, v16i) ? 2 : 1;
+   const TileMode mode = row_mode(g);
+   const SmallChoice c = small_choice(ctx, g, mode);
+   if (c.tile == 0) {
+      if (c.mi == 1) return c.nj == 1 ? launch_direct_as<Mma, OUT, 1, 1>(ctx, g, mode) : launch_direct_as<Mma, OUT, 1, 2>(ctx, g, mode);
+      return c.nj == 1 ? launch_direct_as<Mma, OUT, 2, 1>(ctx, g, mode) : launch_direct_as<Mma, OUT, 2, 2>(ctx, g, mode);
+   }
+   if (mode == CHUNK_ROWS)
+      return c.tile == 64 ? launch_tiled<Mma, BK, NSETS, 1, 1, OUT, false>(ctx, g) : launch_tiled<Mma, BK, NSETS, 2, 2, OUT, false>(ctx, g);
+   if (mode == DWORD_ROWS)
+      return c.tile == 64 ? launch_tiled_impl<Mma, BK, 1, 1, 1, OUT, false, DWORD_ROWS>(ctx, g) : launch_tiled_impl<Mma, BK, 1, 2, 2, OUT, false, DWORD_ROWS>(ctx, g);
+   return c.tile == 64 ? launch_tiled_impl<Mma, BK, 1, 1, 1, OUT, false, ANY_ROWS>(ctx, g) : launch_tiled_impl<Mma, BK, 1, 2, 2, OUT, false, ANY_ROWS>(ctx, g);
+}
+
+// Products on operands with rows of whole, aligned 16-byte chunks along K: A [M,K], B^T [N,K].
+template <class Mma, int OUT>
+int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
+{
+   constexpr bool IS_INT = __is_same(typename Mma::Acc, v16i);
+   // 128 bytes of K per stage; int8 keeps two register sets in flight, fp8 (twice the
+   // fragment registers) one.
+   constexpr int BK = 128;
+   constexpr int NSETS = IS_INT ? 2 : 1;
+   if constexpr (IS_INT && OUT != SOFIE_OUT_BF16) {
+      if (few_rows_whole(ctx, g) || few_rows_sliced(ctx, g)) return launch_few_rows<OUT>(ctx, g);
+   }
+   if (big_product(g)) {
+      // descriptor offsets are 32-bit: a 256-row panel plus K must stay below 2 GiB
+      if ((size_t)256 * g.lda + g.K < (1u << 31) && (size_t)256 * g.ldb + g.K < (1u << 31))
+         return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT>(ctx, g);
+      return launch_tiled<Mma, BK, NSETS, 4, 4, OUT, false>(ctx, g);
+   }
+   if constexpr (IS_INT) {
+      // a long K with few 128 x 128 tiles is cut into slices of K: 128 x 128 tiles write int32 partial sums per slice
+      // (integer sums, so the result does not depend on the cut), a second kernel adds them and converts
+      int splits = 1, kslice = 0;
+      if (split_k_plan(ctx, g, splits, kslice)) return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, splits, kslice);
+   }
+   return launch_small<Mma, OUT>(ctx, g);
+}
+
+// Operands the fast kernels cannot read as they lie (rows that are no whole 16-byte chunks, B [K,N]) copied into rows
+// they can (k_copy_operands); a B promised constant is copied by the first call only. *done stays false where there is no
+// scratch memory for it (while a graph is recorded, inside the no-allocation entry point): the caller then takes a kernel
+// that reads the operands where they are.
+template <class Mma>
+int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool copy_b, bool *done)
+{
+   *done = false;
+   CopyOperandsArgs c{};
+   c.A = g.A; c.B = g.B;
+   c.M = g.M; c.N = g.N; c.K = g.K; c.lda = g.lda; c.ldb = g.ldb;
+   c.Kp = cdiv(g.K, 16) * 16;
+   c.kn = !transB;
+   const size_t a_bytes = copy_a ? (((size_t)g.M * c.Kp + 255) & ~(size_t)255) : 0, b_bytes = copy_b ? (((size_t)g.N * c.Kp + 255) & ~(size_t)255) : 0;
+   GemmArgs h = g;
+   if (copy_a) h.lda = c.Kp;
+   if (copy_b) h.ldb = c.Kp;
+   // with rows of B alone copied the product keeps its K: the zeros behind it would meet whatever follows A's rows
+   const bool padded = copy_a || g.K == c.Kp;
+   if (padded) h.K = c.Kp;
+   const size_t sums = padded ? nk_scratch_bytes<Mma>(ctx, h) : 0;
+   if (a_bytes + b_bytes + sums >= ((size_t)1 << 40) || !workspace_has_room(ctx, a_bytes + b_bytes + sums)) return SOFIE_HIP_OK;
+   void *bp = nullptr;
+   bool fresh = copy_b;
+   if (copy_b) {
+      const int layout[] = {3, g.K, g.N, g.ldb, transB};
+      if (int rc = packed_weights(ctx, g.B, layout_key(layout, 5), b_bytes, &bp, &fresh)) return rc;
+   }
+   const bool b_in_scratch = copy_b && (bp == ctx->workspace || bp == ctx->static_scratch);
+   h.scratch_used = a_bytes + (b_in_scratch ? b_bytes : 0);
+   void *base = nullptr;
+   if (h.scratch_used + sums)
+      if (int rc = workspace(ctx, h.scratch_used + sums, &base)) return rc;
+   c.Ap = static_cast<unsigned char *>(base);
+   c.Bp = b_in_scratch ? static_cast<unsigned char *>(base) + a_bytes : static_cast<unsigned char *>(bp);
+   if (copy_a) h.A = c.Ap;
+   if (copy_b) h.B = c.Bp;
+   const size_t blocks_a = copy_a ? ((size_t)g.M * (c.Kp / 16) + 255) / 256 : 0;
+   size_t blocks_b = 0;
+   c.groups_k = cdiv(c.Kp, 128);
+   if (fresh) blocks_b = c.kn ? (size_t)c.groups_k * cdiv(g.N, 128) : ((size_t)g.N * (c.Kp / 16) + 255) / 256;
+   if (blocks_a + blocks_b >= ((size_t)1 << 31)) return SOFIE_HIP_OK;
+   c.blocks_a = (int)blocks_a;
+   if (blocks_a + blocks_b) {
+      hipLaunchKernelGGL(k_copy_operands, dim3((unsigned)(blocks_a + blocks_b)), dim3(256), 0, ctx->stream, c);
+      if (int rc = check_launch(ctx, "k_copy_operands")) return rc;
+   }
+   g = h;
+   *done = true;
+   return SOFIE_HIP_OK;
 }
 
 template <class Mma, int OUT>
@@ -1465,84 +1932,69 @@ int dispatch(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
 {
    constexpr bool IS_INT = __is_same(typename Mma::Acc, v16i);
    constexpr int ESZ = OutSize<OUT>::value;
-   const bool a_ok = g.K % 16 == 0 && g.lda % 16 == 0 && aligned16(g.A);
-   const bool b_nk_ok = transB && g.ldb % 16 == 0 && aligned16(g.B);
-   const bool b_kn_ok = !transB && g.ldb % 4 == 0 && g.N % 4 == 0 && (reinterpret_cast<uintptr_t>(g.B) & 3u) == 0;
-   g.vec_store = ((size_t)g.ldy * ESZ) % 16 == 0 && aligned16(g.Y);
-   // K = 0 (an empty sum: the outputs are the epilogue of zero) takes the plain kernel, whose K loop runs zero times
-   if (g.K == 0) return launch_simple<IS_INT, OUT>(ctx, g, transB);
-   if constexpr (IS_INT && OUT != SOFIE_OUT_BF16) {
-      if (transB && g.N <= 16 && a_ok && g.ldb % 16 == 0 && aligned16(g.B) && (size_t)g.M * 16 < ((size_t)1 << 40))
-         return launch_skinny<OUT>(ctx, g);
-   }
-   if (!a_ok || !(b_nk_ok || b_kn_ok)) return launch_simple<IS_INT, OUT>(ctx, g, transB);
-   if constexpr (IS_INT && OUT != SOFIE_OUT_BF16) {
-      // a small batch on a layer of 2 MB or more: a pass over B with K in slices (8 x 4096 x 4096: 9.1 against 15.1 us; a
-      // layer of 1 MB is faster on tiles in one launch: 6.0 against 7.2 us)
-      if (transB && g.M <= 32 && g.N >= 64 && g.K >= 512 && (size_t)g.N * g.K >= ((size_t)2 << 20) &&
-          (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31))
-         return launch_few_rows<OUT>(ctx, g);
-   }
-   const bool big = (size_t)g.M * g.N >= (size_t)256 * 256 * 128 && g.M >= 256 && g.N >= 256;
-   // 128 bytes of K per stage; int8 keeps two register sets in flight, fp8 (twice the
-   // fragment registers) one.
    constexpr int BK = 128;
    constexpr int NSETS = IS_INT ? 2 : 1;
-   if (transB) {
-      // descriptor offsets are 32-bit: a 256-row panel plus K must stay below 2 GiB
-      const bool fits = (size_t)256 * g.lda + g.K < (1u << 31) && (size_t)256 * g.ldb + g.K < (1u << 31);
-      if (big && fits) return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT>(ctx, g);
-      if (big) return launch_tiled<Mma, BK, NSETS, 4, 4, OUT, false>(ctx, g);
-      // a long K with few 128 x 128 tiles (a wide fully connected layer on a small batch x width):
-      // 64 x 64 tiles put four times as many workgroups on the device
-      if constexpr (IS_INT) {
-         // ... and a longer one is cut into slices of K: 128 x 128 tiles write int32 partial sums per slice
-         // (integer sums, so the result does not depend on the cut), a second kernel adds them and converts
-         int splits = 1, kslice = 0;
-         if (split_k_plan(ctx, g, splits, kslice)) return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, splits, kslice);
+   const bool a_ok = g.K % 16 == 0 && g.lda % 16 == 0 && aligned16(g.A);
+   const bool b_nk_ok = transB && g.K % 16 == 0 && g.ldb % 16 == 0 && aligned16(g.B);
+   const bool b_kn_ok = !transB && g.K % 16 == 0 && g.ldb % 4 == 0 && g.N % 4 == 0 && (reinterpret_cast<uintptr_t>(g.B) & 3u) == 0;
+   g.vec_store = ((size_t)g.ldy * ESZ) % 16 == 0 && aligned16(g.Y);
+   if (a_ok && b_nk_ok && g.K > 0) return dispatch_nk<Mma, OUT>(ctx, g);
+   const bool big = big_product(g);
+   if (a_ok && b_kn_ok && g.K > 0) {
+      if (big && g.ldb % 16 == 0 && aligned16(g.B) && (size_t)256 * g.lda + g.K < (1u << 31) &&
+          (size_t)(g.K + 128) * g.ldb < (1u << 31)) {
+         // B [K,N] as it lies: rows of k go to LDS and the transposing LDS read builds the operand
+         return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT, true>(ctx, g);
       }
-      if (cdiv(g.M, 128) * cdiv(g.N, 128) * 2 <= ctx->num_cus && g.K >= 1024)
-         return launch_tiled<Mma, BK, NSETS, 1, 1, OUT, false>(ctx, g);
-      return launch_tiled<Mma, BK, NSETS, 2, 2, OUT, false>(ctx, g);
-   }
-   if (big && g.ldb % 16 == 0 && aligned16(g.B) && (size_t)256 * g.lda + g.K < (1u << 31) &&
-       (size_t)(g.K + 128) * g.ldb < (1u << 31)) {
-      // B [K,N] as it lies: rows of k go to LDS and the transposing LDS read builds the operand
-      return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT, true>(ctx, g);
-   }
-   if (big && g.K % 16 == 0 && (size_t)256 * g.lda + g.K < (1u << 31) && (size_t)257 * g.K < (1u << 31)) {
-      // B [K,N] -> B^T [N,K] in the context's scratch buffer, then the K-contiguous kernel.
-      // A caller that reuses B (weights) should transpose once and call with transB = 1.
-      void *bt = nullptr;
-      if (int rc = workspace(ctx, (size_t)g.N * g.K, &bt)) return rc;
-      if (int rc = transpose_bytes(ctx, g.B, static_cast<unsigned char *>(bt), g.K, g.N, g.ldb, g.K)) return rc;
-      g.B = static_cast<const uint8_t *>(bt);
-      g.ldb = g.K;
-      return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT>(ctx, g);
-   }
-   if (big) return launch_tiled<Mma, BK, NSETS, 4, 4, OUT, true>(ctx, g);
-   // Products of fewer tiles: a pass that transposes B in front (N * K bytes, into the context's scratch buffer, or once
-   // per weight tensor when the caller promised constant weights) costs less than the byte transposes in every
-   // workgroup's K loop, from one row of A upwards (2048^3: 20.2 against 23.7 us, 512 x 512 x 4096: 15.9 against 37.1,
-   // 8 x 4096 x 4096: 28.7 against 45.3, 1 x 1024 x 1024: 9.4 against 16.1). A B^T of at most the fixed scratch array's
-   // size, so that the no-allocation entry point takes the same path.
-   if (g.K % 16 == 0 && (size_t)g.N * g.K <= (size_t)SOFIE_HIP_NOALLOC_SCRATCH_BYTES) {
-      void *bt = nullptr;
-      bool fresh = true;
-      const int layout[] = {2, g.K, g.N, g.ldb};
-      if (int rc = packed_weights(ctx, g.B, layout_key(layout, 4), (size_t)g.N * g.K, &bt, &fresh)) return rc;
-      if (fresh)
+      if (big && (size_t)256 * g.lda + g.K < (1u << 31) && (size_t)257 * g.K < (1u << 31)) {
+         // B [K,N] -> B^T [N,K] in the context's scratch buffer, then the K-contiguous kernel.
+         // A caller that reuses B (weights) should transpose once and call with transB = 1.
+         void *bt = nullptr;
+         if (int rc = workspace(ctx, (size_t)g.N * g.K, &bt)) return rc;
          if (int rc = transpose_bytes(ctx, g.B, static_cast<unsigned char *>(bt), g.K, g.N, g.ldb, g.K)) return rc;
-      g.B = static_cast<const uint8_t *>(bt);
-      g.ldb = g.K;
-      // a copy of its own (constant weights): every choice of the [N,K] case is open; a copy in the scratch buffer
-      // leaves the kernels that need no scratch memory themselves
-      if (bt != ctx->workspace && bt != ctx->static_scratch) return dispatch<Mma, OUT>(ctx, g, 1);
-      if (cdiv(g.M, 128) * cdiv(g.N, 128) * 2 <= ctx->num_cus && g.K >= 1024)
-         return launch_tiled<Mma, BK, NSETS, 1, 1, OUT, false>(ctx, g);
-      return launch_tiled<Mma, BK, NSETS, 2, 2, OUT, false>(ctx, g);
+         g.B = static_cast<const uint8_t *>(bt);
+         g.ldb = g.K;
+         return launch_dma<Mma, SOFIE_DMA_BK, SOFIE_DMA_NST, OUT>(ctx, g);
+      }
+      // Products of fewer tiles: a pass that transposes B in front (N * K bytes, into the context's scratch buffer, or once
+      // per weight tensor when the caller promised constant weights) costs less than the byte transposes in every
+      // workgroup's K loop, from one row of A upwards (2048^3: 20.2 against 23.7 us, 512 x 512 x 4096: 15.9 against 37.1,
+      // 8 x 4096 x 4096: 28.7 against 45.3, 1 x 1024 x 1024: 9.4 against 16.1). A B^T of at most the fixed scratch array's
+      // size, so that the no-allocation entry point takes the same path.
+      if (!big && (size_t)g.N * g.K <= (size_t)SOFIE_HIP_NOALLOC_SCRATCH_BYTES) {
+         void *bt = nullptr;
+         bool fresh = true;
+         const int layout[] = {2, g.K, g.N, g.ldb};
+         if (int rc = packed_weights(ctx, g.B, layout_key(layout, 4), (size_t)g.N * g.K, &bt, &fresh)) return rc;
+         if (fresh)
+            if (int rc = transpose_bytes(ctx, g.B, static_cast<unsigned char *>(bt), g.K, g.N, g.ldb, g.K)) return rc;
+         g.B = static_cast<const uint8_t *>(bt);
+         g.ldb = g.K;
+         // a copy of its own (constant weights): every choice of the [N,K] case is open; a copy in the scratch buffer
+         // leaves the kernels that need no scratch memory themselves
+         if (bt != ctx->workspace && bt != ctx->static_scratch) return dispatch_nk<Mma, OUT>(ctx, g);
+         if (cdiv(g.M, 128) * cdiv(g.N, 128) * 2 <= ctx->num_cus) return launch_tiled<Mma, BK, NSETS, 1, 1, OUT, false>(ctx, g);
+         return launch_tiled<Mma, BK, NSETS, 2, 2, OUT, false>(ctx, g);
+      }
    }
-   return launch_tiled<Mma, BK, NSETS, 2, 2, OUT, true>(ctx, g);
+   if (g.K < 16) return launch_simple<IS_INT, OUT>(ctx, g, transB);
+   // Rows that are no whole 16-byte chunks. A large product copies its operands into rows that are, for the kernels with
+   // 256 x 256 tiles (2100 x 4101 x 1001: 22 us with the copy of A, 26 with both, 35 on 128 x 128 tiles that load odd rows;
+   // 8000 x 8001 x 257: 44 / 46 / 77; 1166 x 2937 x 2491, which has too few such tiles: 26 / 31 / 24); a smaller one with
+   // B [K,N] only transposes B.
+   bool done = false;
+   if (big) {
+      if (int rc = copy_operands<Mma>(ctx, g, transB, !a_ok, !b_nk_ok, &done)) return rc;
+      if (done) return dispatch_nk<Mma, OUT>(ctx, g);
+   } else if (!transB) {
+      if (int rc = copy_operands<Mma>(ctx, g, transB, false, true, &done)) return rc;
+      if (done) transB = 1;
+   }
+   if (transB) return launch_small<Mma, OUT>(ctx, g);
+   // B [K,N] and no memory for a copy
+   if (g.N < 4) return launch_simple<IS_INT, OUT>(ctx, g, transB);
+   if (cdiv(g.M, 128) * cdiv(g.N, 128) * 2 <= ctx->num_cus) return launch_tiled_impl<Mma, BK, 1, 1, 1, OUT, true, ANY_ROWS>(ctx, g);
+   return launch_tiled_impl<Mma, BK, 1, 2, 2, OUT, true, ANY_ROWS>(ctx, g);
 }
 
 }  // namespace

@@ -52,6 +52,7 @@ struct GemmArgs {
    // bytes and writes its tile into the slice's own copy of Y, `ysplit` bytes after the previous one
    int splits, kslice;
    long long ysplit;
+   size_t scratch_used;   // bytes at the start of the scratch buffer that hold copies of this call's operands
 };
 
 template <int OUT> struct OutSize { static constexpr int value = 4; };
@@ -202,8 +203,9 @@ __device__ __forceinline__ void tile_epilogue_wave(const GemmArgs &g, typename M
          if (m < g.M && (FULLN || nfirst < g.N)) {
             const v4i v = *reinterpret_cast<const v4i *>(stg + row * SROW + cc * 16);
             unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)m * g.ldy + nfirst) * ESZ;
-            if (FULLN || (g.vec_store && nfirst + 16 / ESZ <= g.N)) {
-               if (write_through) store16_wt(out, v);
+            if (FULLN || nfirst + 16 / ESZ <= g.N) {
+               if (!FULLN && !g.vec_store) __builtin_memcpy(out, &v, 16);      // rows that start anywhere
+               else if (write_through) store16_wt(out, v);
                else *reinterpret_cast<v4i *>(out) = v;
             } else {
                const unsigned char *src = stg + row * SROW + cc * 16;
@@ -414,8 +416,9 @@ __device__ __forceinline__ void tile_epilogue_wave16(const GemmArgs &g, v4i (&ac
          if (m < g.M && nfirst < g.N) {
             const v4i v = *reinterpret_cast<const v4i *>(stg + row * SROW + cc * 16);
             unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)m * g.ldy + nfirst) * ESZ;
-            if (g.vec_store && nfirst + 16 / ESZ <= g.N) {
-               store16_wt(out, v);
+            if (nfirst + 16 / ESZ <= g.N) {
+               if (g.vec_store) store16_wt(out, v);
+               else __builtin_memcpy(out, &v, 16);      // rows that start anywhere
             } else {
                const unsigned char *src = stg + row * SROW + cc * 16;
                const int cnt = (g.N - nfirst) < (16 / ESZ) ? (g.N - nfirst) : (16 / ESZ);

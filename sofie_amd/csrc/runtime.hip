@@ -149,6 +149,12 @@ int packed_weights(sofie_hip_ctx *ctx, const void *w, unsigned long long key, si
    return workspace(ctx, bytes, ptr);
 }
 
+bool workspace_has_room(const sofie_hip_ctx *ctx, size_t bytes)
+{
+   if (ctx->no_alloc) return ctx->static_scratch && bytes <= (size_t)SOFIE_HIP_NOALLOC_SCRATCH_BYTES;
+   return bytes <= ctx->workspace_bytes || (!ctx->capturing && ctx->live_graphs == 0);
+}
+
 int workspace(sofie_hip_ctx *ctx, size_t bytes, void **ptr)
 {
    if (ctx->no_alloc) {   // inside the no-allocation entry point: the fixed array or nothing

@@ -1,0 +1,129 @@
+"""One-byte products on operands of any size and alignment: rows that start at any byte, K that is no multiple of 16, both
+storage orders of B. Covers the kernels of small products (k_gemm_bytes_direct on 16 and 32 rows and columns, k_gemm_bytes
+on 64 x 64 and 128 x 128 tiles, each for rows of whole dwords and of any bytes), the copies that large products make
+(k_copy_operands), and the paths without memory for a copy."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from oracle import oracle
+from sofie_amd import lib as L
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sofie_amd import ops as o
+    return o
+
+
+def rng(seed):
+    return np.random.default_rng(seed)
+
+
+def rows_at(ctx, a, ld, offset):
+    """The matrix on the device with rows `ld` bytes apart, the first `offset` bytes into its buffer (which ends with the
+    last row); returns (buffer, address)."""
+    buf = np.full(offset + (a.shape[0] - 1) * ld + a.shape[1], 0x55, np.uint8)
+    for i, row in enumerate(a.view(np.uint8)):
+        buf[offset + i * ld:offset + i * ld + a.shape[1]] = row
+    t = torch.from_numpy(buf).to(ctx.device)
+    return t, t.data_ptr() + offset
+
+
+# one K below and above a chunk of 16 and a step of 128, K whose last chunk holds one byte, single rows and columns, tiles
+# that end one row or column behind a boundary
+SHAPES = [(1, 4, 16), (1, 5, 17), (3, 1, 31), (16, 16, 127), (17, 33, 129), (33, 47, 50), (2, 300, 1000), (65, 66, 257), (5, 2, 4099),
+          (70, 13, 1041), (256, 1000, 1000), (130, 300, 515), (300, 257, 2049), (700, 650, 397)]
+
+
+@pytest.mark.parametrize("transB", [True, False])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_int8_product_of_any_rows(ops, M, N, K, transB):
+    """Bit-exact against the oracle for the three output kinds; operands at an odd and at a four-byte offset."""
+    r = rng(1000 + M + N + K)
+    A = r.integers(-127, 128, (M, K)).astype(np.int8)
+    B = r.integers(-127, 128, (N, K) if transB else (K, N)).astype(np.int8)
+    scale = (r.uniform(20.0, 60.0, N) / (73.3 * 73.3 * np.sqrt(K))).astype(np.float32)
+    bias = r.integers(-2000, 2000, N).astype(np.int32)
+    acc = oracle.igemm_s8(A, B, transB) + bias[None, :]
+    ctx = ops.default_context()
+    sd, bd = ctx.dev(scale), ctx.dev(bias)
+    for offset, pad in ((0, 0), (3, 2), (4, -K % 4)):
+        (ta, pa), (tb, pb) = rows_at(ctx, A, K + pad, offset), rows_at(ctx, B, B.shape[1] + pad, offset)
+        for out, want in ((L.OUT_S32, acc), (L.OUT_S8, oracle.qgemm_s8(A, B, scale, bias, transB, zpy=3, relu=True)),
+                          (L.OUT_F32, oracle.qgemm_s8_f32out(A, B, scale, bias, transB, relu=True))):
+            y = ctx.empty((M, N), {L.OUT_S32: torch.int32, L.OUT_S8: torch.int8, L.OUT_F32: torch.float32}[out])
+            ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, int(transB), M, N, K, C.c_void_p(pa), K + pad, C.c_void_p(pb), B.shape[1] + pad,
+                                                 ctx.ptr(sd), ctx.ptr(bd), 3, L.ACT_RELU, ctx.ptr(y), N, out))
+            ctx.sync()
+            assert np.array_equal(y.cpu().numpy(), want), (offset, pad, out)
+
+
+@pytest.mark.parametrize("transB", [True, False])
+@pytest.mark.parametrize("M,N,K", [(2100, 4099, 131), (1025, 8200, 48)])
+def test_large_int8_product_copies_ragged_operands(ops, M, N, K, transB):
+    """Products of 128 tiles of 256 x 256 and more: operands copied into whole chunks (A alone where B has them), sampled rows
+    against the oracle; with the constant-weights promise B is copied by the first call only and the results stay."""
+    r = rng(1100 + K)
+    A = r.integers(-127, 128, (M, K)).astype(np.int8)
+    B = r.integers(-127, 128, (N, K) if transB else (K, N)).astype(np.int8)
+    rows = np.concatenate([np.arange(0, 16), r.integers(0, M, 16), np.arange(M - 16, M)])
+    want = oracle.igemm_s8(A[rows], B, transB)
+    for promise in (0, 1):
+        ctx = ops.Context(0)
+        assert ctx.lib.sofie_hip_constant_weights(ctx.h, promise) == 0
+        a, b = ctx.dev(A), ctx.dev(B)
+        for _ in range(2):
+            y = ctx.empty((M, N), torch.int32)
+            ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, int(transB), M, N, K, ctx.ptr(a), K, ctx.ptr(b), B.shape[1], None, None, 0,
+                                                 L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32))
+            ctx.sync()
+            assert np.array_equal(y.cpu().numpy()[rows], want)
+        ctx.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 70, 333), (9, 3, 100)])
+def test_any_rows_without_memory_for_a_copy(ops, M, N, K):
+    """B [K,N] of odd rows in a call that is recorded on a fresh context (no scratch buffer exists and none may be made):
+    a kernel that reads B where it lies runs, and every replay gives the oracle's result."""
+    r = rng(1200 + K)
+    A = r.integers(-127, 128, (M, K)).astype(np.int8)
+    B = r.integers(-127, 128, (K, N)).astype(np.int8)
+    want = oracle.igemm_s8(A, B)
+    ctx = ops.Context(0, stream=torch.cuda.Stream())
+    a, b, y = ctx.dev(A), ctx.dev(B), ctx.empty((M, N), torch.int32)
+    torch.cuda.synchronize()
+    graph = C.c_void_p()
+    ctx.check(ctx.lib.sofie_hip_capture_begin(ctx.h))
+    rc = ctx.lib.sofie_hip_qgemm_s8(ctx.h, 0, M, N, K, ctx.ptr(a), K, ctx.ptr(b), N, None, None, 0, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32)
+    ctx.check(ctx.lib.sofie_hip_capture_end(ctx.h, C.byref(graph)))
+    ctx.check(rc)
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_graph_launch(ctx.h, graph))
+        ctx.sync()
+        assert np.array_equal(y.cpu().numpy(), want)
+    ctx.check(ctx.lib.sofie_hip_graph_destroy(ctx.h, graph))
+    ctx.close()
+
+
+@pytest.mark.parametrize("transB", [True, False])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 16), (17, 33, 129), (33, 47, 50), (256, 500, 1001), (300, 1030, 333), (1, 9, 4001), (2100, 4099, 67)])
+def test_fp8_product_of_any_rows(ops, M, N, K, transB):
+    """Against the float64 product of the same e4m3 operands: |d| <= 7 * 2^-13 * sum|a_k b_k| (what the matrix instruction's sums of
+    eight products may drop), plus 2^-8 |ref| for a bf16 result."""
+    g = torch.Generator(device="cuda").manual_seed(1300 + M + N + K)
+    A = torch.randn(M, K, device="cuda", generator=g).to(torch.float8_e4m3fn)
+    B = torch.randn(*((N, K) if transB else (K, N)), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    bias = torch.randn(N, device="cuda", generator=g)
+    a, b = A.double(), (B.t() if transB else B).double().contiguous()
+    ref, mag = a @ b + bias.double(), a.abs() @ b.abs()
+    for out in (L.OUT_F32, L.OUT_BF16):
+        y = ops.gemm_fp8(A.view(torch.uint8), B.view(torch.uint8), 1.0, 1.0, bias, transB, out)
+        tol = (2.0 ** -8 if out == L.OUT_BF16 else 2.0 ** -23) * ref.abs() + 7 * 2.0 ** -13 * mag
+        assert bool(((y.double() - ref).abs() <= tol).all())
