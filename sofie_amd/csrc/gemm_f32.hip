@@ -1,13 +1,6 @@
-// fp32 GEMM on the matrix cores (v_mfma_f32_32x32x2_f32) with a fused
-// alpha / beta*bias / ReLU epilogue.
-//
-// 256 threads = 4 wavefronts (2x2), each owning TI x TJ tiles of 32x32. Operands are staged
-// in LDS k-major ([k][row]) so that the one-float-per-lane MFMA operand read is a conflict-free
-// ds_read_b32 for either storage order of A and B; the accumulator layout puts 32 consecutive
-// output columns in 32 consecutive lanes, so results are stored straight from registers as
-// 128-byte row segments. Loads are guarded scalar loads: no alignment or size restrictions.
-// Roofline: MFMA fp32 (256 flop/clk/CU); each K-step of 16 issues 8*TI*TJ MFMAs of 64 cycles
-// per wavefront against 16 scalar loads per thread.
+// fp32 GEMM on the matrix cores with a fused alpha / beta*bias / ReLU epilogue: k_gemm_f32_dma (v_mfma_f32_32x32x2_f32) for
+// operands that can be fetched 16 bytes at a time, k_gemm_f32 (v_mfma_f32_16x16x4_f32) for all others, k_gemm_f32_skinny for
+// few rows. Roofline: MFMA fp32 (256 flop/clk/CU).
 #include <cstdint>
 #include <type_traits>
 
@@ -35,134 +28,288 @@ struct GemmF32Args {
    float *partial;
 };
 
-constexpr int BK = 16;
-
-// Stage a [rows x BK] block of a matrix into LDS as dst[k][row].
-// k_major_src: the source is stored [K][rows] (row index contiguous); else [rows][K].
-template <int ROWS, int LD>
-__device__ __forceinline__ void fetch(float (&reg)[ROWS * BK / 256], const float *src, int ld, bool k_major_src,
-                                      int row0, int k0, int nrows, int K, int tid)
+// Workgroup id -> tile, in groups of 4 rows of tiles, so that the workgroups in flight share rows of A and columns of B in an
+// L2. Workgroups are dealt to the 8 XCDs in turn: renumbered so that an XCD (an L2) works on consecutive tiles.
+__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int &tm, int &tn)
 {
-#pragma unroll
-   for (int i = 0; i < ROWS * BK / 256; ++i) {
-      const int e = i * 256 + tid;
-      int r, k;
-      if (k_major_src) { k = e / ROWS; r = e % ROWS; }
-      else { r = e / BK; k = e % BK; }
-      const int gr = row0 + r, gk = k0 + k;
-      float v = 0.0f;
-      if (gr < nrows && gk < K) v = k_major_src ? src[(size_t)gk * ld + gr] : src[(size_t)gr * ld + gk];
-      reg[i] = v;
+   {
+      const int tiles = tiles_m * tiles_n, xcd = pid & 7, base = tiles >> 3, rem = tiles & 7;
+      pid = (pid >> 3) + xcd * base + (xcd < rem ? xcd : rem);
    }
+   const int width = 4 * tiles_n, group = pid / width, first = group * 4;
+   const int gsize = tiles_m - first < 4 ? tiles_m - first : 4;
+   tm = first + (pid % width) % gsize;
+   tn = (pid % width) / gsize;
 }
 
-template <int ROWS, int LD>
-__device__ __forceinline__ void stash(const float (&reg)[ROWS * BK / 256], float *dst, bool k_major_src, int tid)
+// A, B and Y of product `index` of a stack (row-major over the leading dimensions, last dimension fastest).
+__device__ __forceinline__ void select_product(GemmF32Args &g, long long index)
 {
+   long long rem = index, oa = 0, ob = 0;
+   // (constant subscripts: with a run-time one the whole argument block would move to scratch memory)
 #pragma unroll
-   for (int i = 0; i < ROWS * BK / 256; ++i) {
-      const int e = i * 256 + tid;
-      int r, k;
-      if (k_major_src) { k = e / ROWS; r = e % ROWS; }
-      else { r = e / BK; k = e % BK; }
-      dst[k * LD + r] = reg[i];
+   for (int d = SOFIE_GEMM_MAX_LEAD - 1; d >= 0; --d) {
+      if (d >= g.n_lead) continue;
+      const long long pos = rem % g.lead[d];
+      rem /= g.lead[d];
+      oa += pos * g.sa[d];
+      ob += pos * g.sb[d];
    }
+   g.A += oa;
+   g.B += ob;
+   g.Y += index * g.stride_y;
 }
 
-template <int TI, int TJ>
-__global__ void __launch_bounds__(256) k_gemm_f32(GemmF32Args g)
+// alpha * v + beta * bias, ReLU, for columns n .. n + 3 of row m.
+__device__ __forceinline__ v4f finish4(const GemmF32Args &g, v4f v, int m, int n)
 {
-   constexpr int BM = 2 * TI * 32, BN = 2 * TJ * 32;
-   constexpr int LDA = BM + 4, LDB = BN + 4;
-   __shared__ float sA[2][BK * LDA];
-   __shared__ float sB[2][BK * LDB];
-
-   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-   const int wm = wave >> 1, wn = wave & 1;
-   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-   if (g.n_lead > 0) {
-      // this workgroup's product of the stack: its position along every leading dimension, last dimension fastest
-      long long rem = (long long)blockIdx.z + g.z0, oa = 0, ob = 0;
-      const long long index = rem;
-      for (int d = g.n_lead - 1; d >= 0; --d) {
-         const long long pos = rem % g.lead[d];
-         rem /= g.lead[d];
-         oa += pos * g.sa[d];
-         ob += pos * g.sb[d];
-      }
-      g.A += oa;
-      g.B += ob;
-      g.Y += index * g.stride_y;
+#pragma unroll
+   for (int e = 0; e < 4; ++e) {
+      v[e] = __fmul_rn(g.alpha, v[e]);
+      if (n + e >= g.N) continue;
+      if (g.bias_kind == SOFIE_BIAS_ROW) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, g.bias[n + e]));
+      else if (g.bias_kind == SOFIE_BIAS_FULL) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n + e]));
+      else if (g.bias_kind == SOFIE_BIAS_COL) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, g.bias[m]));
+      if (g.relu) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
    }
-
-   float ra[BM * BK / 256], rb[BN * BK / 256];
-   v16f acc[TI][TJ];
-#pragma unroll
-   for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j)
-#pragma unroll
-         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-   const bool a_kmajor = g.transA != 0;   // A stored [K][M]
-   const bool b_kmajor = g.transB == 0;   // B stored [K][N]
-   const int nk = (g.K + BK - 1) / BK;
-
-   fetch<BM, LDA>(ra, g.A, g.lda, a_kmajor, m0, 0, g.M, g.K, tid);
-   fetch<BN, LDB>(rb, g.B, g.ldb, b_kmajor, n0, 0, g.N, g.K, tid);
-   stash<BM, LDA>(ra, sA[0], a_kmajor, tid);
-   stash<BN, LDB>(rb, sB[0], b_kmajor, tid);
-   __syncthreads();
-
-   const int fr = lane & 31, fk = lane >> 5;
-   for (int kt = 0; kt < nk; ++kt) {
-      const int cur = kt & 1;
-      if (kt + 1 < nk) {
-         fetch<BM, LDA>(ra, g.A, g.lda, a_kmajor, m0, (kt + 1) * BK, g.M, g.K, tid);
-         fetch<BN, LDB>(rb, g.B, g.ldb, b_kmajor, n0, (kt + 1) * BK, g.N, g.K, tid);
-      }
-      const float *a = sA[cur] + fk * LDA + wm * TI * 32 + fr;
-      const float *b = sB[cur] + fk * LDB + wn * TJ * 32 + fr;
-#pragma unroll
-      for (int s = 0; s < BK / 2; ++s) {
-         float fa[TI], fb[TJ];
-#pragma unroll
-         for (int i = 0; i < TI; ++i) fa[i] = a[2 * s * LDA + i * 32];
-#pragma unroll
-         for (int j = 0; j < TJ; ++j) fb[j] = b[2 * s * LDB + j * 32];
-#pragma unroll
-         for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
-      }
-      if (kt + 1 < nk) {
-         stash<BM, LDA>(ra, sA[cur ^ 1], a_kmajor, tid);
-         stash<BN, LDB>(rb, sB[cur ^ 1], b_kmajor, tid);
-      }
-      __syncthreads();
+   return v;
+}
+__device__ __forceinline__ void store4(const GemmF32Args &g, v4f v, int m, int n)
+{
+   float *o = g.Y + (size_t)m * g.ldy + n;
+   if (n + 4 <= g.N) {
+      __builtin_memcpy(o, &v, 16);       // rows may start on any float
+      return;
    }
+#pragma unroll
+   for (int e = 0; e < 3; ++e)
+      if (n + e < g.N) o[e] = v[e];
+}
 
+// Products of any sizes, leading dimensions and storage (A_KM: A stored [K][M], B_KM: B stored [K][N]). 256 threads = 4
+// wavefronts in 2 x 2, each with MI x NJ tiles of 16 x 16 (v_mfma_f32_16x16x4_f32: tiles of 16 let a product take workgroup
+// tiles of 32 to 128 rows and columns, so that their number suits the device: 1500 x 1001 is 256 tiles of 96 x 64). Both
+// operand tiles travel global memory -> LDS without registers, 16 bytes per lane (buffer_load_dwordx4 ... lds, which takes any
+// address on a dword; 4 bytes per lane cost the same time per request, 33 cycles of a compute unit), in 2 or 3 stages of 32 k:
+//   * inside 16 k lane group kg (lane / 16) supplies k = 4 kg + e to matrix instruction e;
+//   * an operand with rows along K lies in rows of 8 chunks of 16 bytes, chunk c of row r in slot c ^ ((r >> 1) & 7): the 16
+//     rows a lane group reads with one 16-byte read per lane fall on 16 slots;
+//   * an operand with rows along M or N lies in rows of k, rotated by 16 columns per four k (one 4-byte read per
+//     instruction, the lane groups on different banks).
+// Cells outside the matrices ask for an offset outside the descriptor and arrive as zeros, or, behind M and N, hold
+// what lies there and are not stored. Only where a 16-byte piece would straddle the end of K (rows along K) or of the
+// whole matrix (rows along N, last row) the last step travels 4 bytes per lane. Bound: fp32 matrix instructions.
+template <bool KM, int ROWS>
+struct F32Operand {
+   static constexpr int BK = 32;
+   static constexpr int NRQ = ROWS / 32;                                             // requests per stage
+   static constexpr int NV = KM ? (ROWS == 128 ? 2 : ROWS == 96 ? 3 : 1) : 1;        // different lane offsets among them
+   static constexpr int KPR = 1024 / ROWS;                                           // KM: rows of k per request (but for 96 columns)
+   static constexpr unsigned OUTSIDE = 0x80000000u;
+   const float *base;
+   rsrc_t rs;                      // rows along K: the tile's rows
+   unsigned voff[NV];
+   int kofs[NV];                   // first k of the lane's 16 bytes inside the stage (KM: of the request)
+   unsigned ld4;
+   int ld, K, rows, first, tid;
+   bool straddles;                 // the last step has pieces that are inside in part
+   unsigned row_offset[KM ? 1 : NRQ];      // rows along K: uniform offsets of the requests' rows
+
+   __device__ __forceinline__ void init(const float *base_, int ld_, int first_, int count, int K_, int tid_)
+   {
+      ld = ld_;
+      ld4 = (unsigned)ld_ * 4u;
+      K = K_;
+      first = first_;
+      tid = tid_;
+      rows = count - first < ROWS ? count - first : ROWS;
+      if constexpr (KM) {
+         base = base_ + first;
+         straddles = (rows & 3) != 0;
 #pragma unroll
-   for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-         const int n = n0 + wn * TJ * 32 + j * 32 + fr;
-         if (n >= g.N) continue;
-         float brow = 0.0f;
-         if (g.bias_kind == SOFIE_BIAS_ROW) brow = __fmul_rn(g.beta, g.bias[n]);
-#pragma unroll
-         for (int r = 0; r < 16; ++r) {
-            const int m = m0 + wm * TI * 32 + i * 32 + (r >> 2) * 8 + fk * 4 + (r & 3);
-            if (m >= g.M) continue;
-            float v = __fmul_rn(g.alpha, acc[i][j][r]);
-            if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, brow);
-            else if (g.bias_kind == SOFIE_BIAS_FULL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n]));
-            else if (g.bias_kind == SOFIE_BIAS_COL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[m]));
-            if (g.relu) v = v > 0.0f ? v : 0.0f;
-            g.Y[(size_t)m * g.ldy + n] = v;
+         for (int v = 0; v < NV; ++v) {
+            const int idx = v * 256 + tid, k = idx / (ROWS / 4), pos = idx % (ROWS / 4) * 4;
+            const int col = (pos + ROWS - 16 * ((k >> 2) & 3) % ROWS) % ROWS;
+            kofs[v] = NV == 2 ? k - v * KPR : k;
+            voff[v] = col < rows ? (unsigned)kofs[v] * ld4 + (unsigned)col * 4u : OUTSIDE;
          }
+      } else {
+         base = base_ + (size_t)first * ld;
+         straddles = (K & 3) != 0;
+         rs = make_rsrc(base, (unsigned)rows * ld4);
+         const int row = tid >> 3;
+         kofs[0] = ((tid & 7) ^ ((row >> 1) & 7)) * 4;
+         voff[0] = (unsigned)row * ld4 + (unsigned)kofs[0] * 4u;
+#pragma unroll
+         for (int u = 0; u < NRQ; ++u) row_offset[u] = u * 32 < rows ? (unsigned)u * 32u * ld4 : 0u;
       }
+   }
+   // The cells of K-step kt into LDS byte address dst. WHOLE: the step ends in front of K (a wavefront has its SIMD to itself
+   // here, so every instruction of the loop is time: no checks). A uniform offset never exceeds the descriptor's range
+   // (requests of rows that do not exist ask for the tile's first rows, whose results are not stored).
+   template <bool WHOLE>
+   __device__ __forceinline__ void request(int kt, unsigned dst, int wave) const
+   {
+      const int k0 = kt * BK, left = WHOLE ? BK : K - k0 < BK ? K - k0 : BK;
+      if constexpr (KM) {
+         // a descriptor per step: its rows of k (any number of steps, a matrix of any size)
+         const bool last = !WHOLE && k0 + BK >= K;
+         const rsrc_t step = make_rsrc(base + (left > 0 ? (size_t)k0 * ld : 0),
+                                       left <= 0 ? 0u : last ? (unsigned)(left - 1) * ld4 + (unsigned)rows * 4u : BK * ld4);
+         if (!WHOLE && straddles && last && left > 0) {
+            for (int u = 0; u < ROWS / 8; ++u) {
+               const int idx = u * 256 + tid, k = idx / ROWS, pos = idx % ROWS;
+               const int col = (pos + ROWS - 16 * ((k >> 2) & 3) % ROWS) % ROWS;
+               dma4(step, dst + u * 1024 + wave * 256, (int)(col < rows && k < left ? (unsigned)k * ld4 + (unsigned)col * 4u : OUTSIDE), 0);
+            }
+            return;
+         }
+#pragma unroll
+         for (int u = 0; u < NRQ; ++u) {
+            const int k = NV == 3 ? 0 : u * KPR;
+            const unsigned v = WHOLE || k + kofs[u % NV] < left ? voff[u % NV] : OUTSIDE;
+            dma16(step, dst + u * 4096 + wave * 1024, (int)v, (int)(WHOLE || k < left ? (unsigned)k * ld4 : 0u));
+         }
+      } else {
+         const unsigned k4 = left > 0 ? (unsigned)k0 * 4u : 0u;
+         if (!WHOLE && straddles && left < BK && left > 0) {
+            for (int u = 0; u < ROWS / 8; ++u) {
+               const int row = u * 8 + (tid >> 5), pos = tid & 31;
+               const int k = (((pos >> 2) ^ ((row >> 1) & 7)) << 2) + (pos & 3);
+               dma4(rs, dst + u * 1024 + wave * 256, (int)(row < rows && k < left ? (unsigned)row * ld4 + (unsigned)k * 4u : OUTSIDE), (int)k4);
+            }
+            return;
+         }
+         const unsigned v = WHOLE || kofs[0] < left ? voff[0] : OUTSIDE;
+#pragma unroll
+         for (int u = 0; u < NRQ; ++u) dma16(rs, dst + u * 4096 + wave * 1024, (int)v, (int)(row_offset[u] + k4));
+      }
+   }
+};
+
+// Registers of a lane's reads of one operand tile: T tiles of 16 rows (columns) from `first` on.
+template <bool KM, int ROWS, int T>
+struct F32Fragments {
+   int at[KM ? T : 2];
+   __device__ __forceinline__ void init(int first, int r16, int kg)
+   {
+      if constexpr (KM) {
+#pragma unroll
+         for (int t = 0; t < T; ++t) at[t] = 4 * kg * ROWS + (first + t * 16 + 16 * kg) % ROWS + r16;
+      } else {
+#pragma unroll
+         for (int s = 0; s < 2; ++s) at[s] = (first + r16) * 32 + (((s * 4 + kg) ^ ((r16 >> 1) & 7)) << 2);
+      }
+   }
+   __device__ __forceinline__ v4f read(const float *tile, int s, int t) const
+   {
+      if constexpr (KM) {
+         v4f f;
+#pragma unroll
+         for (int e = 0; e < 4; ++e) f[e] = tile[at[t] + (s * 16 + e) * ROWS];
+         return f;
+      } else {
+         return *reinterpret_cast<const v4f *>(tile + at[s] + t * 16 * 32);
+      }
+   }
+};
+
+template <bool A_KM, bool B_KM, int MI, int NJ>
+__global__ void __launch_bounds__(256, MI * NJ >= 9 ? 2 : 3) k_gemm_f32(GemmF32Args g)
+{
+   constexpr int BM = 32 * MI, BN = 32 * NJ, BK = 32, STAGE = (BM + BN) * BK;
+   constexpr int NST = BM + BN > 192 ? 2 : 3;
+   constexpr int RQ = F32Operand<A_KM, BM>::NRQ + F32Operand<B_KM, BN>::NRQ;      // requests per wavefront and stage, at least
+   extern __shared__ __align__(16) unsigned char smem_raw[];
+   float *const lds = reinterpret_cast<float *>(smem_raw);
+   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)smem_raw;
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, kg = lane >> 4;
+   if (g.n_lead > 0) select_product(g, (long long)blockIdx.z + g.z0);
+   int tm, tn;
+   tile_of(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   int kt_begin = 0, kt_end = (g.K + BK - 1) / BK;
+   if (gridDim.y > 1) {      // K in slices: raw sums into the slice's plane of the scratch buffer
+      const int per = (kt_end + (int)gridDim.y - 1) / (int)gridDim.y;
+      kt_begin = (int)blockIdx.y * per;
+      kt_end = kt_end < kt_begin + per ? kt_end : kt_begin + per;
+      g.Y = g.partial + (size_t)blockIdx.y * g.M * g.N;
+      g.ldy = g.N;
+      g.alpha = 1.0f;
+      g.bias_kind = SOFIE_BIAS_NONE;
+      g.relu = 0;
+   }
+   F32Operand<A_KM, BM> oa;
+   F32Operand<B_KM, BN> ob;
+   oa.init(g.A, g.lda, m0, g.M, g.K, tid);
+   ob.init(g.B, g.ldb, n0, g.N, g.K, tid);
+   F32Fragments<A_KM, BM, MI> ra;
+   F32Fragments<B_KM, BN, NJ> rb;
+   ra.init(wm * 16 * MI, r16, kg);
+   rb.init(wn * 16 * NJ, r16, kg);
+   v4f acc[MI][NJ];
+#pragma unroll
+   for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+   auto request = [&](auto whole, int kt, int stage) {
+      // (a step behind the last one is requested again with nothing in it, so that the waits count the same requests)
+      const unsigned dst = lds0 + (unsigned)(stage * STAGE * 4);
+      oa.template request<decltype(whole)::value>(kt, dst, wave);
+      ob.template request<decltype(whole)::value>(kt, dst + BM * BK * 4, wave);
+   };
+   auto multiply = [&](const float *tile) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+         v4f fa[MI], fb[NJ];
+#pragma unroll
+         for (int i = 0; i < MI; ++i) fa[i] = ra.read(tile, s, i);
+#pragma unroll
+         for (int j = 0; j < NJ; ++j) fb[j] = rb.read(tile + BM * BK, s, j);
+         // rows of the result tile are columns n (the B operand first): a lane ends up with 4 consecutive columns of a row
+#pragma unroll
+         for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+               for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][e], fa[i][e], acc[i][j], 0, 0, 0);
+      }
+   };
+#pragma unroll
+   for (int d = 0; d < NST - 1; ++d) request(std::false_type{}, kt_begin + d, d);
+   int kt = kt_begin;
+   // steps whose requests (NST - 1 steps ahead) all end in front of K, then the others
+   const int whole_steps = g.K / BK < kt_end ? g.K / BK : kt_end;
+   for (; kt + 2 * NST - 2 < whole_steps; kt += NST) {
+#pragma unroll
+      for (int d = 0; d < NST; ++d) {
+         wait_vmcnt<(NST - 2) * RQ>();
+         __syncthreads();      // stage d has landed for every wavefront, and everybody is done with the one in front of it
+         request(std::true_type{}, kt + d + NST - 1, (d + NST - 1) % NST);
+         multiply(lds + d * STAGE);
+      }
+   }
+   for (; kt < kt_end; kt += NST) {
+#pragma unroll
+      for (int d = 0; d < NST; ++d) {
+         if (kt + d >= kt_end) break;
+         wait_vmcnt<(NST - 2) * RQ>();
+         __syncthreads();
+         request(std::false_type{}, kt + d + NST - 1, (d + NST - 1) % NST);
+         multiply(lds + d * STAGE);
+      }
+   }
+   wait_vmcnt<0>();            // requests of stages nobody reads may not outlive the workgroup
+#pragma unroll
+   for (int i = 0; i < MI; ++i) {
+      const int m = m0 + wm * 16 * MI + i * 16 + r16;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+         const int n = n0 + wn * 16 * NJ + j * 16 + kg * 4;
+         if (m < g.M && n < g.N) store4(g, finish4(g, acc[i][j], m, n), m, n);
+      }
+   }
 }
 
 // The same product for operands that allow it (A [M][K] row-major, K a multiple of 32, 16-byte aligned rows), with
@@ -191,21 +338,8 @@ __global__ void __launch_bounds__(256, T == 2 ? 2 : 4) k_gemm_f32_dma(GemmF32Arg
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int wm = wave >> 1, wn = wave & 1;
    const int fr = lane & 31, fk = lane >> 5;
-   // tiles in groups of 4 rows of tiles, so that the workgroups in flight share rows of A and columns of B in an L2
    int tm, tn;
-   {
-      const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-      // workgroups are dealt to the 8 XCDs in turn: renumbered so that an XCD (an L2) works on consecutive tiles
-      int pid = blockIdx.x;
-      {
-         const int tiles = tiles_m * tiles_n, xcd = pid & 7, base = tiles >> 3, rem = tiles & 7;
-         pid = (pid >> 3) + xcd * base + (xcd < rem ? xcd : rem);
-      }
-      const int width = 4 * tiles_n, group = pid / width, first = group * 4;
-      const int gsize = tiles_m - first < 4 ? tiles_m - first : 4;
-      tm = first + (pid % width) % gsize;
-      tn = (pid % width) / gsize;
-   }
+   tile_of(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
    const int rows_a = g.M - m0 < BM ? g.M - m0 : BM, rows_b = g.N - n0 < BN ? g.N - n0 : BN;
    // K in slices (few tiles, long K): this workgroup's steps of 32 k, raw sums into its plane of the scratch buffer
@@ -334,6 +468,139 @@ __global__ void __launch_bounds__(256, T == 2 ? 2 : 4) k_gemm_f32_dma(GemmF32Arg
    }
 }
 
+// Small products of any storage and alignment: a workgroup owns 16 MI rows x 16 NJ columns and all of K. Its eight
+// wavefronts take the chunks of 32 k in turn, DEPTH chunks of loads in flight each, straight from global memory into the
+// operand registers (lane group kg supplies k = 8 kg + e of a chunk to instruction e), no LDS and no barrier on the way;
+// their sums meet in LDS in a fixed order. A product this small is latency: one trip to memory, where the tiled kernel makes
+// one per K-step and the products with K in slices launch twice.
+template <bool A_KM, bool B_KM, int MI, int NJ>
+__global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(GemmF32Args g)
+{
+   constexpr int CH = 32, STEP = 8 * CH;
+   constexpr int DEPTH = MI * NJ == 1 ? 3 : 2;
+   constexpr int V = MI * NJ * 64;                     // quads of output columns of the tile
+   __shared__ __align__(16) v4f red[8][V];
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int r16 = lane & 15, kg = lane >> 4;
+   if (g.n_lead > 0) select_product(g, (long long)blockIdx.z + g.z0);
+   int tm, tn;
+   tile_of(blockIdx.x, (g.M + 16 * MI - 1) / (16 * MI), (g.N + 16 * NJ - 1) / (16 * NJ), tm, tn);
+   const int m0 = tm * 16 * MI, n0 = tn * 16 * NJ;
+   // rows and columns behind the matrix are copies of the last one; their results are not stored
+   const float *pa[MI], *pb[NJ];
+#pragma unroll
+   for (int i = 0; i < MI; ++i) {
+      const int m = m0 + i * 16 + r16 < g.M ? m0 + i * 16 + r16 : g.M - 1;
+      pa[i] = A_KM ? g.A + m : g.A + (size_t)m * g.lda;
+   }
+#pragma unroll
+   for (int j = 0; j < NJ; ++j) {
+      const int n = n0 + j * 16 + r16 < g.N ? n0 + j * 16 + r16 : g.N - 1;
+      pb[j] = B_KM ? g.B + n : g.B + (size_t)n * g.ldb;
+   }
+   struct Chunk {
+      v4f a[MI][2], b[NJ][2];
+   };
+   // every load stays inside its row (column): the last ones are moved down to end with it
+   auto fetch = [&](v4f &v, const float *p, int ld, bool km, int k) {
+      if (km) {
+#pragma unroll
+         for (int e = 0; e < 4; ++e) v[e] = p[(size_t)(k + e < g.K ? k + e : g.K - 1) * ld];
+      } else {
+         __builtin_memcpy(&v, p + (k < g.K - 4 ? k : g.K - 4), 16);
+      }
+   };
+   auto load = [&](Chunk &c, int k0) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+         for (int i = 0; i < MI; ++i) fetch(c.a[i][h], pa[i], g.lda, A_KM, k0 + kg * 8 + h * 4);
+#pragma unroll
+         for (int j = 0; j < NJ; ++j) fetch(c.b[j][h], pb[j], g.ldb, B_KM, k0 + kg * 8 + h * 4);
+      }
+   };
+   v4f acc[MI][NJ];
+#pragma unroll
+   for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+   // values of k .. k + 3 out of a load that may have been moved down, zero behind K
+   auto trim = [&](v4f v, bool km, int k) {
+      const int drop = km ? 0 : k - (g.K - 4);
+      v4f r = v;
+      if (drop > 0) {
+         if (drop & 1) r = v4f{r[1], r[2], r[3], 0.0f};
+         if (drop & 2) r = v4f{r[2], r[3], 0.0f, 0.0f};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = k + e < g.K ? r[e] : 0.0f;
+      return r;
+   };
+   auto multiply = [&](Chunk &c, int k0) {
+      if (k0 + CH > g.K) {      // uniform: the last chunk
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            const int k = k0 + kg * 8 + h * 4;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) c.a[i][h] = trim(c.a[i][h], A_KM, k);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) c.b[j][h] = trim(c.b[j][h], B_KM, k);
+         }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+         for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+               for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c.b[j][h][e], c.a[i][h][e], acc[i][j], 0, 0, 0);
+   };
+   Chunk c[DEPTH];
+   int k0 = wave * CH;
+#pragma unroll
+   for (int d = 0; d < DEPTH; ++d) load(c[d], k0 + d * STEP);
+   while (k0 < g.K) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+         if (k0 < g.K) multiply(c[d], k0);
+         if (k0 + DEPTH * STEP < g.K) load(c[d], k0 + DEPTH * STEP);
+         k0 += STEP;
+      }
+   }
+#pragma unroll
+   for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) red[wave][(i * NJ + j) * 64 + lane] = acc[i][j];
+   __syncthreads();
+   const int m = m0 + (tid / (64 * NJ)) * 16 + (tid & 15), n = n0 + (tid / 64 % NJ) * 16 + ((tid >> 4) & 3) * 4;
+   if (tid >= V || m >= g.M || n >= g.N) return;
+   v4f s = red[0][tid];
+#pragma unroll
+   for (int w = 1; w < 8; ++w)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = __fadd_rn(s[e], red[w][tid][e]);
+   store4(g, finish4(g, s, m, n), m, n);
+}
+
+// One thread per output: matrices whose rows are too long for the 32-bit offsets of the kernels above (2^24 floats).
+__global__ void __launch_bounds__(256) k_gemm_f32_plain(GemmF32Args g)
+{
+   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+   if (idx >= (size_t)g.M * g.N) return;
+   if (g.n_lead > 0) select_product(g, (long long)blockIdx.z + g.z0);
+   const int m = (int)(idx / g.N), n = (int)(idx % g.N);
+   float v = 0.0f;
+   for (int k = 0; k < g.K; ++k)
+      v = fmaf(g.transA ? g.A[(size_t)k * g.lda + m] : g.A[(size_t)m * g.lda + k], g.transB ? g.B[(size_t)n * g.ldb + k] : g.B[(size_t)k * g.ldb + n], v);
+   v = __fmul_rn(g.alpha, v);
+   if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[n]));
+   else if (g.bias_kind == SOFIE_BIAS_FULL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n]));
+   else if (g.bias_kind == SOFIE_BIAS_COL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[m]));
+   if (g.relu) v = v > 0.0f ? v : 0.0f;
+   g.Y[(size_t)m * g.ldy + n] = v;
+}
+
 // Few rows of A (M <= 64: a layer on a small batch): the product is a pass over B, bound by memory, and tiles of
 // 64 x 64 outputs would leave most of the device idle. Here a wavefront owns all rows of A (MT tiles of T = 16 rows,
 // v_mfma_f32_16x16x4_f32) and 4 T = 64 columns: its accumulators are MT x 4 tiles of T x T (rows of A x columns), and B
@@ -387,6 +654,14 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
    } else {
       const int n = c0 + 4 * fr;
       b_off[0] = n < g.N ? (unsigned)((4 * fk * g.ldb + n) * 4) : OUTSIDE;
+   }
+   // beta * bias of the lane's four columns, requested ahead of the loop (one load per output behind it was most of a
+   // short product's time: 52 x 1113 x 184 17.6 us)
+   float brow[4];
+#pragma unroll
+   for (int q = 0; q < 4; ++q) {
+      const int n = B_NK ? c0 + T * q + fr : c0 + 4 * fr + q;
+      brow[q] = g.bias_kind == SOFIE_BIAS_ROW && n < g.N ? __fmul_rn(g.beta, g.bias[n]) : 0.0f;
    }
    struct Chunk {
       v4f a[MT], b[4];
@@ -472,10 +747,10 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
    float *const out = last ? g.Y : partial + (size_t)blockIdx.y * g.M * g.N;
    const int ldo = last ? g.ldy : g.N;
    const bool vec_out = !last || (g.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(g.Y) & 15u) == 0);   // rows of whole 16-byte chunks
-   auto finish = [&](float v, int m, int n) {
+   auto finish = [&](float v, int q, int m, int n) {
       if (!last) return v;
       v = __fmul_rn(g.alpha, v);
-      if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[n]));
+      if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, brow[q]);
       else if (g.bias_kind == SOFIE_BIAS_FULL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n]));
       else if (g.bias_kind == SOFIE_BIAS_COL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[m]));
       if (g.relu) v = v > 0.0f ? v : 0.0f;
@@ -491,14 +766,14 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                const int n = c0 + T * q + fr;
-               if (n < g.N) out[(size_t)m * ldo + n] = finish(acc[t][q][r], m, n);
+               if (n < g.N) out[(size_t)m * ldo + n] = finish(acc[t][q][r], q, m, n);
             }
          } else {
             const int n = c0 + 4 * fr;     // N is a multiple of 4 on this path: the four columns are inside together
             if (n < g.N) {
                float *o = out + (size_t)m * ldo + n;
-               const v4f v = {finish(acc[t][0][r], m, n), finish(acc[t][1][r], m, n + 1), finish(acc[t][2][r], m, n + 2),
-                              finish(acc[t][3][r], m, n + 3)};
+               const v4f v = {finish(acc[t][0][r], 0, m, n), finish(acc[t][1][r], 1, m, n + 1), finish(acc[t][2][r], 2, m, n + 2),
+                              finish(acc[t][3][r], 3, m, n + 3)};
                if (vec_out) *reinterpret_cast<v4f *>(o) = v;
                else {
 #pragma unroll
@@ -571,6 +846,115 @@ int launch_skinny(sofie_hip_ctx *ctx, GemmF32Args &g)
    return g.transB ? launch_skinny_as<true, 16, 4>(ctx, g) : launch_skinny_as<false, 16, 4>(ctx, g);
 }
 
+template <bool A_KM, bool B_KM, int MI, int NJ>
+int launch_tiles_as(sofie_hip_ctx *ctx, GemmF32Args &g, int splits, unsigned nz)
+{
+   constexpr int BM = 32 * MI, BN = 32 * NJ, NST = BM + BN > 192 ? 2 : 3;
+   if (splits > 1) {
+      void *ws = nullptr;
+      if (int rc = workspace(ctx, (size_t)splits * g.M * g.N * sizeof(float), &ws)) return rc;
+      g.partial = static_cast<float *>(ws);
+   }
+   constexpr auto kern = k_gemm_f32<A_KM, B_KM, MI, NJ>;
+   SOFIE_LARGE_LDS(kern);
+   hipLaunchKernelGGL(kern, dim3(cdiv(g.M, BM) * cdiv(g.N, BN), splits, nz), dim3(256), NST * (BM + BN) * 32 * 4, ctx->stream, g);
+   if (int rc = check_launch(ctx, "k_gemm_f32")) return rc;
+   if (splits == 1) return SOFIE_HIP_OK;
+   hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(g.M * g.N, 256)), dim3(256), 0, ctx->stream, g, g.partial, splits);
+   return check_launch(ctx, "k_gemm_f32_skinny_finish");
+}
+
+template <bool A_KM, bool B_KM, int MI, int NJ>
+int launch_direct_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz)
+{
+   hipLaunchKernelGGL((k_gemm_f32_direct<A_KM, B_KM, MI, NJ>), dim3(cdiv(g.M, 16 * MI) * cdiv(g.N, 16 * NJ), 1, nz), dim3(512), 0, ctx->stream, g);
+   return check_launch(ctx, "k_gemm_f32_direct");
+}
+
+// The kernel for operands of any kind, by an estimate of its time behind the launch.
+//   direct   1 us per round of resident workgroups, and the larger of its matrix instructions (550 GFLOP/s per compute unit) and
+//            of what it reads (a compute unit takes in 43 bytes per ns)
+//   tiles    the measured time of a K-step of 32, of a workgroup alone on its compute unit and of one among others (128 x 128:
+//            1.95 / 1.91 us, of which 1.71 are its matrix instructions), and 2 us around it
+//   slices   5 us for the pass that adds them, and their sums written and read at 6 TB/s
+// Fitted to the times of every kernel on 34 sizes, 10 x 64 x 16 to 4000 x 4001 x 4002. Where the lines fall: 90 x 90 x 360 5.4 us
+// direct, 6.4 on 32 x 32 tiles, 12.3 on 64 x 64; 1500 x 1001 x 1111 85 / 38 / 42, 34 on 32 x 64; 256 x 256 x 12800 39 direct, 90 on
+// 32 x 32 tiles and 25 with them in 8 slices; 4000 x 4001 x 4002 978 on 64 x 64, 965 on 128 x 128.
+struct GeneralChoice {
+   bool direct;
+   int mi, nj, splits;
+   float us;
+};
+constexpr int kDirectTiles[4][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}};
+struct TileCost {
+   int mi, nj;
+   float alone, among;
+};
+constexpr TileCost kTileCosts[6] = {{1, 1, 0.21f, 0.176f}, {1, 2, 0.36f, 0.275f}, {2, 1, 0.36f, 0.275f}, {2, 2, 0.60f, 0.51f}, {3, 2, 0.85f, 0.78f}, {4, 4, 1.95f, 1.91f}};
+
+GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, bool one_launch)
+{
+   GeneralChoice best = {false, 1, 1, 1, 1e30f};
+   const int cus = ctx->num_cus;
+   auto consider = [&](bool direct, int mi, int nj, int splits, float us) {
+      if (us < best.us) best = {direct, mi, nj, splits, us};
+   };
+   if (g.K >= 4 && g.bias_kind != SOFIE_BIAS_FULL)
+      for (const auto &t : kDirectTiles) {
+         const int mi = t[0], nj = t[1], resident = mi * nj == 4 ? 1 : 2;
+         const long long per_cu = ((long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj) * nz + cus - 1) / cus;
+         const float mfma = (float)per_cu * 512.0f * mi * nj * g.K / 550e3f, reads = (float)per_cu * 64.0f * (mi + nj) * g.K / 43e3f;
+         consider(true, mi, nj, 1, 0.5f + (float)((per_cu + resident - 1) / resident) + (mfma > reads ? mfma : reads));
+      }
+   const int steps = cdiv(g.K, 32);
+   for (const auto &t : kTileCosts) {
+      const long long tiles = (long long)cdiv(g.M, 32 * t.mi) * cdiv(g.N, 32 * t.nj) * nz;
+      for (int s = 1; s <= 16; s = s < 4 ? s + 1 : s * 2) {
+         if (s > 1 && (one_launch || steps / s < 4 || (size_t)g.M * g.N >= ((size_t)1 << 28))) break;
+         const long long per_cu = (tiles * s + cus - 1) / cus;
+         const float step = per_cu == 1 ? t.alone : (float)per_cu * t.among;
+         consider(false, t.mi, t.nj, s, 2.0f + step * cdiv(steps, s) + (s > 1 ? 5.0f + 8.0f * s * (float)g.M * g.N / 6e6f : 0.0f));
+      }
+   }
+   return best;
+}
+
+template <bool A_KM, bool B_KM>
+int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_launch)
+{
+   const GeneralChoice c = general_choice(ctx, g, nz, one_launch);
+   if (c.direct) {
+      switch (c.mi * 10 + c.nj) {
+      case 11: return launch_direct_as<A_KM, B_KM, 1, 1>(ctx, g, nz);
+      case 12: return launch_direct_as<A_KM, B_KM, 1, 2>(ctx, g, nz);
+      case 21: return launch_direct_as<A_KM, B_KM, 2, 1>(ctx, g, nz);
+      default: return launch_direct_as<A_KM, B_KM, 2, 2>(ctx, g, nz);
+      }
+   }
+   switch (c.mi * 10 + c.nj) {
+   case 11: return launch_tiles_as<A_KM, B_KM, 1, 1>(ctx, g, c.splits, nz);
+   case 12: return launch_tiles_as<A_KM, B_KM, 1, 2>(ctx, g, c.splits, nz);
+   case 21: return launch_tiles_as<A_KM, B_KM, 2, 1>(ctx, g, c.splits, nz);
+   case 22: return launch_tiles_as<A_KM, B_KM, 2, 2>(ctx, g, c.splits, nz);
+   case 32: return launch_tiles_as<A_KM, B_KM, 3, 2>(ctx, g, c.splits, nz);
+   default: return launch_tiles_as<A_KM, B_KM, 4, 4>(ctx, g, c.splits, nz);
+   }
+}
+
+// Operands of any size, alignment and storage; nz products of a stack (one_launch: K is not cut).
+int launch_general(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_launch)
+{
+   // 32-bit offsets: 128 rows of an operand with rows along K, 32 of the others
+   if (g.lda >= (1 << 22) || g.ldb >= (1 << 22)) {
+      const size_t blocks = ((size_t)g.M * g.N + 255) / 256;
+      SOFIE_REQUIRE(ctx, blocks < ((size_t)1 << 31), "output too large");
+      hipLaunchKernelGGL(k_gemm_f32_plain, dim3((unsigned)blocks, 1, nz), dim3(256), 0, ctx->stream, g);
+      return check_launch(ctx, "k_gemm_f32_plain");
+   }
+   if (g.transA) return g.transB ? launch_general_as<true, false>(ctx, g, nz, one_launch) : launch_general_as<true, true>(ctx, g, nz, one_launch);
+   return g.transB ? launch_general_as<false, false>(ctx, g, nz, one_launch) : launch_general_as<false, true>(ctx, g, nz, one_launch);
+}
+
 }  // namespace
 
 extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, int M, int N, int K, float alpha,
@@ -609,7 +993,8 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
                     (size_t)128 * ldy * 4 < (1u << 31) && (size_t)cdiv(M, tile) * cdiv(N, tile) < (1u << 30);
    // a few rows of A on a B of some size: a pass over B (k_gemm_f32_skinny); needs whole 16-byte chunks per lane. With 33 to
    // 64 rows and thousands of column tiles the 64 x 64 tiles below fill the device and reuse B from LDS.
-   const bool skinny = (M <= 32 || (M <= 64 && N < 8192)) && !transA && K >= 64 && K % 4 == 0 && (size_t)N * K >= 64 * 1024 && lda % 4 == 0 && ldb % 4 == 0 &&
+   // ... and more than 32 rows on 16 M elements of B are faster on tiles with K in slices: 64 x 4096 x 4096 27 against 39 us.
+   const bool skinny = (M <= 32 || (M <= 64 && N < 8192 && (size_t)N * K < ((size_t)1 << 24))) && !transA && K >= 64 && K % 4 == 0 && (size_t)N * K >= 64 * 1024 && lda % 4 == 0 && ldb % 4 == 0 &&
                        (transB || N % 4 == 0) && aligned16(A) && aligned16(B) &&
                        (size_t)M * lda * 4 < (1u << 31) && (size_t)(transB ? N : K) * ldb * 4 < (1u << 31) &&
                        (size_t)M * ldy < (1u << 31);
@@ -643,12 +1028,9 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
       if (splits == 1) return SOFIE_HIP_OK;
       hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(M * N, 256)), dim3(256), 0, ctx->stream, g, g.partial, splits);
       return check_launch(ctx, "k_gemm_f32_skinny_finish");
-   } else if (small) {
-      hipLaunchKernelGGL((k_gemm_f32<1, 1>), dim3(cdiv(N, 64), cdiv(M, 64)), dim3(256), 0, ctx->stream, g);
-   } else {
-      hipLaunchKernelGGL((k_gemm_f32<2, 2>), dim3(cdiv(N, 128), cdiv(M, 128)), dim3(256), 0, ctx->stream, g);
    }
-   return check_launch(ctx, "k_gemm_f32");
+   // (a bias given for every output element keeps to one launch)
+   return launch_general(ctx, g, 1, bias_kind == SOFIE_BIAS_FULL);
 }
 
 extern "C" int sofie_hip_gemm_f32_stacked(sofie_hip_ctx *ctx, int transA, int transB, int M, int N, int K, float alpha,
@@ -680,10 +1062,7 @@ extern "C" int sofie_hip_gemm_f32_stacked(sofie_hip_ctx *ctx, int transA, int tr
    for (long long z0 = 0; z0 < stack; z0 += 65535) {
       const unsigned nz = (unsigned)((stack - z0) < 65535 ? (stack - z0) : 65535);
       g.z0 = (int)z0;
-      const bool small = (size_t)cdiv(M, 128) * cdiv(N, 128) * nz < 256;
-      if (small) hipLaunchKernelGGL((k_gemm_f32<1, 1>), dim3(cdiv(N, 64), cdiv(M, 64), nz), dim3(256), 0, ctx->stream, g);
-      else hipLaunchKernelGGL((k_gemm_f32<2, 2>), dim3(cdiv(N, 128), cdiv(M, 128), nz), dim3(256), 0, ctx->stream, g);
-      if (int rc = check_launch(ctx, "k_gemm_f32_stacked")) return rc;
+      if (int rc = launch_general(ctx, g, nz, true)) return rc;
    }
    return SOFIE_HIP_OK;
 }

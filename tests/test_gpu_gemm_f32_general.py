@@ -1,0 +1,60 @@
+"""fp32 products of any size, alignment and storage: k_gemm_f32_direct (16 and 32 rows and columns per workgroup) and
+k_gemm_f32 (tiles of 32 x 32 to 128 x 128, K in one piece or in slices), every transposition, against float64."""
+import numpy as np
+import pytest
+
+from sofie_amd import lib as L
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sofie_amd import ops as o
+    return o
+
+
+# (M, N, K): a single element, K below the four of a load, one k and one row or column behind a chunk (4, 32), a tile
+# (16, 32, 64, 96, 128) or a wavefront's share; K long enough for slices (few tiles) and a size for each tile shape
+SIZES = [(1, 1, 1), (3, 5, 2), (16, 16, 32), (17, 33, 31), (33, 17, 65), (65, 129, 100), (130, 67, 19), (97, 64, 33), (64, 64, 2049),
+         (300, 200, 1025), (10, 1000, 999), (700, 33, 77), (1100, 1000, 130), (2050, 1030, 67)]
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_gemm_f32_of_any_kind(ops, M, N, K, tA, tB):
+    """1e-5 of the largest output: sums of fp32 products in another order differ by about sqrt(K) 2^-24 of the terms' root
+    mean square times sqrt(K). Leading dimensions equal to the sizes and three floats wider, every bias kind."""
+    g = torch.Generator(device="cuda").manual_seed(100 * M + 10 * N + K)
+    ctx = ops.default_context()
+
+    def matrix(rows, cols, pad):
+        return torch.randn(rows, cols + pad, device="cuda", generator=g)
+    for pad, kind in ((0, L.BIAS_ROW), (3, L.BIAS_NONE), (0, L.BIAS_FULL), (3, L.BIAS_COL)):
+        A = matrix(K, M, pad) if tA else matrix(M, K, pad)
+        B = matrix(N, K, pad) if tB else matrix(K, N, pad)
+        a = A[:, :M].t() if tA else A[:, :K]
+        b = B[:, :K].t() if tB else B[:, :N]
+        bias = {L.BIAS_NONE: None, L.BIAS_ROW: torch.randn(N, device="cuda", generator=g), L.BIAS_FULL: torch.randn(M, N, device="cuda", generator=g),
+                L.BIAS_COL: torch.randn(M, device="cuda", generator=g)}[kind]
+        beta = 0.0 if bias is None else 2.0
+        y = ctx.empty((M, N), torch.float32)
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_gemm_f32(ctx.h, tA, tB, M, N, K, 0.5, ctx.ptr(A), A.shape[1], ctx.ptr(B), B.shape[1], beta, ctx.ptr(bias), kind,
+                                             ctx.ptr(y), N, L.ACT_RELU))
+        ctx.sync()
+        ref = 0.5 * (a.double().contiguous() @ b.double().contiguous())
+        if bias is not None:
+            ref = ref + beta * (bias.double()[:, None] if kind == L.BIAS_COL else bias.double())
+        ref = ref.clamp(min=0)
+        assert float((y.double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max()))
+
+
+def test_gemm_f32_slices_give_the_same_bits_twice(ops):
+    """Few tiles and a long K without alignment: slices of K in a fixed order."""
+    r = np.random.default_rng(7)
+    A, B = r.standard_normal((70, 6001)).astype(np.float32), r.standard_normal((6001, 90)).astype(np.float32)
+    y = ops.gemm_f32(A, B, beta=0.0)
+    assert np.array_equal(y, ops.gemm_f32(A, B, beta=0.0))
+    assert np.max(np.abs(y - A.astype(np.float64) @ B.astype(np.float64))) <= 1e-5 * np.max(np.abs(y))
