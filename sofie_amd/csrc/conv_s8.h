@@ -32,4 +32,9 @@ int qconv_ring(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done);
 // same whole images in both. *done tells whether the launch was made (if not, nothing was launched).
 int qconv_ring_pair(sofie_hip_ctx *ctx, const QConvArgs &g1, const QConvArgs &g2, bool *done);
 
+// Any channel counts, kernel sizes, strides, pads and layouts, one group, int8 output, optionally with a 2x2 stride-2 max
+// pooling. scratch: qconv_any_scratch(g) bytes of the context's scratch buffer (0: the kernel does not take the problem).
+size_t qconv_any_scratch(const QConvArgs &g);
+int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *done);
+
 }  // namespace sofie

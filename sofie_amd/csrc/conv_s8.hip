@@ -681,9 +681,45 @@ int run(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch)
                                  g.pool_kw, 0, 0, 0, 0, g.pool_sh, g.pool_sw);
 }
 
+// What the kernels of fixed channel multiples leave: k_qconv_any, with a pooling other than 2x2 behind it as a pass of its own.
+// Without room for its copies (a recording does not let the scratch buffer grow) nothing is launched and *done stays false.
+int run_any(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
+{
+   *done = false;
+   QConvArgs h = g;
+   size_t need = qconv_any_scratch(h), conv_bytes = 0;
+   if (!need && g.pool_kh != 0) {
+      if (mfma_shape(g) || (g.C == 1 && g.KH == 3 && g.KW == 3)) return SOFIE_HIP_OK;   // the convolution has a kernel of its own
+      h.pool_kh = h.pool_kw = h.pool_sh = h.pool_sw = 0;
+      h.PH = g.OH; h.PW = g.OW;
+      need = qconv_any_scratch(h);
+      conv_bytes = up256((size_t)g.N * g.OC * g.OH * g.OW);
+   }
+   if (!need || !workspace_has_room(ctx, conv_bytes + need)) return SOFIE_HIP_OK;
+   void *ws = nullptr;
+   if (int rc = workspace(ctx, conv_bytes + need, &ws)) return rc;
+   int8_t *const scratch = static_cast<int8_t *>(ws);
+   if (conv_bytes) h.y = scratch;
+   if (int rc = qconv_any(ctx, h, scratch + conv_bytes, done)) return rc;
+   if (!*done || !conv_bytes) return SOFIE_HIP_OK;
+   return sofie_hip_maxpool2d_s8(ctx, scratch, static_cast<int8_t *>(g.y), g.y_nhwc ? SOFIE_LAYOUT_NHWC : SOFIE_LAYOUT_NCHW, g.N, g.OC,
+                                 g.OH, g.OW, g.pool_kh, g.pool_kw, 0, 0, 0, 0, g.pool_sh, g.pool_sw);
+}
+
 template <int OUT>
 int run(sofie_hip_ctx *ctx, const QConvArgs &g)
 {
+   if constexpr (OUT == SOFIE_OUT_S8) {
+      bool done = false;
+      if (int rc = qconv_first_layer(ctx, g, &done)) return rc;
+      if (done) return SOFIE_HIP_OK;
+      if (int rc = launch_mfma<OUT>(ctx, g, &done)) return rc;
+      if (done) return SOFIE_HIP_OK;
+      if (!mfma_shape(g) || (g.x_nhwc && g.y_nhwc && g.w_ohwi)) {
+         if (int rc = run_any(ctx, g, &done)) return rc;
+         if (done) return SOFIE_HIP_OK;
+      }
+   }
    void *ws = nullptr;
    const size_t need = run_scratch_bytes(g);
    if (need)
@@ -844,6 +880,11 @@ extern "C" int sofie_hip_quantize_qconv2d_s8(sofie_hip_ctx *ctx, const float *x,
    bool done = false;
    if (int rc = qconv_first_layer(ctx, g, &done)) return rc;
    if (done) return SOFIE_HIP_OK;
+   // channel counts that the int8 kernels do not take: the copy that k_qconv_any reads is quantized while it is made
+   if (!mfma_shape(g)) {
+      if (int rc = run_any(ctx, g, &done)) return rc;
+      if (done) return SOFIE_HIP_OK;
+   }
    // otherwise: quantize into scratch memory, then the int8 path
    g.xf = nullptr;
    const size_t xbytes = up256((size_t)N * C * H * W);

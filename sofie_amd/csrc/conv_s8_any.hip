@@ -1,0 +1,483 @@
+// int8 convolution of any channel counts, kernel sizes, strides and pads (one group, int8 output) on the matrix cores.
+//
+// Implicit GEMM on v_mfma_i32_16x16x64_i8: rows are output pixels, columns output channels, K = 16-byte chunks of the
+// input. A lane's operand of a K-step (64 bytes) is one chunk of its pixel, loaded straight into registers at
+// base(pixel) + offset(chunk); the offsets of all chunks stand in a small LDS table. Two forms of the input:
+//   * in place (BOUNDS): channels-last, C a multiple of 16, 16-byte aligned. A chunk lies inside one tap; a chunk outside
+//     the image is replaced by the zero-point.
+//   * a copy in scratch memory, [N][H + pads][W + pads][Cp], Cp = C rounded up to whole dwords, pads filled with the
+//     zero-point: written by k_qconv_any_input from channels-last or channel-plane int8 or from the float tensor that
+//     QuantizeLinear would read. One kernel row of a window is then KW * Cp contiguous bytes, which are cut into chunks
+//     together (a 7x7 kernel on 3 channels: 14 chunks instead of 49), and no tap needs a bounds check.
+// The weights are copied fragment by fragment ([16 channels][K-step][lane][16 bytes], zeros behind the last channel and the
+// last tap), so that what an operand reads behind a row or a pixel is multiplied by 0 and a fragment is 1 KB in one piece.
+//
+// Bound. The vector cache hands a CU 64 bytes a cycle: an operand fragment of 1 KB costs 16 cycles of it, a matrix
+// instruction 16 cycles of one of four SIMDs, so 64 pixels x 64 channels per wavefront with the weights in LDS balance the
+// two. Measurements stand at the rules of choose().
+#include <math.h>
+
+#include "conv_s8.h"
+#include "gemm_tile.h"
+
+using namespace sofie;
+
+namespace {
+
+struct AnyArgs {
+   const int8_t *x;         // channels-last input or its padded copy
+   const int8_t *w;         // fragments of the weights
+   const int32_t *bias;
+   const float *scale;
+   int8_t *y;
+   unsigned xbytes, wbytes; // sizes of x and w: loads behind them return 0
+   int M, OC;               // output pixels (pooled ones with the fused pooling), output channels
+   int OH, OW;              // extent of the pixel grid of M
+   int H, W, C;             // BOUNDS: the image
+   int img, row;            // bytes of an image and of a row
+   int sh, sw, ph, pw;      // BOUNDS: pads; otherwise 0
+   int pix;                 // bytes of a pixel
+   int run16;               // 16-byte chunks of a kernel row
+   int S, chunks;           // K-steps of 64 bytes, chunks of 16 bytes in them that carry weights
+   int nob;                 // blocks of NB*16 channels
+   int ntiles, per;         // pixel tiles, consecutive tiles of a workgroup
+   int total;               // workgroups with work (the grid is rounded up to the XCDs)
+   int nhwc_out, plane;
+   unsigned fill;
+   int zp, lo;
+   FastDiv dOW, dOH, dRun, dC16, dPlane;
+};
+
+constexpr unsigned OUTSIDE = 0x80000000u;
+
+// MB x NB tiles of 16 pixels x 16 channels per wavefront; NW wavefronts, groups of WK of them share their pixels and deal
+// the K-steps among themselves; D fragments of every pixel tile in flight. POOL: the four pixel tiles are the positions of
+// a 2x2 window with stride 2. BLDS: the weights of the workgroup's channels stay in LDS while it walks over its tiles.
+template <int MB, int NB, int NW, int WK, int D, bool BOUNDS, bool POOL, bool BLDS>
+__global__ void __launch_bounds__(NW * 64) k_qconv_any(AnyArgs a)
+{
+   static_assert(!POOL || MB == 4, "the four window positions are the four pixel tiles");
+   static_assert(!BLDS || WK == 1, "the dealt K-steps read their weights from memory");
+   constexpr int MBP = POOL ? 1 : MB;
+   constexpr int TM = (NW / WK) * MBP * 16;
+   constexpr int OCT = NB * 16;
+   extern __shared__ __align__(16) unsigned char smem[];
+   float *const s_scale = reinterpret_cast<float *>(smem);
+   int *const s_bias = reinterpret_cast<int *>(s_scale + OCT);
+   v2i *const tab = reinterpret_cast<v2i *>(s_bias + OCT);                         // [S * 4] offset, (row << 16 | column) of a chunk
+   unsigned char *const big = reinterpret_cast<unsigned char *>(tab + a.S * 4);    // weights (BLDS) or partial sums (WK > 1)
+
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int l16 = lane & 15, kg = lane >> 4;
+   const int wp = wave / WK, wk = wave % WK;
+   // workgroups of one XCD (every eighth) take neighbouring pixel tiles: the rows that two tiles share are in its L2
+   const int idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+   if (idx >= a.total) return;
+   const int ob = idx % a.nob;
+   const int t0 = (idx / a.nob) * a.per, t1 = min(t0 + a.per, a.ntiles);
+   const int n0 = ob * OCT;
+
+   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(a.x), 0, a.xbytes, 0x00020000);
+   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(a.w), 0, a.wbytes, 0x00020000);
+
+   if constexpr (BLDS) {
+      // the fragments of NB tiles are contiguous: a linear copy by LDS-DMA, 1 KB per wavefront and request
+      const rsrc_t rs = make_rsrc(a.w, a.wbytes);
+      const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)big;
+      for (int f = wave; f < NB * a.S; f += NW) dma16(rs, lds0 + f * 1024, lane * 16, (ob * NB * a.S + f) * 1024);
+   }
+   for (int q = tid; q < a.S * 4; q += NW * 64) {
+      const int kh = fdiv(q, a.dRun), r = q - kh * a.run16;
+      const int kw = BOUNDS ? fdiv(r, a.dC16) : 0;
+      // chunks behind the last kernel row carry zero weights: they read the first chunk again
+      tab[q] = q < a.chunks ? v2i{kh * a.row + r * 16, kh << 16 | kw} : v2i{0, 0};
+   }
+   if (tid < OCT) {
+      const int n = n0 + tid;
+      s_scale[tid] = n < a.OC ? a.scale[n] : 0.0f;
+      s_bias[tid] = a.bias && n < a.OC ? a.bias[n] : 0;
+   }
+   if constexpr (BLDS) wait_vmcnt<0>();
+   __syncthreads();
+
+   const int s_per = (a.S + WK - 1) / WK;
+   const int s0 = wk * s_per, s1 = min(s0 + s_per, a.S);
+   const float zpo = (float)(a.zp + 128), lof = (float)(a.lo + 128);
+
+   // sums of a tile (POOL: of the four positions) -> requantised bytes of pixel m, channels n0 + 16 i + 4 kg ..
+   auto finish = [&](const v4i *s, int i, int m) {
+      const v4f sc = *reinterpret_cast<const v4f *>(s_scale + i * 16 + kg * 4);
+      const v4i bi = *reinterpret_cast<const v4i *>(s_bias + i * 16 + kg * 4);
+      unsigned pk = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+         int v = s[0][t];
+         if constexpr (POOL) {   // the requantisation is monotonic: falling for a negative scale
+            const int hi = max(max(s[0][t], s[1][t]), max(s[2][t], s[3][t])), lo = min(min(s[0][t], s[1][t]), min(s[2][t], s[3][t]));
+            v = sc[t] < 0.0f ? lo : hi;
+         }
+         const float r = __fmul_rn(__int2float_rn(v + bi[t]), sc[t]);
+         pk = __builtin_amdgcn_cvt_pk_u8_f32(fmaxf(__fadd_rn(rintf(r), zpo), lof), t, pk);
+      }
+      pk ^= 0x80808080u;
+      const int oc = n0 + i * 16 + kg * 4;
+      if (m >= a.M || oc >= a.OC) return;
+      if (a.nhwc_out) {
+         int8_t *const p = a.y + (size_t)m * a.OC + oc;
+         if (oc + 4 <= a.OC) __builtin_memcpy(p, &pk, 4);
+         else
+            for (int t = 0; t < a.OC - oc; ++t) p[t] = (int8_t)(pk >> (8 * t));
+      } else {
+         const int n = fdiv(m, a.dPlane);
+         int8_t *const p = a.y + ((size_t)n * a.OC + oc) * a.plane + (m - n * a.plane);
+         for (int t = 0; t < min(4, a.OC - oc); ++t) p[(size_t)t * a.plane] = (int8_t)(pk >> (8 * t));
+      }
+   };
+
+   for (int tile = t0; tile < t1; ++tile) {
+      int base[MB], ih0[MB], iw0[MB];
+#pragma unroll
+      for (int j = 0; j < MB; ++j) {
+         int m = tile * TM + (POOL ? wp * 16 : (wp * MB + j) * 16) + l16;
+         m = m < a.M ? m : a.M - 1;
+         const int R = fdiv(m, a.dOW), n = fdiv(R, a.dOH);
+         int oh = R - n * a.OH, ow = m - R * a.OW;
+         if constexpr (POOL) { oh = 2 * oh + (j >> 1); ow = 2 * ow + (j & 1); }
+         ih0[j] = oh * a.sh - a.ph;
+         iw0[j] = ow * a.sw - a.pw;
+         base[j] = n * a.img + ih0[j] * a.row + iw0[j] * a.pix;
+      }
+      v4i acc[NB][MB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+         for (int j = 0; j < MB; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+
+      v4i fa[D][MB], fb[BLDS ? 1 : D][NB];
+      int pad[D][MB];      // BOUNDS: the zero-point where the chunk lies outside the image (its load returns 0), else 0
+      auto load = [&](int buf, int s) {
+         const v2i e = tab[s * 4 + kg];
+#pragma unroll
+         for (int j = 0; j < MB; ++j) {
+            unsigned off = (unsigned)(base[j] + e[0]);
+            if constexpr (BOUNDS) {
+               const bool in = (unsigned)(ih0[j] + (e[1] >> 16)) < (unsigned)a.H & (unsigned)(iw0[j] + (e[1] & 0xffff)) < (unsigned)a.W;
+               off = in ? off : OUTSIDE;
+               pad[buf][j] = in ? 0 : (int)a.fill;
+            }
+            fa[buf][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+         }
+         if constexpr (!BLDS) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+               fb[buf][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, lane * 16, ((ob * NB + i) * a.S + s) * 1024, 0));
+         }
+      };
+      auto mma = [&](int buf, int s) {
+         v4i b[NB];
+#pragma unroll
+         for (int i = 0; i < NB; ++i) {
+            if constexpr (BLDS) b[i] = *reinterpret_cast<const v4i *>(big + (i * a.S + s) * 1024 + lane * 16);
+            else b[i] = fb[buf][i];
+         }
+#pragma unroll
+         for (int j = 0; j < MB; ++j) {
+            v4i f = fa[buf][j];
+            if constexpr (BOUNDS) {
+#pragma unroll
+               for (int t = 0; t < 4; ++t) f[t] |= pad[buf][j];
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[i], f, acc[i][j], 0, 0, 0);
+         }
+      };
+      if (s0 < s1) {
+#pragma unroll
+         for (int u = 0; u < D; ++u) load(u, min(s0 + u, s1 - 1));
+         int s = s0;
+         for (; s + D < s1; s += D) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+               mma(u, s + u);
+               load(u, min(s + u + D, s1 - 1));
+            }
+         }
+#pragma unroll
+         for (int u = 0; u < D; ++u)
+            if (s + u < s1) mma(u, s + u);
+      }
+      const int m0 = tile * TM + wp * MBP * 16 + l16;
+      if constexpr (WK == 1) {
+#pragma unroll
+         for (int i = 0; i < NB; ++i) {
+            if constexpr (POOL) finish(acc[i], i, m0);
+            else
+#pragma unroll
+               for (int j = 0; j < MB; ++j) finish(&acc[i][j], i, m0 + j * 16);
+         }
+      } else {
+         // sums of the wavefronts that share these pixels, added by whichever of them owns the unit
+         v4i *const part = reinterpret_cast<v4i *>(big) + (size_t)wp * WK * NB * MB * 64;
+#pragma unroll
+         for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < MB; ++j) part[((wk * NB + i) * MB + j) * 64 + lane] = acc[i][j];
+         __syncthreads();
+         constexpr int UNIT = POOL ? MB : 1;
+         for (int u = wk; u < NB * MB / UNIT; u += WK) {
+            v4i v[UNIT];
+#pragma unroll
+            for (int e = 0; e < UNIT; ++e) {
+               v[e] = part[(u * UNIT + e) * 64 + lane];
+#pragma unroll
+               for (int k = 1; k < WK; ++k) v[e] += part[(k * NB * MB + u * UNIT + e) * 64 + lane];
+            }
+            if constexpr (POOL) finish(v, u, m0);
+            else finish(v, u / MB, m0 + (u % MB) * 16);
+         }
+         if (tile + 1 < t1) __syncthreads();
+      }
+   }
+}
+
+// Weights in fragment order: one thread per 16 bytes, [channel tile][K-step][lane].
+__global__ void __launch_bounds__(256) k_qconv_any_weights(const int8_t *w, v4i *dst, int total, int S, int run16, FastDiv dS, FastDiv dRun,
+                                                           FastDiv dPix, int pix, int OC, int C, int KH, int KW, int ohwi)
+{
+   const int id = blockIdx.x * 256 + threadIdx.x;
+   if (id >= total) return;
+   const int lane = id & 63, fs = id >> 6;
+   const int t = fdiv(fs, dS), s = fs - t * S;
+   const int oc = t * 16 + (lane & 15), q = s * 4 + (lane >> 4);
+   const int kh = fdiv(q, dRun), r0 = (q - kh * run16) * 16;
+   int8_t v[16];
+#pragma unroll
+   for (int b = 0; b < 16; ++b) {
+      const int r = r0 + b, kw = fdiv(r, dPix), c = r - kw * pix;
+      const bool ok = oc < OC && kh < KH && kw < KW && c < C;
+      const size_t off = !ok ? 0 : ohwi ? (((size_t)oc * KH + kh) * KW + kw) * C + c : (((size_t)oc * C + c) * KH + kh) * KW + kw;
+      const int8_t e = w[off];
+      v[b] = ok ? e : (int8_t)0;
+   }
+   v4i o;
+   __builtin_memcpy(&o, v, 16);
+   dst[id] = o;
+}
+
+// The padded copy of the input, one thread per dword. FROM: 0 channels-last int8, 1 int8 planes, 2 float planes (quantized).
+template <int FROM>
+__global__ void __launch_bounds__(256) k_qconv_any_input(QConvArgs g, unsigned *dst, int total, int HP, int WP, int cd, FastDiv dcd,
+                                                         FastDiv dWP, FastDiv dHP)
+{
+   const int id = blockIdx.x * 256 + threadIdx.x;
+   if (id >= total) return;
+   // dword of a pixel fastest where the source is channels-last (contiguous reads); the column fastest where it is planes
+   int n, r, c, k;
+   if constexpr (FROM == 0) {
+      const int p = fdiv(id, dcd), R = fdiv(p, dWP);
+      k = id - p * cd;
+      c = p - R * WP;
+      n = fdiv(R, dHP);
+      r = R - n * HP;
+   } else {
+      const int p = fdiv(id, dWP), R = fdiv(p, dcd);
+      c = id - p * WP;
+      k = p - R * cd;
+      n = fdiv(R, dHP);
+      r = R - n * HP;
+   }
+   const int ih = r - g.ph, iw = c - g.pw;
+   unsigned v = 0x01010101u * (unsigned)(g.zpx & 0xff);
+   if (ih >= 0 && ih < g.H && iw >= 0 && iw < g.W) {
+      const int left = g.C - 4 * k;      // channels of this dword that exist (the others meet zero weights)
+      if constexpr (FROM == 0) {
+         const int8_t *p = g.x + (((size_t)n * g.H + ih) * g.W + iw) * g.C + 4 * k;
+         if (left >= 4) __builtin_memcpy(&v, p, 4);
+         else {
+            v = 0;
+            for (int t = 0; t < left; ++t) v |= (unsigned)(uint8_t)p[t] << (8 * t);
+         }
+      } else if (left <= 0) {
+         v = 0;
+      } else {
+         const size_t plane = (size_t)g.H * g.W;
+         const size_t off = ((size_t)n * g.C + 4 * k) * plane + (size_t)ih * g.W + iw;
+         v = 0;
+         if constexpr (FROM == 1) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+               const unsigned e = (uint8_t)g.x[off + (t < left ? t : 0) * plane];
+               v |= t < left ? e << (8 * t) : 0u;
+            }
+         } else {
+            float f[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) f[t] = g.xf[off + (t < left ? t : 0) * plane];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+               float q = rintf(__fdiv_rn(f[t], g.xscale));
+               q = fminf(fmaxf(q, -1024.0f), 1024.0f);
+               const int e = min(127, max(-128, (int)q + g.zpx));
+               v |= t < left ? (unsigned)(e & 0xff) << (8 * t) : 0u;
+            }
+         }
+      }
+   }
+   dst[FROM == 0 ? id : (((size_t)n * HP + r) * WP + c) * cd + k] = v;
+}
+
+size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// Sizes that the launch and the scratch memory are planned by.
+struct Plan {
+   bool ok, copy;         // copy: the input goes through the padded copy
+   int pix, HP, WP, run16, S, nt;
+   size_t xbytes, wbytes;
+};
+
+Plan plan(const QConvArgs &g)
+{
+   Plan p{};
+   const bool pool = g.pool_kh != 0;
+   if (g.groups != 1 || !g.scale) return p;
+   if (pool && !(g.pool_kh == 2 && g.pool_kw == 2 && g.pool_sh == 2 && g.pool_sw == 2)) return p;
+   p.copy = g.xf || !g.x_nhwc || g.C % 16 != 0 || !aligned16(g.x);
+   p.HP = g.H + g.ph + g.pbh;
+   p.WP = g.W + g.pw + g.pbw;
+   // pixels of whole dwords; from 64 channels on of whole chunks, so that no operand load crosses a cache line
+   p.pix = !p.copy ? g.C : g.C >= 64 ? (g.C + 15) & ~15 : (g.C + 3) & ~3;
+   const long long run = (long long)g.KW * p.pix, chunks = (run + 15) / 16 * g.KH;
+   if (chunks > 4096 || g.KH > 0x7fff || g.KW > 0xffff) return p;
+   p.run16 = (int)((run + 15) / 16);
+   p.S = (int)((chunks + 3) / 4);
+   p.nt = cdiv(g.OC, 16);
+   p.wbytes = (size_t)(p.nt + 3) * p.S * 1024;   // the last block of up to four channel tiles may hang over by three
+   const size_t in = p.copy ? (size_t)g.N * p.HP * p.WP * p.pix : (size_t)g.N * g.H * g.W * g.C;
+   // 64 bytes behind the copy: a kernel row's last chunk reads up to 15 bytes behind the last pixel
+   p.xbytes = p.copy ? in + 64 : in;
+   const long long rows = (long long)g.N * p.HP, M = (long long)g.N * g.PH * g.PW;
+   p.ok = p.xbytes < ((size_t)1 << 30) && p.wbytes < ((size_t)1 << 30) && rows < (1ll << 31) && M < (1ll << 30) && g.OC < (1 << 24);
+   return p;
+}
+
+}  // namespace
+
+namespace sofie {
+
+size_t qconv_any_scratch(const QConvArgs &g)
+{
+   const Plan p = plan(g);
+   return !p.ok ? 0 : up256(p.copy ? p.xbytes : 0) + up256(p.wbytes);
+}
+
+int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *done)
+{
+   *done = false;
+   const Plan p = plan(g);
+   if (!p.ok) return SOFIE_HIP_OK;
+   const bool pool = g.pool_kh != 0;
+   int8_t *const xs = scratch, *const ws_own = scratch + up256(p.copy ? p.xbytes : 0);
+   // weights: kept under the constant-weights promise, otherwise (and where packed_weights has only the start of the scratch
+   // buffer to give) in this call's part of the scratch buffer
+   void *ws = nullptr;
+   bool fresh = true;
+   const int layout[] = {4, g.OC, g.C, g.KH, g.KW, p.pix, g.w_ohwi};
+   if (ctx->constant_weights)
+      if (int rc = packed_weights(ctx, g.w, layout_key(layout, 7), p.wbytes, &ws, &fresh)) return rc;
+   if (!ws || ws == ctx->workspace) ws = ws_own;
+   if (fresh) {
+      const int total = (int)(p.wbytes / 16);
+      hipLaunchKernelGGL(k_qconv_any_weights, dim3(cdiv(total, 256)), dim3(256), 0, ctx->stream, g.w, static_cast<v4i *>(ws), total, p.S,
+                         p.run16, make_fastdiv(p.S), make_fastdiv(p.run16), make_fastdiv(p.pix), p.pix, g.OC, g.C, g.KH, g.KW, g.w_ohwi);
+      if (int rc = check_launch(ctx, "k_qconv_any_weights")) return rc;
+   }
+   if (p.copy) {
+      const int cd = p.pix / 4, total = g.N * p.HP * p.WP * cd;
+      const dim3 grid((unsigned)cdiv(total, 256)), block(256);
+      unsigned *const dst = reinterpret_cast<unsigned *>(xs);
+      const FastDiv dcd = make_fastdiv(cd), dWP = make_fastdiv(p.WP), dHP = make_fastdiv(p.HP);
+      if (g.xf) hipLaunchKernelGGL(k_qconv_any_input<2>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
+      else if (!g.x_nhwc) hipLaunchKernelGGL(k_qconv_any_input<1>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
+      else hipLaunchKernelGGL(k_qconv_any_input<0>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
+      if (int rc = check_launch(ctx, "k_qconv_any_input")) return rc;
+   }
+   AnyArgs a{};
+   a.x = p.copy ? xs : g.x;
+   a.w = static_cast<const int8_t *>(ws);
+   a.bias = g.bias; a.scale = g.scale; a.y = static_cast<int8_t *>(g.y);
+   a.xbytes = (unsigned)p.xbytes; a.wbytes = (unsigned)p.wbytes;
+   a.OC = g.OC; a.OH = g.PH; a.OW = g.PW; a.M = g.N * g.PH * g.PW;
+   a.H = g.H; a.W = g.W; a.C = g.C;
+   a.pix = p.pix;
+   a.row = (p.copy ? p.WP : g.W) * p.pix;
+   a.img = (p.copy ? p.HP : g.H) * a.row;
+   a.sh = g.sh; a.sw = g.sw;
+   a.ph = p.copy ? 0 : g.ph; a.pw = p.copy ? 0 : g.pw;
+   a.run16 = p.run16; a.S = p.S; a.chunks = p.run16 * g.KH;
+   a.nhwc_out = g.y_nhwc; a.plane = g.PH * g.PW;
+   a.fill = 0x01010101u * (unsigned)(g.zpx & 0xff);
+   a.zp = g.zpy; a.lo = g.lo;
+   a.dOW = make_fastdiv(a.OW); a.dOH = make_fastdiv(a.OH); a.dRun = make_fastdiv(p.run16); a.dC16 = make_fastdiv(cdiv(p.pix, 16));
+   a.dPlane = make_fastdiv(a.plane);
+   const bool bounds = !p.copy && (g.ph || g.pw || g.pbh || g.pbw);
+
+   const int cus = ctx->num_cus;
+   const size_t tab_bytes = (size_t)p.S * 32;
+   auto go = [&](auto kern, int nb, int nw, int wk, int mbp, size_t big, int resident) {
+      const int tm = nw / wk * mbp * 16;
+      a.nob = cdiv(p.nt, nb);
+      a.ntiles = cdiv(a.M, tm);
+      a.per = 1;
+      if (resident) {      // persistent: one round of workgroups
+         int groups = cus * resident / a.nob;
+         if (groups < 1) groups = 1;
+         a.per = cdiv(a.ntiles, groups);
+      }
+      a.total = cdiv(a.ntiles, a.per) * a.nob;
+      hipLaunchKernelGGL(kern, dim3((unsigned)((a.total + 7) & ~7)), dim3(nw * 64), (size_t)nb * 16 * 8 + tab_bytes + big, ctx->stream, a);
+      *done = true;
+      return check_launch(ctx, "k_qconv_any");
+   };
+#define SOFIE_ANY(MB_, MBPOOL_, NB_, NW_, WK_, D_, BLDS_, big_, resident_)                                                   \
+   do {                                                                                                                      \
+      constexpr auto kb = k_qconv_any<MB_, NB_, NW_, WK_, D_, true, false, BLDS_>, kn = k_qconv_any<MB_, NB_, NW_, WK_, D_, false, false, BLDS_>, \
+                     pb = k_qconv_any<4, NB_, NW_, WK_, D_, true, true, BLDS_>, pn = k_qconv_any<4, NB_, NW_, WK_, D_, false, true, BLDS_>; \
+      SOFIE_LARGE_LDS(kb); SOFIE_LARGE_LDS(kn); SOFIE_LARGE_LDS(pb); SOFIE_LARGE_LDS(pn);                                    \
+      return go(pool ? (bounds ? pb : pn) : (bounds ? kb : kn), NB_, NW_, WK_, pool ? 1 : MB_, big_, resident_);             \
+   } while (0)
+   // channels per workgroup: up to four tiles of 16, as few idle ones as possible
+   auto even = [&](int most) { return cdiv(p.nt, cdiv(p.nt, most)); };
+   const int mb = pool ? 1 : 4;
+   int nb = even(4);
+   while (nb > 1 && (size_t)nb * p.S * 1024 > (size_t)144 * 1024) nb = even(nb - 1);
+   const size_t wlds = (size_t)nb * p.S * 1024;
+   const long long big_tiles = (long long)cdiv(a.M, 4 * mb * 16) * cdiv(p.nt, nb);
+   if (big_tiles >= cus && wlds <= (size_t)144 * 1024) {
+      if (wlds + tab_bytes <= (size_t)50 * 1024 || big_tiles < 2 * cus) {
+         const int resident = (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024)) > 3 ? 3 : (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024));
+         if (nb == 1) SOFIE_ANY(4, 4, 1, 4, 1, 4, true, wlds, resident);
+         if (nb == 2) SOFIE_ANY(4, 4, 2, 4, 1, 4, true, wlds, resident);
+         if (nb == 3) SOFIE_ANY(4, 4, 3, 4, 1, 3, true, wlds, resident);
+         SOFIE_ANY(4, 4, 4, 4, 1, 3, true, wlds, resident);
+      }
+      if (nb == 1) SOFIE_ANY(4, 4, 1, 8, 1, 4, true, wlds, 1);
+      if (nb == 2) SOFIE_ANY(4, 4, 2, 8, 1, 4, true, wlds, 1);
+      if (nb == 3) SOFIE_ANY(4, 4, 3, 8, 1, 3, true, wlds, 1);
+      SOFIE_ANY(4, 4, 4, 8, 1, 3, true, wlds, 1);
+   }
+   // fewer tiles: smaller ones, weights from memory; few K-steps are not worth dealing out
+   const long long mid_tiles = (long long)cdiv(a.M, 4 * (pool ? 1 : 2) * 16) * cdiv(p.nt, even(4));
+   if (mid_tiles >= cus || p.S < 4) {
+      nb = mid_tiles >= cus ? even(4) : 1;
+      if (nb == 1) SOFIE_ANY(2, 4, 1, 4, 1, 4, false, 0, 0);
+      if (nb == 2) SOFIE_ANY(2, 4, 2, 4, 1, 3, false, 0, 0);
+      if (nb == 3) SOFIE_ANY(2, 4, 3, 4, 1, 3, false, 0, 0);
+      SOFIE_ANY(2, 4, 4, 4, 1, 3, false, 0, 0);
+   }
+   if ((long long)cdiv(a.M, 16) * cdiv(p.nt, 2) >= cus && p.nt > 1)
+      SOFIE_ANY(1, 4, 2, 8, 8, 4, false, (size_t)8 * 2 * (pool ? 4 : 1) * 1024, 0);
+   SOFIE_ANY(1, 4, 1, 8, 8, 4, false, (size_t)8 * 1 * (pool ? 4 : 1) * 1024, 0);
+#undef SOFIE_ANY
+}
+
+}  // namespace sofie
