@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "conv_f32.h"
 #include "gemm_tile.h"
 
 using namespace sofie;
@@ -643,6 +644,60 @@ inline size_t dma_lds_budget(const sofie_hip_ctx *ctx, size_t workgroups, int ma
    return best == 3 ? (size_t)52 * 1024 : (size_t)(160 * 1024) / best - 512;
 }
 
+// What conv_f32_any needs to know, but for the phases.
+ConvProblem problem_of(const ConvArgs &g)
+{
+   ConvProblem p{};
+   p.x = g.x; p.w = g.w; p.bias = g.bias; p.y = g.y;
+   p.N = g.N; p.C = g.C; p.H = g.H; p.W = g.W; p.OC = g.OC; p.groups = g.groups;
+   p.sh = g.sh; p.sw = g.sw; p.dh = g.dh; p.dw = g.dw; p.relu = g.relu;
+   p.KH0 = g.KH0; p.KW0 = g.KW0; p.OH0 = g.OH0; p.OW0 = g.OW0;
+   p.transposed = g.transposed;
+   return p;
+}
+
+// The whole of g (its one phase, or all of them) on k_conv_f32_any; *done stays false where it does not take it.
+int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done)
+{
+   ConvProblem p = problem_of(g);
+   p.nphases = g.nphases > 1 ? g.nphases : 1;
+   p.phase[0] = {g.OH, g.OW, g.KH, g.KW, g.ph, g.pw, g.th0, g.ths, g.tw0, g.tws, g.oy0, g.oys, g.ox0, g.oxs};
+   for (int i = 0; i < g.nphases && g.nphases > 1; ++i) {
+      const PhaseArgs &f = g.phase[i];
+      p.phase[i] = {f.OH, f.OW, f.KH, f.KW, f.ph, f.pw, f.th0, g.ths, f.tw0, g.tws, f.oy0, g.oys, f.ox0, g.oxs};
+   }
+   return conv_f32_any(ctx, p, done);
+}
+
+// Whether a layer that k_conv2d_f32_dma takes (full channel blocks of an even K) runs on k_conv_f32_any all the same.
+// With the constant-weights promise from 7 million multiply-adds on (us, k_conv2d_f32_dma / k_conv_f32_any: 7.4 M 8.2 / 4.8,
+// 231 M 17.3 / 10.5, 472 M 19.8 / 16.7, 944 M 31.7 / 25.4, 59 G 910 / 900); below, both are a launch's latency, and the tests
+// of the kept layouts name the older kernel there. Without it the weights are laid out in front of every call, and the
+// fragments of k_conv_f32_any (whole tiles of 16 channels and 32 k) cost more to write: from 2^29 on, where that no longer
+// counts (944 M 34.2 / 29.4; 472 M 21.8 / 22.3, 84 M 1x1 11.3 / 12.4, 231 M 19.7 / 15.5, 12 M 10.7 / 9.7).
+bool beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
+{
+   double outputs = (double)g.OH * g.OW, taps = (double)g.KH * g.KW;
+   if (g.nphases > 1) {
+      outputs = (double)g.H * g.W;
+      taps = (double)g.KH0 * g.KW0;
+   }
+   const double madds = (double)g.N * g.OC * g.icg * outputs * taps;
+   // Short sums for whole tiles of channels: the stores of a tile of 64 x 128 come in longer pieces (7x8x144x144 -> 39: 21.8
+   // against 24.5 us, 6x6x30x30 -> 128 transposed 4x4: 10.1 against 14.0).
+   const int phases = g.nphases > 1 ? g.nphases : 1;
+   if (g.icg <= 16 && g.icg * taps <= 72 * phases && g.ocg >= 32 && (double)g.OH * g.OW >= 256.0 * phases) return false;
+   // Long sums of phases that fill tiles of 64 channels x 128 pixels: there k_conv2d_f32_dma reads each input cell once for all
+   // taps and stores two pixels apart in longer pieces (64x128x28x28 -> 64, 4x4: 123.9 against 126.3 us; where a quarter
+   // of the tiles is empty, 40x144x7x7 -> 232: 56 against 28).
+   if (g.nphases > 1 && g.icg * taps >= 256.0 * phases) {
+      const double area = (double)g.phase[0].OH * g.phase[0].OW;
+      const double full = g.ocg / (64.0 * cdiv(g.ocg, 64)) * area / (128.0 * cdiv((int)area, 128));
+      if (full >= 0.85) return false;
+   }
+   return madds >= (ctx->constant_weights ? 7.0e6 : 536870912.0);
+}
+
 template <int TI, int TJ>
 int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
 {
@@ -658,7 +713,7 @@ int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
    const size_t budget = 52 * 1024;
    *done = false;
    const int octiles = cdiv(g.ocg, BOC);
-   if ((size_t)g.groups * octiles > 65535 || g.N > 65535) return SOFIE_HIP_OK;
+   if ((size_t)g.groups * octiles > 65535 || g.N > 65535) return run_any(ctx, g, done);
    if (!g.transposed) {
       // First choice: operands by LDS-DMA under the matrix loop (k_conv2d_f32_dma), on a copy of the weights laid out
       // for it (a small kernel in front). The largest full channel block with an even K whose two LDS buffers fit the
@@ -744,6 +799,10 @@ int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
          }
       }
    }
+   if (!g.transposed || (g.uh == 1 && g.uw == 1)) {
+      if (int rc = run_any(ctx, g, done)) return rc;
+      if (*done) return SOFIE_HIP_OK;
+   }
    int icb = 96 / KHW;
    if (icb < 1) icb = 1;
    if (icb > g.icg) icb = g.icg;
@@ -785,7 +844,7 @@ int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
    const size_t budget = 52 * 1024;
    *done = false;
    const int octiles = cdiv(g.ocg, BOC);
-   if ((size_t)g.groups * octiles > 65535 || (size_t)g.N * g.nphases > 65535) return SOFIE_HIP_OK;
+   if ((size_t)g.groups * octiles > 65535 || (size_t)g.N * g.nphases > 65535) return run_any(ctx, g, done);
    size_t lds_max = 0;
    int tiles_max = 0;
    // First choice: operands by LDS-DMA under the matrix loop, on sub-kernels gathered into the [K][channel] order (a
@@ -895,6 +954,8 @@ int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
       lds_max = 0;
       tiles_max = 0;
    }
+   if (int rc = run_any(ctx, g, done)) return rc;
+   if (*done) return SOFIE_HIP_OK;
    for (int i = 0; i < g.nphases; ++i) {
       PhaseArgs &p = g.phase[i];
       const int KHW = p.KH * p.KW;
@@ -945,6 +1006,10 @@ int run_conv(sofie_hip_ctx *ctx, ConvArgs &g)
    g.dOW = make_fastdiv((unsigned)g.OW);
    bool done = false;
    int rc;
+   if (beyond_dma(ctx, g) && (!g.transposed || (g.uh == 1 && g.uw == 1))) {
+      rc = run_any(ctx, g, &done);
+      if (rc || done) return rc;
+   }
    // 128 channels x 128 pixels per workgroup where that gives every compute unit a tile, else 64 x 128, else 64 x 64: a
    // layer on one image or a few has too few of the large tiles to fill the device (one 56x56 image, 64 -> 128
    // channels: 25 tiles of 128 x 128, 98 of 64 x 64)
@@ -1139,6 +1204,10 @@ extern "C" int sofie_hip_conv_transpose2d_f32(sofie_hip_ctx *ctx, const float *x
       if (ok && all.nphases > 1) {
          all.dUH = make_fastdiv(1u); all.dUW = make_fastdiv(1u); all.dOW = make_fastdiv(1u);
          bool done = false;
+         if (beyond_dma(ctx, all)) {
+            if (int rc = run_any(ctx, all, &done)) return rc;
+            if (done) return SOFIE_HIP_OK;
+         }
          // tiles as for the plain convolution: the largest that still give every compute unit one
          auto tiles = [&](int boc, int bp) {
             size_t t = 0;

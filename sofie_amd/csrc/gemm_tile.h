@@ -524,6 +524,17 @@ __device__ __forceinline__ void store4_buf(rsrc_t rs, float v, unsigned voff, un
                 : "memory");
 }
 
+// 16 bytes per lane the same way. The wait states belong to the store: its data registers must not be written by the next
+// instruction, which the compiler sees to only for stores whose uniform offset is a constant (lanes 12 to 15 of a row had the
+// next address in their third float now and then).
+__device__ __forceinline__ void store16_buf(rsrc_t rs, v4f v, unsigned voff, unsigned soff)
+{
+   asm volatile("buffer_store_dwordx4 %0, %1, %2, %3 offen\n\ts_nop 1"
+                :
+                : "v"(v), "v"(voff), "s"(rs), "s"(__builtin_amdgcn_readfirstlane((int)soff))
+                : "memory");
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()
 {
