@@ -519,11 +519,13 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(G
          for (int j = 0; j < NJ; ++j) fetch(c.b[j][h], pb[j], g.ldb, B_KM, k0 + kg * 8 + h * 4);
       }
    };
-   v4f acc[MI][NJ];
+   // two sums per output: shorter chains of rounded additions (relative error of two layers of 1024 1.6e-7 -> 1.25e-7) that do not wait
+   // for each other (16 x 300 x 300 4.3 -> 4.0 us)
+   v4f acc[2][MI][NJ];
 #pragma unroll
    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < NJ; ++j) acc[0][i][j] = acc[1][i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
    // values of k .. k + 3 out of a load that may have been moved down, zero behind K
    auto trim = [&](v4f v, bool km, int k) {
       const int drop = km ? 0 : k - (g.K - 4);
@@ -554,7 +556,7 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(G
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
-               for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c.b[j][h][e], c.a[i][h][e], acc[i][j], 0, 0, 0);
+               for (int j = 0; j < NJ; ++j) acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c.b[j][h][e], c.a[i][h][e], acc[h][i][j], 0, 0, 0);
    };
    Chunk c[DEPTH];
    int k0 = wave * CH;
@@ -571,7 +573,7 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(G
 #pragma unroll
    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) red[wave][(i * NJ + j) * 64 + lane] = acc[i][j];
+      for (int j = 0; j < NJ; ++j) red[wave][(i * NJ + j) * 64 + lane] = acc[0][i][j] + acc[1][i][j];
    __syncthreads();
    const int m = m0 + (tid / (64 * NJ)) * 16 + (tid & 15), n = n0 + (tid / 64 % NJ) * 16 + ((tid >> 4) & 3) * 4;
    if (tid >= V || m >= g.M || n >= g.N) return;
@@ -1069,12 +1071,15 @@ extern "C" int sofie_hip_gemm_f32_stacked(sofie_hip_ctx *ctx, int transA, int tr
 
 // ------------------------------------------------------------------------------------------------------------
 // A chain of small fully connected layers in one launch: y = act_L(... act_1(x W_1 + b_1) ... W_L + b_L).
-// A multilayer perceptron on a few hundred rows is three kernel launches of a few microseconds each and nothing
-// else: the matrix cores have nothing to chew on (8.65 MFLOP for 256 rows of 64 -> 128 -> 64 -> 8) and the time
-// is the launches. Here a workgroup carries R rows through every layer with the activations in LDS; the weights
-// (W_l [K_l, N_l], row-major) come straight from L2, one coalesced row of N_l per step of k. With N_l below the
-// 256 threads of the workgroup the threads also split K: thread (o, part) sums its share of k for output o, the
-// partial sums meet in LDS. Plain fp32 fused multiply-adds in a fixed order per output; no matrix instructions.
+// A workgroup carries 16 RT rows through every layer with the activations in LDS, on v_mfma_f32_16x16x4_f32. The weights
+// (W_l [K_l, N_l], row-major) go straight from the L2 into the instruction's operand registers, 4 bytes per lane of any
+// dword: a piece is 64 rows of k x 16 columns, 16 loads. A wavefront's pieces form one list over all column tiles, parts of K and
+// layers, and the loads of the next piece are always under way while one is multiplied: the first weights (and biases) of a layer
+// arrive under the layer before it. Against one thread per output and 1, 4 or 8 rows per workgroup (us): 64-128-64-8 on 256 rows
+// 7.5 -> 6.6, on 16384 27.4 -> 12.5; 20-32-32-1 on 4096 15.5 -> 5.3; 100-487-13 on 8192 34.8 -> 16.7. What bounds it: launch and memory latency for a small network on a few rows; a
+// compute unit's share of the L2 (about 57 B/ns, every workgroup reads all weights) up to 16 rows for each of them; the
+// matrix instructions above.
+// A layer with fewer column tiles than the workgroup has wavefronts deals the pieces of K to parts, added in LDS in order.
 namespace {
 
 struct MlpArgs {
@@ -1084,84 +1089,165 @@ struct MlpArgs {
    int relu[SOFIE_MLP_MAX_LAYERS];
    const float *x;
    float *y;
-   int n_layers, M, ldx, ldy, maxd;
+   int n_layers, M, ldx, ldy;
+   int ld[2];   // floats per row of the two activation buffers: the inputs of even and of odd layers
+   int psh[SOFIE_MLP_MAX_LAYERS];   // the pieces of a layer's K are dealt to 1 << psh parts
 };
 
-template <int R>
-__global__ void __launch_bounds__(256) k_mlp_f32(MlpArgs a)
+template <int RT, int NW>
+__global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
 {
+   constexpr int ROWS = 16 * RT;
+   // sums per output: shorter chains of rounded additions, and matrix instructions that do not wait for each other
+   constexpr int CH = RT == 4 ? 2 : 4;
    extern __shared__ __align__(16) float s_mlp[];
-   float *buf_in = s_mlp, *buf_out = s_mlp + R * a.maxd;     // activations of the rows, [R][maxd] each
-   float *part = s_mlp + 2 * R * a.maxd;                     // [256][R] partial sums
-   const int tid = threadIdx.x;
-   const int row0 = blockIdx.x * R;
-   {
-      const int K0 = a.dims[0];
-      for (int idx = tid; idx < R * K0; idx += 256) {
-         const int r = idx / K0, k = idx - r * K0;
-         buf_in[r * a.maxd + k] = row0 + r < a.M ? a.x[(size_t)(row0 + r) * a.ldx + k] : 0.0f;
+   float *const buf[2] = {s_mlp, s_mlp + ROWS * a.ld[0]};
+   float *const part = s_mlp + ROWS * (a.ld[0] + a.ld[1]);     // [wavefront][RT][lane][4] sums of parts of K
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int c = lane & 15, kg = lane >> 4;
+   const int row0 = blockIdx.x * ROWS;
+
+   // the next piece whose weights are requested: layer, unit (column tile and part), piece of K; and what its layer's pieces share
+   int fl = -1, fu = 0, fp = 0, fK = 0, fN = 0, fsh = 0, funits = 0;
+   __amdgpu_buffer_rsrc_t fw, fb;
+   auto settle = [&] {       // onto the first piece of this wavefront at or behind unit fu
+      while (fu >= funits) {
+         if (++fl >= a.n_layers) return;
+         fK = a.dims[fl];
+         fN = a.dims[fl + 1];
+         fsh = a.psh[fl];
+         funits = ((fN + 15) >> 4) << fsh;
+         fu = wave;
+         // rows behind K lie outside the descriptor and arrive as zeros; columns behind N hold other weights and end in
+         // columns of the result that are dropped
+         fw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.W[fl]), 0, fK * fN * 4, 0x00020000);
+         fb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.bias[fl]), 0, a.bias[fl] ? fN * 4 : 0, 0x00020000);
+      }
+      fp = fu & ((1 << fsh) - 1);
+   };
+   float nw[16], nb = 0.0f;
+   auto fetch = [&] {
+      if (fl >= a.n_layers) return;
+      const int n = (fu >> fsh) * 16 + c, row = fN * 4;
+      const int at = (fp * 64 + 4 * kg) * row + n * 4;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+         if (fp * 64 + s * 16 < fK) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+               nw[4 * s + e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fw, at + (16 * s + e) * row, 0, 0));
+         }
+      nb = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(fb, n * 4, 0, 0));
+      fp += 1 << fsh;
+      if (fp * 64 >= fK) {
+         fu += NW;
+         settle();
+      }
+   };
+   settle();
+   fetch();
+
+   {  // the rows of x, with zeros up to a whole 16 of K and for rows behind M
+      const int K = a.dims[0], KP = (K + 15) & ~15;
+      for (int k = lane; k < KP; k += 64) {
+         float v[ROWS / NW];
+#pragma unroll
+         for (int i = 0; i < ROWS / NW; ++i) {
+            const int row = row0 + i * NW + wave;
+            v[i] = row < a.M && k < K ? a.x[(size_t)row * a.ldx + k] : 0.0f;
+         }
+#pragma unroll
+         for (int i = 0; i < ROWS / NW; ++i) buf[0][(i * NW + wave) * a.ld[0] + k] = v[i];
       }
    }
    __syncthreads();
+
    for (int l = 0; l < a.n_layers; ++l) {
-      const int K = a.dims[l], N = a.dims[l + 1];
-      const float *__restrict__ W = a.W[l];
-      const bool last = l + 1 == a.n_layers;
-      // columns per pass (a power of two, at most 256) and the parts K is cut into
-      int n2 = 1;
-      while (n2 < N && n2 < 256) n2 <<= 1;
-      const int parts = 256 / n2;
-      const int kc = (K + parts - 1) / parts;
-      const int oc = tid & (n2 - 1), pt = tid / n2;
-      const int k0 = pt * kc, k1 = k0 + kc < K ? k0 + kc : K;
-      for (int o0 = 0; o0 < N; o0 += n2) {
-         const int o = o0 + oc;
-         float acc[R];
+      const int K = a.dims[l], N = a.dims[l + 1], ldi = a.ld[l & 1], ldo = a.ld[(l + 1) & 1];
+      const float *in = l & 1 ? buf[1] : buf[0];
+      float *out = l & 1 ? buf[0] : buf[1];
+      const bool last = l + 1 == a.n_layers, relu = a.relu[l];
+      const int sh = a.psh[l], parts = 1 << sh, tiles = (N + 15) >> 4, pieces = (K + 63) >> 6;
+      // columns behind N become the zeros up to a whole 16 of the next layer's K
+      auto finish = [&](int r, int n, float v) {
+         if (relu) v = fmaxf(v, 0.0f);
+         if (!last) out[r * ldo + n] = n < N ? v : 0.0f;
+         else if (n < N && row0 + r < a.M) a.y[(size_t)(row0 + r) * a.ldy + n] = v;
+      };
+      for (int u = wave; u < tiles << sh; u += NW) {
+         const int t = u >> sh, p = u & (parts - 1);
+         v4f acc[RT][CH];
 #pragma unroll
-         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-         if (o < N) {
-            const float *w = W + (size_t)k0 * N + o;
-#pragma unroll 8
-            for (int k = k0; k < k1; ++k) {
-               const float wv = *w;
-               w += N;
+         for (int i = 0; i < RT; ++i)
 #pragma unroll
-               for (int r = 0; r < R; ++r) acc[r] = fmaf(buf_in[r * a.maxd + k], wv, acc[r]);
+            for (int h = 0; h < CH; ++h) acc[i][h] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+         float bias = 0.0f;
+         for (int q = p; q < pieces; q += parts) {
+            float w[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) w[e] = nw[e];
+            bias = nb;
+            fetch();
+            const float *ap = in + c * ldi + q * 64 + 4 * kg;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+               if (q * 64 + s * 16 >= K) break;
+#pragma unroll
+               for (int i = 0; i < RT; ++i) {
+                  const v4f f = *reinterpret_cast<const v4f *>(ap + i * 16 * ldi + s * 16);
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) acc[i][e % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[e], w[4 * s + e], acc[i][e % CH], 0, 0, 0);
+               }
             }
          }
-         auto finish = [&](int r, int oo, float v) {
-            if (a.bias[l]) v += a.bias[l][oo];
-            if (a.relu[l]) v = fmaxf(v, 0.0f);
-            if (last) {
-               if (row0 + r < a.M) a.y[(size_t)(row0 + r) * a.ldy + oo] = v;
-            } else {
-               buf_out[r * a.maxd + oo] = v;
-            }
-         };
-         if (parts == 1) {
-            // 256 columns per pass: every thread holds the complete sums of its column
-            if (o < N) {
+         // a lane has rows 4 kg .. 4 kg + 3 of column c
 #pragma unroll
-               for (int r = 0; r < R; ++r) finish(r, o, acc[r]);
-            }
-         } else {
+         for (int i = 0; i < RT; ++i) {
+            v4f sum = acc[i][0] + acc[i][1];
+            if constexpr (CH == 4) sum += acc[i][2] + acc[i][3];
+            if (parts > 1) *reinterpret_cast<v4f *>(part + ((u * RT + i) * 64 + lane) * 4) = sum;
 #pragma unroll
-            for (int r = 0; r < R; ++r) part[tid * R + r] = acc[r];
-            __syncthreads();
-            // the parts of an output are added in order by one thread per (row, output)
-            for (int idx = tid; idx < R * n2; idx += 256) {
-               const int r = idx / n2, c = idx - r * n2;
-               if (o0 + c >= N) continue;
-               float v = 0.0f;
-               for (int p = 0; p < parts; ++p) v += part[(p * n2 + c) * R + r];
-               finish(r, o0 + c, v);
-            }
+            for (int e = 0; e < 4; ++e)
+               if (parts == 1) finish(i * 16 + kg * 4 + e, t * 16 + c, sum[e] + bias);
          }
-         if (parts > 1) __syncthreads();   // the partial sums are read before the next pass overwrites them
+      }
+      if (parts > 1) {
+         __syncthreads();
+         for (int idx = tid; idx < tiles * RT * 256; idx += NW * 64) {
+            const int t = idx / (RT * 256), o = idx - t * (RT * 256), ln = (o >> 2) & 63, n = t * 16 + (ln & 15);
+            float v = part[t * parts * (RT * 256) + o];
+            for (int p = 1; p < parts; ++p) v += part[(t * parts + p) * (RT * 256) + o];
+            if (a.bias[l] && n < N) v += a.bias[l][n];
+            finish((o >> 8) * 16 + (ln >> 4) * 4 + (o & 3), n, v);
+         }
       }
       __syncthreads();
-      float *t = buf_in; buf_in = buf_out; buf_out = t;
    }
+}
+
+template <int RT, int NW>
+int launch_mlp(sofie_hip_ctx *ctx, MlpArgs &a, size_t lds)
+{
+   SOFIE_LARGE_LDS((k_mlp_f32<RT, NW>));
+   for (int l = 0; l < a.n_layers; ++l) {
+      const int tiles = cdiv(a.dims[l + 1], 16), pieces = cdiv(a.dims[l], 64);
+      for (a.psh[l] = 0; (2 * tiles << a.psh[l]) <= NW && (2 << a.psh[l]) <= pieces;) ++a.psh[l];
+   }
+   hipLaunchKernelGGL((k_mlp_f32<RT, NW>), dim3((unsigned)cdiv(a.M, 16 * RT)), dim3(NW * 64), lds, ctx->stream, a);
+   return check_launch(ctx, "k_mlp_f32");
+}
+
+// A layer as a product of its own (lda and ldy: of x and y for the first and the last, else of the scratch buffer).
+GemmF32Args mlp_layer(const MlpArgs &a, int l, const float *in, int lda, float *out, int ldy)
+{
+   GemmF32Args g{};
+   g.A = in; g.B = a.W[l]; g.bias = a.bias[l]; g.Y = out;
+   g.M = a.M; g.N = a.dims[l + 1]; g.K = a.dims[l];
+   g.lda = lda; g.ldb = g.N; g.ldy = ldy;
+   g.alpha = 1.0f; g.beta = a.bias[l] ? 1.0f : 0.0f;
+   g.bias_kind = a.bias[l] ? SOFIE_BIAS_ROW : SOFIE_BIAS_NONE;
+   g.relu = a.relu[l];
+   return g;
 }
 
 }  // namespace
@@ -1174,11 +1260,9 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    SOFIE_REQUIRE(ctx, n_layers >= 1 && n_layers <= SOFIE_MLP_MAX_LAYERS && dims && W && act, "bad layer list");
    SOFIE_REQUIRE(ctx, M >= 0, "negative dimension");
    MlpArgs a{};
-   int maxd = 0;
    for (int l = 0; l <= n_layers; ++l) {
       SOFIE_REQUIRE(ctx, dims[l] >= 1 && dims[l] <= SOFIE_MLP_MAX_WIDTH, "layer width out of range");
       a.dims[l] = dims[l];
-      if (dims[l] > maxd) maxd = dims[l];
    }
    for (int l = 0; l < n_layers; ++l) {
       SOFIE_REQUIRE(ctx, W[l], "null weight matrix");
@@ -1191,19 +1275,49 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    SOFIE_REQUIRE(ctx, x && y, "null operand");
    SOFIE_REQUIRE(ctx, ldx >= dims[0] && ldy >= dims[n_layers], "leading dimension too small");
    a.x = x; a.y = y; a.n_layers = n_layers; a.M = M; a.ldx = ldx; a.ldy = ldy;
-   a.maxd = (maxd + 3) & ~3;
-   // rows per workgroup: one while that still gives every CU a workgroup, more when there are rows to share the
-   // weight traffic between
+   // a row of a buffer: the widest layer it holds, up to a whole 16, and 4 floats that keep neighbouring rows on other banks
+   for (int l = 0; l < n_layers; ++l) {
+      const int w = ((dims[l] + 15) & ~15) + 4;
+      if (w > a.ld[l & 1]) a.ld[l & 1] = w;
+   }
+   auto lds = [&](int rt, int waves) { return (size_t)(16 * rt * (a.ld[0] + a.ld[1]) + waves * rt * 256) * sizeof(float); };
+   // 16 rows per workgroup while that is at most one workgroup per compute unit; more rows share a pass over the weights above
+   // it, as far as the activations fit (16 rows of the widest layers take 148 KB)
    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-   const int R = M <= 2 * cus ? 1 : M <= 8 * cus ? 4 : 8;
-   const size_t lds = ((size_t)2 * R * a.maxd + (size_t)256 * R) * sizeof(float);
-   const dim3 grid((unsigned)cdiv(M, R)), block(256);
-   // (up to 72 KB of LDS at the widest layers: above the default limit of a launch)
-   SOFIE_LARGE_LDS(k_mlp_f32<1>);
-   SOFIE_LARGE_LDS(k_mlp_f32<4>);
-   SOFIE_LARGE_LDS(k_mlp_f32<8>);
-   if (R == 1) hipLaunchKernelGGL(k_mlp_f32<1>, grid, block, lds, ctx->stream, a);
-   else if (R == 4) hipLaunchKernelGGL(k_mlp_f32<4>, grid, block, lds, ctx->stream, a);
-   else hipLaunchKernelGGL(k_mlp_f32<8>, grid, block, lds, ctx->stream, a);
-   return check_launch(ctx, "k_mlp_f32");
+   const int rt = M > 64 * cus && lds(4, 8) <= (size_t)kMaxDynamicLds ? 4 : M > 16 * cus && lds(2, 8) <= (size_t)kMaxDynamicLds ? 2 : 1;
+   // In one launch every workgroup takes in all weights, 43 bytes per ns and compute unit, which a launch per layer (2.8 us each)
+   // shares out: the shorter estimate, and a single layer is a product in any case. One launch against a launch per layer:
+   // 64-128-64-8 on 256 rows 6.6 / 13.4 us, 256-256-256-16 on 512 rows 18.5 / 12.8, 1024-1024-1024 on 256 rows 199 / 22.5.
+   const int per_cu = cdiv(cdiv(M, 16 * rt), cus);
+   float one = 3.0f + n_layers, each = 0.0f;
+   for (int l = 0; l < n_layers; ++l) {
+      const float weights = (float)((dims[l] + 63) & ~63) * (float)((dims[l + 1] + 15) & ~15);
+      const float reads = weights * 4.0f / 43e3f, mfma = weights * 32.0f * rt / 550e3f;
+      one += per_cu * (reads > mfma ? reads : mfma);
+      each += 2.8f + general_choice(ctx, mlp_layer(a, l, x, dims[l], y, dims[l + 1]), 1, true).us;
+   }
+   int widest = 0;
+   for (int l = 1; l < n_layers; ++l)
+      if (dims[l] > widest) widest = dims[l];
+   // (memory between the layers: without it, as while a graph is recorded on a context that has none, one launch does)
+   const size_t floats = (size_t)M * widest;
+   if ((n_layers == 1 || each < one) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
+      void *ws = nullptr;
+      if (n_layers == 1 || (workspace_has_room(ctx, 2 * floats * sizeof(float)) && workspace(ctx, 2 * floats * sizeof(float), &ws) == SOFIE_HIP_OK)) {
+         const float *in = x;
+         int lda = ldx;
+         for (int l = 0; l < n_layers; ++l) {
+            const bool last = l + 1 == n_layers;
+            float *out = last ? y : static_cast<float *>(ws) + (l & 1) * floats;
+            GemmF32Args g = mlp_layer(a, l, in, lda, out, last ? ldy : dims[l + 1]);
+            if (int rc = launch_general(ctx, g, 1, true)) return rc;
+            in = out;
+            lda = dims[l + 1];
+         }
+         return SOFIE_HIP_OK;
+      }
+   }
+   if (rt == 4) return launch_mlp<4, 8>(ctx, a, lds(4, 8));
+   if (rt == 2) return launch_mlp<2, 8>(ctx, a, lds(2, 8));
+   return launch_mlp<1, 16>(ctx, a, lds(1, 16));
 }

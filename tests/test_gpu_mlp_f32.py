@@ -1,0 +1,93 @@
+"""The one-launch chain of fully connected layers at the edges of its tiles: 16 rows and 16 columns of an output tile, pieces of 64
+rows of a weight matrix, parts of K, and the rows per workgroup (16, 32, 64 by the number of rows and the widths)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sofie_amd import ops as o
+    return o
+
+
+def exact_and_bound(x, Ws, bs, relus):
+    """The float64 result, and a bound on what fp32 sums of K products and a bias in any order are away from it, carried through
+    the layers (ReLU passes an error on or takes it away)."""
+    h, err = x.astype(np.float64), np.zeros_like(x, dtype=np.float64)
+    for W, b, relu in zip(Ws, bs, relus):
+        W, b = W.astype(np.float64), 0.0 if b is None else b.astype(np.float64)
+        mag = (np.abs(h) + err) @ np.abs(W) + np.abs(b)
+        err = err @ np.abs(W) + (W.shape[0] + 1) * 2.0 ** -24 * 1.01 * mag
+        h = h @ W + b
+        if relu:
+            h = np.maximum(h, 0.0)
+    return h, err
+
+
+@pytest.mark.parametrize("M,dims", [(1, [1, 1]), (15, [16, 16]), (17, [17, 15, 1]), (16, [64, 16, 64]), (33, [65, 63, 127, 5]),
+                                    (256, [64, 128, 64, 8]), (5, [1024, 1024, 1024]), (3, [129, 33, 257]), (40, [20] * 17),
+                                    (4097, [60, 33, 9]), (4097, [512, 500, 7]), (4111, [700, 601, 3]), (16385, [50, 129, 66, 8]),
+                                    (16400, [300, 257])])
+def test_mlp_f32_edges(ops, M, dims):
+    r = np.random.default_rng(M + sum(dims))
+    n = len(dims) - 1
+    x = r.standard_normal((M, dims[0])).astype(np.float32)
+    Ws = [(r.standard_normal((a, b)) / np.sqrt(a)).astype(np.float32) for a, b in zip(dims, dims[1:])]
+    bs = [r.standard_normal(b).astype(np.float32) if i % 3 != 1 else None for i, b in enumerate(dims[1:])]
+    relus = [i + 1 < n for i in range(n)]
+    h, err = exact_and_bound(x, Ws, bs, relus)
+    got = ops.mlp_f32(x, Ws, bs, relus).astype(np.float64)
+    assert got.shape == h.shape
+    assert np.all(np.abs(got - h) <= err), (M, dims, np.max(np.abs(got - h) / err))
+
+
+@pytest.mark.parametrize("M,dims", [(5, [1024, 1024, 1024]), (70, [300, 257, 300, 10])])
+def test_mlp_f32_recorded_without_scratch_memory(ops, M, dims):
+    """Wide layers take a launch each, with scratch memory between them; a recording on a context that has none takes one launch
+    for all of them, and every replay gives the same result."""
+    ctx = ops.Context(0, stream=torch.cuda.Stream())
+    r = np.random.default_rng(7)
+    n = len(dims) - 1
+    Ws = [(r.standard_normal((a, b)) / np.sqrt(a)).astype(np.float32) for a, b in zip(dims, dims[1:])]
+    bs = [r.standard_normal(b).astype(np.float32) for b in dims[1:]]
+    x = r.standard_normal((M, dims[0])).astype(np.float32)
+    h, err = exact_and_bound(x, Ws, bs, [True] * n)
+    xd, wd, bd = ctx.dev(x, torch.float32), [ctx.dev(w, torch.float32) for w in Ws], [ctx.dev(b, torch.float32) for b in bs]
+    y = torch.zeros((M, dims[-1]), device="cuda")
+    args = (n, (C.c_int * (n + 1))(*dims), (C.c_void_p * n)(*[t.data_ptr() for t in wd]), (C.c_void_p * n)(*[t.data_ptr() for t in bd]),
+            (C.c_int * n)(*[1] * n), C.c_void_p(xd.data_ptr()), dims[0], C.c_void_p(y.data_ptr()), dims[-1], M)
+    torch.cuda.synchronize()
+    graph = C.c_void_p()
+    ctx.check(ctx.lib.sofie_hip_capture_begin(ctx.h))
+    ctx.check(ctx.lib.sofie_hip_mlp_f32(ctx.h, *args))
+    ctx.check(ctx.lib.sofie_hip_capture_end(ctx.h, C.byref(graph)))
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_graph_launch(ctx.h, graph))
+        ctx.check(ctx.lib.sofie_hip_sync(ctx.h))
+        assert np.all(np.abs(y.cpu().numpy() - h) <= err)
+    ctx.check(ctx.lib.sofie_hip_graph_destroy(ctx.h, graph))
+    y.zero_()
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_mlp_f32(ctx.h, *args))      # the scratch buffer may grow now
+    ctx.check(ctx.lib.sofie_hip_sync(ctx.h))
+    assert np.all(np.abs(y.cpu().numpy() - h) <= err)
+    ctx.close()
+
+
+@pytest.mark.parametrize("N", [5, 17, 100])
+def test_mlp_f32_infinite_weight_stays_in_its_column(ops, N):
+    """Lanes behind a layer's last column hold weights of the next row; nothing of theirs reaches a result."""
+    r = np.random.default_rng(N)
+    x = r.uniform(0.5, 1.0, (20, 37)).astype(np.float32)
+    W = r.standard_normal((37, N)).astype(np.float32)
+    ref = ops.mlp_f32(x, [W], [None], [False])
+    W[:, 0] = np.inf
+    got = ops.mlp_f32(x, [W], [None], [False])
+    assert np.all(got[:, 0] == np.inf) and np.array_equal(got[:, 1:], ref[:, 1:])
