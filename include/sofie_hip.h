@@ -160,9 +160,10 @@ int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, int M, int N,
  * values or NULL (bias itself may be NULL), act[l-1] SOFIE_ACT_NONE or SOFIE_ACT_RELU. Replaces n_layers times the
  * sequence the reference emits per Gemm (ROperator_Gemm.hxx:292-390: bias copy, BLAS::sgemm_, ReLU loop) when every
  * layer is small (widths up to SOFIE_MLP_MAX_WIDTH): the intermediate activations never leave the chip and the
- * chain costs one launch, or one per layer where that is faster (weights of hundreds of kilobytes on few rows). The emitter joins Gemm operators into such a call when each one's output feeds only the
- * next (RModel::FuseGemmChain). Sums are fp32 in an order that depends on the widths and on M alone; the result
- * agrees with the separate calls to the usual 1e-5 relative tolerance, not bit for bit. */
+ * chain costs one launch, or one per layer where that is faster (weights of hundreds of kilobytes on few rows, with
+ * scratch memory between the layers). The emitter joins Gemm operators into such a call when each one's output feeds
+ * only the next (RModel::FuseGemmChain). Sums are fp32 in a fixed order for a given way; the result agrees with the
+ * separate calls to the usual 1e-5 relative tolerance, not bit for bit. */
 #define SOFIE_MLP_MAX_LAYERS 16
 #define SOFIE_MLP_MAX_WIDTH 1024
 int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *dims, const float *const *W,

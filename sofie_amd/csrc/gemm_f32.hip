@@ -519,8 +519,8 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(G
          for (int j = 0; j < NJ; ++j) fetch(c.b[j][h], pb[j], g.ldb, B_KM, k0 + kg * 8 + h * 4);
       }
    };
-   // two sums per output: shorter chains of rounded additions (relative error of two layers of 1024 1.6e-7 -> 1.25e-7) that do not wait
-   // for each other (16 x 300 x 300 4.3 -> 4.0 us)
+   // two sums per output: shorter chains of rounded additions (relative error of two layers of 1024 1.6e-7 -> 1.25e-7) that do
+   // not wait for each other (four layers of 300 on 16 rows 17.8 -> 16.1 us)
    v4f acc[2][MI][NJ];
 #pragma unroll
    for (int i = 0; i < MI; ++i)
@@ -1076,9 +1076,9 @@ extern "C" int sofie_hip_gemm_f32_stacked(sofie_hip_ctx *ctx, int transA, int tr
 // dword: a piece is 64 rows of k x 16 columns, 16 loads. A wavefront's pieces form one list over all column tiles, parts of K and
 // layers, and the loads of the next piece are always under way while one is multiplied: the first weights (and biases) of a layer
 // arrive under the layer before it. Against one thread per output and 1, 4 or 8 rows per workgroup (us): 64-128-64-8 on 256 rows
-// 7.5 -> 6.6, on 16384 27.4 -> 12.5; 20-32-32-1 on 4096 15.5 -> 5.3; 100-487-13 on 8192 34.8 -> 16.7. What bounds it: launch and memory latency for a small network on a few rows; a
-// compute unit's share of the L2 (about 57 B/ns, every workgroup reads all weights) up to 16 rows for each of them; the
-// matrix instructions above.
+// 7.5 -> 6.6, on 16384 27.4 -> 12.5; 20-32-32-1 on 4096 15.5 -> 5.3; 100-487-13 on 8192 34.8 -> 16.7. What bounds it: launch and
+// memory latency for a small network on a few rows; a compute unit's share of the L2 (43 B/ns measured, every workgroup reads all
+// weights) up to 16 rows for each of them; the matrix instructions above.
 // A layer with fewer column tiles than the workgroup has wavefronts deals the pieces of K to parts, added in LDS in order.
 namespace {
 
