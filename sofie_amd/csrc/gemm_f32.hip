@@ -1091,6 +1091,7 @@ struct MlpArgs {
    float *y;
    int n_layers, M, ldx, ldy;
    int ld[2];   // floats per row of the two activation buffers: the inputs of even and of odd layers
+   int maxd;    // k_mlp_f32_row: the widest layer
    int psh[SOFIE_MLP_MAX_LAYERS];   // the pieces of a layer's K are dealt to 1 << psh parts
 };
 
@@ -1205,10 +1206,11 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
          for (int i = 0; i < RT; ++i) {
             v4f sum = acc[i][0] + acc[i][1];
             if constexpr (CH == 4) sum += acc[i][2] + acc[i][3];
+            if (p == 0) sum += bias;
             if (parts > 1) *reinterpret_cast<v4f *>(part + ((u * RT + i) * 64 + lane) * 4) = sum;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-               if (parts == 1) finish(i * 16 + kg * 4 + e, t * 16 + c, sum[e] + bias);
+               if (parts == 1) finish(i * 16 + kg * 4 + e, t * 16 + c, sum[e]);
          }
       }
       if (parts > 1) {
@@ -1217,11 +1219,91 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
             const int t = idx / (RT * 256), o = idx - t * (RT * 256), ln = (o >> 2) & 63, n = t * 16 + (ln & 15);
             float v = part[t * parts * (RT * 256) + o];
             for (int p = 1; p < parts; ++p) v += part[(t * parts + p) * (RT * 256) + o];
-            if (a.bias[l] && n < N) v += a.bias[l][n];
             finish((o >> 8) * 16 + (ln >> 4) * 4 + (o & 3), n, v);
          }
       }
       __syncthreads();
+   }
+}
+
+// One row per workgroup and one output per thread, plain fused multiply-adds: a layer of fewer than 256 outputs is cut into parts of
+// K whose sums meet in LDS. For up to two rows per compute unit, where it is the shorter chain of waits (us, against k_mlp_f32):
+// 144-128-41 on 256 rows 6.1 / 7.2, 147-112-128-32-95-23 10.8 / 12.2, 8-500-9 6.1 / 6.6; not with a layer of 8 outputs or fewer
+// (32 parts and more, added one after the other): 64-128-64-8 7.5 / 6.6, 20-32-32-1 16.0 / 5.3.
+__global__ void __launch_bounds__(256) k_mlp_f32_row(MlpArgs a)
+{
+   constexpr int R = 1;
+   extern __shared__ __align__(16) float s_mlp[];
+   float *buf_in = s_mlp, *buf_out = s_mlp + R * a.maxd;     // activations of the rows, [R][maxd] each
+   float *part = s_mlp + 2 * R * a.maxd;                     // [256][R] partial sums
+   const int tid = threadIdx.x;
+   const int row0 = blockIdx.x * R;
+   {
+      const int K0 = a.dims[0];
+      for (int idx = tid; idx < R * K0; idx += 256) {
+         const int r = idx / K0, k = idx - r * K0;
+         buf_in[r * a.maxd + k] = row0 + r < a.M ? a.x[(size_t)(row0 + r) * a.ldx + k] : 0.0f;
+      }
+   }
+   __syncthreads();
+   for (int l = 0; l < a.n_layers; ++l) {
+      const int K = a.dims[l], N = a.dims[l + 1];
+      const float *__restrict__ W = a.W[l];
+      const bool last = l + 1 == a.n_layers;
+      // columns per pass (a power of two, at most 256) and the parts K is cut into
+      int n2 = 1;
+      while (n2 < N && n2 < 256) n2 <<= 1;
+      const int parts = 256 / n2;
+      const int kc = (K + parts - 1) / parts;
+      const int oc = tid & (n2 - 1), pt = tid / n2;
+      const int k0 = pt * kc, k1 = k0 + kc < K ? k0 + kc : K;
+      for (int o0 = 0; o0 < N; o0 += n2) {
+         const int o = o0 + oc;
+         float acc[R];
+#pragma unroll
+         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+         if (o < N) {
+            const float *w = W + (size_t)k0 * N + o;
+#pragma unroll 8
+            for (int k = k0; k < k1; ++k) {
+               const float wv = *w;
+               w += N;
+#pragma unroll
+               for (int r = 0; r < R; ++r) acc[r] = fmaf(buf_in[r * a.maxd + k], wv, acc[r]);
+            }
+         }
+         auto finish = [&](int r, int oo, float v) {
+            if (a.bias[l]) v += a.bias[l][oo];
+            if (a.relu[l]) v = fmaxf(v, 0.0f);
+            if (last) {
+               if (row0 + r < a.M) a.y[(size_t)(row0 + r) * a.ldy + oo] = v;
+            } else {
+               buf_out[r * a.maxd + oo] = v;
+            }
+         };
+         if (parts == 1) {
+            // 256 columns per pass: every thread holds the complete sums of its column
+            if (o < N) {
+#pragma unroll
+               for (int r = 0; r < R; ++r) finish(r, o, acc[r]);
+            }
+         } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) part[tid * R + r] = acc[r];
+            __syncthreads();
+            // the parts of an output are added in order by one thread per (row, output)
+            for (int idx = tid; idx < R * n2; idx += 256) {
+               const int r = idx / n2, c = idx - r * n2;
+               if (o0 + c >= N) continue;
+               float v = 0.0f;
+               for (int p = 0; p < parts; ++p) v += part[(p * n2 + c) * R + r];
+               finish(r, o0 + c, v);
+            }
+         }
+         if (parts > 1) __syncthreads();   // the partial sums are read before the next pass overwrites them
+      }
+      __syncthreads();
+      float *t = buf_in; buf_in = buf_out; buf_out = t;
    }
 }
 
@@ -1316,6 +1398,15 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
          }
          return SOFIE_HIP_OK;
       }
+   }
+   int narrowest = dims[1];
+   for (int l = 0; l <= n_layers; ++l) {
+      if (dims[l] > a.maxd) a.maxd = dims[l];
+      if (l > 0 && dims[l] < narrowest) narrowest = dims[l];
+   }
+   if (M <= 2 * cus && narrowest > 8) {
+      hipLaunchKernelGGL(k_mlp_f32_row, dim3((unsigned)M), dim3(256), (2 * a.maxd + 256) * sizeof(float), ctx->stream, a);
+      return check_launch(ctx, "k_mlp_f32_row");
    }
    if (rt == 4) return launch_mlp<4, 8>(ctx, a, lds(4, 8));
    if (rt == 2) return launch_mlp<2, 8>(ctx, a, lds(2, 8));
