@@ -19,10 +19,13 @@ def ops():
 # (16, 32, 64, 96, 128) or a wavefront's share; K long enough for slices (few tiles) and a size for each tile shape
 SIZES = [(1, 1, 1), (3, 5, 2), (16, 16, 32), (17, 33, 31), (33, 17, 65), (65, 129, 100), (130, 67, 19), (97, 64, 33), (64, 64, 2049),
          (300, 200, 1025), (10, 1000, 999), (700, 33, 77), (1100, 1000, 130), (2050, 1030, 67)]
+# rows and columns that are no whole fours, K in whole steps of 32: the last step of an operand stored along M or N must not be
+# requested 16 bytes at a time, and it is the last one of a round of stages (two: an odd number of steps, three: 2 mod 3)
+STRADDLING = [(1501, 1001, 1024), (301, 1003, 256), (130, 1002, 160), (2049, 1031, 96), (258, 257, 4096)]
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("M,N,K", SIZES + STRADDLING)
 def test_gemm_f32_of_any_kind(ops, M, N, K, tA, tB):
     """1e-5 of the largest output: sums of fp32 products in another order differ by about sqrt(K) 2^-24 of the terms' root
     mean square times sqrt(K). Leading dimensions equal to the sizes and three floats wider, every bias kind."""
