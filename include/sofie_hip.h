@@ -78,6 +78,11 @@ int sofie_hip_destroy(sofie_hip_ctx *ctx);
  * (sofie_hip_conv2d_f32: [K][channel]; sofie_hip_conv_transpose2d_f32: the gathered sub-kernels of the output phases)
  * in a buffer of its own per tensor and geometry, made by the first call, instead of making it in front of every
  * launch in the scratch buffer; at most SOFIE_HIP_PACKED_MAX tensors, later ones are laid out per call as before.
+ * The promise also covers a B given [K,N] (transB = 0) to sofie_hip_qgemm_s8 or sofie_hip_gemm_fp8 where that call
+ * transposes it in front of its kernel: K and lda multiples of 16 and A on a 16-byte address, N and ldb multiples of 4
+ * and B on a 4-byte address, N * K at most SOFIE_HIP_NOALLOC_SCRATCH_BYTES, and M < 256, N < 256 or M * N < 2^23. The
+ * transposed copy is kept then; a program that computes such a B between calls makes them on a context without the
+ * promise. Every other operand of a product is read as it is at the time of the call.
  * on = 0 frees the copies. Not allowed while a graph is recorded; a new tensor met while a graph is recorded is laid
  * out per call. A generated Session makes the promise in its constructor: its weights are uploaded once and never
  * written again. The reference re-lays a Conv's weights inside every infer call (ROperator_Conv.hxx:342-362); no

@@ -1876,9 +1876,9 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
 }
 
 // Operands the fast kernels cannot read as they lie (rows that are no whole 16-byte chunks, B [K,N]) copied into rows
-// they can (k_copy_operands); a B promised constant is copied by the first call only. *done stays false where there is no
-// scratch memory for it (while a graph is recorded, inside the no-allocation entry point): the caller then takes a kernel
-// that reads the operands where they are.
+// they can (k_copy_operands), by every call: the constant-weights promise does not name these operands, B may be computed
+// between two calls. *done stays false where there is no scratch memory for it (while a graph is recorded, inside the
+// no-allocation entry point): the caller then takes a kernel that reads the operands where they are.
 template <class Mma>
 int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool copy_b, bool *done)
 {
@@ -1896,32 +1896,23 @@ int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool
    const bool padded = copy_a || g.K == c.Kp;
    if (padded) h.K = c.Kp;
    const size_t sums = padded ? nk_scratch_bytes<Mma>(ctx, h) : 0;
-   if (a_bytes + b_bytes + sums >= ((size_t)1 << 40) || !workspace_has_room(ctx, a_bytes + b_bytes + sums)) return SOFIE_HIP_OK;
-   void *bp = nullptr;
-   bool fresh = copy_b;
-   if (copy_b) {
-      const int layout[] = {3, g.K, g.N, g.ldb, transB};
-      if (int rc = packed_weights(ctx, g.B, layout_key(layout, 5), b_bytes, &bp, &fresh)) return rc;
-   }
-   const bool b_in_scratch = copy_b && (bp == ctx->workspace || bp == ctx->static_scratch);
-   h.scratch_used = a_bytes + (b_in_scratch ? b_bytes : 0);
-   void *base = nullptr;
-   if (h.scratch_used + sums)
-      if (int rc = workspace(ctx, h.scratch_used + sums, &base)) return rc;
-   c.Ap = static_cast<unsigned char *>(base);
-   c.Bp = b_in_scratch ? static_cast<unsigned char *>(base) + a_bytes : static_cast<unsigned char *>(bp);
-   if (copy_a) h.A = c.Ap;
-   if (copy_b) h.B = c.Bp;
+   h.scratch_used = a_bytes + b_bytes;
    const size_t blocks_a = copy_a ? ((size_t)g.M * (c.Kp / 16) + 255) / 256 : 0;
    size_t blocks_b = 0;
    c.groups_k = cdiv(c.Kp, 128);
-   if (fresh) blocks_b = c.kn ? (size_t)c.groups_k * cdiv(g.N, 128) : ((size_t)g.N * (c.Kp / 16) + 255) / 256;
-   if (blocks_a + blocks_b >= ((size_t)1 << 31)) return SOFIE_HIP_OK;
+   if (copy_b) blocks_b = c.kn ? (size_t)c.groups_k * cdiv(g.N, 128) : ((size_t)g.N * (c.Kp / 16) + 255) / 256;
+   if (a_bytes + b_bytes + sums >= ((size_t)1 << 40) || blocks_a + blocks_b >= ((size_t)1 << 31) ||
+       !workspace_has_room(ctx, a_bytes + b_bytes + sums))
+      return SOFIE_HIP_OK;
+   void *base = nullptr;
+   if (int rc = workspace(ctx, a_bytes + b_bytes + sums, &base)) return rc;
+   c.Ap = static_cast<unsigned char *>(base);
+   c.Bp = c.Ap + a_bytes;
+   if (copy_a) h.A = c.Ap;
+   if (copy_b) h.B = c.Bp;
    c.blocks_a = (int)blocks_a;
-   if (blocks_a + blocks_b) {
-      hipLaunchKernelGGL(k_copy_operands, dim3((unsigned)(blocks_a + blocks_b)), dim3(256), 0, ctx->stream, c);
-      if (int rc = check_launch(ctx, "k_copy_operands")) return rc;
-   }
+   hipLaunchKernelGGL(k_copy_operands, dim3((unsigned)(blocks_a + blocks_b)), dim3(256), 0, ctx->stream, c);
+   if (int rc = check_launch(ctx, "k_copy_operands")) return rc;
    g = h;
    *done = true;
    return SOFIE_HIP_OK;

@@ -67,7 +67,7 @@ def test_int8_product_of_any_rows(ops, M, N, K, transB):
 @pytest.mark.parametrize("M,N,K", [(2100, 4099, 131), (1025, 8200, 48)])
 def test_large_int8_product_copies_ragged_operands(ops, M, N, K, transB):
     """Products of 128 tiles of 256 x 256 and more: operands copied into whole chunks (A alone where B has them), sampled rows
-    against the oracle; with the constant-weights promise B is copied by the first call only and the results stay."""
+    against the oracle, with and without the constant-weights promise."""
     r = rng(1100 + K)
     A = r.integers(-127, 128, (M, K)).astype(np.int8)
     B = r.integers(-127, 128, (N, K) if transB else (K, N)).astype(np.int8)
@@ -84,6 +84,29 @@ def test_large_int8_product_copies_ragged_operands(ops, M, N, K, transB):
             ctx.sync()
             assert np.array_equal(y.cpu().numpy()[rows], want)
         ctx.close()
+
+
+@pytest.mark.parametrize("M,N,K,transB", [(256, 1000, 1000, False), (40, 70, 333, False), (2100, 4099, 67, False), (2100, 4099, 67, True),
+                                          (2048, 4096, 72, False)])
+def test_operand_changed_between_calls_under_the_promise(ops, M, N, K, transB):
+    """The constant-weights promise does not name the operands of these products: B rewritten in place between two calls (as a
+    tensor that a program computes is) gives the product with what it holds then."""
+    r = rng(1150 + K)
+    A = r.integers(-127, 128, (M, K)).astype(np.int8)
+    rows = np.unique(np.concatenate([np.arange(0, min(M, 16)), r.integers(0, M, 16), [M - 1]]))
+    ctx = ops.Context(0)
+    assert ctx.lib.sofie_hip_constant_weights(ctx.h, 1) == 0
+    a, b = ctx.dev(A), ctx.empty((N, K) if transB else (K, N), torch.int8)
+    for _ in range(3):
+        B = r.integers(-127, 128, (N, K) if transB else (K, N)).astype(np.int8)
+        b.copy_(torch.from_numpy(B))
+        y = ctx.empty((M, N), torch.int32)
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, int(transB), M, N, K, ctx.ptr(a), K, ctx.ptr(b), B.shape[1], None, None, 0, L.ACT_NONE,
+                                             ctx.ptr(y), N, L.OUT_S32))
+        ctx.sync()
+        assert np.array_equal(y.cpu().numpy()[rows], oracle.igemm_s8(A[rows], B, transB))
+    ctx.close()
 
 
 @pytest.mark.parametrize("M,N,K", [(40, 70, 333), (9, 3, 100)])
