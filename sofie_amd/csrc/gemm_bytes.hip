@@ -1678,15 +1678,6 @@ SmallChoice small_choice(const sofie_hip_ctx *ctx, const GemmArgs &g, TileMode m
    return best;
 }
 
-// Scratch memory of a call behind the operand copies it may already hold there (g.scratch_used bytes, reserved together
-// with this by copy_operands, so that the buffer does not move under the copies).
-int call_scratch(sofie_hip_ctx *ctx, const GemmArgs &g, size_t bytes, void **ptr)
-{
-   if (int rc = workspace(ctx, g.scratch_used + bytes, ptr)) return rc;
-   *ptr = static_cast<unsigned char *>(*ptr) + g.scratch_used;
-   return SOFIE_HIP_OK;
-}
-
 // At most 16 rows on a B of some size, in one launch with K cut inside the workgroups only: enough columns for a
 // workgroup of 16 columns on at least every second compute unit, and a K of which everything is requested at once (at
 // 8 x 8192 x 8192 k_gemm_bytes_direct is ahead, 12.7 against 14.5 us; up to K = 4096 the two are equal: 16 x 4096 x 4096 5.9 / 6.1).
@@ -1729,7 +1720,7 @@ int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g)
    const int splits = few_rows_splits(ctx, g, &kslice);
    const int ldp = cdiv(g.N, 4) * 4;
    void *part = nullptr;
-   if (int rc = call_scratch(ctx, g, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
+   if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
    const dim3 grid(blocks, splits);
    hipLaunchKernelGGL(k_qgemm_few_rows, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
    if (int rc = check_launch(ctx, "k_qgemm_few_rows")) return rc;
@@ -1747,7 +1738,7 @@ int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, int splits, int kslice, cons
 {
    const int ldp = cdiv(g.N, 4) * 4;
    void *part = nullptr;
-   if (int rc = call_scratch(ctx, g, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
+   if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
    GemmArgs p = g;
    p.Y = part;
    p.ldy = ldp;
@@ -1815,19 +1806,6 @@ bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, int &splits, int 
 }
 
 bool big_product(const GemmArgs &g) { return (size_t)g.M * g.N >= (size_t)256 * 256 * 128 && g.M >= 256 && g.N >= 256; }
-// Scratch bytes dispatch_nk needs for the partial sums of this product.
-template <class Mma>
-size_t nk_scratch_bytes(const sofie_hip_ctx *ctx, const GemmArgs &g)
-{
-   if constexpr (__is_same(typename Mma::Acc, v16i)) {
-      const size_t sums = (size_t)g.M * (cdiv(g.N, 4) * 4) * sizeof(int);
-      int splits = 1, kslice = 0;
-      if (few_rows_whole(ctx, g)) return 0;
-      if (few_rows_sliced(ctx, g)) return few_rows_splits(ctx, g, &kslice) * sums;
-      if (!big_product(g) && split_k_plan(ctx, g, splits, kslice)) return splits * sums;
-   }
-   return 0;
-}
 
 // Products of fewer than 128 tiles of 256 x 256, A [M,K] and B^T [N,K] with K >= 16 in rows that may start anywhere.
 template <class Mma, int OUT>
@@ -1879,7 +1857,6 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
 // they can (k_copy_operands), by every call: the constant-weights promise does not name these operands, B may be computed
 // between two calls. *done stays false where there is no scratch memory for it (while a graph is recorded, inside the
 // no-allocation entry point): the caller then takes a kernel that reads the operands where they are.
-template <class Mma>
 int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool copy_b, bool *done)
 {
    *done = false;
@@ -1893,19 +1870,14 @@ int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool
    if (copy_a) h.lda = c.Kp;
    if (copy_b) h.ldb = c.Kp;
    // with rows of B alone copied the product keeps its K: the zeros behind it would meet whatever follows A's rows
-   const bool padded = copy_a || g.K == c.Kp;
-   if (padded) h.K = c.Kp;
-   const size_t sums = padded ? nk_scratch_bytes<Mma>(ctx, h) : 0;
-   h.scratch_used = a_bytes + b_bytes;
+   if (copy_a) h.K = c.Kp;
    const size_t blocks_a = copy_a ? ((size_t)g.M * (c.Kp / 16) + 255) / 256 : 0;
    size_t blocks_b = 0;
    c.groups_k = cdiv(c.Kp, 128);
    if (copy_b) blocks_b = c.kn ? (size_t)c.groups_k * cdiv(g.N, 128) : ((size_t)g.N * (c.Kp / 16) + 255) / 256;
-   if (a_bytes + b_bytes + sums >= ((size_t)1 << 40) || blocks_a + blocks_b >= ((size_t)1 << 31) ||
-       !workspace_has_room(ctx, a_bytes + b_bytes + sums))
-      return SOFIE_HIP_OK;
+   if (blocks_a + blocks_b >= ((size_t)1 << 31) || !workspace_has_room(ctx, a_bytes + b_bytes)) return SOFIE_HIP_OK;
    void *base = nullptr;
-   if (int rc = workspace(ctx, a_bytes + b_bytes + sums, &base)) return rc;
+   if (int rc = workspace(ctx, a_bytes + b_bytes, &base)) return rc;
    c.Ap = static_cast<unsigned char *>(base);
    c.Bp = c.Ap + a_bytes;
    if (copy_a) h.A = c.Ap;
@@ -1975,10 +1947,10 @@ int dispatch(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
    // B [K,N] only transposes B.
    bool done = false;
    if (big) {
-      if (int rc = copy_operands<Mma>(ctx, g, transB, !a_ok, !b_nk_ok, &done)) return rc;
+      if (int rc = copy_operands(ctx, g, transB, !a_ok, !b_nk_ok, &done)) return rc;
       if (done) return dispatch_nk<Mma, OUT>(ctx, g);
    } else if (!transB) {
-      if (int rc = copy_operands<Mma>(ctx, g, transB, false, true, &done)) return rc;
+      if (int rc = copy_operands(ctx, g, transB, false, true, &done)) return rc;
       if (done) transB = 1;
    }
    if (transB) return launch_small<Mma, OUT>(ctx, g);

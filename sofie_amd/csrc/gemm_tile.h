@@ -52,7 +52,6 @@ struct GemmArgs {
    // bytes and writes its tile into the slice's own copy of Y, `ysplit` bytes after the previous one
    int splits, kslice;
    long long ysplit;
-   size_t scratch_used;   // bytes at the start of the scratch buffer that hold copies of this call's operands
 };
 
 template <int OUT> struct OutSize { static constexpr int value = 4; };
