@@ -49,6 +49,8 @@ int workspace(sofie_hip_ctx *ctx, size_t bytes, void **ptr);
 // Whether workspace() would hand out this many bytes in the present state of the context (a recording, recorded graphs
 // and the no-allocation entry point do not let the buffer grow).
 bool workspace_has_room(const sofie_hip_ctx *ctx, size_t bytes);
+// The scratch buffer for a caller that has another way without it: null where it has no room, or the device no memory.
+void *workspace_if_room(sofie_hip_ctx *ctx, size_t bytes);
 int check_launch(sofie_hip_ctx *ctx, const char *what);
 // Where a kernel's own layout of the weight tensor `w` goes: the context's scratch buffer (*fresh = true: fill it now), or,
 // when the caller has promised that its weights do not change (sofie_hip_constant_weights), a buffer kept for this

@@ -767,11 +767,6 @@ template <bool A_KM, bool B_KM, int MI, int NJ>
 int launch_tiles_as(sofie_hip_ctx *ctx, GemmF32Args &g, int splits, unsigned nz)
 {
    constexpr int BM = 32 * MI, BN = 32 * NJ, NST = BM + BN > 192 ? 2 : 3;
-   if (splits > 1) {
-      void *ws = nullptr;
-      if (int rc = workspace(ctx, (size_t)splits * g.M * g.N * sizeof(float), &ws)) return rc;
-      g.partial = static_cast<float *>(ws);
-   }
    constexpr auto kern = k_gemm_f32<A_KM, B_KM, MI, NJ>;
    SOFIE_LARGE_LDS(kern);
    hipLaunchKernelGGL(kern, dim3(cdiv(g.M, BM) * cdiv(g.N, BN), splits, nz), dim3(256), NST * (BM + BN) * 32 * 4, ctx->stream, g);
@@ -839,7 +834,12 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
 template <bool A_KM, bool B_KM>
 int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_launch)
 {
-   const GeneralChoice c = general_choice(ctx, g, nz, one_launch);
+   GeneralChoice c = general_choice(ctx, g, nz, one_launch);
+   if (c.splits > 1) {
+      // without memory for the slices' sums (while a graph is recorded or alive) K stays in one piece
+      g.partial = static_cast<float *>(workspace_if_room(ctx, (size_t)c.splits * g.M * g.N * sizeof(float)));
+      if (!g.partial) c = general_choice(ctx, g, nz, true);
+   }
    if (c.direct) {
       switch (c.mi * 10 + c.nj) {
       case 11: return launch_direct_as<A_KM, B_KM, 1, 1>(ctx, g, nz);

@@ -193,6 +193,12 @@ int workspace(sofie_hip_ctx *ctx, size_t bytes, void **ptr)
    return SOFIE_HIP_OK;
 }
 
+void *workspace_if_room(sofie_hip_ctx *ctx, size_t bytes)
+{
+   void *ptr = nullptr;
+   return workspace_has_room(ctx, bytes) && workspace(ctx, bytes, &ptr) == SOFIE_HIP_OK ? ptr : nullptr;
+}
+
 int check_launch(sofie_hip_ctx *ctx, const char *what)
 {
    hipError_t e = hipGetLastError();

@@ -1,5 +1,7 @@
 """fp32 products of any size, alignment and storage: k_gemm_f32_direct (16 and 32 rows and columns per workgroup) and
 k_gemm_f32 (tiles of 32 x 32 to 128 x 128, K in one piece or in slices), every transposition, against float64."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -61,3 +63,39 @@ def test_gemm_f32_slices_give_the_same_bits_twice(ops):
     y = ops.gemm_f32(A, B, beta=0.0)
     assert np.array_equal(y, ops.gemm_f32(A, B, beta=0.0))
     assert np.max(np.abs(y - A.astype(np.float64) @ B.astype(np.float64))) <= 1e-5 * np.max(np.abs(y))
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (1, 1)])
+def test_gemm_f32_without_memory_for_slices(ops, tA, tB):
+    """A long K on few tiles, recorded on a context that has no scratch buffer, and called while the graph is alive, when the
+    buffer may not grow: K stays in one piece. Every replay and the eager call against float64; the slices come back with
+    the graph gone."""
+    M, N, K = 70, 90, 6001
+    r = np.random.default_rng(11)
+    A, B = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    ctx = ops.Context(0, stream=torch.cuda.Stream())
+    a, b = ctx.dev(np.ascontiguousarray(A.T) if tA else A), ctx.dev(np.ascontiguousarray(B.T) if tB else B)
+    y = ctx.empty((M, N), torch.float32)
+
+    def call():
+        return ctx.lib.sofie_hip_gemm_f32(ctx.h, tA, tB, M, N, K, 1.0, ctx.ptr(a), a.shape[1], ctx.ptr(b), b.shape[1], 0.0, None, L.BIAS_NONE,
+                                          ctx.ptr(y), N, L.ACT_NONE)
+
+    def check(run):
+        y.zero_()
+        torch.cuda.synchronize()
+        ctx.check(run())
+        ctx.sync()
+        assert np.max(np.abs(y.cpu().numpy() - ref)) <= 1e-5 * np.max(np.abs(ref))
+    graph = C.c_void_p()
+    ctx.check(ctx.lib.sofie_hip_capture_begin(ctx.h))
+    rc = call()
+    ctx.check(ctx.lib.sofie_hip_capture_end(ctx.h, C.byref(graph)))
+    ctx.check(rc)
+    for _ in range(3):
+        check(lambda: ctx.lib.sofie_hip_graph_launch(ctx.h, graph))
+        check(call)
+    ctx.check(ctx.lib.sofie_hip_graph_destroy(ctx.h, graph))
+    check(call)
+    ctx.close()
