@@ -1846,9 +1846,13 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
    }
    if constexpr (IS_INT) {
       // a long K with few 128 x 128 tiles is cut into slices of K: 128 x 128 tiles write int32 partial sums per slice
-      // (integer sums, so the result does not depend on the cut), a second kernel adds them and converts
+      // (integer sums, so the result does not depend on the cut), a second kernel adds them and converts. At most 16 columns
+      // (the last layer of a classifier) go without slices where there is no memory for their sums: a call that needs
+      // none can always be recorded.
       int splits = 1, kslice = 0;
-      if (split_k_plan(ctx, g, splits, kslice)) return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, splits, kslice);
+      if (split_k_plan(ctx, g, splits, kslice) &&
+          (g.N > 16 || workspace_has_room(ctx, (size_t)splits * g.M * (cdiv(g.N, 4) * 4) * sizeof(int))))
+         return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, splits, kslice);
    }
    return launch_small<Mma, OUT>(ctx, g);
 }

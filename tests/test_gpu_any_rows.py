@@ -109,20 +109,22 @@ def test_operand_changed_between_calls_under_the_promise(ops, M, N, K, transB):
     ctx.close()
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 70, 333), (9, 3, 100)])
-def test_any_rows_without_memory_for_a_copy(ops, M, N, K):
-    """B [K,N] of odd rows in a call that is recorded on a fresh context (no scratch buffer exists and none may be made):
-    a kernel that reads B where it lies runs, and every replay gives the oracle's result."""
+@pytest.mark.parametrize("M,N,K,transB", [(40, 70, 333, False), (9, 3, 100, False), (1024, 16, 16384, True), (300, 5, 32768, True)])
+def test_any_rows_without_memory_for_a_copy(ops, M, N, K, transB):
+    """B [K,N] of odd rows, and a long K on at most 16 columns, in a call that is recorded on a fresh context (no scratch buffer
+    exists and none may be made): a kernel that reads B where it lies and writes no partial sums runs, and every replay
+    gives the oracle's result."""
     r = rng(1200 + K)
     A = r.integers(-127, 128, (M, K)).astype(np.int8)
-    B = r.integers(-127, 128, (K, N)).astype(np.int8)
-    want = oracle.igemm_s8(A, B)
+    B = r.integers(-127, 128, (N, K) if transB else (K, N)).astype(np.int8)
+    want = oracle.igemm_s8(A, B, transB)
     ctx = ops.Context(0, stream=torch.cuda.Stream())
     a, b, y = ctx.dev(A), ctx.dev(B), ctx.empty((M, N), torch.int32)
     torch.cuda.synchronize()
     graph = C.c_void_p()
     ctx.check(ctx.lib.sofie_hip_capture_begin(ctx.h))
-    rc = ctx.lib.sofie_hip_qgemm_s8(ctx.h, 0, M, N, K, ctx.ptr(a), K, ctx.ptr(b), N, None, None, 0, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32)
+    rc = ctx.lib.sofie_hip_qgemm_s8(ctx.h, int(transB), M, N, K, ctx.ptr(a), K, ctx.ptr(b), B.shape[1], None, None, 0, L.ACT_NONE, ctx.ptr(y), N,
+                                    L.OUT_S32)
     ctx.check(ctx.lib.sofie_hip_capture_end(ctx.h, C.byref(graph)))
     ctx.check(rc)
     for _ in range(3):
