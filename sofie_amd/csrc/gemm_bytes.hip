@@ -1684,7 +1684,7 @@ SmallChoice small_choice(const sofie_hip_ctx *ctx, const GemmArgs &g, TileMode m
 bool few_rows_whole(const sofie_hip_ctx *ctx, const GemmArgs &g)
 {
    return g.M <= 16 && cdiv(g.N, 16) * 2 >= ctx->num_cus && g.K >= 512 && g.K <= 4096 && (size_t)g.N * g.K >= ((size_t)2 << 20) &&
-          (size_t)g.N * g.ldb + g.K < (1u << 31);
+          (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);      // 32-bit offsets
 }
 // ... or with K in slices, for fewer columns and a long K: 4 x 64 x 65536 16.7 against 41.5 us in one launch
 // (k_gemm_bytes_direct), 16 x 1024 x 32768 18.3 / 29.9, 8 x 256 x 16384 10.0 / 13.3, 8 x 1024 x 8192 8.5 / 7.9. The second

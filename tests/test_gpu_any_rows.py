@@ -137,6 +137,22 @@ def test_any_rows_without_memory_for_a_copy(ops, M, N, K, transB):
     ctx.close()
 
 
+def test_few_rows_that_lie_far_apart(ops):
+    """16 rows of A 300 MB apart, on a B that the kernel for few rows takes otherwise: its offsets are 32 bits wide."""
+    M, N, K, lda = 16, 2048, 1024, 300_000_000
+    r = rng(1250)
+    A, B = r.integers(-127, 128, (M, K)).astype(np.int8), r.integers(-127, 128, (N, K)).astype(np.int8)
+    ctx = ops.default_context()
+    a = torch.zeros((M - 1) * lda + K, dtype=torch.int8, device=ctx.device)
+    for i in range(M):
+        a[i * lda:i * lda + K] = torch.from_numpy(A[i]).to(ctx.device)
+    b, y = ctx.dev(B), ctx.empty((M, N), torch.int32)
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, 1, M, N, K, ctx.ptr(a), lda, ctx.ptr(b), K, None, None, 0, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32))
+    ctx.sync()
+    assert np.array_equal(y.cpu().numpy(), oracle.igemm_s8(A, B, True))
+
+
 @pytest.mark.parametrize("transB", [True, False])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 16), (17, 33, 129), (33, 47, 50), (256, 500, 1001), (300, 1030, 333), (1, 9, 4001), (2100, 4099, 67)])
 def test_fp8_product_of_any_rows(ops, M, N, K, transB):
