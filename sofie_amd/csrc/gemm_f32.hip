@@ -500,10 +500,10 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 2 : 4) k_gemm_f32_direct(G
    store4(g, finish4(g, s, m, n), m, n);
 }
 
-// One thread per output: matrices whose rows are too long for the 32-bit offsets of the kernels above (2^24 floats).
+// One thread per output: K below the eight where operands would be shared, on rows of millions of floats.
 __global__ void __launch_bounds__(256) k_gemm_f32_plain(GemmF32Args g)
 {
-   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+   const size_t idx = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
    if (idx >= (size_t)g.M * g.N) return;
    if (g.n_lead > 0) select_product(g, (long long)blockIdx.z + g.z0);
    const int m = (int)(idx / g.N), n = (int)(idx % g.N);
@@ -804,23 +804,31 @@ struct TileCost {
 };
 constexpr TileCost kTileCosts[6] = {{1, 1, 0.21f, 0.176f}, {1, 2, 0.36f, 0.275f}, {2, 1, 0.36f, 0.275f}, {2, 2, 0.60f, 0.51f}, {3, 2, 0.85f, 0.78f}, {4, 4, 1.95f, 1.91f}};
 
+// The tiled kernel's offsets are 32 bits wide: a K-step's 32 rows of an operand stored along M or N, a tile's rows of one along
+// K. k_gemm_f32_direct takes any leading dimension. A launch holds fewer than 2^32 threads. us = 1e30: nothing fits (K below
+// four on rows of 2^24 floats).
 GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, bool one_launch)
 {
    GeneralChoice best = {false, 1, 1, 1, 1e30f};
+   auto offsets_fit = [](bool km, int ld, int rows) { return (long long)(km ? 32 : rows) * ld * 4 < (1ll << 31); };
    const int cus = ctx->num_cus;
    auto consider = [&](bool direct, int mi, int nj, int splits, float us) {
       if (us < best.us) best = {direct, mi, nj, splits, us};
    };
-   if (g.K >= 4 && g.bias_kind != SOFIE_BIAS_FULL)
+   auto consider_direct = [&] {
       for (const auto &t : kDirectTiles) {
          const int mi = t[0], nj = t[1], resident = mi * nj == 4 ? 1 : 2;
-         const long long per_cu = ((long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj) * nz + cus - 1) / cus;
+         const long long tiles = (long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj), per_cu = (tiles * nz + cus - 1) / cus;
+         if (tiles >= (1ll << 32) / 512) continue;
          const float mfma = (float)per_cu * 512.0f * mi * nj * g.K / 550e3f, reads = (float)per_cu * 64.0f * (mi + nj) * g.K / 43e3f;
          consider(true, mi, nj, 1, 0.5f + (float)((per_cu + resident - 1) / resident) + (mfma > reads ? mfma : reads));
       }
+   };
+   if (g.K >= 4 && g.bias_kind != SOFIE_BIAS_FULL) consider_direct();
    const int steps = cdiv(g.K, 32);
    for (const auto &t : kTileCosts) {
       const long long tiles = (long long)cdiv(g.M, 32 * t.mi) * cdiv(g.N, 32 * t.nj) * nz;
+      if (!offsets_fit(g.transA, g.lda, 32 * t.mi) || !offsets_fit(!g.transB, g.ldb, 32 * t.nj) || tiles / nz >= (1ll << 32) / 256) continue;
       for (int s = 1; s <= 16; s = s < 4 ? s + 1 : s * 2) {
          if (s > 1 && (one_launch || steps / s < 4 || (size_t)g.M * g.N >= ((size_t)1 << 28))) break;
          const long long per_cu = (tiles * s + cus - 1) / cus;
@@ -828,18 +836,13 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
          consider(false, t.mi, t.nj, s, 2.0f + step * cdiv(steps, s) + (s > 1 ? 5.0f + 8.0f * s * (float)g.M * g.N / 6e6f : 0.0f));
       }
    }
+   if (g.K >= 4 && best.us >= 1e30f) consider_direct();
    return best;
 }
 
 template <bool A_KM, bool B_KM>
-int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_launch)
+int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, const GeneralChoice &c)
 {
-   GeneralChoice c = general_choice(ctx, g, nz, one_launch);
-   if (c.splits > 1) {
-      // without memory for the slices' sums (while a graph is recorded or alive) K stays in one piece
-      g.partial = static_cast<float *>(workspace_if_room(ctx, (size_t)c.splits * g.M * g.N * sizeof(float)));
-      if (!g.partial) c = general_choice(ctx, g, nz, true);
-   }
    if (c.direct) {
       switch (c.mi * 10 + c.nj) {
       case 11: return launch_direct_as<A_KM, B_KM, 1, 1>(ctx, g, nz);
@@ -861,15 +864,21 @@ int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_
 // Operands of any size, alignment and storage; nz products of a stack (one_launch: K is not cut).
 int launch_general(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_launch)
 {
-   // 32-bit offsets: 128 rows of an operand with rows along K, 32 of the others
-   if (g.lda >= (1 << 22) || g.ldb >= (1 << 22)) {
-      const size_t blocks = ((size_t)g.M * g.N + 255) / 256;
-      SOFIE_REQUIRE(ctx, blocks < ((size_t)1 << 31), "output too large");
-      hipLaunchKernelGGL(k_gemm_f32_plain, dim3((unsigned)blocks, 1, nz), dim3(256), 0, ctx->stream, g);
+   GeneralChoice c = general_choice(ctx, g, nz, one_launch);
+   if (c.splits > 1) {
+      // without memory for the slices' sums (while a graph is recorded or alive) K stays in one piece
+      g.partial = static_cast<float *>(workspace_if_room(ctx, (size_t)c.splits * g.M * g.N * sizeof(float)));
+      if (!g.partial) c = general_choice(ctx, g, nz, true);
+   }
+   // a handful of k on rows of millions: a thread per output is the shortest way there (4194305 x 7 x 5: 161 us against
+   // 264 on tiles)
+   if (c.us >= 1e30f || (g.K < 8 && (g.lda >= (1 << 22) || g.ldb >= (1 << 22)))) {
+      const size_t blocks = ((size_t)g.M * g.N + 255) / 256, across = blocks < ((size_t)1 << 23) ? blocks : (size_t)1 << 23;
+      hipLaunchKernelGGL(k_gemm_f32_plain, dim3((unsigned)across, (unsigned)((blocks + across - 1) / across), nz), dim3(256), 0, ctx->stream, g);
       return check_launch(ctx, "k_gemm_f32_plain");
    }
-   if (g.transA) return g.transB ? launch_general_as<true, false>(ctx, g, nz, one_launch) : launch_general_as<true, true>(ctx, g, nz, one_launch);
-   return g.transB ? launch_general_as<false, false>(ctx, g, nz, one_launch) : launch_general_as<false, true>(ctx, g, nz, one_launch);
+   if (g.transA) return g.transB ? launch_general_as<true, false>(ctx, g, nz, c) : launch_general_as<true, true>(ctx, g, nz, c);
+   return g.transB ? launch_general_as<false, false>(ctx, g, nz, c) : launch_general_as<false, true>(ctx, g, nz, c);
 }
 
 }  // namespace

@@ -97,6 +97,10 @@ template <int ROWS> int check_all()
             if ((long long)count * K > 150000 && !(count == 1001 && K == 1024 && pad == 0)) continue;
             bad += check<true, ROWS>(count, K, pad) + check<false, ROWS>(count, K, pad);
          }
+   // the longest rows whose offsets fit 32 bits: a step's 32 rows, or a tile's
+   const int longest_km = (1 << 24) - 1, longest = (int)((1ll << 31) / 4 / ROWS) - 1;
+   for (int K : {31, 33, 64})
+      for (int count : {31, 128, 130}) bad += check<true, ROWS>(count, K, longest_km - count) + check<false, ROWS>(count, K, longest - K);
    return bad;
 }
 

@@ -65,6 +65,44 @@ def test_gemm_f32_slices_give_the_same_bits_twice(ops):
     assert np.max(np.abs(y - A.astype(np.float64) @ B.astype(np.float64))) <= 1e-5 * np.max(np.abs(y))
 
 
+@pytest.mark.parametrize("M,N,K,tA,tB,lda,ldb,kernel",
+                         [(37, 70, 50, 0, 0, 1 << 22, 1 << 22, "k_gemm_f32_direct"), (300, 250, 200, 0, 1, (1 << 22) + 1, (1 << 22) - 3, "k_gemm_f32_direct"),
+                          (4000, 650, 64, 0, 0, 0, (1 << 24) - 1, "k_gemm_f32"), (4000, 650, 64, 1, 0, (1 << 24) + 1, (1 << 22) + 2, "k_gemm_f32_direct"),
+                          (40, 100, 64, 0, 1, (1 << 24) - 1, (1 << 23) + 1, "k_gemm_f32_direct"), (9, 20, 3, 0, 0, 0, (1 << 24) + 3, "k_gemm_f32_plain"),
+                          (21, 9, 7, 1, 1, (1 << 22) + 1, 0, "k_gemm_f32_plain")])
+def test_gemm_f32_rows_far_apart(ops, M, N, K, tA, tB, lda, ldb, kernel):
+    """Leading dimensions around those where a tile's 32-bit offsets end (2^22 to 2^24 floats): the kernel that takes them, a row
+    bias and (not where a thread per output is the rule) a full one, against float64."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    ctx = ops.Context(0)
+
+    def strided(rows, cols, ld):
+        ld = ld or cols
+        buf = torch.empty((rows - 1) * ld + cols, device="cuda")
+        view = torch.as_strided(buf, (rows, cols), (ld, 1))
+        view.copy_(torch.randn(rows, cols, device="cuda", generator=g))
+        return buf, view, ld
+    a, av, lda = strided(*((K, M) if tA else (M, K)), lda)
+    b, bv, ldb = strided(*((N, K) if tB else (K, N)), ldb)
+    ref = (av.t() if tA else av).double().contiguous() @ (bv.t() if tB else bv).double().contiguous()
+    y = ctx.empty((M, N), torch.float32)
+    buf, n = C.create_string_buffer(4096), C.c_int(-1)
+    for kind, bias in ((L.BIAS_ROW, torch.randn(N, device="cuda", generator=g)), (L.BIAS_FULL, torch.randn(M, N, device="cuda", generator=g))):
+        y.zero_()
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+        ctx.check(ctx.lib.sofie_hip_gemm_f32(ctx.h, tA, tB, M, N, K, 1.0, ctx.ptr(a), lda, ctx.ptr(b), ldb, 1.0, ctx.ptr(bias), kind, ctx.ptr(y), N,
+                                             L.ACT_NONE))
+        ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
+        names = [line.split()[0] for line in buf.value.decode().splitlines()]
+        ctx.sync()
+        want = ref + bias.double()
+        assert float((y.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
+        assert kind == L.BIAS_FULL or names[0] == kernel, names
+        assert K < 8 or "k_gemm_f32_plain" not in names, names
+    ctx.close()
+
+
 @pytest.mark.parametrize("tA,tB", [(0, 0), (1, 1)])
 def test_gemm_f32_without_memory_for_slices(ops, tA, tB):
     """A long K on few tiles, recorded on a context that has no scratch buffer, and called while the graph is alive, when the
