@@ -1960,6 +1960,16 @@ int dispatch(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
    if (transB) return launch_small<Mma, OUT>(ctx, g);
    // B [K,N] and no memory for a copy
    if (g.N < 4) return launch_simple<IS_INT, OUT>(ctx, g, transB);
+   if (a_ok && b_kn_ok) {
+      // whole, aligned chunks: 128 x 128 tiles of them, 1.1 us per K-step (1.5 ragged), or 64 x 64 tiles of rows of any bytes, 1.1 us,
+      // each by its rounds over the device (B not to be copied, us: 256x8192x8192 81 / 145, 512x4096x12288 104 / 211, 384x8192x8192
+      // 82 on these and 101 on 128 x 128 tiles of rows of any bytes; 64x8192x8192 97 / 75, 256x2064x16400 180 / 135)
+      const long long cus = ctx->num_cus, rounds = ((long long)cdiv(g.M, 128) * cdiv(g.N, 128) + cus - 1) / cus,
+                      rounds64 = ((long long)cdiv(g.M, 64) * cdiv(g.N, 64) + cus - 1) / cus;
+      const bool whole = g.M % 128 == 0 && g.N % 128 == 0 && g.K % BK == 0;
+      if ((whole ? 1.1f : 1.5f) * rounds <= 1.1f * rounds64) return launch_tiled<Mma, BK, NSETS, 2, 2, OUT, true>(ctx, g);
+      return launch_tiled_impl<Mma, BK, 1, 1, 1, OUT, true, ANY_ROWS>(ctx, g);
+   }
    if (cdiv(g.M, 128) * cdiv(g.N, 128) * 2 <= ctx->num_cus) return launch_tiled_impl<Mma, BK, 1, 1, 1, OUT, true, ANY_ROWS>(ctx, g);
    return launch_tiled_impl<Mma, BK, 1, 2, 2, OUT, true, ANY_ROWS>(ctx, g);
 }

@@ -137,6 +137,21 @@ def test_any_rows_without_memory_for_a_copy(ops, M, N, K, transB):
     ctx.close()
 
 
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 8320), (300, 4100, 8208), (64, 4100, 8208)])
+def test_aligned_product_whose_b_may_not_be_copied(ops, M, N, K):
+    """B [K,N] of more bytes than the entry point that allocates nothing has scratch memory: read where it lies, on 128 x 128
+    tiles (whole and ragged ones) or on 64 x 64 tiles; sampled rows against the oracle."""
+    r = rng(1270 + M)
+    A, B = r.integers(-127, 128, (M, K)).astype(np.int8), r.integers(-127, 128, (K, N)).astype(np.int8)
+    rows = np.unique(np.concatenate([np.arange(0, 4), r.integers(0, M, 6), [M - 1]]))
+    ctx = ops.default_context()
+    a, b, y = ctx.dev(A), ctx.dev(B), ctx.empty((M, N), torch.int32)
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_qgemm_s8_noalloc(ctx.h, 0, M, N, K, ctx.ptr(a), K, ctx.ptr(b), N, None, None, 0, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32))
+    ctx.sync()
+    assert np.array_equal(y.cpu().numpy()[rows], oracle.igemm_s8(A[rows], B))
+
+
 def test_few_rows_that_lie_far_apart(ops):
     """16 rows of A 300 MB apart, on a B that the kernel for few rows takes otherwise: its offsets are 32 bits wide."""
     M, N, K, lda = 16, 2048, 1024, 300_000_000
