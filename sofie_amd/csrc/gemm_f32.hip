@@ -1305,9 +1305,11 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    int widest = 0;
    for (int l = 1; l < n_layers; ++l)
       if (dims[l] > widest) widest = dims[l];
-   // (memory between the layers: without it, as while a graph is recorded on a context that has none, one launch does)
+   // (memory between the layers: without it, as while a graph is recorded on a context that has none, one launch does. One
+   // layer written over its own input stays with the kernels that take in a workgroup's rows before they write them.)
    const size_t floats = (size_t)M * widest;
-   if ((n_layers == 1 || each < one) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
+   const bool in_place = n_layers == 1 && x < y + (size_t)(M - 1) * ldy + dims[1] && y < x + (size_t)(M - 1) * ldx + dims[0];
+   if (((n_layers == 1 && !in_place) || (n_layers > 1 && each < one)) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
       void *ws = nullptr;
       if (n_layers == 1 || (workspace_has_room(ctx, 2 * floats * sizeof(float)) && workspace(ctx, 2 * floats * sizeof(float), &ws) == SOFIE_HIP_OK)) {
          const float *in = x;

@@ -81,6 +81,27 @@ def test_mlp_f32_recorded_without_scratch_memory(ops, M, dims):
     ctx.close()
 
 
+@pytest.mark.parametrize("M,dims", [(3, [40, 40]), (700, [40, 24]), (5000, [300, 300]), (40000, [500, 500]), (300, [64, 100, 64]), (300, [600, 700, 600])])
+def test_mlp_f32_over_its_own_input(ops, M, dims):
+    """y is x: every row is taken in before anything of it is written, whatever the number of layers and the kernel."""
+    r = np.random.default_rng(M)
+    n, ld = len(dims) - 1, dims[0]
+    Ws = [(r.standard_normal((a, b)) / np.sqrt(a)).astype(np.float32) for a, b in zip(dims, dims[1:])]
+    bs = [r.standard_normal(b).astype(np.float32) for b in dims[1:]]
+    x = r.standard_normal((M, ld)).astype(np.float32)
+    h, err = exact_and_bound(x, Ws, bs, [True] * n)
+    ctx = ops.default_context()
+    xd, wd, bd = ctx.dev(x.copy()), [ctx.dev(w) for w in Ws], [ctx.dev(b) for b in bs]
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_mlp_f32(ctx.h, n, (C.c_int * (n + 1))(*dims), (C.c_void_p * n)(*[t.data_ptr() for t in wd]),
+                                        (C.c_void_p * n)(*[t.data_ptr() for t in bd]), (C.c_int * n)(*[1] * n), C.c_void_p(xd.data_ptr()), ld,
+                                        C.c_void_p(xd.data_ptr()), ld, M))
+    ctx.sync()
+    got = xd.cpu().numpy()
+    assert np.all(np.abs(got[:, :dims[-1]] - h) <= err)
+    assert np.array_equal(got[:, dims[-1]:], x[:, dims[-1]:])
+
+
 @pytest.mark.parametrize("N", [5, 17, 100])
 def test_mlp_f32_infinite_weight_stays_in_its_column(ops, N):
     """Lanes behind a layer's last column hold weights of the next row; nothing of theirs reaches a result."""
