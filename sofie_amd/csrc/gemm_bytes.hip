@@ -1859,8 +1859,8 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
 
 // Operands the fast kernels cannot read as they lie (rows that are no whole 16-byte chunks, B [K,N]) copied into rows
 // they can (k_copy_operands), by every call: the constant-weights promise does not name these operands, B may be computed
-// between two calls. *done stays false where there is no scratch memory for it (while a graph is recorded, inside the
-// no-allocation entry point): the caller then takes a kernel that reads the operands where they are.
+// between two calls. *done stays false where there is no memory for it (while a graph is recorded, inside the
+// no-allocation entry point, on a full device): the caller then takes a kernel that reads the operands where they are.
 int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool copy_b, bool *done)
 {
    *done = false;
@@ -1879,10 +1879,9 @@ int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool
    size_t blocks_b = 0;
    c.groups_k = cdiv(c.Kp, 128);
    if (copy_b) blocks_b = c.kn ? (size_t)c.groups_k * cdiv(g.N, 128) : ((size_t)g.N * (c.Kp / 16) + 255) / 256;
-   if (blocks_a + blocks_b >= ((size_t)1 << 31) || !workspace_has_room(ctx, a_bytes + b_bytes)) return SOFIE_HIP_OK;
-   void *base = nullptr;
-   if (int rc = workspace(ctx, a_bytes + b_bytes, &base)) return rc;
-   c.Ap = static_cast<unsigned char *>(base);
+   if (blocks_a + blocks_b >= ((size_t)1 << 24)) return SOFIE_HIP_OK;      // a launch holds fewer than 2^32 threads
+   c.Ap = static_cast<unsigned char *>(workspace_if_room(ctx, a_bytes + b_bytes));
+   if (!c.Ap) return SOFIE_HIP_OK;
    c.Bp = c.Ap + a_bytes;
    if (copy_a) h.A = c.Ap;
    if (copy_b) h.B = c.Bp;

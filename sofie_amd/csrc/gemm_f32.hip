@@ -1310,13 +1310,13 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    const size_t floats = (size_t)M * widest;
    const bool in_place = n_layers == 1 && x < y + (size_t)(M - 1) * ldy + dims[1] && y < x + (size_t)(M - 1) * ldx + dims[0];
    if (((n_layers == 1 && !in_place) || (n_layers > 1 && each < one)) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
-      void *ws = nullptr;
-      if (n_layers == 1 || (workspace_has_room(ctx, 2 * floats * sizeof(float)) && workspace(ctx, 2 * floats * sizeof(float), &ws) == SOFIE_HIP_OK)) {
+      float *const ws = n_layers == 1 ? nullptr : static_cast<float *>(workspace_if_room(ctx, 2 * floats * sizeof(float)));
+      if (n_layers == 1 || ws) {
          const float *in = x;
          int lda = ldx;
          for (int l = 0; l < n_layers; ++l) {
             const bool last = l + 1 == n_layers;
-            float *out = last ? y : static_cast<float *>(ws) + (l & 1) * floats;
+            float *out = last ? y : ws + (l & 1) * floats;
             GemmF32Args g = mlp_layer(a, l, in, lda, out, last ? ldy : dims[l + 1]);
             if (int rc = launch_general(ctx, g, 1, true)) return rc;
             in = out;
