@@ -35,6 +35,7 @@ int qconv_ring_pair(sofie_hip_ctx *ctx, const QConvArgs &g1, const QConvArgs &g2
 // Any channel counts, kernel sizes, strides, pads and layouts, one group, int8 output, optionally with a 2x2 stride-2 max
 // pooling. scratch: qconv_any_scratch(g) bytes of the context's scratch buffer (0: the kernel does not take the problem).
 size_t qconv_any_scratch(const QConvArgs &g);
+bool qconv_any_pays(const sofie_hip_ctx *ctx, const QConvArgs &g);      // against the kernel of one thread per output
 int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *done);
 
 }  // namespace sofie

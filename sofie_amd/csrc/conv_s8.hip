@@ -682,7 +682,8 @@ int run(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch)
 }
 
 // What the kernels of fixed channel multiples leave: k_qconv_any, with a pooling other than 2x2 behind it as a pass of its own.
-// Without memory for its copies (a recording does not let the scratch buffer grow) nothing is launched and *done stays false.
+// Where that is the longer way, or without memory for its copies (a recording does not let the scratch buffer grow), nothing is
+// launched and *done stays false.
 int run_any(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
 {
    *done = false;
@@ -695,7 +696,8 @@ int run_any(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
       need = qconv_any_scratch(h);
       conv_bytes = up256((size_t)g.N * g.OC * g.OH * g.OW);
    }
-   int8_t *const scratch = need ? static_cast<int8_t *>(workspace_if_room(ctx, conv_bytes + need)) : nullptr;
+   if (!need || !qconv_any_pays(ctx, h)) return SOFIE_HIP_OK;
+   int8_t *const scratch = static_cast<int8_t *>(workspace_if_room(ctx, conv_bytes + need));
    if (!scratch) return SOFIE_HIP_OK;
    if (conv_bytes) h.y = scratch;
    if (int rc = qconv_any(ctx, h, scratch + conv_bytes, done)) return rc;

@@ -370,6 +370,21 @@ size_t qconv_any_scratch(const QConvArgs &g)
    return !p.ok ? 0 : up256(p.copy ? p.xbytes : 0) + up256(p.wbytes);
 }
 
+// One thread per output is the shorter way for a layer of a few million multiply-adds on few channels: one launch, where this one
+// has a copy of the weights in front of it (2.7 us, unless it is kept) and one of the input (2.8 us, unless it is read in place),
+// but a chain of K loads. Both estimates are fits to 1714 layers of 1 to 256 channels (9 % rms for the single thread's; what is
+// chosen is more than 10 % behind the other in 10 of them without kept weights and in 6 with them). us, one thread / this without
+// and with kept weights: 8x9x11x11 -> 85, 1x1 4.8 / 10.6 / 8.4; 1x3x32x32 -> 16, 3x3 6.8 / 10.9 / 8.2; 2x12x16x16 -> 20, 3x3
+// 16.1 / 11.0 / 8.3; 1x16x14x14 -> 32, 3x3 in place 20.2 / 8.0 / 5.4.
+bool qconv_any_pays(const sofie_hip_ctx *ctx, const QConvArgs &g)
+{
+   const double K = (double)g.C * g.KH * g.KW, outputs = (double)g.N * g.OC * g.OH * g.OW;
+   // (what is fused here is a pass of its own there)
+   const double passes = (g.pool_kh != 0 ? 4.0 : 0.0) + (g.xf ? 4.0 : 0.0);
+   const double plain = 4.0 + passes + (g.x_nhwc ? 0.076 : 0.111) * K + 0.08 * g.KH * g.KW + 0.26e-6 * outputs * K + 2.9e-6 * outputs;
+   return plain >= 5.0 + (plan(g).copy ? 2.8 : 0.0) + (ctx->constant_weights ? 0.0 : 2.7);
+}
+
 int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *done)
 {
    *done = false;

@@ -38,6 +38,10 @@ SHAPES = [
     (20, 20, 41, 39, 40, 3, 3, (1, 1), (0, 1)),     # large tiles, three channel tiles
     (20, 64, 41, 39, 61, 5, 5, (1, 1), (2, 2)),     # large tiles, more weights than a third of the LDS
     (9, 128, 33, 33, 100, 7, 7, (1, 1), (3, 3)),    # weights of one channel tile are all that fits the LDS
+    # the short sums above once more with the pixels from which on they are this kernel's
+    (3, 16, 90, 70, 17, 1, 1, (1, 1), (0, 0)),      # one K-step that is a quarter full, no bounds
+    (9, 1, 140, 130, 8, 5, 5, (1, 1), (2, 2)),      # one channel
+    (20, 5, 62, 61, 9, 2, 3, (1, 2), (0, 1)),       # K of 30 bytes, uneven kernel, stride and pads
 ]
 
 
@@ -88,6 +92,33 @@ def test_float_input_is_quantized_into_the_copy(ops, shape):
     want = oracle.qconv2d_s8(q, wt, scale, bias, pads, strides, 1, -128, -128, True)
     got = ops.quantize_qconv2d_s8(x, 1.0 / 255.0, -128, wt, scale, bias, pads, strides, 1, -128, True, y_layout=L.LAYOUT_NHWC)
     assert np.array_equal(got.transpose(0, 3, 1, 2), want)
+
+
+@pytest.mark.parametrize("shape,kernels", [((8, 9, 11, 11, 85, 1, 1), ("k_qconv_simple", "k_qconv_simple")),
+                                           ((2, 9, 12, 12, 50, 3, 3), ("k_qconv_any", "k_qconv_any")),
+                                           ((1, 6, 10, 10, 20, 3, 3), ("k_qconv_simple", "k_qconv_any")),
+                                           ((1, 16, 14, 14, 32, 3, 3), ("k_qconv_any", "k_qconv_any"))])
+def test_small_layers_take_the_shorter_way(ops, shape, kernels):
+    """The kernel of a small layer without and with kept weights, at the second call; bytes against the oracle."""
+    n, c, h, w, oc, kh, kw = shape
+    p = kh // 2
+    x, wt, scale, bias = make(np.random.default_rng(c), n, c, h, w, oc, kh, kw, False)
+    want = oracle.qconv2d_s8(x, wt, scale, bias, (p, p), (1, 1), 1, 0, -9, False).transpose(0, 2, 3, 1)
+    for promise, kernel in zip((0, 1), kernels):
+        ctx = ops.Context(0)
+        assert ctx.lib.sofie_hip_constant_weights(ctx.h, promise) == 0
+        xd, wd = ctx.dev(np.ascontiguousarray(x.transpose(0, 2, 3, 1))), ctx.dev(np.ascontiguousarray(wt.transpose(0, 2, 3, 1)))
+        sd, bd, y = ctx.dev(scale), ctx.dev(bias), ctx.empty(want.shape, torch.int8)
+        buf, m = C.create_string_buffer(4096), C.c_int(-1)
+        for _ in range(2):
+            ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+            ctx.check(ctx.lib.sofie_hip_qconv2d_s8(ctx.h, ctx.ptr(xd), L.LAYOUT_NHWC, ctx.ptr(wd), L.LAYOUT_NHWC, ctx.ptr(bd), ctx.ptr(sd), ctx.ptr(y),
+                                                   L.LAYOUT_NHWC, n, c, h, w, oc, kh, kw, p, p, p, p, 1, 1, 1, 0, -9, L.ACT_NONE, L.OUT_S8))
+            ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(m)))
+            ctx.sync()
+            assert np.array_equal(y.cpu().numpy(), want)
+        assert [line.split()[0] for line in buf.value.decode().splitlines()][-1] == kernel
+        ctx.close()
 
 
 @pytest.mark.parametrize("promise", [0, 1])
