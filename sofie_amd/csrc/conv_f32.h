@@ -24,7 +24,8 @@ struct ConvProblem {
    ConvPhase phase[4];
 };
 
-// Runs the problem on k_conv_f32_any (conv_f32_any.hip); *done stays false where it does not take it.
-int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, bool *done);
+// Runs the problem on k_conv_f32_any (conv_f32_any.hip); *done stays false where it does not take it, or where its estimate
+// is above the microseconds of the caller's other way.
+int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done);
 
 }  // namespace sofie

@@ -11,6 +11,8 @@
 // consecutive pixels of one channel plane: coalesced NCHW stores, bias and ReLU fused.
 // Roofline: MFMA fp32; per K-step of 2 each wavefront issues TI*TJ MFMAs (64 cycles each)
 // against TI+TJ+1 ds_read_b32.
+#include <math.h>
+
 #include <type_traits>
 
 #include "common.h"
@@ -656,8 +658,9 @@ ConvProblem problem_of(const ConvArgs &g)
    return p;
 }
 
-// The whole of g (its one phase, or all of them) on k_conv_f32_any; *done stays false where it does not take it.
-int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done)
+// The whole of g (its one phase, or all of them) on k_conv_f32_any; *done stays false where it does not take it, or where
+// other_us is the shorter way.
+int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us = HUGE_VAL)
 {
    ConvProblem p = problem_of(g);
    p.nphases = g.nphases > 1 ? g.nphases : 1;
@@ -666,7 +669,7 @@ int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done)
       const PhaseArgs &f = g.phase[i];
       p.phase[i] = {f.OH, f.OW, f.KH, f.KW, f.ph, f.pw, f.th0, g.ths, f.tw0, g.tws, f.oy0, g.oys, f.ox0, g.oxs};
    }
-   return conv_f32_any(ctx, p, done);
+   return conv_f32_any(ctx, p, other_us, done);
 }
 
 // Whether a layer that k_conv2d_f32_dma takes (full channel blocks of an even K) runs on k_conv_f32_any all the same.
@@ -696,6 +699,19 @@ bool beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
       if (full >= 0.85) return false;
    }
    return madds >= (ctx->constant_weights ? 7.0e6 : 536870912.0);
+}
+
+// Microseconds of k_conv2d_f32 for a sum of one channel block (K below 96), on weights as they lie: fits to 1770 convolutions and to 292
+// transposed ones in phases (12 and 13 % rms). patch: floats of a tile's input cells; tiles, work, cells: tiles, tiles x K and
+// tiles x patch over all phases, the former two by the tile's size. Without kept weights k_conv_f32_any has a launch in front of it,
+// and is the longer way for small layers (us, this / k_conv_f32_any: 1x10x28x28 -> 10, 1x1 5.8 / 7.3; 16x3x32x32 -> 24, 3x3 7.3 / 8.4;
+// 1x256x14x14 in 256 groups 6.6 / 10.9; 1x33x33x33 -> 33, 3x3, K = 297 37 / 10).
+// Up to 14 us only: above, the launch in front matters less than what the estimates are off.
+double staged_us(bool phases, int K, double patch, double tiles, double work, double cells, double outputs)
+{
+   const double us = phases ? 7.0 + 0.058 * K + 0.55e-3 * patch + 0.96e-3 * tiles + 91e-6 * work + 0.72e-6 * cells + 2.7e-6 * outputs
+                            : 4.85 + 0.053 * K + 0.51e-3 * patch + 1.48e-3 * tiles + 53e-6 * work + 0.27e-6 * cells + 1.73e-6 * outputs;
+   return us < 14.0 ? us : HUGE_VAL;
 }
 
 template <int TI, int TJ>
@@ -800,7 +816,11 @@ int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
       }
    }
    if (!g.transposed || (g.uh == 1 && g.uw == 1)) {
-      if (int rc = run_any(ctx, g, done)) return rc;
+      const int K = g.icg * KHW;
+      const double patch = (double)g.icg * g.PH * g.PW, tiles = (double)cdiv(OHW, BP) * g.groups * octiles * g.N;
+      const bool staged = !ctx->constant_weights && !g.transposed && K < 96 && (((K + 1) & ~1) * (LDW + 1.0) + patch) * 4 <= (double)budget;
+      const double other = staged ? staged_us(false, K, patch, tiles * TI * TJ, tiles * TI * TJ * K, tiles * patch, (double)g.N * g.OC * OHW) : HUGE_VAL;
+      if (int rc = run_any(ctx, g, done, other)) return rc;
       if (*done) return SOFIE_HIP_OK;
    }
    int icb = 96 / KHW;
@@ -954,8 +974,26 @@ int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
       lds_max = 0;
       tiles_max = 0;
    }
-   if (int rc = run_any(ctx, g, done)) return rc;
-   if (*done) return SOFIE_HIP_OK;
+   {
+      bool staged = !ctx->constant_weights;
+      int K = 0;
+      double patch = 0.0, all_tiles = 0.0, work = 0.0, cells = 0.0;
+      for (int i = 0; i < g.nphases && staged; ++i) {
+         const PhaseArgs &p = g.phase[i];
+         const int k = g.icg * p.KH * p.KW, rows = (BP + p.OW - 2) / p.OW + 1;
+         const double cut = (double)g.icg * ((rows < p.OH ? rows : p.OH) - 1 + p.KH) * (p.OW - 1 + p.KW);
+         const double tiles = (double)cdiv(p.OH * p.OW, BP) * g.groups * octiles * g.N;
+         staged = k < 96 && (((k + 1) & ~1) * (LDW + 1.0) + cut) * 4 <= (double)budget;
+         if (k > K) K = k;
+         if (cut > patch) patch = cut;
+         all_tiles += tiles * TI * TJ;
+         work += tiles * TI * TJ * k;
+         cells += tiles * cut;
+      }
+      const double other = staged ? staged_us(true, K, patch, all_tiles, work, cells, (double)g.N * g.OC * g.OH0 * g.OW0) : HUGE_VAL;
+      if (int rc = run_any(ctx, g, done, other)) return rc;
+      if (*done) return SOFIE_HIP_OK;
+   }
    for (int i = 0; i < g.nphases; ++i) {
       PhaseArgs &p = g.phase[i];
       const int KHW = p.KH * p.KW;

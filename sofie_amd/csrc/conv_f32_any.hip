@@ -453,7 +453,7 @@ int launch(sofie_hip_ctx *ctx, const AnyArgs &g, int nphases, int mode, int stor
 
 }  // namespace
 
-int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, bool *done)
+int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done)
 {
    *done = false;
    const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
@@ -538,41 +538,11 @@ int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, bool *done)
    if (per > (size_t)p.N) per = (size_t)p.N;
    if (per < 1) return SOFIE_HIP_OK;
 
-   int key[8 + 7 * MAX_PHASES] = {quad ? 4 : 3, p.groups, g.ocg, g.icg, p.KH0, p.KW0, p.transposed, p.nphases};
-   for (int i = 0; i < p.nphases; ++i) {
-      const AnyPhase &q = g.phase[i];
-      const int v[7] = {q.KH, q.KW, q.th0, q.ths, q.tw0, q.tws, q.wofs};
-      for (int e = 0; e < 7; ++e) key[8 + 7 * i + e] = v[e];
-   }
    const int mode = quad ? LOOKED_UP : pad ? TESTED : INSIDE;
-   void *ws = nullptr;
-   bool fresh = true;
-   // (while a graph is recorded the scratch buffer may be too small: the general kernel needs none)
-   if (packed_weights(ctx, p.w, layout_key(key, 8 + 7 * p.nphases), wbytes, &ws, &fresh)) return SOFIE_HIP_OK;
-   if (fresh) {
-      WeightArgs a{};
-      a.w = p.w; a.dst = static_cast<float *>(ws);
-      a.icg = g.icg; a.ocg = g.ocg; a.octiles = g.octiles; a.CB = g.CB; a.nblocks = g.nblocks; a.quad = quad;
-      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.total4 = (int)(wfloats / 4);
-      for (int i = 0; i < MAX_PHASES; ++i) a.phase[i] = g.phase[i];
-      hipLaunchKernelGGL(k_conv_f32_any_weights, dim3((unsigned)cdiv(a.total4, 256)), dim3(256), 0, ctx->stream, a);
-      if (int rc = check_launch(ctx, "k_conv_f32_any_weights")) return rc;
-   }
-   g.w = static_cast<const float *>(ws);
-   g.bias = p.bias;
-   g.H = p.H; g.W = p.W; g.groups = p.groups; g.sh = p.sh; g.sw = p.sw; g.dh = p.dh; g.dw = p.dw; g.relu = p.relu;
-   g.chw4 = (int)image;
-   g.hw4 = p.H * p.W * 4;
-   g.ocplane4 = (int)out_image;
-   g.plane4 = p.OH0 * p.OW0 * 4;
-   g.OW0 = p.OW0;
+   g.groups = p.groups;
    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-   for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
-      const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
-      g.x = p.x + n0 * (image / 4);
-      g.y = p.y + n0 * (out_image / 4);
-      g.xbytes = (unsigned)(n * image);
-      g.ybytes = (unsigned)(n * out_image);
+   // the form for a launch on n images, and the pixels of g for it
+   auto choose = [&](size_t n) {
       // the pixels a form works on: those of each phase, or in a pair as many columns in both
       auto set_pixels = [&](int store) {
          for (int i = 0; i < p.nphases; ++i) {
@@ -612,7 +582,48 @@ int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, bool *done)
             form.time = estimate(g, p.nphases, cus, mode, form);
             if (best.ti == 0 || form.time < best.time) best = form;
          }
-      if (best.ti == 0) return set_error(ctx, SOFIE_HIP_EINVAL, "%s: no form fits", __func__);
+      return best;
+   };
+   Form best = choose(per);
+   if (best.ti == 0) return SOFIE_HIP_OK;
+   // against what the caller has instead (the estimate's unit is a cycle at 2400 MHz; weights that are not kept are laid out in
+   // front of the launch, 3.1 us)
+   if (other_us < 0.95 * (best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1))) return SOFIE_HIP_OK;
+
+   int key[8 + 7 * MAX_PHASES] = {quad ? 4 : 3, p.groups, g.ocg, g.icg, p.KH0, p.KW0, p.transposed, p.nphases};
+   for (int i = 0; i < p.nphases; ++i) {
+      const AnyPhase &q = g.phase[i];
+      const int v[7] = {q.KH, q.KW, q.th0, q.ths, q.tw0, q.tws, q.wofs};
+      for (int e = 0; e < 7; ++e) key[8 + 7 * i + e] = v[e];
+   }
+   void *ws = nullptr;
+   bool fresh = true;
+   // (while a graph is recorded the scratch buffer may be too small: the general kernel needs none)
+   if (packed_weights(ctx, p.w, layout_key(key, 8 + 7 * p.nphases), wbytes, &ws, &fresh)) return SOFIE_HIP_OK;
+   if (fresh) {
+      WeightArgs a{};
+      a.w = p.w; a.dst = static_cast<float *>(ws);
+      a.icg = g.icg; a.ocg = g.ocg; a.octiles = g.octiles; a.CB = g.CB; a.nblocks = g.nblocks; a.quad = quad;
+      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.total4 = (int)(wfloats / 4);
+      for (int i = 0; i < MAX_PHASES; ++i) a.phase[i] = g.phase[i];
+      hipLaunchKernelGGL(k_conv_f32_any_weights, dim3((unsigned)cdiv(a.total4, 256)), dim3(256), 0, ctx->stream, a);
+      if (int rc = check_launch(ctx, "k_conv_f32_any_weights")) return rc;
+   }
+   g.w = static_cast<const float *>(ws);
+   g.bias = p.bias;
+   g.H = p.H; g.W = p.W; g.sh = p.sh; g.sw = p.sw; g.dh = p.dh; g.dw = p.dw; g.relu = p.relu;
+   g.chw4 = (int)image;
+   g.hw4 = p.H * p.W * 4;
+   g.ocplane4 = (int)out_image;
+   g.plane4 = p.OH0 * p.OW0 * 4;
+   g.OW0 = p.OW0;
+   for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
+      const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
+      g.x = p.x + n0 * (image / 4);
+      g.y = p.y + n0 * (out_image / 4);
+      g.xbytes = (unsigned)(n * image);
+      g.ybytes = (unsigned)(n * out_image);
+      if (n != per) best = choose(n);
       g.ks = best.ks;
       g.oblocks = cdiv(g.octiles, best.ti);
       g.dOB = make_fastdiv((unsigned)(g.oblocks * g.groups));

@@ -1,6 +1,8 @@
 """fp32 convolutions of any channels, kernels, strides, dilations, groups and pads, and transposed ones, against float64: every
 form of k_conv_f32_any (16 to 96 channels x 16 or 32 pixels per wavefront, K shared by one to eight wavefronts, the three kinds of
 stores), the tables of all taps, of four channels' taps and of finished offsets, and kernels it leaves to k_conv2d_f32."""
+import ctypes as C
+
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -11,6 +13,15 @@ pytestmark = pytest.mark.gpu
 def ops():
     from sofie_amd import ops as o
     return o
+
+
+@pytest.fixture(scope="module")
+def kept(ops):
+    """A context that keeps its weights in the kernels' layouts: small layers run on k_conv_f32_any there, too."""
+    ctx = ops.Context(0)
+    ctx.check(ctx.lib.sofie_hip_constant_weights(ctx.h, 1))
+    yield ctx
+    ctx.close()
 
 
 # N, C, H, W, OC, KH, KW, stride, (top, left, bottom, right), dilation, groups
@@ -42,20 +53,23 @@ def close(y, ref):
 
 
 @pytest.mark.parametrize("shape", CONV)
-def test_conv_of_any_kind(ops, shape):
+def test_conv_of_any_kind(ops, kept, shape):
     n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
     g = torch.Generator(device="cuda").manual_seed(n * 1000 + c * 10 + oc)
     x = torch.randn(n, c, h, w, device="cuda", generator=g)
     wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * (c // groups * kh * kw) ** -0.5
     bias = torch.randn(oc, device="cuda", generator=g)
     torch.cuda.synchronize()
-    y = ops.conv2d_f32(x, wt, bias, pads, s, d, groups, relu=True)
-    z = ops.conv2d_f32(x, wt, None, pads, s, d, groups)
-    ops.default_context().sync()
     t, l, b, r = pads
     ref = torch.nn.functional.conv2d(torch.nn.functional.pad(x.cpu().double(), (l, r, t, b)), wt.cpu().double(), None, s, 0, d, groups)
-    assert close(z.cpu(), ref)
-    assert close(y.cpu(), (ref + bias.cpu().double()[:, None, None]).clamp(min=0))
+    for ctx in (ops.default_context(), kept):
+        y = ops.conv2d_f32(x, wt, bias, pads, s, d, groups, relu=True, ctx=ctx)
+        z = ops.conv2d_f32(x, wt, None, pads, s, d, groups, ctx=ctx)
+        ctx.sync()
+        assert close(z.cpu(), ref)
+        assert close(y.cpu(), (ref + bias.cpu().double()[:, None, None]).clamp(min=0))
+    kept.check(kept.lib.sofie_hip_constant_weights(kept.h, 0))      # this tensor's memory is freed
+    kept.check(kept.lib.sofie_hip_constant_weights(kept.h, 1))
 
 
 # N, C, H, W, OC/groups, KH, KW, stride, (top, left, bottom, right), dilation, groups, output padding
@@ -73,21 +87,79 @@ CONVT = [
 
 
 @pytest.mark.parametrize("shape", CONVT)
-def test_conv_transpose_of_any_kind(ops, shape):
+def test_conv_transpose_of_any_kind(ops, kept, shape):
     n, c, h, w, ocg, kh, kw, s, pads, d, groups, extra = shape
     g = torch.Generator(device="cuda").manual_seed(n * 1000 + c * 10 + ocg)
     x = torch.randn(n, c, h, w, device="cuda", generator=g)
     wt = torch.randn(c, ocg, kh, kw, device="cuda", generator=g) * (c // groups * kh * kw) ** -0.5
     bias = torch.randn(ocg * groups, device="cuda", generator=g)
     torch.cuda.synchronize()
-    y = ops.conv_transpose2d_f32(x, wt, bias, pads, s, d, groups, extra)
-    ops.default_context().sync()
+    ys = []
+    for ctx in (ops.default_context(), kept):
+        ys.append(ops.conv_transpose2d_f32(x, wt, bias, pads, s, d, groups, extra, ctx=ctx))
+        ctx.sync()
+    kept.check(kept.lib.sofie_hip_constant_weights(kept.h, 0))      # this tensor's memory is freed
+    kept.check(kept.lib.sofie_hip_constant_weights(kept.h, 1))
     full = torch.nn.functional.conv_transpose2d(x.cpu().double(), wt.cpu().double(), bias.cpu().double(), s, 0, 0, groups, d)
     full = torch.nn.functional.pad(full, (0, max(0, extra[1] - pads[3]), 0, max(0, extra[0] - pads[2])))
     if full.shape != (n, ocg * groups, s[0] * (h - 1) + d[0] * (kh - 1) + 1, s[1] * (w - 1) + d[1] * (kw - 1) + 1):
         full[:, :, s[0] * (h - 1) + d[0] * (kh - 1) + 1:] = bias.cpu().double()[:, None, None]
         full[:, :, :, s[1] * (w - 1) + d[1] * (kw - 1) + 1:] = bias.cpu().double()[:, None, None]
-    assert close(y.cpu(), full[:, :, pads[0]:pads[0] + y.shape[2], pads[1]:pads[1] + y.shape[3]])
+    for y in ys:
+        assert close(y.cpu(), full[:, :, pads[0]:pads[0] + y.shape[2], pads[1]:pads[1] + y.shape[3]])
+
+
+# (shape as above), the last kernel of a second call without and with kept weights
+ROUTES = [
+    ((1, 10, 28, 28, 10, 1, 1, 1), ("k_conv2d_f32", "k_conv_f32_any")),              # one launch against a pass over the weights and one
+    ((16, 3, 32, 32, 24, 3, 3, 1), ("k_conv2d_f32", "k_conv_f32_any")),
+    ((1, 256, 14, 14, 256, 3, 3, 256), ("k_conv2d_f32", "k_conv_f32_any")),
+    ((1, 33, 33, 33, 33, 3, 3, 1), ("k_conv_f32_any", "k_conv_f32_any")),            # a long sum: the pass pays
+    ((32, 5, 60, 60, 40, 3, 3, 1), ("k_conv_f32_any", "k_conv_f32_any")),            # many tiles
+]
+
+
+@pytest.mark.parametrize("shape,kernels", ROUTES)
+def test_layers_take_the_shorter_way(ops, shape, kernels):
+    n, c, h, w, oc, kh, kw, groups = shape
+    g = torch.Generator(device="cuda").manual_seed(n * 1000 + c * 10 + oc)
+    x, wt = torch.randn(n, c, h, w, device="cuda", generator=g), torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g)
+    torch.cuda.synchronize()
+    ref = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), None, 1, kh // 2, 1, groups)
+    buf, m = C.create_string_buffer(4096), C.c_int(-1)
+    for promise, kernel in zip((0, 1), kernels):
+        ctx = ops.Context(0)
+        ctx.check(ctx.lib.sofie_hip_constant_weights(ctx.h, promise))
+        for _ in range(2):
+            ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+            y = ops.conv2d_f32(x, wt, None, (kh // 2, kh // 2), (1, 1), (1, 1), groups, ctx=ctx)
+            ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(m)))
+            ctx.sync()
+            assert close(y.cpu(), ref)
+        assert [line.split()[0] for line in buf.value.decode().splitlines()][-1] == kernel
+        ctx.close()
+
+
+@pytest.mark.parametrize("shape,kernels", [((5, 3, 20, 20, 12, 3, 2), ("k_conv2d_f32_phases", "k_conv_f32_any")),
+                                           ((5, 61, 20, 20, 12, 3, 2), ("k_conv_f32_any", "k_conv_f32_any"))])
+def test_transposed_layers_take_the_shorter_way(ops, shape, kernels):
+    n, c, h, w, oc, k, s = shape
+    g = torch.Generator(device="cuda").manual_seed(c)
+    x, wt = torch.randn(n, c, h, w, device="cuda", generator=g), torch.randn(c, oc, k, k, device="cuda", generator=g)
+    torch.cuda.synchronize()
+    ref = torch.nn.functional.conv_transpose2d(x.cpu().double(), wt.cpu().double(), None, s, 1)
+    buf, m = C.create_string_buffer(4096), C.c_int(-1)
+    for promise, kernel in zip((0, 1), kernels):
+        ctx = ops.Context(0)
+        ctx.check(ctx.lib.sofie_hip_constant_weights(ctx.h, promise))
+        for _ in range(2):
+            ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+            y = ops.conv_transpose2d_f32(x, wt, None, (1, 1, 1, 1), (s, s), (1, 1), 1, (0, 0), ctx=ctx)
+            ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(m)))
+            ctx.sync()
+            assert close(y.cpu(), ref)
+        assert [line.split()[0] for line in buf.value.decode().splitlines()][-1] == kernel
+        ctx.close()
 
 
 def test_a_value_outside_the_sum_stays_outside(ops):
