@@ -701,6 +701,37 @@ bool beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
    return madds >= (ctx->constant_weights ? 7.0e6 : 536870912.0);
 }
 
+// Tiles of 64 ti channels x 64 tj pixels for a convolution of one phase, and how many: 128 x 128 per workgroup where that gives
+// every compute unit a tile, else 64 x 128, else 64 x 64: a layer on one image or a few has too few of the large tiles to fill
+// the device (one 56x56 image, 64 -> 128 channels: 25 tiles of 128 x 128, 98 of 64 x 64).
+struct Tiling {
+   int ti, tj;
+   size_t tiles;
+};
+Tiling tiling_of(const sofie_hip_ctx *ctx, const ConvArgs &g)
+{
+   auto tiles = [&](int boc, int bp) { return (size_t)cdiv(g.OH * g.OW, bp) * g.groups * cdiv(g.ocg, boc) * g.N; };
+   if (g.ocg > 64 && tiles(128, 128) >= (size_t)ctx->num_cus) return {2, 2, tiles(128, 128)};
+   if (tiles(64, 128) >= (size_t)ctx->num_cus) return {1, 2, tiles(64, 128)};
+   return {1, 1, tiles(64, 64)};
+}
+
+// Microseconds of k_conv2d_f32_dma for a short sum that is beyond_dma, where the two kernels are close: 3x3 on 6 to 27 input
+// channels, an even number. A fit to 528 layers (12 % rms; without it k_conv_f32_any was more than 5 % behind on 217 of them, with it
+// on 81). us, k_conv2d_f32_dma / k_conv_f32_any: 2x18x155x155 -> 212 41 / 60, 55x16x60x60 -> 64 41 / 50, 10x16x116x116 -> 176
+// 95 / 85, 1x10x101x101 -> 64 13.3 / 8.6.
+double dma_us(const sofie_hip_ctx *ctx, const ConvArgs &g)
+{
+   const double K = 9.0 * g.icg;
+   if (g.nphases > 1 || g.transposed || g.KH != 3 || g.KW != 3 || g.icg % 2 != 0 || g.icg < 6 || K > 250.0 || g.ocg < 40) return HUGE_VAL;
+   const Tiling t = tiling_of(ctx, g);
+   if (t.tiles < (size_t)ctx->num_cus) return HUGE_VAL;      // the other one shares K among wavefronts
+   const double size = t.ti * t.tj, tiles = (double)t.tiles, rounds = ceil(tiles / (3.0 * ctx->num_cus)), idle = 1.0 - tiles / (3.0 * ctx->num_cus);
+   const double us = 4.4 + 0.009 * K + 0.36e-6 * g.N * g.OC * g.OH * g.OW + size * (tiles * (0.72e-3 + 47.7e-6 * K) + rounds * 9.2e-3 * K +
+                     (idle > 0.0 ? idle * 6.4e-3 * K : 0.0));
+   return us + (ctx->constant_weights ? 0.0 : 3.1);
+}
+
 // Microseconds of k_conv2d_f32 for a sum of one channel block (K below 96), on weights as they lie: fits to 1770 convolutions and to 292
 // transposed ones in phases (12 and 13 % rms). patch: floats of a tile's input cells; tiles, work, cells: tiles, tiles x K and
 // tiles x patch over all phases, the former two by the tile's size. Without kept weights k_conv_f32_any has a launch in front of it,
@@ -1045,16 +1076,12 @@ int run_conv(sofie_hip_ctx *ctx, ConvArgs &g)
    bool done = false;
    int rc;
    if (beyond_dma(ctx, g) && (!g.transposed || (g.uh == 1 && g.uw == 1))) {
-      rc = run_any(ctx, g, &done);
+      rc = run_any(ctx, g, &done, dma_us(ctx, g));
       if (rc || done) return rc;
    }
-   // 128 channels x 128 pixels per workgroup where that gives every compute unit a tile, else 64 x 128, else 64 x 64: a
-   // layer on one image or a few has too few of the large tiles to fill the device (one 56x56 image, 64 -> 128
-   // channels: 25 tiles of 128 x 128, 98 of 64 x 64)
-   const size_t pixels = (size_t)g.OH * g.OW;
-   auto tiles = [&](int boc, int bp) { return (size_t)cdiv((int)pixels, bp) * g.groups * cdiv(g.ocg, boc) * g.N; };
-   if (g.ocg > 64 && tiles(128, 128) >= (size_t)ctx->num_cus) rc = launch<2, 2>(ctx, g, &done);
-   else if (tiles(64, 128) >= (size_t)ctx->num_cus) rc = launch<1, 2>(ctx, g, &done);
+   const Tiling t = tiling_of(ctx, g);
+   if (t.ti == 2) rc = launch<2, 2>(ctx, g, &done);
+   else if (t.tj == 2) rc = launch<1, 2>(ctx, g, &done);
    else rc = launch<1, 1>(ctx, g, &done);
    if (rc || done) return rc;
    const size_t total = (size_t)g.N * g.OC * g.OH * g.OW;

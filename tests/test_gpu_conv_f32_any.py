@@ -116,6 +116,9 @@ ROUTES = [
     ((1, 256, 14, 14, 256, 3, 3, 256), ("k_conv2d_f32", "k_conv_f32_any")),
     ((1, 33, 33, 33, 33, 3, 3, 1), ("k_conv_f32_any", "k_conv_f32_any")),            # a long sum: the pass pays
     ((32, 5, 60, 60, 40, 3, 3, 1), ("k_conv_f32_any", "k_conv_f32_any")),            # many tiles
+    # short sums on an even number of channels
+    ((55, 16, 60, 60, 64, 3, 3, 1), ("k_conv2d_f32_dma_pairs", "k_conv2d_f32_dma_pairs")),
+    ((1, 10, 101, 101, 64, 3, 3, 1), ("k_conv_f32_split_finish", "k_conv_f32_any")),
 ]
 
 
