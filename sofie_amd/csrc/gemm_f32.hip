@@ -588,14 +588,6 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
       const int n = c0 + 4 * fr;
       b_off[0] = n < g.N ? (unsigned)((4 * fk * g.ldb + n) * 4) : OUTSIDE;
    }
-   // beta * bias of the lane's four columns, requested ahead of the loop (one load per output behind it was most of a
-   // short product's time: 52 x 1113 x 184 17.6 us)
-   float brow[4];
-#pragma unroll
-   for (int q = 0; q < 4; ++q) {
-      const int n = B_NK ? c0 + T * q + fr : c0 + 4 * fr + q;
-      brow[q] = g.bias_kind == SOFIE_BIAS_ROW && n < g.N ? __fmul_rn(g.beta, g.bias[n]) : 0.0f;
-   }
    struct Chunk {
       v4f a[MT], b[4];
    };
@@ -641,6 +633,16 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
    load(c0_, k0);
    load(c1_, k0 + STEP);
    load(c2_, k0 + 2 * STEP);
+   // the bias of the lane's four columns, requested behind the first operands and ahead of the loop, which does not wait for it (one
+   // load per output behind the loop was most of a short product's time: 52 x 1113 x 184 17.6 us; beta * bias in front of it
+   // cost 0.6 us, also where a slice has no use for it: 2 x 192 x 5828 8.7 against 7.8 us)
+   const bool last = splits == 1;
+   float brow[4];
+#pragma unroll
+   for (int q = 0; q < 4; ++q) {
+      const int n = B_NK ? c0 + T * q + fr : c0 + 4 * fr + q;
+      brow[q] = last && g.bias_kind == SOFIE_BIAS_ROW && n < g.N ? g.bias[n] : 0.0f;
+   }
    for (; k0 < k_end; k0 += STEP) {
       load(c3_, k0 + 3 * STEP);
       multiply(c0_);
@@ -676,14 +678,13 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
    if (wave == 0) add(red);
    if (wave != 0) return;
    // tile (t, q), register r of a lane: row t * T + Tile::row(r, kg); column c0 + 4 j + q (B [K][N]) or c0 + T q + j
-   const bool last = splits == 1;
    float *const out = last ? g.Y : partial + (size_t)blockIdx.y * g.M * g.N;
    const int ldo = last ? g.ldy : g.N;
    const bool vec_out = !last || (g.ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(g.Y) & 15u) == 0);   // rows of whole 16-byte chunks
    auto finish = [&](float v, int q, int m, int n) {
       if (!last) return v;
       v = __fmul_rn(g.alpha, v);
-      if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, brow[q]);
+      if (g.bias_kind == SOFIE_BIAS_ROW) v = __fadd_rn(v, __fmul_rn(g.beta, brow[q]));
       else if (g.bias_kind == SOFIE_BIAS_FULL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n]));
       else if (g.bias_kind == SOFIE_BIAS_COL) v = __fadd_rn(v, __fmul_rn(g.beta, g.bias[m]));
       if (g.relu) v = v > 0.0f ? v : 0.0f;
