@@ -14,6 +14,7 @@
 // 8 XCDs) owns a compact rectangle of output tiles and its L2 sees each operand panel once.
 #include "common.h"
 #include "gemm_tile.h"
+#include "row_chunk.h"
 
 using namespace sofie;
 
@@ -46,49 +47,6 @@ __device__ __forceinline__ void tile_of_workgroup(int pid, int tiles_m, int tile
 //   DWORD_ROWS   ... multiples of 4 with K >= 16
 //   ANY_ROWS     nothing but K >= 16 (and N >= 4 with B [K,N])
 enum TileMode { WHOLE_TILES, CHUNK_ROWS, DWORD_ROWS, ANY_ROWS };
-
-// Bytes k .. k + 15 of a row of K >= 16 bytes that starts at any address, zero behind K. load_row_chunk requests the dwords
-// they lie in (loads from odd addresses are taken apart lane by lane: 256 x 1000 x 1001 in k_gemm_bytes_direct took 13.6 us
-// with them and 5.7 us with K = 1000), row_chunk puts them together once they are there. A chunk that would run over the
-// end of the row is requested so that it ends there and is moved down. No byte outside the aligned dwords of the row is
-// touched. SHIFTS: some row or K is no multiple of four bytes (without it the fifth dword is not requested).
-struct RowChunk {
-   v4i d;
-   int e;
-};
-template <bool SHIFTS>
-__device__ __forceinline__ void load_row_chunk(RowChunk &c, const unsigned char *row, int k, int K)
-{
-   const unsigned char *p = row + (k < K - 16 ? k : K - 16);
-   const int sh = (int)(reinterpret_cast<uintptr_t>(p) & 3u);
-   p -= sh;
-   __builtin_memcpy(&c.d, __builtin_assume_aligned(p, 4), 16);
-   if constexpr (SHIFTS) c.e = *reinterpret_cast<const int *>(p + (sh ? 16 : 12));
-}
-template <bool SHIFTS>
-__device__ __forceinline__ v4i row_chunk(const RowChunk &c, const unsigned char *row, int k, int K)
-{
-   v4i v = c.d;
-   if constexpr (SHIFTS) {
-      const unsigned sh = (unsigned)((reinterpret_cast<uintptr_t>(row) + (k < K - 16 ? k : K - 16)) & 3u);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-         v[i] = (int)__builtin_amdgcn_alignbyte((unsigned)(i < 3 ? c.d[i + 1] : c.e), (unsigned)c.d[i], sh);
-   }
-   return v;
-}
-__device__ __forceinline__ v4i trim_row_chunk(v4i v, int k, int K)
-{
-   const int drop = k - (K - 16);      // bytes in front of k that load_row_chunk had to take along
-   if (drop <= 0) return v;
-   if (drop >= 16) return v4i{0, 0, 0, 0};
-   typedef unsigned long long u64;
-   const u64 lo = ((u64)(unsigned)v[1] << 32) | (unsigned)v[0], hi = ((u64)(unsigned)v[3] << 32) | (unsigned)v[2];
-   const int bits = drop * 8;
-   const u64 rl = bits < 64 ? (lo >> bits) | (hi << (64 - bits)) : hi >> (bits - 64);
-   const u64 rh = bits < 64 ? hi >> bits : 0;
-   return v4i{(int)(unsigned)rl, (int)(unsigned)(rl >> 32), (int)(unsigned)rh, (int)(unsigned)(rh >> 32)};
-}
 
 template <class Mma, int BK, int NSETS, int TI, int TJ, int OUT, bool B_KN, TileMode MODE>
 __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_gemm_bytes(GemmArgs g)

@@ -63,6 +63,36 @@ def test_int8_product_of_any_rows(ops, M, N, K, transB):
             assert np.array_equal(y.cpu().numpy(), want), (offset, pad, out)
 
 
+# a size for each number of rows and columns of k_gemm_bytes_direct (16 x 16, 16 x 32, 32 x 16, 32 x 32)
+@pytest.mark.parametrize("M,N", [(40, 100), (200, 500), (1088, 100), (500, 272)])
+@pytest.mark.parametrize("K", [41, 45, 46, 47, 44, 300, 1001])
+def test_last_chunk_of_every_direct_form(ops, M, N, K):
+    """The bytes behind K are cut off by moving the last chunk of a row down: 1 to 15 bytes, in every form of the kernel and for every kind
+    of output. int8 against the oracle bit by bit; e4m3 within 7 * 2^-13 of the sum of the products' magnitudes (the matrix
+    instruction's own cut) and a rounding to bfloat16 (2^-8)."""
+    r = rng(1050 + M + K)
+    ctx = ops.default_context()
+    A, B = r.integers(-127, 128, (M, K)).astype(np.int8), r.integers(-127, 128, (N, K)).astype(np.int8)
+    scale = (r.uniform(20.0, 60.0, N) / (73.3 * 73.3 * np.sqrt(K))).astype(np.float32)
+    bias = r.integers(-2000, 2000, N).astype(np.int32)
+    a, b, sd, bd = ctx.dev(A), ctx.dev(B), ctx.dev(scale), ctx.dev(bias)
+    for out, want in ((L.OUT_S32, oracle.igemm_s8(A, B, True) + bias[None, :]), (L.OUT_S8, oracle.qgemm_s8(A, B, scale, bias, True, zpy=3)),
+                      (L.OUT_F32, oracle.qgemm_s8_f32out(A, B, scale, bias, True))):
+        y = ctx.empty((M, N), {L.OUT_S32: torch.int32, L.OUT_S8: torch.int8, L.OUT_F32: torch.float32}[out])
+        ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, 1, M, N, K, ctx.ptr(a), K, ctx.ptr(b), K, ctx.ptr(sd), ctx.ptr(bd), 3, L.ACT_NONE, ctx.ptr(y), N, out))
+        ctx.sync()
+        assert np.array_equal(y.cpu().numpy(), want), out
+    fa, fb = (torch.from_numpy(r.standard_normal(s).astype(np.float32)).to(torch.float8_e4m3fn) for s in ((M, K), (N, K)))
+    want, mag = fa.double() @ fb.double().t(), fa.double().abs() @ fb.double().abs().t()
+    ad, bd8 = fa.view(torch.uint8).cuda(), fb.view(torch.uint8).cuda()
+    for out, kind, rounding in ((L.OUT_F32, torch.float32, 0.0), (L.OUT_BF16, torch.bfloat16, 2.0 ** -8)):
+        y = ctx.empty((M, N), kind)
+        torch.cuda.synchronize()
+        ctx.check(ctx.lib.sofie_hip_gemm_fp8(ctx.h, 1, M, N, K, ctx.ptr(ad), K, ctx.ptr(bd8), K, 1.0, 1.0, None, ctx.ptr(y), N, out))
+        ctx.sync()
+        assert bool(((y.cpu().double() - want).abs() <= 7 * 2.0 ** -13 * mag + rounding * want.abs()).all()), out
+
+
 @pytest.mark.parametrize("transB", [True, False])
 @pytest.mark.parametrize("M,N,K", [(2100, 4099, 131), (1025, 8200, 48)])
 def test_large_int8_product_copies_ragged_operands(ops, M, N, K, transB):
