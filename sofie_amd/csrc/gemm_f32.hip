@@ -1256,8 +1256,16 @@ int launch_mlp(sofie_hip_ctx *ctx, MlpArgs &a, size_t lds)
       const int tiles = cdiv(a.dims[l + 1], 16), pieces = cdiv(a.dims[l], 64);
       for (a.psh[l] = 0; (2 * tiles << a.psh[l]) <= NW && (2 << a.psh[l]) <= pieces;) ++a.psh[l];
    }
-   hipLaunchKernelGGL((k_mlp_f32<RT, NW>), dim3((unsigned)cdiv(a.M, 16 * RT)), dim3(NW * 64), lds, ctx->stream, a);
-   return check_launch(ctx, "k_mlp_f32");
+   // a launch holds fewer than 2^32 threads: 67 million rows at 16 per workgroup of 1024
+   const int M = a.M, most = (1 << 21) * 16 * RT;
+   for (int row = 0;; row += most) {
+      a.M = M - row < most ? M - row : most;
+      hipLaunchKernelGGL((k_mlp_f32<RT, NW>), dim3((unsigned)cdiv(a.M, 16 * RT)), dim3(NW * 64), lds, ctx->stream, a);
+      if (int rc = check_launch(ctx, "k_mlp_f32")) return rc;
+      if (M - row <= most) return SOFIE_HIP_OK;
+      a.x += (size_t)most * a.ldx;
+      a.y += (size_t)most * a.ldy;
+   }
 }
 
 // A layer as a product of its own (lda and ldy: of x and y for the first and the last, else of the scratch buffer).

@@ -102,6 +102,26 @@ def test_mlp_f32_over_its_own_input(ops, M, dims):
     assert np.array_equal(got[:, dims[-1]:], x[:, dims[-1]:])
 
 
+def test_mlp_f32_rows_of_several_launches(ops):
+    """2^26 rows of 16 per workgroup of 1024 threads: as many threads as a launch does not hold any more."""
+    M, dims = (1 << 26) + 3, [1, 600, 600, 1]
+    r = np.random.default_rng(26)
+    Ws = [(r.standard_normal((a, b)) / np.sqrt(a)).astype(np.float32) for a, b in zip(dims, dims[1:])]
+    bs = [r.standard_normal(b).astype(np.float32) for b in dims[1:]]
+    ctx = ops.default_context()
+    xd, y = torch.linspace(-3.0, 3.0, M, device="cuda"), torch.zeros(M, device="cuda")
+    wd, bd = [ctx.dev(w) for w in Ws], [ctx.dev(b) for b in bs]
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_mlp_f32(ctx.h, 3, (C.c_int * 4)(*dims), (C.c_void_p * 3)(*[t.data_ptr() for t in wd]),
+                                        (C.c_void_p * 3)(*[t.data_ptr() for t in bd]), (C.c_int * 3)(1, 1, 0), C.c_void_p(xd.data_ptr()), 1,
+                                        C.c_void_p(y.data_ptr()), 1, M))
+    ctx.sync()
+    rows = np.concatenate([np.arange(20), r.integers(0, M, 50), np.arange((1 << 25) - 20, (1 << 25) + 20), np.arange(M - 20, M)])
+    pick = torch.from_numpy(rows).cuda()
+    h, err = exact_and_bound(xd[pick].cpu().numpy()[:, None], Ws, bs, [True, True, False])
+    assert np.all(np.abs(y[pick].cpu().numpy()[:, None] - h) <= err)
+
+
 @pytest.mark.parametrize("N", [5, 17, 100])
 def test_mlp_f32_infinite_weight_stays_in_its_column(ops, N):
     """Lanes behind a layer's last column hold weights of the next row; nothing of theirs reaches a result."""
