@@ -1608,6 +1608,7 @@ TileMode row_mode(const GemmArgs &g)
 //   tiles    0.54 us per K-step of 128 bytes for 128 x 128 tiles, half of that for 64 x 64, 1.3 and 1.6 times as much where
 //            rows are no whole chunks or no whole dwords; 2.5 / 0.8 us for the epilogue; a compute unit takes its tiles in turn
 // Fitted to the times of every kernel on 35 sizes from 1 x 1024 x 1024 to 1166 x 2937 x 2491 and 8001 x 101 x 513 (4.5 to 40 us).
+// A form whose launch would exceed 2^32 threads (64 x 64 tiles: 2^30 rows) is left out.
 struct SmallChoice {
    int tile;          // 64 or 128: k_gemm_bytes on tiles of that size; 0: k_gemm_bytes_direct
    int mi, nj;
@@ -1625,11 +1626,13 @@ SmallChoice small_choice(const sofie_hip_ctx *ctx, const GemmArgs &g, TileMode m
       const int mi = 1 + (i >> 1), nj = 1 + (i & 1);
       const long long wgs = (long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj), per_cu = (wgs + cus - 1) / cus;
       const int resident = mi * nj == 4 ? 1 : 2;
+      if (wgs >= (1ll << 32) / 512) continue;
       consider(0, mi, nj, (float)((per_cu + resident - 1) / resident) + (float)per_cu * 16 * (mi + nj) * g.K / rate);
    }
    const float slower = mode == ANY_ROWS ? 1.6f : mode == DWORD_ROWS ? 1.3f : 1.0f;
    for (int tile = 64; tile <= 128; tile *= 2) {
       const long long wgs = (long long)cdiv(g.M, tile) * cdiv(g.N, tile), per_cu = (wgs + cus - 1) / cus;
+      if (tile == 64 && wgs >= (1ll << 32) / 256) continue;
       const float step = slower * (tile == 64 ? 0.27f : 0.54f), epilogue = tile == 64 ? 0.8f : 2.5f;
       consider(tile, 0, 0, (float)per_cu * (cdiv(g.K, 128) * step + epilogue));
    }

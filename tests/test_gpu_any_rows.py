@@ -139,6 +139,24 @@ def test_operand_changed_between_calls_under_the_promise(ops, M, N, K, transB):
     ctx.close()
 
 
+def test_int8_product_of_a_billion_rows(ops):
+    """2^30 rows: 64 x 64 tiles would be a launch of 2^32 threads."""
+    M, N, K = 1 << 30, 17, 16
+    r = rng(30)
+    ctx = ops.default_context()
+    a = torch.empty((M, K), dtype=torch.int8, device="cuda")
+    a.view(torch.int64).random_()
+    B = r.integers(-127, 128, (N, K)).astype(np.int8)
+    scale = (r.uniform(20.0, 60.0, N) / (73.3 * 73.3 * 4.0)).astype(np.float32)
+    b, sd, y = ctx.dev(B), ctx.dev(scale), torch.zeros((M, N), dtype=torch.int8, device="cuda")
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, 1, M, N, K, ctx.ptr(a), K, ctx.ptr(b), K, ctx.ptr(sd), None, 0, L.ACT_NONE, ctx.ptr(y), N,
+                                         L.OUT_S8))
+    ctx.sync()
+    pick = torch.from_numpy(np.concatenate([np.arange(200), r.integers(0, M, 500), np.arange(M - 200, M)])).cuda()
+    assert np.array_equal(y[pick].cpu().numpy(), oracle.qgemm_s8(a[pick].cpu().numpy(), B, scale, None, True))
+
+
 @pytest.mark.parametrize("M,N,K,transB", [(40, 70, 333, False), (9, 3, 100, False), (1024, 16, 16384, True), (300, 5, 32768, True)])
 def test_any_rows_without_memory_for_a_copy(ops, M, N, K, transB):
     """B [K,N] of odd rows, and a long K on at most 16 columns, in a call that is recorded on a fresh context (no scratch buffer
