@@ -1854,6 +1854,19 @@ int copy_operands(sofie_hip_ctx *ctx, GemmArgs &g, int transB, bool copy_a, bool
    return SOFIE_HIP_OK;
 }
 
+// Whether a product with B [K,N] off whole chunks is shorter with a thread per output than with B copied in front of it: one launch
+// against two, a chain of K loads (of K conversions for e4m3). Both are estimates: 1x1x16 4.1 against 6.6 us, 5x5223x18 4.5 / 8.2,
+// 53x305x23 5.0 / 7.4, 8x64x34 5.7 / 7.6, 56x3657x35 7.3 / 8.7, 8x3x56 7.0 / 7.9; e4m3 64x14x16 5.8 / 7.2, 20x256x18 6.5 / 7.2.
+template <bool IS_INT>
+bool simple_pays(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   GemmArgs copied = g;
+   copied.B = nullptr;
+   copied.ldb = 0;
+   const float plain = 3.1f + (IS_INT ? 0.07f : 0.17f) * g.K + (IS_INT ? 0.22e-6f : 0.4e-6f) * g.M * g.N * g.K;
+   return plain < 6.8f + small_choice(ctx, copied, row_mode(copied)).us;
+}
+
 template <class Mma, int OUT>
 int dispatch(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
 {
@@ -1914,6 +1927,7 @@ int dispatch(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
       if (int rc = copy_operands(ctx, g, transB, !a_ok, !b_nk_ok, &done)) return rc;
       if (done) return dispatch_nk<Mma, OUT>(ctx, g);
    } else if (!transB) {
+      if (simple_pays<IS_INT>(ctx, g)) return launch_simple<IS_INT, OUT>(ctx, g, transB);
       if (int rc = copy_operands(ctx, g, transB, false, true, &done)) return rc;
       if (done) transB = 1;
    }

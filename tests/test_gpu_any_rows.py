@@ -139,6 +139,25 @@ def test_operand_changed_between_calls_under_the_promise(ops, M, N, K, transB):
     ctx.close()
 
 
+@pytest.mark.parametrize("M,N,K,kernels", [(1, 1, 16, ["k_gemm_bytes_simple"]), (53, 305, 23, ["k_gemm_bytes_simple"]),
+                                           (8, 64, 34, ["k_gemm_bytes_simple"]), (40, 70, 333, ["k_copy_operands", "k_gemm_bytes_direct"])])
+def test_short_sums_take_the_shorter_way(ops, M, N, K, kernels):
+    """B [K,N] of odd rows: a thread per output where that is one launch of less time than the copy and the product."""
+    r = rng(1300 + K)
+    A, B = r.integers(-127, 128, (M, K)).astype(np.int8), r.integers(-127, 128, (K, N)).astype(np.int8)
+    ctx = ops.Context(0)
+    (a, pa), (b, pb), y = rows_at(ctx, A, K, 0), rows_at(ctx, B, N, 3), ctx.empty((M, N), torch.int32)
+    buf, n = C.create_string_buffer(4096), C.c_int(-1)
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+    ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, 0, M, N, K, C.c_void_p(pa), K, C.c_void_p(pb), N, None, None, 0, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S32))
+    ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
+    ctx.sync()
+    assert [l.split()[0] for l in buf.value.decode().splitlines()] == kernels
+    assert np.array_equal(y.cpu().numpy(), oracle.igemm_s8(A, B, False))
+    ctx.close()
+
+
 def test_int8_product_of_a_billion_rows(ops):
     """2^30 rows: 64 x 64 tiles would be a launch of 2^32 threads."""
     M, N, K = 1 << 30, 17, 16
