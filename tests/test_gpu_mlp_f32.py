@@ -132,3 +132,37 @@ def test_mlp_f32_infinite_weight_stays_in_its_column(ops, N):
     W[:, 0] = np.inf
     got = ops.mlp_f32(x, [W], [None], [False])
     assert np.all(got[:, 0] == np.inf) and np.array_equal(got[:, 1:], ref[:, 1:])
+
+
+@pytest.mark.parametrize("M,N1,N2,kernel", [(20, 5, 17, "k_mlp_f32"), (600, 17, 5, "k_mlp_f32"), (5000, 100, 30, "k_mlp_f32"),
+                                            (9000, 33, 9, "k_mlp_f32"), (17500, 30, 12, "k_mlp_f32"), (20, 30, 17, "k_mlp_f32_row"),
+                                            (500, 100, 9, "k_mlp_f32_row")])
+def test_mlp_f32_chain_keeps_infinite_weights_in_their_columns(ops, M, N1, N2, kernel):
+    """The same inside the chain kernels, on 16, 32 and 64 rows per workgroup and on one: an infinite column of the last layer (the
+    lanes behind its last column hold it too) is its column of the result, a column of minus infinity of the first layer is
+    a zero behind the ReLU."""
+    r = np.random.default_rng(M + N1)
+    dims = [37, N1, N2]
+    x = r.uniform(0.5, 1.0, (M, 37)).astype(np.float32)
+    Ws = [r.uniform(0.1, 1.0, (a, b)).astype(np.float32) for a, b in zip(dims, dims[1:])]
+    Ws[0][:, 0], Ws[1][0, :] = -1.0, 0.0
+    ctx = ops.default_context()
+
+    def run():
+        buf, n = C.create_string_buffer(4096), C.c_int(-1)
+        assert ctx.lib.sofie_hip_trace_begin(ctx.h) == 0
+        try:
+            y = ops.mlp_f32(x, Ws, [None, None], [True, False])
+        finally:
+            assert ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)) == 0
+        assert [l.split()[0] for l in buf.value.decode().splitlines()] == [kernel]
+        return y
+
+    ref = run()
+    assert np.all(np.isfinite(ref))
+    Ws[1][1:, 0] = np.inf
+    got = run()
+    assert np.all(got[:, 0] == np.inf) and np.array_equal(got[:, 1:], ref[:, 1:])
+    Ws[0][:, 0] = -np.inf
+    again = run()
+    assert np.array_equal(again, got)
