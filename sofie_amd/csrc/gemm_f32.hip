@@ -1319,12 +1319,20 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    // In one launch every workgroup takes in all weights, 43 bytes per ns and compute unit, which a launch per layer (2.8 us each)
    // shares out: the shorter estimate, and a single layer is a product in any case. One launch against a launch per layer:
    // 64-128-64-8 on 256 rows 6.6 / 13.4 us, 256-256-256-16 on 512 rows 18.5 / 12.8, 1024-1024-1024 on 256 rows 199 / 22.5.
+   // (k_mlp_f32_row: the weights as often as a compute unit has rows; 8-16-768 on 8 rows 6.0 us, 6.9 in two launches.)
    const int per_cu = cdiv(cdiv(M, 16 * rt), cus);
-   float one = 3.0f + n_layers, each = 0.0f;
+   int narrowest = dims[1];
+   float one = 3.0f + n_layers, each = 0.0f, row = one;
+   for (int l = 0; l <= n_layers; ++l) {
+      if (dims[l] > a.maxd) a.maxd = dims[l];
+      if (l > 0 && dims[l] < narrowest) narrowest = dims[l];
+   }
+   const bool by_rows = M <= 2 * cus && narrowest > 8;
    for (int l = 0; l < n_layers; ++l) {
       const float weights = (float)((dims[l] + 63) & ~63) * (float)((dims[l + 1] + 15) & ~15);
       const float reads = weights * 4.0f / 43e3f, mfma = weights * 32.0f * rt / 550e3f;
       one += per_cu * (reads > mfma ? reads : mfma);
+      row += cdiv(M, cus) * 4.0f * dims[l] * dims[l + 1] / 43e3f;
       each += 2.8f + general_choice(ctx, mlp_layer(a, l, x, dims[l], y, dims[l + 1]), 1, true).us;
    }
    int widest = 0;
@@ -1334,7 +1342,7 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    // layer written over its own input stays with the kernels that take in a workgroup's rows before they write them.)
    const size_t floats = (size_t)M * widest;
    const bool in_place = n_layers == 1 && x < y + (size_t)(M - 1) * ldy + dims[1] && y < x + (size_t)(M - 1) * ldx + dims[0];
-   if (((n_layers == 1 && !in_place) || (n_layers > 1 && each < one)) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
+   if (((n_layers == 1 && !in_place) || (n_layers > 1 && each < (by_rows && row < one ? row : one))) && ldx < (1 << 22) && floats < ((size_t)1 << 28)) {
       float *const ws = n_layers == 1 ? nullptr : static_cast<float *>(workspace_if_room(ctx, 2 * floats * sizeof(float)));
       if (n_layers == 1 || ws) {
          const float *in = x;
@@ -1350,12 +1358,7 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
          return SOFIE_HIP_OK;
       }
    }
-   int narrowest = dims[1];
-   for (int l = 0; l <= n_layers; ++l) {
-      if (dims[l] > a.maxd) a.maxd = dims[l];
-      if (l > 0 && dims[l] < narrowest) narrowest = dims[l];
-   }
-   if (M <= 2 * cus && narrowest > 8) {
+   if (by_rows) {
       hipLaunchKernelGGL(k_mlp_f32_row, dim3((unsigned)M), dim3(256), (2 * a.maxd + 256) * sizeof(float), ctx->stream, a);
       return check_launch(ctx, "k_mlp_f32_row");
    }

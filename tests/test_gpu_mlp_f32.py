@@ -136,7 +136,7 @@ def test_mlp_f32_infinite_weight_stays_in_its_column(ops, N):
 
 @pytest.mark.parametrize("M,N1,N2,kernel", [(20, 5, 17, "k_mlp_f32"), (600, 17, 5, "k_mlp_f32"), (5000, 100, 30, "k_mlp_f32"),
                                             (9000, 33, 9, "k_mlp_f32"), (17500, 30, 12, "k_mlp_f32"), (20, 30, 17, "k_mlp_f32_row"),
-                                            (500, 100, 9, "k_mlp_f32_row")])
+                                            (500, 100, 9, "k_mlp_f32_row"), (8, 16, 768, "k_mlp_f32_row")])
 def test_mlp_f32_chain_keeps_infinite_weights_in_their_columns(ops, M, N1, N2, kernel):
     """The same inside the chain kernels, on 16, 32 and 64 rows per workgroup and on one: an infinite column of the last layer (the
     lanes behind its last column hold it too) is its column of the result, a column of minus infinity of the first layer is
