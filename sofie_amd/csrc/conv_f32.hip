@@ -737,6 +737,8 @@ double dma_us(const sofie_hip_ctx *ctx, const ConvArgs &g)
 // tiles x patch over all phases, the former two by the tile's size. Without kept weights k_conv_f32_any has a launch in front of it,
 // and is the longer way for small layers (us, this / k_conv_f32_any: 1x10x28x28 -> 10, 1x1 5.8 / 7.3; 16x3x32x32 -> 24, 3x3 7.3 / 8.4;
 // 1x256x14x14 in 256 groups 6.6 / 10.9; 1x33x33x33 -> 33, 3x3, K = 297 37 / 10).
+// A transposed convolution of unit stride, or of a stride whose phases are a launch each, counts as a plain one (5x3x65x64 -> 4, 3x3
+// s3 61.9 / 76.8).
 // Up to 14 us only: above, the launch in front matters less than what the estimates are off.
 double staged_us(bool phases, int K, double patch, double tiles, double work, double cells, double outputs)
 {
@@ -849,7 +851,7 @@ int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
    if (!g.transposed || (g.uh == 1 && g.uw == 1)) {
       const int K = g.icg * KHW;
       const double patch = (double)g.icg * g.PH * g.PW, tiles = (double)cdiv(OHW, BP) * g.groups * octiles * g.N;
-      const bool staged = !ctx->constant_weights && !g.transposed && K < 96 && (((K + 1) & ~1) * (LDW + 1.0) + patch) * 4 <= (double)budget;
+      const bool staged = !ctx->constant_weights && K < 96 && (((K + 1) & ~1) * (LDW + 1.0) + patch) * 4 <= (double)budget;
       const double other = staged ? staged_us(false, K, patch, tiles * TI * TJ, tiles * TI * TJ * K, tiles * patch, (double)g.N * g.OC * OHW) : HUGE_VAL;
       if (int rc = run_any(ctx, g, done, other)) return rc;
       if (*done) return SOFIE_HIP_OK;

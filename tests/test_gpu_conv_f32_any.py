@@ -144,7 +144,9 @@ def test_layers_take_the_shorter_way(ops, shape, kernels):
 
 
 @pytest.mark.parametrize("shape,kernels", [((5, 3, 20, 20, 12, 3, 2), ("k_conv2d_f32_phases", "k_conv_f32_any")),
-                                           ((5, 61, 20, 20, 12, 3, 2), ("k_conv_f32_any", "k_conv_f32_any"))])
+                                           ((5, 61, 20, 20, 12, 3, 2), ("k_conv_f32_any", "k_conv_f32_any")),
+                                           ((9, 1, 39, 16, 16, 4, 1), ("k_conv2d_f32", "k_conv_f32_any")),
+                                           ((5, 3, 65, 64, 4, 3, 3), ("k_conv2d_f32", "k_conv_f32_any"))])
 def test_transposed_layers_take_the_shorter_way(ops, shape, kernels):
     n, c, h, w, oc, k, s = shape
     g = torch.Generator(device="cuda").manual_seed(c)
