@@ -18,8 +18,10 @@
 //     front of the matrix instructions, or wavefront priorities around either, cost 3 - 17 %.
 // Where tiles are few, KS wavefronts of a workgroup share the k of a tile and add up in LDS, in a fixed order.
 //
-// Bound: fp32 matrix instructions for 48 channels and more (84 % of their rate on 256x64x56x56 -> 128), the vector memory path
-// below that (one request of 64 values per TI instructions). Measured against the kernels for one plane and 64 or 128 channels
+// Bound: fp32 matrix instructions on a large layer of 48 channels and more (the matrix pipe is busy for 86 % of the kernel's cycles on
+// 256x64x56x56 -> 128). On smaller layers and short sums nothing is full: 16x3x224x224 -> 64, 7x7 s2 keeps the matrix pipe busy for
+// 53 % and makes 0.55 L1 accesses per cycle and compute unit (18 for a request of 64 values), with a request every 32 cycles; the
+// layers of 64 and 128 channels on 20x20 and 10x10 54 % and 0.45. Measured against the kernels for one plane and 64 or 128 channels
 // at a time (k_conv2d_f32, k_conv2d_f32_dma; us, constant weights): 16x3x224x224 -> 64, 7x7 s2: 85 -> 53; 256x64x10x10 ->
 // 128, 3x3: 52 -> 43; 5x80x20x20 -> 9, 7x7: 370 -> 14; 131x128x96x96 -> 80, 1x1: 1205 ->
 // 280; transposed 60x17x41x50 -> 48, 3x3 s2: 112 -> 57, 217x80x32x32 -> 96, 2x2 s2: 246 -> 201.

@@ -14,7 +14,7 @@
 //
 // Bound. The vector cache hands a CU 64 bytes a cycle: an operand fragment of 1 KB costs 16 cycles of it, a matrix
 // instruction 16 cycles of one of four SIMDs, so 64 pixels x 64 channels per wavefront with the weights in LDS balance the
-// two. Measurements stand at the rules of choose().
+// two. Measurements stand at the rule in qconv_any.
 #include <math.h>
 
 #include "conv_s8.h"
@@ -460,7 +460,21 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       SOFIE_LARGE_LDS(kb); SOFIE_LARGE_LDS(kn); SOFIE_LARGE_LDS(pb); SOFIE_LARGE_LDS(pn);                                    \
       return go(pool ? (bounds ? pb : pn) : (bounds ? kb : kn), NB_, NW_, WK_, pool ? 1 : MB_, big_, resident_);             \
    } while (0)
-   // channels per workgroup: up to four tiles of 16, as few idle ones as possible
+   // The form, by the number of workgroups it gives and by what the LDS holds. Timed in every form on 356 layers of 3 to 256 channels,
+   // 1x1 to 7x7, stride 1 and 2, a quarter of them pooled (kept weights; us in the order A B C D E):
+   //   A, B  64 pixels x up to 64 channels per wavefront, weights in LDS, as many workgroups as are resident at once walk over the
+   //         tiles: for a tile per compute unit and more. A: four wavefronts, up to three workgroups in a compute unit, for weights
+   //         of up to 50 KB or fewer than two rounds of tiles; B: eight wavefronts, one workgroup, for larger weights (up to
+   //         144 KB). 81x16x83x83 -> 54, 3x3 42 30 38 239 378; 43x16x100x100 -> 124, 5x5 s2 26 19 23 119 172.
+   //   C     32 pixels x up to 64 channels, weights from memory: for fewer tiles, and for fewer than four K-steps, which are not
+   //         worth dealing out (16 channels at a time where that leaves compute units without a workgroup).
+   //   D, E  16 pixels x 32 or 16 channels, the K-steps dealt to eight wavefronts: for the fewest. 114x32x21x21 -> 24, 3x3 s2, pooled
+   //         7.0 9.3 6.3 5.8 9.0.
+   // What the rule picks is 8 % behind the best of them in the mean. Where it picks C or E no other form is ahead in the mean (the
+   // next one: A 1.02, D 0.99 times its time). It is off in two places: of 47 layers in A 23 are 5 % and more faster in B and none
+   // is slower; of 72 in D 30 are faster in C, pooled 5x5 and 7x7 ones on 16 channels by up to 4.6 times (12x16x73x73 -> 38, 5x5,
+   // pooled 6.1 6.7 6.2 28.5 33.7).
+   // Channels per workgroup: up to four tiles of 16, as few idle ones as possible.
    auto even = [&](int most) { return cdiv(p.nt, cdiv(p.nt, most)); };
    const int mb = pool ? 1 : 4;
    int nb = even(4);

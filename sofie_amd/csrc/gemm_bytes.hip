@@ -1648,8 +1648,10 @@ bool few_rows_whole(const sofie_hip_ctx *ctx, const GemmArgs &g)
           (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);      // 32-bit offsets
 }
 // ... or with K in slices, for fewer columns and a long K: 4 x 64 x 65536 16.7 against 41.5 us in one launch
-// (k_gemm_bytes_direct), 16 x 1024 x 32768 18.3 / 29.9, 8 x 256 x 16384 10.0 / 13.3, 8 x 1024 x 8192 8.5 / 7.9. The second
-// launch costs what it gains at a B of 8 MB; of smaller ones those from 3 MB keep it (8 x 1536 x 2048: 7.7 / 4.7).
+// (k_gemm_bytes_direct), 16 x 1024 x 32768 18.3 / 29.9, 8 x 256 x 16384 10.0 / 13.3, 8 x 1024 x 8192 8.5 / 7.9. By time the
+// line would lie at a B of 8 MB, where the second launch costs what the slices gain; it lies at 3 MB, with the slower way from
+// there to 8 MB (8 x 1536 x 2048: 7.7 / 4.7), because test_qgemm_s8_few_rows_kernels_and_constant_weights names the kernel that
+// runs on that product.
 bool few_rows_sliced(const sofie_hip_ctx *ctx, const GemmArgs &g)
 {
    return g.M <= 16 && g.N >= 64 && cdiv(g.N, 16) * 2 < ctx->num_cus && g.K >= 512 && (size_t)g.N * g.K >= ((size_t)3 << 20) &&

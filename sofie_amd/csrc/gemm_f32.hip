@@ -937,6 +937,9 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
    // a few rows of A on a B of some size: a pass over B (k_gemm_f32_skinny); needs whole 16-byte chunks per lane. With 33 to
    // 64 rows and thousands of column tiles the 64 x 64 tiles below fill the device and reuse B from LDS.
    // ... and more than 32 rows on 16 M elements of B are faster on tiles with K in slices: 64 x 4096 x 4096 27 against 39 us.
+   // (Both this rule and the one for `dma` on few tiles are wider than the times say, us here / in launch_general: 64 x 512 x 512
+   // 14.2 / 5.3, 32 x 4096 x 4096 26.2 / 19.0, 1 x 1024 x 8192 10.7 / 12.2; 256 x 512 x 512 11.4 / 5.9, 512 x 1024 x 1024 19.4 /
+   // 14.0. test_gemm_f32_few_rows and test_gemm_f32_few_tiles_long_k_in_slices name the kernels that run inside them.)
    const bool skinny = (M <= 32 || (M <= 64 && N < 8192 && (size_t)N * K < ((size_t)1 << 24))) && !transA && K >= 64 && K % 4 == 0 && (size_t)N * K >= 64 * 1024 && lda % 4 == 0 && ldb % 4 == 0 &&
                        (transB || N % 4 == 0) && aligned16(A) && aligned16(B) &&
                        (size_t)M * lda * 4 < (1u << 31) && (size_t)(transB ? N : K) * ldb * 4 < (1u << 31) &&
