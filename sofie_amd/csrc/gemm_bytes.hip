@@ -384,12 +384,6 @@ __global__ void __launch_bounds__(256, (TI * TJ >= 16 || NSETS > 2) ? 1 : 2) k_g
 #ifndef SOFIE_GEMM16
 #define SOFIE_GEMM16 1
 #endif
-// Ablation builds of k_gemm_dma16 for timing only (make ABLATE=...; the results are wrong by construction): bit 0 leaves
-// out the LDS-DMA requests after the first two K-steps, bit 1 the fragment reads after the first K-step, bit 2 the matrix
-// instructions. Waits, barriers, prologue and epilogue stay. 0 in the library that is shipped.
-#ifndef SOFIE_GEMM_ABLATE
-#define SOFIE_GEMM_ABLATE 0
-#endif
 template <int S> struct StageTag { static constexpr int value = S; };
 
 // LDS of k_gemm_dma: [A stage 0][A stage 1][B stage 0][B stage 1], BM*BK (BN*BK) bytes each. Both stages of an
@@ -852,51 +846,36 @@ __global__ void __launch_bounds__(512, 2) k_gemm_dma16(GemmArgs g)
    }
    barrier();
    if (group == 1) barrier();
-   constexpr bool NO_REQUESTS = (SOFIE_GEMM_ABLATE & 1) != 0, NO_READS = (SOFIE_GEMM_ABLATE & 2) != 0,
-                  NO_MFMA = (SOFIE_GEMM_ABLATE & 4) != 0;
    v4i fn[NSUB][NI], fm[NSUB][MJ];          // (inside a K-step in effect: every step rewrites all of them)
    auto kstep = [&](int t, auto tag) {
       constexpr int S = decltype(tag)::value;
-      if (t > 0 && !NO_REQUESTS) request(t + 1, 1 - S);
-      if (!NO_READS || t == 0) {
+      if (t > 0) request(t + 1, 1 - S);
 #pragma unroll
-         for (int sub = 0; sub < NSUB; ++sub) {
+      for (int sub = 0; sub < NSUB; ++sub) {
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-               if constexpr (B_KN) fn[sub][i] = load_frag_kn(i, S * BBYTES, sub);
-               else fn[sub][i] = *reinterpret_cast<const v4i *>(n_base[sub] + i * 16 * BK + S * BBYTES);
-            }
-#pragma unroll
-            for (int j = 0; j < MJ; ++j) fm[sub][j] = *reinterpret_cast<const v4i *>(m_base[sub] + j * 16 * BK + S * ABYTES);
+         for (int i = 0; i < NI; ++i) {
+            if constexpr (B_KN) fn[sub][i] = load_frag_kn(i, S * BBYTES, sub);
+            else fn[sub][i] = *reinterpret_cast<const v4i *>(n_base[sub] + i * 16 * BK + S * BBYTES);
          }
+#pragma unroll
+         for (int j = 0; j < MJ; ++j) fm[sub][j] = *reinterpret_cast<const v4i *>(m_base[sub] + j * 16 * BK + S * ABYTES);
       }
       __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
       if (group == 1) wait_vmcnt<0>();
       barrier();
-      if constexpr (NO_MFMA) {
-         // the fragments stay "used", so that their reads are not removed with the instructions that consume them
+      // The m tiles are walked back and forth (0..3 with an even n tile, 3..0 with an odd one): every instruction
+      // then shares one operand with the one before it. 51.1 - 51.7 against 51.6 - 52.2 us (B [K,N]) and 48.8 - 49.4
+      // against 49.6 - 50.4 us (B [N,K]) at 4096^3, alternating in one process; with the n tiles innermost, or the
+      // two K halves of a tile one behind the other, nothing or a loss.
 #pragma unroll
-         for (int sub = 0; sub < NSUB; ++sub) {
+      for (int sub = 0; sub < NSUB; ++sub)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) asm volatile("" ::"v"(fn[sub][i]));
+         for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int j = 0; j < MJ; ++j) asm volatile("" ::"v"(fm[sub][j]));
-         }
-      } else {
-         // The m tiles are walked back and forth (0..3 with an even n tile, 3..0 with an odd one): every instruction
-         // then shares one operand with the one before it. 51.1 - 51.7 against 51.6 - 52.2 us (B [K,N]) and 48.8 - 49.4
-         // against 49.6 - 50.4 us (B [N,K]) at 4096^3, alternating in one process; with the n tiles innermost, or the
-         // two K halves of a tile one behind the other, nothing or a loss.
-#pragma unroll
-         for (int sub = 0; sub < NSUB; ++sub)
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-#pragma unroll
-               for (int jj = 0; jj < MJ; ++jj) {
-                  const int j = (i & 1) ? MJ - 1 - jj : jj;
-                  acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fn[sub][i], fm[sub][j], acc[i][j], 0, 0, 0);
-               }
-      }
+            for (int jj = 0; jj < MJ; ++jj) {
+               const int j = (i & 1) ? MJ - 1 - jj : jj;
+               acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fn[sub][i], fm[sub][j], acc[i][j], 0, 0, 0);
+            }
       if (group == 0) wait_vmcnt<0>();
       if (group == 0 || t + 1 < nk) barrier();
    };
