@@ -1422,7 +1422,7 @@ template <> struct SelectMma16<MmaF8> { typedef Mma16F8 type; };
 // straight from global memory into the operand registers: lane (row % 16, kq) loads the 32 bytes kq of its rows' chunks
 // (the order of K inside a chunk is the same for A and B and does not matter), no LDS and no barrier on the way. The
 // wavefronts' sums meet in LDS and every four of them leave as one store. A product this small is latency: one trip to
-// memory for everything, where the tiled kernel makes one per K-step (256 x 1000 x 1000: 5.4 us against 12.2 on 128 x 128
+// memory for everything, where the tiled kernel makes one per K-step (256 x 1000 x 1000: 4.6 us against 12.2 on 128 x 128
 // tiles, 6.2 on 64 x 64; 8 x 1001 x 1001: 5.3 / 11.5 / 6.7; 4096 x 16 x 12800: 14 / 70 / 38; all read at up to 43 bytes
 // per ns and compute unit, which is what a larger product pays for its smaller tiles).
 // Two workgroups per compute unit (128 registers) but for 32 x 32 tiles, whose operands would not fit them.
@@ -1509,10 +1509,13 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 1 : 4) k_gemm_bytes_direct
          for (int j = 0; j < NJ; ++j) acc[i][j] = Mma::mma(b[j][0], b[j][1], a[i][0], a[i][1], acc[i][j]);
    };
    constexpr int STEP = 8 * 128;
+   // (chunks behind K are not requested: every lane would ask for the last bytes of its row once more, which took longer than the
+   // product; 512 x 512 x 1024 8.2 us with them, 4.5 without, 64 x 2491 x 1024 8.1 / 4.5, 256 x 1000 x 1000 5.8 / 4.6)
    Chunk c[DEPTH];
    int k0 = wave * 128;
 #pragma unroll
-   for (int d = 0; d < DEPTH; ++d) load(c[d], k0 + d * STEP);
+   for (int d = 0; d < DEPTH; ++d)
+      if (k0 + d * STEP < g.K) load(c[d], k0 + d * STEP);
    while (k0 < g.K) {
 #pragma unroll
       for (int d = 0; d < DEPTH; ++d) {
