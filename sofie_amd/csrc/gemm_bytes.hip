@@ -1245,19 +1245,20 @@ int launch_dma(sofie_hip_ctx *ctx, GemmArgs &g)
    return check_launch(ctx, "k_gemm_dma");
 }
 
-// Few rows of A (M <= 16: a quantised layer on a small batch) with B [N][K]: the product is a pass over B, bound by
-// memory, and 64 x 64 tiles would give a handful of compute units all the work. A wavefront owns all rows of A
-// (v_mfma_i32_16x16x64_i8) and 64 columns; B goes from global memory straight into the matrix
+// Few rows of A (M <= 32: a quantised layer on a small batch) with B [N][K]: the product is a pass over B, bound by
+// memory, and 64 x 64 tiles would give a handful of compute units all the work. A wavefront owns all rows of A (MT
+// tiles of 16 rows, v_mfma_i32_16x16x64_i8) and 64 columns; B goes from global memory straight into the matrix
 // instruction's operand registers: lane (j = lane % 16, kq = lane / 16) loads bytes k0 + 16 kq .. + 15 of column 16 q + j,
 // which is its part of the operand of tile q as it stands, and the same bytes of its row of A. The grid is column
 // blocks x slices of K; a wavefront takes a quarter of the slice in chunks of 64 k (consecutive chunks: the two halves
 // of a 128-byte line are fetched one behind the other), three chunks of loads in flight while one is multiplied; the
 // four wavefronts' sums meet in LDS and go to the scratch buffer [slice][M][ldp] that k_splitk_finish adds up and
 // converts (integer sums: the result is that of the unsplit kernels bit for bit).
+template <int MT>
 __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial, int ldp, int kslice)
 {
    constexpr unsigned OUTSIDE = 0x80000000u;
-   __shared__ int red[2 * 4 * 4 * 64];
+   __shared__ int red[2 * MT * 4 * 4 * 64];
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int j = lane & 15, kq = lane >> 4;
    const int c0 = blockIdx.x * 64;
@@ -1268,23 +1269,28 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
       const_cast<uint8_t *>(g.A), 0, (int)((size_t)(g.M - 1) * g.lda + g.K), 0x00020000);
    const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t *>(g.B), 0, (int)((size_t)(g.N - 1) * g.ldb + g.K), 0x00020000);
-   const unsigned a_off = j < g.M ? (unsigned)(j * g.lda + 16 * kq) : OUTSIDE;
-   unsigned b_off[4];
+   unsigned a_off[MT], b_off[4];
+#pragma unroll
+   for (int t = 0; t < MT; ++t) a_off[t] = t * 16 + j < g.M ? (unsigned)((t * 16 + j) * g.lda + 16 * kq) : OUTSIDE;
 #pragma unroll
    for (int q = 0; q < 4; ++q) b_off[q] = c0 + 16 * q + j < g.N ? (unsigned)((c0 + 16 * q + j) * g.ldb + 16 * kq) : OUTSIDE;
    struct Chunk {
-      v4i a, b[4];
+      v4i a[MT], b[4];
    };
    auto load = [&](Chunk &c, int k0) {
       const bool in = k0 + 16 * kq < k_end;     // K and the wavefronts' shares are multiples of 16: a lane's bytes are in or out together
-      c.a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, in ? a_off : OUTSIDE, k0, 0));
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+         c.a[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ars, in ? a_off[t] : OUTSIDE, k0, 0));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
          c.b[q] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(brs, in ? b_off[q] : OUTSIDE, k0, 0));
    };
-   v4i acc[4];
+   v4i acc[MT][4];
 #pragma unroll
-   for (int q = 0; q < 4; ++q) acc[q] = v4i{0, 0, 0, 0};
+   for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[t][q] = v4i{0, 0, 0, 0};
    Chunk c0_, c1_, c2_, c3_;
    int k0 = k_begin;
    load(c0_, k0);
@@ -1293,7 +1299,9 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    for (; k0 < k_end; k0 += 64) {
       load(c3_, k0 + 192);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(c0_.a, c0_.b[q], acc[q], 0, 0, 0);
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+         for (int t = 0; t < MT; ++t) acc[t][q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(c0_.a[t], c0_.b[q], acc[t][q], 0, 0, 0);
       c0_ = c1_;
       c1_ = c2_;
       c2_ = c3_;
@@ -1301,17 +1309,21 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    // wavefronts 2 and 3 hand their sums to 0 and 1, then 1 hands its to 0
    auto put = [&](int *dst) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-         for (int r = 0; r < 4; ++r) dst[(q * 4 + r) * 64 + lane] = acc[q][r];
+         for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dst[((t * 4 + q) * 4 + r) * 64 + lane] = acc[t][q][r];
    };
    auto add = [&](const int *src) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-         for (int r = 0; r < 4; ++r) acc[q][r] += src[(q * 4 + r) * 64 + lane];
+         for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][q][r] += src[((t * 4 + q) * 4 + r) * 64 + lane];
    };
-   constexpr int BLOCK = 4 * 4 * 64;
+   constexpr int BLOCK = MT * 4 * 4 * 64;
    if (wave >= 2) put(red + (wave - 2) * BLOCK);
    __syncthreads();
    if (wave < 2) add(red + wave * BLOCK);
@@ -1320,18 +1332,20 @@ __global__ void __launch_bounds__(256) k_qgemm_few_rows(GemmArgs g, int *partial
    __syncthreads();
    if (wave != 0) return;
    add(red);
-   // tile q, register r: row kq * 4 + r, column c0 + 16 q + j
+   // tile (t, q), register r: row t * 16 + kq * 4 + r, column c0 + 16 q + j
    int *const out = partial + (size_t)blockIdx.y * g.M * ldp;
 #pragma unroll
-   for (int r = 0; r < 4; ++r) {
-      const int m = kq * 4 + r;
-      if (m >= g.M) continue;
+   for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-         const int n = c0 + 16 * q + j;
-         if (n < ldp) out[(size_t)m * ldp + n] = acc[q][r];
+      for (int r = 0; r < 4; ++r) {
+         const int m = t * 16 + kq * 4 + r;
+         if (m >= g.M) continue;
+#pragma unroll
+         for (int q = 0; q < 4; ++q) {
+            const int n = c0 + 16 * q + j;
+            if (n < ldp) out[(size_t)m * ldp + n] = acc[t][q][r];
+         }
       }
-   }
 }
 
 // The same pass over B for at most 16 rows of A and enough columns to give every compute unit a workgroup without
@@ -1623,21 +1637,25 @@ SmallChoice small_choice(const sofie_hip_ctx *ctx, const GemmArgs &g, TileMode m
 
 // At most 16 rows on a B of some size, in one launch with K cut inside the workgroups only: enough columns for a
 // workgroup of 16 columns on at least every second compute unit, and a K of which everything is requested at once (at
-// 8 x 8192 x 8192 k_gemm_bytes_direct is ahead, 12.7 against 14.5 us; up to K = 4096 the two are equal: 16 x 4096 x 4096 5.9 / 6.1).
-bool few_rows_whole(const sofie_hip_ctx *ctx, const GemmArgs &g)
+// 8 x 8192 x 8192 k_gemm_bytes_direct is ahead, 12.7 against 14.5 us; up to K = 4096 the two are equal: 16 x 4096 x 4096 5.9 / 6.1),
+// or one that 128 x 128 tiles would cut (cut: split_k_plan): 3 x 3326 x 16368 10.4 against 19.5 us in slices of tiles.
+bool few_rows_whole(const sofie_hip_ctx *ctx, const GemmArgs &g, bool cut)
 {
-   return g.M <= 16 && cdiv(g.N, 16) * 2 >= ctx->num_cus && g.K >= 512 && g.K <= 4096 && (size_t)g.N * g.K >= ((size_t)2 << 20) &&
+   return g.M <= 16 && cdiv(g.N, 16) * 2 >= ctx->num_cus && g.K >= 512 && (g.K <= 4096 || cut) && (size_t)g.N * g.K >= ((size_t)2 << 20) &&
           (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);      // 32-bit offsets
 }
 // ... or with K in slices, for fewer columns and a long K: 4 x 64 x 65536 16.7 against 41.5 us in one launch
 // (k_gemm_bytes_direct), 16 x 1024 x 32768 18.3 / 29.9, 8 x 256 x 16384 10.0 / 13.3, 8 x 1024 x 8192 8.5 / 7.9. By time the
 // line would lie at a B of 8 MB, where the second launch costs what the slices gain; it lies at 3 MB, with the slower way from
 // there to 8 MB (8 x 1536 x 2048: 7.7 / 4.7), because test_qgemm_s8_few_rows_kernels_and_constant_weights names the kernel that
-// runs on that product.
-bool few_rows_sliced(const sofie_hip_ctx *ctx, const GemmArgs &g)
+// runs on that product. Where 128 x 128 tiles would cut K, this is the better cut for up to 32 rows (us, this / tiles in slices:
+// 2 x 64 x 46736 11.0 / 21.3, 31 x 64 x 60336 16.5 / 26.8, 17 x 287 x 11888 9.2 / 14.2, 32 x 331 x 10736 10.1 / 14.7); with more than 16
+// rows on more than about 1280 columns the tiles are (0.84 - 0.99 of this in the mean over 60 products).
+bool few_rows_sliced(const sofie_hip_ctx *ctx, const GemmArgs &g, bool cut)
 {
-   return g.M <= 16 && g.N >= 64 && cdiv(g.N, 16) * 2 < ctx->num_cus && g.K >= 512 && (size_t)g.N * g.K >= ((size_t)3 << 20) &&
-          (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);
+   const bool pays = g.M <= 16 ? cdiv(g.N, 16) * 2 < ctx->num_cus && g.K >= 512 && (cut || (size_t)g.N * g.K >= ((size_t)3 << 20))
+                               : g.M <= 32 && g.N <= 1280 && cut;
+   return pays && g.N >= 64 && (size_t)g.M * g.lda + g.K < (1u << 31) && (size_t)g.N * g.ldb + g.K < (1u << 31);
 }
 
 // Slices of K so that about eight workgroups per compute unit exist, every wavefront with at least two chunks, and the
@@ -1653,9 +1671,9 @@ int few_rows_splits(const sofie_hip_ctx *ctx, const GemmArgs &g, int *kslice)
 }
 
 template <int OUT>
-int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g)
+int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g, bool whole)
 {
-   if (few_rows_whole(ctx, g)) {
+   if (whole) {
       const int kper = cdiv(cdiv(g.K, 8), 64) * 64;
       hipLaunchKernelGGL((k_qgemm_few_rows_whole<OUT>), dim3(cdiv(g.N, 16)), dim3(512), 0, ctx->stream, g, kper);
       return check_launch(ctx, "k_qgemm_few_rows_whole");
@@ -1667,7 +1685,8 @@ int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g)
    void *part = nullptr;
    if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
    const dim3 grid(blocks, splits);
-   hipLaunchKernelGGL(k_qgemm_few_rows, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
+   if (g.M <= 16) hipLaunchKernelGGL(k_qgemm_few_rows<1>, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
+   else hipLaunchKernelGGL(k_qgemm_few_rows<2>, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
    if (int rc = check_launch(ctx, "k_qgemm_few_rows")) return rc;
    const size_t threads = (size_t)g.M * (ldp / 4);
    hipLaunchKernelGGL((k_splitk_finish<OUT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, g,
@@ -1781,7 +1800,13 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
    constexpr int BK = 128;
    constexpr int NSETS = IS_INT ? 2 : 1;
    if constexpr (IS_INT && OUT != SOFIE_OUT_BF16) {
-      if (few_rows_whole(ctx, g) || few_rows_sliced(ctx, g)) return launch_few_rows<OUT>(ctx, g);
+      int splits = 1, kslice = 0;
+      const bool cut = g.M <= 32 && split_k_plan(ctx, g, splits, kslice);
+      if (few_rows_whole(ctx, g, cut)) return launch_few_rows<OUT>(ctx, g, true);
+      // (tiles in slices need less memory for their sums)
+      if (few_rows_sliced(ctx, g, cut) &&
+          (!cut || workspace_has_room(ctx, (size_t)few_rows_splits(ctx, g, &kslice) * g.M * (cdiv(g.N, 4) * 4) * sizeof(int))))
+         return launch_few_rows<OUT>(ctx, g, false);
    }
    if (big_product(g)) {
       // descriptor offsets are 32-bit: a 256-row panel plus K must stay below 2 GiB

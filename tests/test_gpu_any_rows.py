@@ -63,6 +63,28 @@ def test_int8_product_of_any_rows(ops, M, N, K, transB):
             assert np.array_equal(y.cpu().numpy(), want), (offset, pad, out)
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [(17, 287, 11888, "k_qgemm_few_rows"), (31, 1023, 24000, "k_qgemm_few_rows"),
+                                          (32, 64, 40000, "k_qgemm_few_rows"), (33, 64, 40000, "k_gemm_bytes"),
+                                          (20, 1300, 24000, "k_gemm_bytes"), (2, 64, 46736, "k_qgemm_few_rows"),
+                                          (3, 3326, 16368, "k_qgemm_few_rows_whole")])
+def test_up_to_32_rows_on_a_long_sum_are_a_pass_over_b(ops, M, N, K, kernel):
+    r = rng(1500 + M)
+    A, B = r.integers(-127, 128, (M, K)).astype(np.int8), r.integers(-127, 128, (N, K)).astype(np.int8)
+    scale = (r.uniform(20.0, 60.0, N) / (73.3 * 73.3 * np.sqrt(K))).astype(np.float32)
+    ctx = ops.Context(0)
+    a, b, sd, y = ctx.dev(A), ctx.dev(B), ctx.dev(scale), ctx.empty((M, N), torch.int8)
+    buf, n = C.create_string_buffer(4096), C.c_int(-1)
+    torch.cuda.synchronize()
+    ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+    ctx.check(ctx.lib.sofie_hip_qgemm_s8(ctx.h, 1, M, N, K, ctx.ptr(a), K, ctx.ptr(b), K, ctx.ptr(sd), None, -3, L.ACT_NONE, ctx.ptr(y), N, L.OUT_S8))
+    ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
+    ctx.sync()
+    names = [l.split()[0] for l in buf.value.decode().splitlines()]
+    assert names[0] == kernel, names
+    assert np.array_equal(y.cpu().numpy(), oracle.qgemm_s8(A, B, scale, None, True, zpy=-3))
+    ctx.close()
+
+
 # a size for each number of rows and columns of k_gemm_bytes_direct (16 x 16, 16 x 32, 32 x 16, 32 x 32)
 @pytest.mark.parametrize("M,N", [(40, 100), (200, 500), (1088, 100), (500, 272)])
 @pytest.mark.parametrize("K", [41, 45, 46, 47, 44, 300, 1001])
