@@ -24,8 +24,12 @@ struct ConvProblem {
    ConvPhase phase[4];
 };
 
-// Runs the problem on k_conv_f32_any (conv_f32_any.hip); *done stays false where it does not take it, or where its estimate
-// is above the microseconds of the caller's other way.
-int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done);
+// Runs the problem on k_conv_f32_any (conv_f32_any.hip) or k_conv_f32_split; *done stays false where they do not take it, or where
+// the former's estimate is above the microseconds of the caller's other way. split_only: not on the former.
+int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done, bool split_only = false);
+
+// Runs the problem on k_conv_f32_split (conv_f32_split.hip); *done stays false where it does not take it, or where its estimate is above
+// the microseconds of the caller's other way.
+int conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done);
 
 }  // namespace sofie

@@ -659,8 +659,8 @@ ConvProblem problem_of(const ConvArgs &g)
 }
 
 // The whole of g (its one phase, or all of them) on k_conv_f32_any; *done stays false where it does not take it, or where
-// other_us is the shorter way.
-int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us = HUGE_VAL)
+// other_us is the shorter way. split_only: on k_conv_f32_split or not at all.
+int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us = HUGE_VAL, bool split_only = false)
 {
    ConvProblem p = problem_of(g);
    p.nphases = g.nphases > 1 ? g.nphases : 1;
@@ -669,7 +669,7 @@ int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us =
       const PhaseArgs &f = g.phase[i];
       p.phase[i] = {f.OH, f.OW, f.KH, f.KW, f.ph, f.pw, f.th0, g.ths, f.tw0, g.tws, f.oy0, g.oys, f.ox0, g.oxs};
    }
-   return conv_f32_any(ctx, p, other_us, done);
+   return conv_f32_any(ctx, p, other_us, done, split_only);
 }
 
 // Whether a layer that k_conv2d_f32_dma takes (full channel blocks of an even K) runs on k_conv_f32_any all the same.
@@ -678,7 +678,9 @@ int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us =
 // of the kept layouts name the older kernel there. Without it the weights are laid out in front of every call, and the
 // fragments of k_conv_f32_any (whole tiles of 16 channels and 32 k) cost more to write: from 2^29 on, where that no longer
 // counts (944 M 34.2 / 29.4; 472 M 21.8 / 22.3, 84 M 1x1 11.3 / 12.4, 231 M 19.7 / 15.5, 12 M 10.7 / 9.7).
-bool beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
+// SPLIT: on k_conv_f32_split only, if that is the shorter way.
+enum Beyond { NOT_BEYOND, SPLIT, ANY };
+Beyond beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
 {
    double outputs = (double)g.OH * g.OW, taps = (double)g.KH * g.KW;
    if (g.nphases > 1) {
@@ -689,16 +691,17 @@ bool beyond_dma(const sofie_hip_ctx *ctx, const ConvArgs &g)
    // Short sums for whole tiles of channels: the stores of a tile of 64 x 128 come in longer pieces (7x8x144x144 -> 39: 21.8
    // against 24.5 us, 6x6x30x30 -> 128 transposed 4x4: 10.1 against 14.0).
    const int phases = g.nphases > 1 ? g.nphases : 1;
-   if (g.icg <= 16 && g.icg * taps <= 72 * phases && g.ocg >= 32 && (double)g.OH * g.OW >= 256.0 * phases) return false;
+   if (g.icg <= 16 && g.icg * taps <= 72 * phases && g.ocg >= 32 && (double)g.OH * g.OW >= 256.0 * phases) return NOT_BEYOND;
+   const bool large = madds >= (ctx->constant_weights ? 7.0e6 : 536870912.0);
    // Long sums of phases that fill tiles of 64 channels x 128 pixels: there k_conv2d_f32_dma reads each input cell once for all
    // taps and stores two pixels apart in longer pieces (64x128x28x28 -> 64, 4x4: 123.9 against 126.3 us; where a quarter
    // of the tiles is empty, 40x144x7x7 -> 232: 56 against 28).
    if (g.nphases > 1 && g.icg * taps >= 256.0 * phases) {
       const double area = (double)g.phase[0].OH * g.phase[0].OW;
       const double full = g.ocg / (64.0 * cdiv(g.ocg, 64)) * area / (128.0 * cdiv((int)area, 128));
-      if (full >= 0.85) return false;
+      if (full >= 0.85) return large ? SPLIT : NOT_BEYOND;
    }
-   return madds >= (ctx->constant_weights ? 7.0e6 : 536870912.0);
+   return large ? ANY : NOT_BEYOND;
 }
 
 // Tiles of 64 ti channels x 64 tj pixels for a convolution of one phase, and how many: 128 x 128 per workgroup where that gives
@@ -1077,8 +1080,9 @@ int run_conv(sofie_hip_ctx *ctx, ConvArgs &g)
    g.dOW = make_fastdiv((unsigned)g.OW);
    bool done = false;
    int rc;
-   if (beyond_dma(ctx, g) && (!g.transposed || (g.uh == 1 && g.uw == 1))) {
-      rc = run_any(ctx, g, &done, dma_us(ctx, g));
+   const Beyond beyond = beyond_dma(ctx, g);
+   if (beyond && (!g.transposed || (g.uh == 1 && g.uw == 1))) {
+      rc = run_any(ctx, g, &done, dma_us(ctx, g), beyond == SPLIT);
       if (rc || done) return rc;
    }
    const Tiling t = tiling_of(ctx, g);
@@ -1271,8 +1275,8 @@ extern "C" int sofie_hip_conv_transpose2d_f32(sofie_hip_ctx *ctx, const float *x
       if (ok && all.nphases > 1) {
          all.dUH = make_fastdiv(1u); all.dUW = make_fastdiv(1u); all.dOW = make_fastdiv(1u);
          bool done = false;
-         if (beyond_dma(ctx, all)) {
-            if (int rc = run_any(ctx, all, &done)) return rc;
+         if (const Beyond beyond = beyond_dma(ctx, all)) {
+            if (int rc = run_any(ctx, all, &done, HUGE_VAL, beyond == SPLIT)) return rc;
             if (done) return SOFIE_HIP_OK;
          }
          // tiles as for the plain convolution: the largest that still give every compute unit one

@@ -455,7 +455,7 @@ int launch(sofie_hip_ctx *ctx, const AnyArgs &g, int nphases, int mode, int stor
 
 }  // namespace
 
-int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done)
+int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done, bool split_only)
 {
    *done = false;
    const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
@@ -588,6 +588,9 @@ int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_u
    };
    Form best = choose(per);
    if (best.ti == 0) return SOFIE_HIP_OK;
+   // Longer sums on many tiles are shorter on the bf16 matrix instructions; both estimates are off by some 10 %.
+   if (int rc = conv_f32_split(ctx, p, 0.9 * (best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1)), done); rc || *done) return rc;
+   if (split_only) return SOFIE_HIP_OK;
    // against what the caller has instead (the estimate's unit is a cycle at 2400 MHz; weights that are not kept are laid out in
    // front of the launch, 3.1 us)
    if (other_us < 0.95 * (best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1))) return SOFIE_HIP_OK;

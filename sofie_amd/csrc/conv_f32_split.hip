@@ -1,0 +1,650 @@
+// fp32 NCHW convolutions of any channels, kernels, strides, dilations and groups, and the output phases of transposed ones, as an
+// implicit GEMM on the bf16 matrix instructions with every operand as three bf16 numbers (split_bf16.h): k_conv_f32_split.
+//
+//   Y[oc, pixel] = sum_k W[oc, k] * X[k, pixel],  k = (8 channels, kernel row, kernel column, channel of the 8)
+//
+// A workgroup of four wavefronts (2 x 2) owns 32 TI channels x 32 TJ pixels, a wavefront TI x TJ tiles of 16 x 16.
+//   * X: the input cells of the tile's pixels (halo included, zeros outside the image) lie in LDS as h, m, l of eight channels
+//     each, 48 bytes a cell, CS channels (a slot) at a time: a cell is split once and read by all taps. 16 lanes with neighbouring
+//     cells fall on different banks, at stride 2, too. Two slots: while one is multiplied the threads hold the loads of the slot
+//     after the next in registers; behind a barrier they convert them and put them where the finished slot was. A step of 32 k is
+//     four chunks of 8 channels of a tap, in one list over all slots, so that no step is cut off at a slot's end (9 taps of 16
+//     channels are 4 1/2 steps); a step that reaches into the next slot has a barrier of its own.
+//   * W: a copy laid out as fragments of split numbers [16 channels][step][h, m, l][lane], once per tensor under the
+//     constant-weights promise, else in front of the launch. Straight into registers, a step ahead.
+//   * Pixels run over all images in one row, or, where that costs little, tiles end with an image; wide images are cut into strips.
+// All requests of a slot leave in one step: the fragments behind them wait for them (loads return in order), and one such wait
+// per slot is cheaper than one per step. A bias read behind the loop made the compiler wait for each store in front of the next one
+// (13000 cycles for 16 stores instead of 6800).
+//
+// Bound: the device's power under bf16 matrix instructions on large layers (256x64x56x56 -> 128: 1.65 GHz, the matrix pipe
+// busy for 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
+// smaller ones. Relative error against 64 bits a quarter of the fp32 instructions'. us against k_conv_f32_any and k_conv2d_f32_dma:
+// 256x64x56x56 -> 128, 3x3 906 -> 640 (576 for the first
+// milliseconds); 256x32x20x20 -> 64 47.4 -> 28.5; 256x64x10x10 -> 128 44.4 -> 27.5; 169x80x16x16 -> 128,
+// 5x5 220 -> 116; 16x64x32x32 -> 65, 7x7 107 -> 51; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 101 (89). Three workgroups per compute
+// unit instead of two (fewer cells per thread and slot) were 12 % of the last.
+#include <cmath>
+
+#include "conv_f32.h"
+#include "conv_f32_patch.h"
+#include "gemm_tile.h"
+#include "split_bf16.h"
+
+using namespace sofie;
+
+namespace {
+
+constexpr unsigned OUTSIDE = 0x40000000u;      // no descriptor of this file reaches it
+constexpr int MAX_PHASES = 4;
+constexpr int CELL = 48;                       // LDS bytes of 8 channels of a cell: h, m, l
+constexpr int THREADS = 256;
+
+// Cells x 8 channels of a slot that a thread carries, at most: registers, which decide how many workgroups share a compute unit.
+constexpr int items_of(int ti, int tj, int wo) { return wo == 1 ? 4 : ti * tj > 8 ? 3 : 2; }
+// Workgroups a compute unit holds at once, by registers.
+constexpr int resident_of(int ti, int tj, int wo) { return ti * tj > 8 ? 2 : ti * tj > 4 || wo == 1 ? 3 : 4; }
+
+struct SplitPhase {
+   int P, PHW, panels;        // pixels, of a panel; panels (strips of images)
+   int ws, strips;            // columns of a strip, strips of an image
+   int KH, KW, ph, pw;
+   int HP, PW, cells;         // rows of a panel's input, cells of a row, of a tile's patch
+   int full;                  // pixels of a panel that exist (PHW: up to whole tiles where tiles do not run on into the next panel)
+   int chunks;                // of a slot: 8 channels of a tap each
+   int steps;                 // of four chunks, all of K
+   int wofs;                  // first 16-byte piece of the phase's fragments
+   int OW;
+   int oy0, oys, ox0, oxs;
+   int th0, ths, tw0, tws;
+   FastDiv dPHW, dWS, dHP, dPW, dStrips, dTaps, dKW, dCells;
+};
+
+struct SplitArgs {
+   const float *x, *bias;
+   const v4i *w;
+   float *y;
+   unsigned xbytes, ybytes, wbytes;
+   int H, W, icg, ocg, groups, sh, sw, dh, dw, relu;
+   int CS, nslots;            // channels of a slot, slots
+   int octiles, oblocks;
+   int chw4, hw4, ocplane4, plane4, OW0;
+   int table_bytes, slot_bytes;      // LDS: table of offsets, two slots
+   int nphases;
+   FastDiv dOB, dPhases;
+   SplitPhase phase[MAX_PHASES];
+};
+
+enum { PIXELS, QUADS };
+
+template <int TI, int TJ, int WO, int STORE, bool PHASES>
+__global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_split(SplitArgs g)
+{
+   extern __shared__ __align__(16) unsigned char smem_raw[];
+   constexpr int BP = 4 / WO * TJ * 16, ITEMS = items_of(TI, TJ, WO);
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = wave % WO;
+   // workgroup id -> (pixels, channels, phase): an XCD (an L2) works on consecutive ids; the phases of a tile, which read the same
+   // input and write every other pixel of the same lines, are next to each other, and so are the channel blocks of a pixel block
+   int pid = blockIdx.x, phase = 0;
+   {
+      const int tiles = gridDim.x, xcd = pid & 7, base = tiles >> 3, rem = tiles & 7;
+      pid = (pid >> 3) + xcd * base + (xcd < rem ? xcd : rem);
+   }
+   if constexpr (PHASES) {
+      const int all = pid;
+      pid = fdiv(all, g.dPhases);
+      phase = all - pid * g.nphases;
+   }
+   SplitPhase q = g.phase[0];
+   if constexpr (PHASES) {
+#pragma unroll
+      for (int i = 1; i < MAX_PHASES; ++i)
+         if (phase == i) q = g.phase[i];
+   }
+   const int pb = fdiv(pid, g.dOB), ob = pid - pb * g.oblocks * g.groups;
+   const int grp = ob / g.oblocks, tile0 = (ob - grp * g.oblocks) * TI * WO + wo * TI;
+   const int p0 = pb * BP;
+   if (p0 >= q.P) return;
+   int origin;      // the tile's first row of the panels' inputs
+   {
+      const int panel = fdiv(p0, q.dPHW);
+      origin = panel * q.HP + fdiv(p0 - panel * q.PHW, q.dWS) * g.sh;
+   }
+   unsigned char *const patch = smem_raw + g.table_bytes;
+   unsigned voff[ITEMS];
+   const int items = q.cells * (g.CS >> 3);
+#pragma unroll
+   for (int s = 0; s < ITEMS; ++s) {
+      const int item = s * THREADS + tid, c8 = fdiv(item, q.dCells), cell = item - c8 * q.cells, row = fdiv(cell, q.dPW), col = cell - row * q.PW;
+      const int grow = origin + row, panel = fdiv(grow, q.dHP), n = fdiv(panel, q.dStrips);
+      const int iy = grow - panel * q.HP - q.ph, ix = (panel - n * q.strips) * q.ws * g.sw + col - q.pw;
+      const bool in = item < items && panel < q.panels && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
+      voff[s] = in ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + c8 * 8 * g.hw4) : OUTSIDE;
+   }
+   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.x), 0, (int)g.xbytes, 0x00020000);
+   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<v4i *>(g.w) + q.wofs, 0, (int)(g.wbytes - 16u * (unsigned)q.wofs), 0x00020000);
+   float xr[ITEMS][8];
+   auto fetch = [&](float (&xr)[ITEMS][8], int s, int slot) {
+      const int c0 = slot * g.CS, rem = g.icg - c0;
+      const unsigned soff = (unsigned)(grp * g.icg + c0) * (unsigned)g.hw4;
+      if (rem >= g.CS) {
+#pragma unroll
+         for (int e = 0; e < 8; ++e)
+            xr[s][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)voff[s], (int)(soff + e * (unsigned)g.hw4), 0));
+      } else {
+         // channels behind the group's last one ask for nothing
+         const int left = rem - fdiv(s * THREADS + tid, q.dCells) * 8;
+#pragma unroll
+         for (int e = 0; e < 8; ++e)
+            xr[s][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(e < left ? voff[s] : OUTSIDE), (int)(e < rem ? soff + e * (unsigned)g.hw4 : 0u), 0));
+      }
+   };
+   auto put = [&](const float (&xr)[ITEMS][8], int s, unsigned char *buf) {
+      if (s * THREADS + tid >= items) return;
+      const Split8 v = split8(xr[s]);
+      v8b *const d = reinterpret_cast<v8b *>(buf + (s * THREADS + tid) * CELL);
+      d[0] = v.h;
+      d[1] = v.m;
+      d[2] = v.l;
+   };
+   unsigned wofs[TI];         // uniform: fragments of this wavefront's tiles (those behind the last tile: the last one's)
+#pragma unroll
+   for (int i = 0; i < TI; ++i) {
+      const int t = tile0 + i < g.octiles ? tile0 + i : g.octiles - 1;
+      wofs[i] = (unsigned)__builtin_amdgcn_readfirstlane((grp * g.octiles + t) * q.steps * 3072);
+   }
+   v8b w[TI][3];
+   auto load_w = [&](int i, unsigned step) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+         w[i][p] = __builtin_bit_cast(v8b, __builtin_amdgcn_raw_buffer_load_b128(wrs, lane * 16 + p * 1024, (int)(wofs[i] + step * 3072u), 0));
+   };
+   // everything that comes from memory is requested first; what the loop needs besides is worked out while it travels
+   float second[ITEMS][8];
+#pragma unroll
+   for (int s = 0; s < ITEMS; ++s)
+      if (s * THREADS < items) fetch(xr, s, 0);
+   if (g.nslots > 1) {
+#pragma unroll
+      for (int s = 0; s < ITEMS; ++s)
+         if (s * THREADS < items) fetch(second, s, 1);
+   }
+#pragma unroll
+   for (int i = 0; i < TI; ++i) load_w(i, 0);
+   constexpr int NB = STORE == QUADS ? 1 : 4;
+   float bias[TI][NB];
+#pragma unroll
+   for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int e = 0; e < NB; ++e) {
+         const int oc = (tile0 + i) * 16 + (STORE == QUADS ? r16 : 4 * kg + e);
+         bias[i][e] = g.bias && oc < g.ocg ? g.bias[grp * g.ocg + oc] : 0.0f;
+      }
+   __builtin_amdgcn_sched_barrier(0);
+   const int taps = q.KH * q.KW;
+   int *const table = reinterpret_cast<int *>(smem_raw);
+   // offset of every chunk of two slots (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
+   // first chunks)
+   for (int e = tid; e < 2 * q.chunks; e += THREADS) {
+      const int second = e >= q.chunks, k = second ? e - q.chunks : e, c8 = fdiv(k, q.dTaps), t = k - c8 * taps, a = fdiv(t, q.dKW), b = t - a * q.KW;
+      table[e] = (c8 * q.cells + a * g.dh * q.PW + b * g.dw) * CELL + (g.nslots > 1 ? second * g.slot_bytes : 0);
+   }
+   int base[TJ];
+#pragma unroll
+   for (int j = 0; j < TJ; ++j) {
+      const int p = p0 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), c = r - oy * q.ws;
+      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh - origin) * q.PW + c * g.sw) * CELL : 0;
+   }
+   v4f acc[TI][TJ];
+#pragma unroll
+   for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+   for (int s = 0; s < ITEMS; ++s)
+      if (s * THREADS < items) put(xr, s, patch);
+   if (g.nslots > 1) {
+#pragma unroll
+      for (int s = 0; s < ITEMS; ++s)
+         if (s * THREADS < items) put(second, s, patch + g.slot_bytes);
+   }
+   // (settled here: behind the loop the compiler would wait for the stores in front of each use)
+#pragma unroll
+   for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int e = 0; e < NB; ++e) asm volatile("" : "+v"(bias[i][e]));
+   __syncthreads();
+   int step = 0, place = 0;      // place: first chunk of the step in the table
+   v8b x[TJ][3];
+   auto read_x = [&](int j, int off) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) x[j][p] = *reinterpret_cast<const v8b *>(patch + base[j] + off + p * 16);
+   };
+   for (int slot = 0; slot < g.nslots; ++slot) {
+      const bool last = slot + 1 == g.nslots, more = slot + 2 < g.nslots;
+      const int end_chunk = q.chunks * (slot + 1), end = last ? q.steps : (end_chunk + 3) >> 2;
+      const bool across = !last && (end_chunk & 3) != 0;      // the last step takes chunks of the next slot, too
+      const int begin = step;
+      bool fresh = true;
+      for (; step < end; ++step) {
+         if (across && step + 1 == end) {
+            __syncthreads();
+            fresh = true;
+         }
+         if (fresh) {
+            const int off = table[place + kg];
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) read_x(j, off);
+         }
+         place = place + 4 == 2 * q.chunks ? 0 : place + 4;
+         const int ahead = across ? end - 2 : end - 1;
+         fresh = step >= ahead;
+         const int off = table[(fresh ? 0 : place) + kg];
+         if (more && step == begin) {
+#pragma unroll
+            for (int s = 0; s < ITEMS; ++s)
+               if (s * THREADS < items) fetch(xr, s, slot + 2);
+         }
+         // The six products of a tile one behind the other (17 cycles each; 19 taking turns with another tile's, 27 with seven),
+         // the additions of the tile before in between.
+         v4f t, before;
+#pragma unroll
+         for (int n = 0; n < TI * TJ; ++n) {
+            const int i = n / TJ, j = n % TJ;
+            constexpr int A[6] = {2, 1, 1, 0, 0, 0}, B[6] = {0, 0, 1, 1, 2, 0};
+            t = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < 6; ++m) {
+               t = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[j][A[m]], w[i][B[m]], t, 0, 0, 0)
+                                  : __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][B[m]], x[j][A[m]], t, 0, 0, 0);
+               if (n > 0 && m >= 1 && m < 5) acc[(n - 1) / TJ][(n - 1) % TJ][m - 1] = __fadd_rn(acc[(n - 1) / TJ][(n - 1) % TJ][m - 1], before[m - 1]);
+               __builtin_amdgcn_sched_barrier(0);
+            }
+            before = t;
+            if (i == TI - 1) read_x(j, off);
+            if (j + 1 == TJ) load_w(i, (unsigned)(step + 1));      // (behind the last step: read and not used)
+            __builtin_amdgcn_sched_barrier(0);
+         }
+#pragma unroll
+         for (int e = 0; e < 4; ++e) acc[TI - 1][TJ - 1][e] = __fadd_rn(acc[TI - 1][TJ - 1][e], before[e]);
+      }
+      if (!last) __syncthreads();
+      if (more) {
+#pragma unroll
+         for (int s = 0; s < ITEMS; ++s)
+            if (s * THREADS < items) put(xr, s, patch + (slot & 1) * g.slot_bytes);
+      }
+   }
+
+   // sums that are not finite: again, with fp32 instructions on the operands as they were given
+   v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+   for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+         for (int e = 0; e < 4; ++e) none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
+   const float any = (none[0] + none[1]) + (none[2] + none[3]);
+   int p1 = p0;      // (so that nothing of the pixels' places is kept in registers through the loop)
+   asm volatile("" : "+s"(p1));
+   if (__builtin_amdgcn_ballot_w64(any != 0.0f) != 0) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+         for (int j = 0; j < TJ; ++j) {
+            const int p = p1 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), n = fdiv(panel, q.dStrips);
+            const int iy0 = oy * g.sh - q.ph, ix0 = ((panel - n * q.strips) * q.ws + r - oy * q.ws) * g.sw - q.pw;
+            v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int c0 = 0; c0 < g.icg; c0 += 4) {
+               const int c = c0 + kg;
+               for (int t = 0; t < taps; ++t) {
+                  const int a = fdiv(t, q.dKW), b = t - a * q.KW, iy = iy0 + a * g.dh, ix = ix0 + b * g.dw;
+                  const bool in = p < q.P && r < q.full && c < g.icg && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
+                  const float xv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + (grp * g.icg + c) * g.hw4) : OUTSIDE), 0, 0));
+                  const int chunk = (c >> 3) * taps + t;
+                  const unsigned wat = wofs[i] + (unsigned)((chunk >> 2) * 3072 + ((chunk & 3) * 16 + r16) * 16 + (c & 7) * 2);
+                  __bf16 part[3];
+#pragma unroll
+                  for (int e = 0; e < 3; ++e)
+                     part[e] = __builtin_bit_cast(__bf16, __builtin_amdgcn_raw_buffer_load_b16(wrs, (int)(c < g.icg ? wat + e * 1024 : OUTSIDE), 0, 0));
+                  const float wv = joined(part[0], part[1], part[2]);
+                  sum = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wv, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, sum, 0, 0, 0);
+               }
+            }
+            acc[i][j] = sum;
+         }
+   }
+
+   const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(g.y, 0, (int)g.ybytes, 0x00020000);
+   const rsrc_t yrs4 = make_rsrc(g.y, g.ybytes);
+   auto finish = [&](float v, float b) {
+      if (g.bias) v = __fadd_rn(v, b);
+      return g.relu ? (v > 0.0f ? v : 0.0f) : v;
+   };
+#pragma unroll
+   for (int j = 0; j < TJ; ++j) {
+      const int p = p1 + (wp * TJ + j) * 16 + (STORE == QUADS ? 4 * kg : r16);
+      const int panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), n = fdiv(panel, q.dStrips);
+      const int ox = (panel - n * q.strips) * q.ws + r - oy * q.ws;
+      const bool pixel = p < q.P && r < q.full && ox < q.OW;
+      const unsigned at_pixel = (unsigned)(n * g.ocplane4 + ((q.oy0 + oy * q.oys) * g.OW0 + q.ox0 + ox * q.oxs) * 4);
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+         const int oc = (tile0 + i) * 16;
+         if (oc >= g.ocg) continue;
+         v4f v = acc[i][j];
+         if constexpr (STORE == QUADS) {
+            const bool there = pixel && oc + r16 < g.ocg;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = finish(v[e], bias[i][0]);
+            store16_buf(yrs4, v, there ? at_pixel + (unsigned)(r16 * g.plane4) : OUTSIDE, (unsigned)(grp * g.ocg + oc) * (unsigned)g.plane4);
+         } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+               if (oc + e >= g.ocg) continue;
+               const bool there = pixel && oc + 4 * kg + e < g.ocg;
+               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, finish(v[e], bias[i][STORE == QUADS ? 0 : e])), yrs, (int)(there ? at_pixel + (unsigned)(kg * 4 * g.plane4) : OUTSIDE),
+                                                     (int)((unsigned)(grp * g.ocg + oc + e) * (unsigned)g.plane4), 0);
+            }
+         }
+      }
+   }
+}
+
+struct SplitWeightArgs {
+   const float *w;
+   v4i *dst;
+   int icg, ocg, octiles, KH0, KW0, transposed, total;      // total: triples of 16-byte pieces over all phases
+   SplitPhase phase[MAX_PHASES];
+};
+
+// The fragments [group][16 channels][step][h, m, l][lane][8 of K]; zeros behind the last channel and the last k.
+__global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs g)
+{
+   const int idx = blockIdx.x * 256 + threadIdx.x;
+   if (idx >= g.total) return;
+   SplitPhase q = g.phase[0];
+#pragma unroll
+   for (int i = 1; i < MAX_PHASES; ++i)
+      if (g.phase[i].wofs > 0 && 3 * idx >= g.phase[i].wofs) q = g.phase[i];
+   int r = idx - q.wofs / 3;
+   const int lane = r & 63;
+   r >>= 6;
+   const int step = r % q.steps, tile = r / q.steps;
+   const int oc = (tile % g.octiles) * 16 + (lane & 15), grp = tile / g.octiles;
+   const int chunk = 4 * step + (lane >> 4), c8 = fdiv(chunk, q.dTaps), t = chunk - c8 * q.KH * q.KW;
+   const int ta = fdiv(t, q.dKW), a = q.th0 + ta * q.ths, b = q.tw0 + (t - ta * q.KW) * q.tws;
+   float v[8];
+#pragma unroll
+   for (int e = 0; e < 8; ++e) {
+      const int ic = c8 * 8 + e;
+      const bool in = oc < g.ocg && ic < g.icg;
+      const size_t at = !in ? 0 : g.transposed ? ((size_t)(grp * g.icg + ic) * g.ocg + oc) : ((size_t)(grp * g.ocg + oc) * g.icg + ic);
+      v[e] = in ? g.w[(at * g.KH0 + a) * g.KW0 + b] : 0.0f;
+   }
+   const Split8 s = split8_exact(v);
+   v4i *d = g.dst + q.wofs + ((size_t)tile * q.steps + step) * 192 + lane;
+   d[0] = __builtin_bit_cast(v4i, s.h);
+   d[64] = __builtin_bit_cast(v4i, s.m);
+   d[128] = __builtin_bit_cast(v4i, s.l);
+}
+
+template <int TI, int TJ, int WO>
+int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, int store, long tiles)
+{
+   constexpr auto kern_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false>, kern_q = k_conv_f32_split<TI, TJ, WO, QUADS, false>, kern_t = k_conv_f32_split<TI, TJ, WO, PIXELS, true>;
+   SOFIE_LARGE_LDS(kern_p);
+   SOFIE_LARGE_LDS(kern_q);
+   SOFIE_LARGE_LDS(kern_t);
+   hipLaunchKernelGGL(nphases > 1 ? kern_t : store == QUADS ? kern_q : kern_p, dim3((unsigned)(tiles * nphases)), dim3(THREADS),
+                      (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), ctx->stream, g);
+   return check_launch(ctx, "k_conv_f32_split");
+}
+
+
+struct Form {
+   int ti, tj, wo, cs, strips;
+   int pixels() const { return 64 / wo * tj; }
+   int channels() const { return 16 * wo * ti; }
+   int items() const { return items_of(ti, tj, wo); }
+   double time;
+};
+
+// Geometry of the problem for tiles of bp pixels, slots of cs channels and images in strips; false where a slot is more than the
+// threads of a workgroup carry, or than the LDS holds. pieces: 16-byte pieces of the fragments (which do not depend on cs and strips).
+bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int strips, size_t *pieces)
+{
+   g.CS = cs;
+   g.nslots = cdiv(g.icg, cs);
+   g.slot_bytes = 0;
+   size_t total = 0;
+   int table = 0;
+   for (int i = 0; i < p.nphases; ++i) {
+      const ConvPhase &f = p.phase[i];
+      SplitPhase &q = g.phase[i];
+      const int taps = f.KH * f.KW;
+      q.KH = f.KH; q.KW = f.KW; q.ph = f.ph; q.pw = f.pw;
+      q.OW = f.OW;
+      q.ws = cdiv(f.OW, strips);
+      if (f.OW % 4 == 0) q.ws = (q.ws + 3) & ~3;
+      q.strips = cdiv(f.OW, q.ws);
+      const long full = (long)f.OH * q.ws;
+      // tiles that do not run on into the next panel read fewer rows: where the last one is nearly full
+      const bool apart = (full + bp - 1) / bp * bp * 100 <= full * 104;
+      const long pixels = apart ? (full + bp - 1) / bp * bp : full;
+      const long HP = (long)(f.OH - 1) * p.sh + (long)(f.KH - 1) * p.dh + 1, PW = (long)(q.ws - 1) * p.sw + (long)(f.KW - 1) * p.dw + 1;
+      if (pixels > (1 << 28) || HP > (1 << 28) || PW > 4096) return false;
+      const long cells = split_patch_rows(bp, q.ws, pixels, f.OH, p.sh, f.KH, p.dh, apart) * PW;
+      // (a step reaches into one slot behind its first chunk's)
+      if (cells * (cs / 8) > (long)items * THREADS || (g.nslots > 1 && cs / 8 * taps < 4)) return false;
+      q.full = (int)full;
+      q.PHW = (int)pixels;
+      q.HP = (int)HP;
+      q.PW = (int)PW;
+      q.cells = (int)cells;
+      q.chunks = cs / 8 * taps;
+      q.steps = cdiv(cdiv(g.icg, 8) * taps, 4);
+      q.wofs = (int)total;
+      total += (size_t)p.groups * g.octiles * q.steps * 192;
+      q.oy0 = f.oy0; q.oys = f.oys; q.ox0 = f.ox0; q.oxs = f.oxs;
+      q.th0 = f.th0; q.ths = f.ths; q.tw0 = f.tw0; q.tws = f.tws;
+      if (q.cells * (cs / 8) * CELL > g.slot_bytes) g.slot_bytes = q.cells * (cs / 8) * CELL;
+      if (2 * q.chunks * 4 > table) table = 2 * q.chunks * 4;
+   }
+   *pieces = total;
+   g.table_bytes = (table + 255) & ~255;
+   return total * 16 <= ((size_t)1 << 29) && g.table_bytes + (g.nslots > 1 ? 2 : 1) * g.slot_bytes <= kMaxDynamicLds;
+}
+
+// Microseconds of a form on n images, laid out in g. A workgroup that is alone on its compute unit waits for memory in front of its loop,
+// once per slot and once per step, and for its stores behind it; workgroups that share one wait for each other's matrix
+// instructions (96 cycles a tile and step), operands, stores and conversions. A fit to 1760 timings of 201 convolutions over the ranges
+// of perf/cases.py (8.4 % rms; the form it picks is 1.1 % behind the best one in the mean).
+double estimate(const SplitArgs &g, const ConvProblem &p, int cus, const Form &f, size_t n, bool quads)
+{
+   const int bp = f.pixels(), oblocks = cdiv(g.octiles, f.wo * f.ti), pieces = f.ti * f.tj;
+   const int by_registers = resident_of(f.ti, f.tj, f.wo), by_lds = kMaxDynamicLds / (g.table_bytes + (g.nslots > 1 ? 2 : 1) * g.slot_bytes);
+   const int resident = by_lds < by_registers ? by_lds : by_registers;
+   const double store_alone = p.nphases > 1 ? 280.0 : quads ? 0.0 : 292.0, store = p.nphases > 1 ? 259.0 : quads ? 0.0 : 176.0;
+   double tiles = 0.0, alone = 0.0, work = 0.0;
+   for (int i = 0; i < p.nphases; ++i) {
+      const SplitPhase &q = g.phase[i];
+      const double mma = 96.0 * q.steps * pieces, reads = (double)q.steps * (f.ti + f.tj), items = (double)q.cells * (g.CS / 8) / THREADS;
+      const double t = (double)cdiv((int)n * q.strips * q.PHW, bp) * oblocks * g.groups;
+      const double one = 3344.0 + (287.0 + store_alone) * pieces + g.nslots * (1053.0 + 785.0 * items) + 100.0 * reads + 0.579 * mma;
+      if (one > alone) alone = one;
+      work += t * (0.889 * mma + 33.5 * reads + (151.0 + store) * pieces + 598.0 * g.nslots * items + 527.0);
+      tiles += t;
+   }
+   const double per_cu = tiles / cus, rounds = per_cu / resident, whole = rounds + 0.895 * (std::ceil(rounds) - rounds);
+   const double waits = alone * (whole > 1.0 ? whole : 1.0), busy = std::ceil(per_cu) * work / tiles;
+   const double w2 = waits * waits, b2 = busy * busy;
+   // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings)
+   const SplitPhase &q0 = g.phase[0], &q1 = g.phase[p.nphases - 1];
+   const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.35 : 1.0;
+   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
+}
+
+template <int TI, int TJ, int WO>
+int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, bool quads, long tiles)
+{
+   constexpr auto kern_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false>, kern_q = k_conv_f32_split<TI, TJ, WO, QUADS, false>, kern_t = k_conv_f32_split<TI, TJ, WO, PIXELS, true>;
+   SOFIE_LARGE_LDS(kern_p);
+   SOFIE_LARGE_LDS(kern_q);
+   SOFIE_LARGE_LDS(kern_t);
+   hipLaunchKernelGGL(nphases > 1 ? kern_t : quads ? kern_q : kern_p, dim3((unsigned)(tiles * nphases)), dim3(THREADS),
+                      (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), ctx->stream, g);
+   return check_launch(ctx, "k_conv_f32_split");
+}
+
+}  // namespace
+
+int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done)
+{
+   *done = false;
+   // The shortest form takes 6 us; below 7.5 us the choice among them costs the host more than it gives. Channels that fill little of the
+   // chunks of eight, and short sums, which are their stores (60x1x16x72 -> 247, 3x3 27 us on k_conv_f32_any, 34 here; the tests of the
+   // other kernels name them up to 144 products: 55x16x60x60 -> 64, 3x3, 1x10x101x101 -> 64).
+   const long icg = p.C / p.groups;
+   if (other_us < 7.5 + (ctx->constant_weights ? 0.0 : 4.0) || icg < 6 || (p.nphases == 1 ? icg * p.KH0 * p.KW0 <= 144 : icg * p.KH0 * p.KW0 < 48 * p.nphases)) return SOFIE_HIP_OK;
+   const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
+   // descriptors and OUTSIDE: 1 GiB of images per launch
+   const size_t room = ((size_t)1 << 30) - ((size_t)16 << 20);
+   if (image > room || out_image > room || p.nphases < 1 || p.nphases > MAX_PHASES) return SOFIE_HIP_OK;
+   for (int i = 0; i < p.nphases; ++i) {
+      const ConvPhase &f = p.phase[i];
+      if (f.KH < 1 || f.KW < 1 || f.OH < 1 || f.OW < 1 || (long)f.KH * f.KW > 256) return SOFIE_HIP_OK;
+   }
+   SplitArgs g{};
+   g.icg = p.C / p.groups;
+   g.ocg = p.OC / p.groups;
+   g.groups = p.groups;
+   g.octiles = cdiv(g.ocg, 16);
+   size_t per = room / (image > out_image ? image : out_image);
+   if (per > (size_t)p.N) per = (size_t)p.N;
+   const ConvPhase &f0 = p.phase[0];
+   const bool whole = p.nphases == 1 && f0.oys == 1 && f0.oxs == 1 && f0.oy0 == 0 && f0.ox0 == 0 && f0.OW == p.OW0 && f0.OH == p.OH0;
+   auto quads = [&] { return whole && (g.phase[0].strips == 1 ? (long)p.OH0 * p.OW0 % 4 == 0 : p.OW0 % 4 == 0); };
+   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+   size_t pieces = 0;
+   // the form for a launch on n images: tiles of 32 ti channels x 32 tj pixels, slots of 16 or 32 channels, the images in as many
+   // strips as read least for their pixels
+   auto choose = [&](size_t n) {
+      static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
+      double mma = 0.0;      // matrix instructions per 16 channels and pixel
+      for (int i = 0; i < p.nphases; ++i)
+         mma += (double)n * p.phase[i].OH * p.phase[i].OW * cdiv(cdiv(g.icg, 8) * p.phase[i].KH * p.phase[i].KW, 4) * p.groups * 96.0 / 16.0 / 4.0;
+      Form best{0, 0, 0, 0, 0, other_us};
+      for (const auto &f : forms) {
+         Form form{f[0], f[1], f[2], 16, 0, 0.0};
+         if (f[0] > 1 && f[2] * (f[0] - 1) >= g.octiles) continue;      // tiles of nothing
+         // (cannot be shorter than its matrix instructions)
+         if (mma * cdiv(g.octiles, f[2] * f[0]) * f[2] * f[0] * 0.889 / (2100.0 * cus) + 3.0 >= best.time) continue;
+         for (; form.cs <= 32; form.cs *= 2) {
+            double least = 0.0;
+            form.strips = 0;
+            for (int strips = 1; strips <= 16; ++strips) {
+               if (!lay_out(g, p, form.pixels(), form.items(), form.cs, strips, &pieces)) continue;
+               const SplitPhase &q = g.phase[0];
+               if ((double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
+               const double cost = (double)q.strips * q.PHW * (1.0 + 0.02 * q.cells / form.pixels());
+               if (form.strips == 0 || cost < least) {
+                  least = cost;
+                  form.strips = strips;
+               } else if (strips > form.strips + 1) {
+                  break;
+               }
+            }
+            if (form.strips == 0) continue;
+            lay_out(g, p, form.pixels(), form.items(), form.cs, form.strips, &pieces);
+            form.time = estimate(g, p, cus, form, n, quads());
+            if (form.time < best.time) best = form;
+         }
+      }
+      return best;
+   };
+   // (weights that are not kept are laid out in front of the launch, twice the bytes of k_conv_f32_any's)
+   other_us = (other_us - (ctx->constant_weights ? 0.0 : 4.0)) * ((double)per / (double)p.N);
+   Form best = choose(per);
+   if (best.ti == 0) return SOFIE_HIP_OK;
+   auto prepare = [&] {
+      lay_out(g, p, best.pixels(), best.items(), best.cs, best.strips, &pieces);
+      for (int i = 0; i < p.nphases; ++i) {
+         SplitPhase &q = g.phase[i];
+         q.dPHW = make_fastdiv((unsigned)q.PHW);
+         q.dWS = make_fastdiv((unsigned)q.ws);
+         q.dHP = make_fastdiv((unsigned)q.HP);
+         q.dPW = make_fastdiv((unsigned)q.PW);
+         q.dStrips = make_fastdiv((unsigned)q.strips);
+         q.dTaps = make_fastdiv((unsigned)(q.KH * q.KW));
+         q.dKW = make_fastdiv((unsigned)q.KW);
+         q.dCells = make_fastdiv((unsigned)q.cells);
+      }
+      g.nphases = p.nphases;
+      g.dPhases = make_fastdiv((unsigned)p.nphases);
+      g.oblocks = cdiv(g.octiles, best.wo * best.ti);
+      g.dOB = make_fastdiv((unsigned)(g.oblocks * g.groups));
+   };
+   prepare();
+   // the step behind the last one may be asked for, to no use
+   const size_t wbytes = pieces * 16 + 4096;
+   g.wbytes = (unsigned)wbytes;
+   int key[7 + 7 * MAX_PHASES] = {5, p.groups, g.ocg, g.icg, p.KH0 * 4096 + p.KW0, p.transposed, p.nphases};
+   for (int i = 0; i < p.nphases; ++i) {
+      const SplitPhase &q = g.phase[i];
+      const int v[7] = {q.KH, q.KW, q.th0, q.ths, q.tw0, q.tws, q.wofs};
+      for (int e = 0; e < 7; ++e) key[7 + 7 * i + e] = v[e];
+   }
+   void *ws = nullptr;
+   bool fresh = true;
+   // (while a graph is recorded the scratch buffer may be too small: the caller has other ways)
+   if (packed_weights(ctx, p.w, layout_key(key, 7 + 7 * p.nphases), wbytes, &ws, &fresh)) return SOFIE_HIP_OK;
+   if (fresh) {
+      SplitWeightArgs a{};
+      a.w = p.w; a.dst = static_cast<v4i *>(ws);
+      a.icg = g.icg; a.ocg = g.ocg; a.octiles = g.octiles;
+      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.total = (int)(pieces / 3);
+      for (int i = 0; i < MAX_PHASES; ++i) a.phase[i] = g.phase[i];
+      hipLaunchKernelGGL(k_conv_f32_split_weights, dim3((unsigned)cdiv(a.total, 256)), dim3(256), 0, ctx->stream, a);
+      if (int rc = check_launch(ctx, "k_conv_f32_split_weights")) return rc;
+   }
+   g.w = static_cast<const v4i *>(ws);
+   g.bias = p.bias;
+   g.H = p.H; g.W = p.W; g.sh = p.sh; g.sw = p.sw; g.dh = p.dh; g.dw = p.dw; g.relu = p.relu;
+   g.chw4 = (int)image;
+   g.hw4 = p.H * p.W * 4;
+   g.ocplane4 = (int)out_image;
+   g.plane4 = p.OH0 * p.OW0 * 4;
+   g.OW0 = p.OW0;
+   for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
+      const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
+      if (n != per) {
+         other_us = HUGE_VAL;
+         best = choose(n);
+         prepare();
+      }
+      g.x = p.x + n0 * (image / 4);
+      g.y = p.y + n0 * (out_image / 4);
+      g.xbytes = (unsigned)(n * image);
+      g.ybytes = (unsigned)(n * out_image);
+      long tiles = 0;
+      for (int i = 0; i < p.nphases; ++i) {
+         SplitPhase &q = g.phase[i];
+         q.panels = (int)n * q.strips;
+         q.P = q.panels * q.PHW;
+         const long t = (long)cdiv(q.P, best.pixels()) * g.oblocks * g.groups;
+         if (t > tiles) tiles = t;
+      }
+      int rc = SOFIE_HIP_OK;
+      switch (best.ti * 100 + best.tj * 10 + best.wo) {
+#define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, quads(), tiles); break
+         SOFIE_FORM(4, 4, 2); SOFIE_FORM(3, 4, 2); SOFIE_FORM(2, 4, 2); SOFIE_FORM(4, 2, 2); SOFIE_FORM(2, 2, 2); SOFIE_FORM(1, 4, 2); SOFIE_FORM(1, 2, 2);
+         SOFIE_FORM(1, 4, 1);
+#undef SOFIE_FORM
+      }
+      if (rc) return rc;
+   }
+   *done = true;
+   return SOFIE_HIP_OK;
+}

@@ -1,0 +1,144 @@
+"""fp32 convolutions on k_conv_f32_split (operands as three bf16 numbers): every tile size, slots of 16 and 32 channels, steps that reach
+into the next slot, strips, groups, phases and ragged ends, against float64; error against the fp32 instructions'; values that are
+not finite."""
+import ctypes as C
+
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sofie_amd import ops as o
+    return o
+
+
+@pytest.fixture()
+def kept(ops):
+    """A context that keeps its weights in the kernels' layouts."""
+    ctx = ops.Context(0)
+    ctx.check(ctx.lib.sofie_hip_constant_weights(ctx.h, 1))
+    yield ctx
+    ctx.close()
+
+
+def names_of(ctx, call):
+    buf, n = C.create_string_buffer(4096), C.c_int(-1)
+    ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+    out = call()
+    ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
+    ctx.sync()
+    return out, [line.split()[0] for line in buf.value.decode().splitlines()]
+
+
+# N, C, H, W, OC, KH, KW, stride, (top, left, bottom, right), dilation, groups
+CONV = [
+    (64, 64, 56, 56, 128, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),      # 128 channels x 128 pixels, tiles end with an image
+    (120, 32, 20, 20, 64, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),      # pixels run on across images
+    (256, 64, 10, 10, 128, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),
+    (90, 35, 41, 37, 70, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),       # odd planes (4-byte stores), three channels of the last eight
+    (64, 51, 40, 64, 93, 5, 5, (1, 1), (2, 2, 2, 2), (1, 1), 1),       # 96 channels
+    (17, 64, 168, 38, 28, 7, 7, (1, 1), (3, 3, 3, 3), (1, 1), 1),      # 32 channels, 49 taps
+    (16, 64, 32, 32, 65, 7, 7, (1, 1), (3, 3, 3, 3), (1, 1), 1),       # one channel behind two blocks of 32
+    (7, 64, 158, 64, 231, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),
+    (5, 16, 58, 58, 192, 5, 5, (1, 1), (2, 2, 2, 2), (1, 1), 1),       # a slot and nothing else
+    (192, 12, 16, 64, 66, 5, 5, (1, 1), (2, 2, 2, 2), (1, 1), 1),      # part of a slot
+    (64, 64, 56, 40, 128, 3, 3, (2, 1), (1, 1, 1, 1), (1, 1), 1),      # every other row
+    (20, 90, 60, 61, 96, 3, 3, (1, 1), (2, 0, 1, 3), (2, 3), 2),       # groups, dilations, uneven pads
+    (30, 128, 30, 225, 64, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),     # wide rows in strips, the last one short
+    (300, 24, 7, 5, 160, 5, 4, (1, 1), (2, 2, 2, 1), (1, 1), 1),       # images smaller than a tile
+]
+
+
+def reference(x, w, bias, s, pads, d, groups):
+    t, l, b, r = pads
+    return torch.nn.functional.conv2d(torch.nn.functional.pad(x.cpu().double(), (l, r, t, b)), w.cpu().double(), bias.cpu().double(), s, 0, d, groups)
+
+
+@pytest.mark.parametrize("shape", CONV)
+def test_conv_in_three_parts(ops, kept, shape):
+    """Products of split numbers lose less than 2^-26 each and sums are rounded once per 32 k at their own size, where fp32 products
+    in a row are rounded K times: 1e-5 of the largest output, as for the other fp32 kernels, and 3e-7 in the 2-norm (they show up to
+    1e-6 at these K)."""
+    n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    x = torch.randn(n, c, h, w, device="cuda", generator=g)
+    wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * (c // groups * kh * kw) ** -0.5
+    bias = torch.randn(oc, device="cuda", generator=g)
+    torch.cuda.synchronize()
+    for ctx in (kept, ops.Context(0)):
+        y, names = names_of(ctx, lambda: ops.conv2d_f32(x, wt, bias, pads, s, d, groups, relu=ctx is kept, ctx=ctx))
+        assert "k_conv_f32_split" in names or ctx is not kept, names
+        # some images, the first and the last among them
+        for i in sorted({0, n // 3, n // 2, n - 1}):
+            ref = reference(x[i:i + 1], wt, bias, s, pads, d, groups)
+            ref = ref.clamp(min=0) if ctx is kept else ref
+            err = y[i:i + 1].cpu().double() - ref
+            assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
+            assert "k_conv_f32_split" not in names or float(err.norm()) <= 3e-7 * float(ref.norm()), i
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,k,s", [(64, 128, 28, 28, 64, 4, 2), (30, 143, 32, 34, 181, 4, 2), (30, 64, 26, 15, 93, 4, 2),
+                                            (60, 87, 19, 21, 40, 3, 2), (64, 120, 20, 20, 90, 3, 1)])
+def test_transposed_conv_in_three_parts(ops, kept, n, c, h, w, oc, k, s):
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    x, wt = torch.randn(n, c, h, w, device="cuda", generator=g), torch.randn(c, oc, k, k, device="cuda", generator=g) * (c * k * k) ** -0.5
+    bias = torch.randn(oc, device="cuda", generator=g)
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv_transpose2d_f32(x, wt, bias, (1, 1, 1, 1), (s, s), (1, 1), 1, (0, 0), ctx=kept))
+    assert "k_conv_f32_split" in names or (k == 3 and s == 2), names
+    for i in sorted({0, n // 2, n - 1}):
+        ref = torch.nn.functional.conv_transpose2d(x[i:i + 1].cpu().double(), wt.cpu().double(), bias.cpu().double(), s, 1)
+        assert float((y[i:i + 1].cpu().double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
+
+
+@pytest.mark.parametrize("c,relu", [(72, False), (16, True)])
+def test_values_that_are_not_finite_stay_in_their_windows(ops, kept, c, relu):
+    """Infinities and NaN in cells, weights and products: the parts of a split infinity are no numbers, but its sums are the fp32
+    kernels' again. Zeros, signs and the largest finite numbers, which a rounded bf16 would leave, among them."""
+    g = torch.Generator().manual_seed(c)
+    x, w = torch.randn(40, c, 28, 28, generator=g), torch.randn(96, c, 5, 5, generator=g)
+    x[3, 0, 4, 4], x[3, c - 1, 27, 27], x[9, 5, 0, 13], x[39, 2, 27, 0] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    w[7, 3, 2, 2], w[95, c - 1, 0, 0] = 1e38, float("inf")
+    w[:, 2] = w[:, 2].clamp(-0.5, 0.5)
+    w[11] = 0.0
+    xp = torch.nn.functional.pad(x, (2, 2, 2, 2))      # zeros outside the image are factors like others: with an infinite weight they are NaN
+    ref = torch.nn.functional.conv2d(xp, w)
+    ref = torch.where(ref > 0, ref, torch.zeros(())) if relu else ref
+    xd, wd = x.cuda(), w.cuda()
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv2d_f32(xd, wd, None, (2, 2), (1, 1), (1, 1), 1, relu, ctx=kept))
+    assert names[-1] == "k_conv_f32_split"
+    y = y.cpu()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.sign(y[~fin & ~torch.isnan(ref)]), torch.sign(ref[~fin & ~torch.isnan(ref)]))
+    scale = torch.nn.functional.conv2d(torch.where(torch.isfinite(x), x, torch.zeros(())).abs().double(), torch.where(torch.isfinite(w), w, torch.zeros(())).abs().double(), None, 1, 2)
+    assert bool(((y.double() - ref.double()).abs()[fin] <= 1e-5 * scale[fin] + 1e-30).all())
+
+
+def test_small_and_mixed_magnitudes_keep_their_bits(ops, kept):
+    """Every cell is split by itself: rows 2^60 apart in one tile, and weights near the smallest normal numbers of bf16's lowest part, are
+    as exact as rows of ones."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(64, 64, 28, 28, device="cuda", generator=g) * torch.exp2(torch.randint(-30, 31, (64, 1, 28, 1), device="cuda", generator=g).float())
+    w = torch.randn(96, 64, 3, 1, device="cuda", generator=g) * torch.exp2(torch.randint(-60, 40, (96, 1, 1, 1), device="cuda", generator=g).float())
+    w[:, :, 0], w[:, :, 2] = 0.0, 0.0      # an output row depends on one row of cells
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv2d_f32(x, w, None, (1, 0), (1, 1), (1, 1), 1, ctx=kept))
+    assert names[-1] == "k_conv_f32_split"
+    ref = torch.nn.functional.conv2d(x.double(), w.double(), None, 1, (1, 0)).cpu()
+    size = torch.nn.functional.conv2d(x.double().abs(), w.double().abs(), None, 1, (1, 0)).cpu()
+    assert bool(((y.cpu().double() - ref).abs() <= 2.0 ** -21 * size).all())      # two roundings of 2^-24 per 32 k and 2^-26 per product
+
+
+def test_whole_numbers_are_exact(ops, kept):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-300, 301, (50, 48, 30, 30), device="cuda", generator=g).float()
+    w = torch.randint(-9, 10, (80, 48, 3, 3), device="cuda", generator=g).float()
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv2d_f32(x, w, None, (1, 1), ctx=kept))
+    assert names[-1] == "k_conv_f32_split"
+    assert torch.equal(y.cpu(), torch.nn.functional.conv2d(x.cpu(), w.cpu(), None, 1, 1))
