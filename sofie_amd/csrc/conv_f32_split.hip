@@ -142,11 +142,12 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
    };
    auto put = [&](const float (&xr)[ITEMS][8], int s, unsigned char *buf) {
       if (s * THREADS + tid >= items) return;
-      const Split8 v = split8(xr[s]);
-      v8b *const d = reinterpret_cast<v8b *>(buf + (s * THREADS + tid) * CELL);
-      d[0] = v.h;
-      d[1] = v.m;
-      d[2] = v.l;
+      v4i v[3];
+      split8(xr[s], v);
+      v4i *const d = reinterpret_cast<v4i *>(buf + (s * THREADS + tid) * CELL);
+      d[0] = v[0];
+      d[1] = v[1];
+      d[2] = v[2];
    };
    unsigned wofs[TI];         // uniform: fragments of this wavefront's tiles (those behind the last tile: the last one's)
 #pragma unroll
@@ -389,19 +390,6 @@ __global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs 
    d[64] = __builtin_bit_cast(v4i, s.m);
    d[128] = __builtin_bit_cast(v4i, s.l);
 }
-
-template <int TI, int TJ, int WO>
-int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, int store, long tiles)
-{
-   constexpr auto kern_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false>, kern_q = k_conv_f32_split<TI, TJ, WO, QUADS, false>, kern_t = k_conv_f32_split<TI, TJ, WO, PIXELS, true>;
-   SOFIE_LARGE_LDS(kern_p);
-   SOFIE_LARGE_LDS(kern_q);
-   SOFIE_LARGE_LDS(kern_t);
-   hipLaunchKernelGGL(nphases > 1 ? kern_t : store == QUADS ? kern_q : kern_p, dim3((unsigned)(tiles * nphases)), dim3(THREADS),
-                      (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), ctx->stream, g);
-   return check_launch(ctx, "k_conv_f32_split");
-}
-
 
 struct Form {
    int ti, tj, wo, cs, strips;

@@ -1,102 +1,17 @@
 // fp32 GEMM on the matrix cores with a fused alpha / beta*bias / ReLU epilogue: k_gemm_f32_dma (v_mfma_f32_32x32x2_f32) for
 // operands that can be fetched 16 bytes at a time, k_gemm_f32 (v_mfma_f32_16x16x4_f32) for all others, k_gemm_f32_skinny for
-// few rows. Roofline: MFMA fp32 (256 flop/clk/CU).
+// few rows; k_gemm_f32_split (gemm_f32_split.hip) where its estimate is the shortest. Roofline: MFMA fp32 (256 flop/clk/CU).
 #include <cstdint>
 #include <type_traits>
 
 #include "common.h"
 #include "gemm_tile.h"
+#include "gemm_f32.h"
 #include "gemm_f32_operand.h"
 
 using namespace sofie;
 
 namespace {
-
-struct GemmF32Args {
-   const float *A, *B, *bias;
-   float *Y;
-   int M, N, K, lda, ldb, ldy;
-   int transA, transB;
-   float alpha, beta;
-   int bias_kind, relu;
-   // stacked products (blockIdx.z + z0 = index of the product, row-major over the n_lead leading dimensions):
-   // element strides of A and B along each leading dimension (0 where the operand is broadcast), Y is dense
-   int n_lead, z0;
-   int lead[SOFIE_GEMM_MAX_LEAD];
-   long long sa[SOFIE_GEMM_MAX_LEAD], sb[SOFIE_GEMM_MAX_LEAD];
-   long long stride_y;
-   // k_gemm_f32_dma with K in slices (gridDim.y > 1): a slice's raw sums go to partial [slice][M][N]
-   float *partial;
-};
-
-// Workgroup id -> tile, in groups of 4 rows of tiles, so that the workgroups in flight share rows of A and columns of B in an
-// L2. Workgroups are dealt to the 8 XCDs in turn: renumbered so that an XCD (an L2) works on consecutive tiles.
-__device__ __forceinline__ void tile_of(int pid, int tiles_m, int tiles_n, int &tm, int &tn)
-{
-   {
-      const int tiles = tiles_m * tiles_n, xcd = pid & 7, base = tiles >> 3, rem = tiles & 7;
-      pid = (pid >> 3) + xcd * base + (xcd < rem ? xcd : rem);
-   }
-   const int width = 4 * tiles_n, group = pid / width, first = group * 4;
-   const int gsize = tiles_m - first < 4 ? tiles_m - first : 4;
-   tm = first + (pid % width) % gsize;
-   tn = (pid % width) / gsize;
-}
-
-// A, B and Y of product `index` of a stack (row-major over the leading dimensions, last dimension fastest).
-__device__ __forceinline__ void select_product(GemmF32Args &g, long long index)
-{
-   long long rem = index, oa = 0, ob = 0;
-   // (constant subscripts: with a run-time one the whole argument block would move to scratch memory)
-#pragma unroll
-   for (int d = SOFIE_GEMM_MAX_LEAD - 1; d >= 0; --d) {
-      if (d >= g.n_lead) continue;
-      const long long pos = rem % g.lead[d];
-      rem /= g.lead[d];
-      oa += pos * g.sa[d];
-      ob += pos * g.sb[d];
-   }
-   g.A += oa;
-   g.B += ob;
-   g.Y += index * g.stride_y;
-}
-
-// The bias of columns n .. n + 3 where a row of it is given. (Requested ahead of a kernel's sums: four loads behind them for every
-// four outputs were a third of the time of a product with a short K; 3274 x 7184 x 16 64 us, 2 of K on 3192 x 3280 36.)
-__device__ __forceinline__ v4f bias_row4(const GemmF32Args &g, int n)
-{
-   v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
-   if (g.bias_kind == SOFIE_BIAS_ROW) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-         if (n + e < g.N) b[e] = g.bias[n + e];
-   }
-   return b;
-}
-// alpha * v + beta * bias, ReLU, for columns n .. n + 3 of row m; row: bias_row4 of n.
-__device__ __forceinline__ v4f finish4(const GemmF32Args &g, v4f v, v4f row, int m, int n)
-{
-#pragma unroll
-   for (int e = 0; e < 4; ++e) {
-      v[e] = __fmul_rn(g.alpha, v[e]);
-      if (g.bias_kind == SOFIE_BIAS_ROW) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, row[e]));
-      else if (g.bias_kind == SOFIE_BIAS_FULL && n + e < g.N) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, g.bias[(size_t)m * g.ldy + n + e]));
-      else if (g.bias_kind == SOFIE_BIAS_COL) v[e] = __fadd_rn(v[e], __fmul_rn(g.beta, g.bias[m]));
-      if (g.relu) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
-   }
-   return v;
-}
-__device__ __forceinline__ void store4(const GemmF32Args &g, v4f v, int m, int n)
-{
-   float *o = g.Y + (size_t)m * g.ldy + n;
-   if (n + 4 <= g.N) {
-      __builtin_memcpy(o, &v, 16);       // rows may start on any float
-      return;
-   }
-#pragma unroll
-   for (int e = 0; e < 3; ++e)
-      if (n + e < g.N) o[e] = v[e];
-}
 
 // Products of any sizes, leading dimensions and storage (A_KM: A stored [K][M], B_KM: B stored [K][N]). 256 threads = 4
 // wavefronts in 2 x 2, each with MI x NJ tiles of 16 x 16 (v_mfma_f32_16x16x4_f32: tiles of 16 let a product take workgroup
@@ -744,6 +659,12 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny_finish(GemmF32Args g, c
    g.Y[(size_t)m * g.ldy + n] = v;
 }
 
+int launch_finish(sofie_hip_ctx *ctx, const GemmF32Args &g, int splits)
+{
+   hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(g.M * g.N, 256)), dim3(256), 0, ctx->stream, g, g.partial, splits);
+   return check_launch(ctx, "k_gemm_f32_skinny_finish");
+}
+
 // M <= 64 rows on k_gemm_f32_skinny. Slices of K so that about eight workgroups per compute unit exist, each wavefront
 // with at least four chunks, and so that the partial sums stay below a quarter of B's bytes once they are more than a
 // few megabytes (below that the launch is latency, not traffic).
@@ -767,8 +688,8 @@ int launch_skinny_as(sofie_hip_ctx *ctx, GemmF32Args &g)
    hipLaunchKernelGGL((k_gemm_f32_skinny<B_NK, T, MT>), dim3(blocks, splits), dim3(256), 0, ctx->stream, g, partial, kslice, splits);
    if (int rc = check_launch(ctx, "k_gemm_f32_skinny")) return rc;
    if (splits == 1) return SOFIE_HIP_OK;
-   hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(g.M * g.N, 256)), dim3(256), 0, ctx->stream, g, partial, splits);
-   return check_launch(ctx, "k_gemm_f32_skinny_finish");
+   g.partial = partial;
+   return launch_finish(ctx, g, splits);
 }
 
 int launch_skinny(sofie_hip_ctx *ctx, GemmF32Args &g)
@@ -789,8 +710,7 @@ int launch_tiles_as(sofie_hip_ctx *ctx, GemmF32Args &g, int splits, unsigned nz)
    hipLaunchKernelGGL(kern, dim3(cdiv(g.M, BM) * cdiv(g.N, BN), splits, nz), dim3(256), NST * (BM + BN) * 32 * 4, ctx->stream, g);
    if (int rc = check_launch(ctx, "k_gemm_f32")) return rc;
    if (splits == 1) return SOFIE_HIP_OK;
-   hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(g.M * g.N, 256)), dim3(256), 0, ctx->stream, g, g.partial, splits);
-   return check_launch(ctx, "k_gemm_f32_skinny_finish");
+   return launch_finish(ctx, g, splits);
 }
 
 template <bool A_KM, bool B_KM, int MI, int NJ>
@@ -809,8 +729,9 @@ int launch_direct_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz)
 // Fitted to the times of every kernel on 34 sizes, 10 x 64 x 16 to 4000 x 4001 x 4002. Where the lines fall: 90 x 90 x 360 5.4 us
 // direct, 6.4 on 32 x 32 tiles, 12.3 on 64 x 64; 1500 x 1001 x 1111 85 / 38 / 42, 34 on 32 x 64; 256 x 256 x 12800 39 direct, 90 on
 // 32 x 32 tiles and 25 with them in 8 slices; 4000 x 4001 x 4002 978 on 64 x 64, 965 on 128 x 128.
+enum GeneralKernel { TILES, DIRECT, SPLIT };
 struct GeneralChoice {
-   bool direct;
+   GeneralKernel kernel;
    int mi, nj, splits;
    float us;
 };
@@ -826,11 +747,11 @@ constexpr TileCost kTileCosts[6] = {{1, 1, 0.21f, 0.176f}, {1, 2, 0.36f, 0.275f}
 // four on rows of 2^24 floats).
 GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, bool one_launch)
 {
-   GeneralChoice best = {false, 1, 1, 1, 1e30f};
+   GeneralChoice best = {TILES, 1, 1, 1, 1e30f};
    auto offsets_fit = [](bool km, int ld, int rows) { return (long long)(km ? 32 : rows) * ld * 4 < (1ll << 31); };
    const int cus = ctx->num_cus;
-   auto consider = [&](bool direct, int mi, int nj, int splits, float us) {
-      if (us < best.us) best = {direct, mi, nj, splits, us};
+   auto consider = [&](GeneralKernel kernel, int mi, int nj, int splits, float us) {
+      if (us < best.us) best = {kernel, mi, nj, splits, us};
    };
    auto consider_direct = [&] {
       for (const auto &t : kDirectTiles) {
@@ -838,7 +759,7 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
          const long long tiles = (long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj), per_cu = (tiles * nz + cus - 1) / cus;
          if (tiles >= (1ll << 32) / 512) continue;
          const float mfma = (float)per_cu * 512.0f * mi * nj * g.K / 550e3f, reads = (float)per_cu * 64.0f * (mi + nj) * g.K / 43e3f;
-         consider(true, mi, nj, 1, 0.5f + (float)((per_cu + resident - 1) / resident) + (mfma > reads ? mfma : reads));
+         consider(DIRECT, mi, nj, 1, 0.5f + (float)((per_cu + resident - 1) / resident) + (mfma > reads ? mfma : reads));
       }
    };
    if (g.K >= 4 && g.bias_kind != SOFIE_BIAS_FULL) consider_direct();
@@ -850,9 +771,12 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
          if (s > 1 && (one_launch || steps / s < 4 || (size_t)g.M * g.N >= ((size_t)1 << 28))) break;
          const long long per_cu = (tiles * s + cus - 1) / cus;
          const float step = per_cu == 1 ? t.alone : (float)per_cu * t.among;
-         consider(false, t.mi, t.nj, s, 2.0f + step * cdiv(steps, s) + (s > 1 ? 5.0f + 8.0f * s * (float)g.M * g.N / 6e6f : 0.0f));
+         consider(TILES, t.mi, t.nj, s, 2.0f + step * cdiv(steps, s) + (s > 1 ? 5.0f + 8.0f * s * (float)g.M * g.N / 6e6f : 0.0f));
       }
    }
+   // (operands as three bf16 numbers on the bf16 matrix instructions: 1500 x 1001 x 1111 27 us, 33 on 32 x 64 tiles)
+   const SplitChoice split = gemm_f32_split_choice(ctx, g, nz, one_launch);
+   consider(SPLIT, split.mi, 4, split.splits, split.us);
    if (g.K >= 4 && best.us >= 1e30f) consider_direct();
    return best;
 }
@@ -860,7 +784,7 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
 template <bool A_KM, bool B_KM>
 int launch_general_as(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, const GeneralChoice &c)
 {
-   if (c.direct) {
+   if (c.kernel == DIRECT) {
       switch (c.mi * 10 + c.nj) {
       case 11: return launch_direct_as<A_KM, B_KM, 1, 1>(ctx, g, nz);
       case 12: return launch_direct_as<A_KM, B_KM, 1, 2>(ctx, g, nz);
@@ -893,6 +817,10 @@ int launch_general(sofie_hip_ctx *ctx, GemmF32Args &g, unsigned nz, bool one_lau
       const size_t blocks = ((size_t)g.M * g.N + 255) / 256, across = blocks < ((size_t)1 << 23) ? blocks : (size_t)1 << 23;
       hipLaunchKernelGGL(k_gemm_f32_plain, dim3((unsigned)across, (unsigned)((blocks + across - 1) / across), nz), dim3(256), 0, ctx->stream, g);
       return check_launch(ctx, "k_gemm_f32_plain");
+   }
+   if (c.kernel == SPLIT) {
+      if (int rc = launch_gemm_f32_split(ctx, g, nz, {c.mi, c.splits, c.us})) return rc;
+      return c.splits > 1 ? launch_finish(ctx, g, c.splits) : SOFIE_HIP_OK;
    }
    if (g.transA) return g.transB ? launch_general_as<true, false>(ctx, g, nz, c) : launch_general_as<true, true>(ctx, g, nz, c);
    return g.transB ? launch_general_as<false, false>(ctx, g, nz, c) : launch_general_as<false, true>(ctx, g, nz, c);
@@ -945,7 +873,21 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
                        (size_t)M * lda * 4 < (1u << 31) && (size_t)(transB ? N : K) * ldb * 4 < (1u << 31) &&
                        (size_t)M * ldy < (1u << 31);
    if (skinny) return launch_skinny(ctx, g);
-   if (dma) {
+   // tiles for less than half of the compute units and a K of 16 steps or more: K in slices (of at least 8 steps) so that about two
+   // workgroups per compute unit exist; the slices' sums are added by the pass of the few-rows kernel
+   // (128 x 1024 x 4096: 18.5 against 76.9 us; with a tile for every compute unit slices gain and lose: -6 % .. +14 %)
+   const int tiles = dma ? cdiv(M, tile) * cdiv(N, tile) : 0, steps = K / 32;
+   const bool sliced = small && tiles * 2 <= ctx->num_cus && steps >= 16;
+   // k_gemm_f32_split instead of whole tiles of 24 us and more (by kTileCosts; below that it gains little, and test_gemm_f32_large
+   // names the kernels): us 2048^3 137 / 110, 4096 x 4096 x 3000 700 / 604; 1024^3 here
+   bool split = false;
+   if (dma && !sliced) {
+      const int per_cu = cdiv(tiles, ctx->num_cus);
+      const TileCost &t = small ? kTileCosts[3] : kTileCosts[5];
+      const float us = 2.0f + (per_cu == 1 ? t.alone : (float)per_cu * t.among) * steps;
+      split = us >= 24.0f && gemm_f32_split_choice(ctx, g, 1, true).us < us;
+   }
+   if (dma && !split) {
       constexpr auto kern_nk2 = k_gemm_f32_dma<false, 2>, kern_kn2 = k_gemm_f32_dma<true, 2>;
       constexpr auto kern_nk1 = k_gemm_f32_dma<false, 1>, kern_kn1 = k_gemm_f32_dma<true, 1>;
       SOFIE_LARGE_LDS(kern_nk2);
@@ -953,12 +895,8 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
       SOFIE_LARGE_LDS(kern_nk1);
       SOFIE_LARGE_LDS(kern_kn1);
       const auto kern = small ? (transB ? kern_nk1 : kern_kn1) : (transB ? kern_nk2 : kern_kn2);
-      // tiles for less than half of the compute units and a K of 16 steps or more: K in slices (of at least 8 steps) so
-      // that about two workgroups per compute unit exist; the slices' sums are added by the pass of the few-rows kernel
-      // (128 x 1024 x 4096: 18.5 against 76.9 us; with a tile for every compute unit slices gain and lose: -6 % .. +14 %)
-      const int tiles = cdiv(M, tile) * cdiv(N, tile), steps = K / 32;
       int splits = 1;
-      if (small && tiles * 2 <= ctx->num_cus && steps >= 16) {
+      if (sliced) {
          splits = 2 * ctx->num_cus / tiles;
          if (splits > steps / 8) splits = steps / 8;
          if (splits > 16) splits = 16;
@@ -972,8 +910,7 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
       hipLaunchKernelGGL(kern, dim3(tiles, splits), dim3(256), 2 * (tile + tile) * 32 * 4, ctx->stream, g);
       if (int rc = check_launch(ctx, small ? "k_gemm_f32_dma64" : "k_gemm_f32_dma")) return rc;
       if (splits == 1) return SOFIE_HIP_OK;
-      hipLaunchKernelGGL(k_gemm_f32_skinny_finish, dim3(cdiv(M * N, 256)), dim3(256), 0, ctx->stream, g, g.partial, splits);
-      return check_launch(ctx, "k_gemm_f32_skinny_finish");
+      return launch_finish(ctx, g, splits);
    }
    // (a bias given for every output element keeps to one launch)
    return launch_general(ctx, g, 1, bias_kind == SOFIE_BIAS_FULL);

@@ -25,17 +25,30 @@ struct Split8 {
    v8b h, m, l;
 };
 
-__device__ __forceinline__ Split8 split8(const float (&x)[8])
+// Eight numbers as h, m and l, two at a time: v_cvt_pk_bf16_f32, the two bf16 as fp32 by a shift and a mask, subtractions: eleven
+// instructions a pair (18 where the compiler converted each number by itself). x - h as a sum of products of bf16 (v_dot2c_f32_bf16, seven
+// a pair) waits for the matrix pipe: ns for each v_mfma_f32_16x16x32_bf16, two wavefronts on a SIMD: 7.4 alone, 7.5 with two
+// conversions or subtractions behind it, 9.1 with three; 14.6 with two dot products.
+__device__ __forceinline__ void split8(const float (&x)[8], v4i (&d)[3])
 {
-   Split8 s;
+   v4f r0, r1;
 #pragma unroll
-   for (int e = 0; e < 8; ++e) {
-      s.h[e] = (__bf16)x[e];
-      const float r = x[e] - (float)s.h[e];
-      s.m[e] = (__bf16)r;
-      s.l[e] = (__bf16)(r - (float)s.m[e]);
+   for (int p = 0; p < 4; ++p) {
+      r0[p] = x[2 * p];
+      r1[p] = x[2 * p + 1];
    }
-   return s;
+#pragma unroll
+   for (int part = 0; part < 3; ++part) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+         const unsigned both = f32x2_to_bf16x2(r0[p], r1[p]);
+         d[part][p] = (int)both;
+         if (part < 2) {
+            r0[p] -= __uint_as_float(both << 16);
+            r1[p] -= __uint_as_float(both & 0xffff0000u);
+         }
+      }
+   }
 }
 
 // The same for operands that are laid out once and read back as fp32 (joined) where sums are repeated: an x that is not finite is h
@@ -59,26 +72,6 @@ __device__ __forceinline__ Split8 split8_exact(const float (&x)[8])
 __device__ __forceinline__ float joined(__bf16 h, __bf16 m, __bf16 l)
 {
    return (float)h + ((float)m + (float)l);
-}
-
-// Sums over 32 k: the small products first.
-__device__ __forceinline__ v4f mma_split(const v8b (&a)[3], const v8b (&b)[3])
-{
-   v4f t = {0.0f, 0.0f, 0.0f, 0.0f};
-   t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[0], t, 0, 0, 0);
-   t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[2], t, 0, 0, 0);
-   t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[1], t, 0, 0, 0);
-   t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[0], t, 0, 0, 0);
-   t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], t, 0, 0, 0);
-   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[0], t, 0, 0, 0);
-}
-
-__device__ __forceinline__ bool not_finite(v4f v)
-{
-   bool bad = false;
-#pragma unroll
-   for (int e = 0; e < 4; ++e) bad = bad || (__float_as_uint(v[e]) & 0x7f800000u) == 0x7f800000u;
-   return bad;
 }
 
 }  // namespace sofie

@@ -1,0 +1,103 @@
+"""fp32 products on k_gemm_f32_split (operands as three bf16 numbers): every storage, 32, 64 and 96 rows per workgroup, K in slices, a K of
+one chunk per wavefront and less, rows, columns and K that are no whole fours, against float64; values that are not finite."""
+import ctypes as C
+
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from sofie_amd import lib as L  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from sofie_amd import ops as o
+    return o
+
+
+def product(ctx, a, b, tA, tB, bias, alpha=1.0, beta=1.0, relu=False, pad=0):
+    """The call through the C ABI, rows of all operands `pad` floats further apart than they are long; the result and the kernels' names."""
+    M, N, K = (a.shape[1] if tA else a.shape[0]), (b.shape[0] if tB else b.shape[1]), (a.shape[0] if tA else a.shape[1])
+
+    def wide(t):
+        if not pad:
+            return t
+        w = torch.full((t.shape[0], t.shape[1] + pad), float("nan"), device="cuda")
+        w[:, :t.shape[1]] = t
+        return w
+    a, b, y = wide(a), wide(b), torch.full((M + 2, N + pad), 77.0, device="cuda")
+    torch.cuda.synchronize()
+    buf, n = C.create_string_buffer(4096), C.c_int(-1)
+    ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+    ctx.check(ctx.lib.sofie_hip_gemm_f32(ctx.h, tA, tB, M, N, K, alpha, a.data_ptr(), a.shape[1], b.data_ptr(), b.shape[1], beta if bias is not None else 0.0,
+                                         bias.data_ptr() if bias is not None else None, L.BIAS_ROW if bias is not None else L.BIAS_NONE,
+                                         y[1].data_ptr(), N + pad, L.ACT_RELU if relu else L.ACT_NONE))
+    ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
+    ctx.sync()
+    assert bool((y[0] == 77.0).all() and (y[M + 1] == 77.0).all() and (y[:, N:] == 77.0).all())      # nothing around the result
+    return y[1:M + 1, :N], [line.split()[0] for line in buf.value.decode().splitlines()]
+
+
+# M, N, K; 32 rows per workgroup, 64, 96, K in slices; every storage
+SHAPES = [(64, 6208, 1106), (65, 6209, 1105), (112, 7656, 1284), (97, 6301, 1283), (1500, 1001, 1111), (1501, 1003, 1024), (1441, 1089, 258),
+          (1537, 1023, 257), (4624, 133, 5187), (130, 3633, 4279), (2447, 107, 5990)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_in_three_parts(ops, shape, tA, tB):
+    """Products of split numbers lose less than 2^-26 each and sums are rounded once per 32 k at their own size, where fp32 products in a
+    row are rounded K times: 3e-7 in the 2-norm and 1e-6 of the largest output (fp32 instructions show up to 1.2e-6 at these K).
+    The same bits on a second call."""
+    M, N, K = shape
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randn((K, M) if tA else (M, K), device="cuda", generator=g)
+    b = torch.randn((N, K) if tB else (K, N), device="cuda", generator=g) * K ** -0.5
+    bias = torch.randn(N, device="cuda", generator=g)
+    ref = (a.t() if tA else a).double().contiguous() @ (b.t() if tB else b).double().contiguous()
+    ctx = ops.Context(0)
+    y, names = product(ctx, a, b, tA, tB, bias)
+    want = ref + bias.double()
+    if "k_gemm_f32_split" in names:
+        err = y.double() - want
+        assert float(err.norm()) <= 3e-7 * float(want.norm()) and float(err.abs().max()) <= 1e-6 * float(want.abs().max())
+    else:      # (operands stored along M take 64 rows or nothing)
+        assert tA or K < 300, names
+    assert torch.equal(y, product(ctx, a, b, tA, tB, bias)[0])
+    y, _ = product(ctx, a, b, tA, tB, bias, alpha=-0.5, beta=2.0, relu=True, pad=3)
+    want = (-0.5 * ref + 2.0 * bias.double()).clamp(min=0)
+    assert float((y.double() - want).abs().max()) <= 1e-6 * float(want.abs().max())
+    ctx.close()
+
+
+@pytest.mark.parametrize("tB", [0, 1])
+def test_gemm_in_three_parts_of_values_that_are_not_finite(ops, tB):
+    """Infinities, NaN and sums that overflow stay where fp32 products put them, and finite ones next to them stay right; numbers that
+    bf16 would round up to infinity are finite."""
+    M, N, K = 1500, 1001, 1111
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g)
+    a[3, 7], a[700, 1110], a[1499, 0], a[900, 50], b[50, 1000] = float("inf"), float("nan"), float("-inf"), 3.4e38, 0.25
+    a[40, :] = 0.0
+    a[40, 9], b[9, 33] = 1.0, 3.4028234e38
+    a[41, :] = 3e38
+    b[:, 500] = 1.0
+    ctx = ops.Context(0)
+    y, names = product(ctx, a, b.t().contiguous() if tB else b, 0, tB, None)
+    assert "k_gemm_f32_split" in names, names
+    rows = [3, 40, 41, 700, 900, 1499, 0, 1, 64, 1498]
+    ref = a[rows].cpu().double() @ b.cpu().double()
+    got = y[rows].cpu()
+    ref32 = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+    for i, r in enumerate(rows):
+        if r == 41:      # sums of 3e38 times anything: only the one that must overflow
+            assert float(got[i, 500]) == float("inf")
+            continue
+        assert torch.equal(got[i].isnan(), ref32[i].isnan()), r
+        assert torch.equal(got[i].isinf(), ref32[i].isinf()), r
+        assert torch.equal(torch.sign(got[i][got[i].isinf()]).double(), torch.sign(ref32[i][ref32[i].isinf()])), r
+        fin = ref32[i].isfinite()
+        if bool(fin.any()):
+            assert float((got[i][fin].double() - ref32[i][fin]).abs().max()) <= 1e-5 * float(ref32[i][fin].abs().max()), r
+    ctx.close()
