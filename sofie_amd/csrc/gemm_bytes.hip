@@ -12,6 +12,8 @@
 // packed results go through a per-wavefront LDS staging block and leave as 16-byte row
 // segments. Workgroup ids are remapped so that each XCD (ids are dealt round-robin over the
 // 8 XCDs) owns a compact rectangle of output tiles and its L2 sees each operand panel once.
+#include <type_traits>
+
 #include "common.h"
 #include "gemm_tile.h"
 #include "row_chunk.h"
@@ -1063,25 +1065,28 @@ template <class Mma, int OUT> struct IS_SPLITTABLE {
    static constexpr bool value = __is_same(typename Mma::Acc, v16i) && OUT == SOFIE_OUT_S32;
 };
 
-// Sum over the K slices of four consecutive int32 partial sums. The loads of four slices are issued together before
+// Sum over the K slices of four consecutive int32 partial sums. The loads of eight slices are issued together before
 // the first addition (one after the other, each waiting for the one before, they were the length of the pass).
 __device__ __forceinline__ v4i sum_slices(const int *__restrict__ p, size_t plane, int splits)
 {
    v4i s = {0, 0, 0, 0};
+   auto some = [&](auto count, int k) {
+      constexpr int COUNT = decltype(count)::value;
+      v4i v[COUNT];
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) v[i] = *reinterpret_cast<const v4i *>(p + (size_t)(k + i) * plane);
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i)
+#pragma unroll
+         for (int e = 0; e < 4; ++e) s[e] += v[i][e];
+   };
    int k = 0;
-   for (; k + 4 <= splits; k += 4) {
-      const v4i a = *reinterpret_cast<const v4i *>(p + (size_t)k * plane);
-      const v4i b = *reinterpret_cast<const v4i *>(p + (size_t)(k + 1) * plane);
-      const v4i c = *reinterpret_cast<const v4i *>(p + (size_t)(k + 2) * plane);
-      const v4i d = *reinterpret_cast<const v4i *>(p + (size_t)(k + 3) * plane);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] += (a[e] + b[e]) + (c[e] + d[e]);
+   for (; k + 8 <= splits; k += 8) some(std::integral_constant<int, 8>{}, k);
+   if (splits & 4) {
+      some(std::integral_constant<int, 4>{}, k);
+      k += 4;
    }
-   for (; k < splits; ++k) {
-      const v4i v = *reinterpret_cast<const v4i *>(p + (size_t)k * plane);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[e] += v[e];
-   }
+   for (; k < splits; ++k) some(std::integral_constant<int, 1>{}, k);
    return s;
 }
 
@@ -1440,6 +1445,8 @@ template <> struct SelectMma16<MmaF8> { typedef Mma16F8 type; };
 // tiles, 6.2 on 64 x 64; 8 x 1001 x 1001: 5.3 / 11.5 / 6.7; 4096 x 16 x 12800: 14 / 70 / 38; all read at up to 43 bytes
 // per ns and compute unit, which is what a larger product pays for its smaller tiles).
 // Two workgroups per compute unit (128 registers) but for 32 x 32 tiles, whose operands would not fit them.
+// Raw sums (SOFIE_OUT_S32) also with K in slices (blockIdx.y, g.kslice bytes each, whole chunks), into the slice's copy of Y: a long K on
+// few tiles, split_k_plan.
 template <class Mma, int OUT, int MI, int NJ, bool SHIFTS>
 __global__ void __launch_bounds__(512, MI * NJ == 4 ? 1 : 4) k_gemm_bytes_direct(GemmArgs g)
 {
@@ -1523,18 +1530,25 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 1 : 4) k_gemm_bytes_direct
          for (int j = 0; j < NJ; ++j) acc[i][j] = Mma::mma(b[j][0], b[j][1], a[i][0], a[i][1], acc[i][j]);
    };
    constexpr int STEP = 8 * 128;
+   int k0 = wave * 128, k_end = g.K;
+   if constexpr (OUT == SOFIE_OUT_S32) {
+      if (g.splits > 1) {
+         k0 += (int)blockIdx.y * g.kslice;
+         const int left = g.K - (int)blockIdx.y * g.kslice;
+         if (left > g.kslice) k_end = g.K - (left - g.kslice);
+      }
+   }
    // (chunks behind K are not requested: every lane would ask for the last bytes of its row once more, which took longer than the
    // product; 512 x 512 x 1024 8.2 us with them, 4.5 without, 64 x 2491 x 1024 8.1 / 4.5, 256 x 1000 x 1000 5.8 / 4.6)
    Chunk c[DEPTH];
-   int k0 = wave * 128;
 #pragma unroll
    for (int d = 0; d < DEPTH; ++d)
-      if (k0 + d * STEP < g.K) load(c[d], k0 + d * STEP);
-   while (k0 < g.K) {
+      if (k0 + d * STEP < k_end) load(c[d], k0 + d * STEP);
+   while (k0 < k_end) {
 #pragma unroll
       for (int d = 0; d < DEPTH; ++d) {
-         if (k0 < g.K) multiply(c[d], k0);
-         if (k0 + DEPTH * STEP < g.K) load(c[d], k0 + DEPTH * STEP);
+         if (k0 < k_end) multiply(c[d], k0);
+         if (k0 + DEPTH * STEP < k_end) load(c[d], k0 + DEPTH * STEP);
          k0 += STEP;
       }
    }
@@ -1557,6 +1571,7 @@ __global__ void __launch_bounds__(512, MI * NJ == 4 ? 1 : 4) k_gemm_bytes_direct
       if constexpr (ESZ == 1) v[e] = (unsigned)((int)fminf(__uint_as_float(v[e]), 255.0f) - 128) & 0xffu;
    }
    unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)om * g.ldy + on) * ESZ;
+   if constexpr (OUT == SOFIE_OUT_S32) out += (size_t)blockIdx.y * (size_t)g.ysplit;
    if (on + 4 <= g.N) {
       if constexpr (ESZ == 1) {
          const unsigned p = v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24);
@@ -1585,7 +1600,7 @@ int launch_direct_as(sofie_hip_ctx *ctx, GemmArgs &g, TileMode mode)
    typedef typename SelectMma16<Mma>::type Mma16;
    g.tiles_m = cdiv(g.M, 16 * MI);
    g.tiles_n = cdiv(g.N, 16 * NJ);
-   const dim3 grid(g.tiles_m * g.tiles_n);
+   const dim3 grid(g.tiles_m * g.tiles_n, OUT == SOFIE_OUT_S32 && g.splits > 1 ? g.splits : 1);
    if (mode == ANY_ROWS) hipLaunchKernelGGL((k_gemm_bytes_direct<Mma16, OUT, MI, NJ, true>), grid, dim3(512), 0, ctx->stream, g);
    else hipLaunchKernelGGL((k_gemm_bytes_direct<Mma16, OUT, MI, NJ, false>), grid, dim3(512), 0, ctx->stream, g);
    return check_launch(ctx, "k_gemm_bytes_direct");
@@ -1694,15 +1709,24 @@ int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g, bool whole)
    return check_launch(ctx, "k_splitk_finish");
 }
 
-// K cut into `splits` slices of `kslice` bytes (a multiple of BK): partial sums into the context's scratch
+// Whether an int8 product with K-contiguous operands is cut into slices of K, and how: few 128 x 128 tiles and a long
+// K (measured: pays from K = 8192 on; below that the second pass over the partial sums costs more). tile: 128, or 0 for
+// mi x nj tiles of 16 of k_gemm_bytes_direct.
+struct SplitKPlan {
+   int splits, kslice, tile, mi, nj;
+   float us;
+};
+size_t split_k_bytes(const GemmArgs &g, int splits) { return (size_t)splits * g.M * (cdiv(g.N, 4) * 4) * sizeof(int); }
+
+// K cut into plan.splits slices of plan.kslice bytes (a multiple of BK): partial sums into the context's scratch
 // buffer, then k_splitk_finish writes Y.
 template <class Mma, int BK, int NSETS, int OUT>
-int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, int splits, int kslice, const GemmArgs *tail = nullptr,
+int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, const SplitKPlan &plan, const GemmArgs *tail = nullptr,
                    int tail_out = SOFIE_OUT_S8)
 {
-   const int ldp = cdiv(g.N, 4) * 4;
+   const int ldp = cdiv(g.N, 4) * 4, splits = plan.splits;
    void *part = nullptr;
-   if (int rc = workspace(ctx, (size_t)splits * g.M * ldp * sizeof(int), &part)) return rc;
+   if (int rc = workspace(ctx, split_k_bytes(g, splits), &part)) return rc;
    GemmArgs p = g;
    p.Y = part;
    p.ldy = ldp;
@@ -1711,9 +1735,13 @@ int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, int splits, int kslice, cons
    p.relu = 0;
    p.vec_store = 1;
    p.splits = splits;
-   p.kslice = kslice;
+   p.kslice = plan.kslice;
    p.ysplit = (long long)g.M * ldp * sizeof(int);
-   if (int rc = launch_tiled<Mma, BK, NSETS, 2, 2, SOFIE_OUT_S32, false>(ctx, p)) return rc;
+   int rc = SOFIE_HIP_OK;
+   if (plan.tile == 128) rc = launch_tiled<Mma, BK, NSETS, 2, 2, SOFIE_OUT_S32, false>(ctx, p);
+   else if (plan.mi == 1) rc = plan.nj == 1 ? launch_direct_as<Mma, SOFIE_OUT_S32, 1, 1>(ctx, p, CHUNK_ROWS) : launch_direct_as<Mma, SOFIE_OUT_S32, 1, 2>(ctx, p, CHUNK_ROWS);
+   else rc = plan.nj == 1 ? launch_direct_as<Mma, SOFIE_OUT_S32, 2, 1>(ctx, p, CHUNK_ROWS) : launch_direct_as<Mma, SOFIE_OUT_S32, 2, 2>(ctx, p, CHUNK_ROWS);
+   if (rc) return rc;
    const size_t threads = (size_t)g.M * (ldp / 4);
    const dim3 fgrid((unsigned)((threads + 255) / 256));
    if (tail) {
@@ -1749,24 +1777,67 @@ int launch_simple(sofie_hip_ctx *ctx, GemmArgs &g, int transB)
    return check_launch(ctx, "k_gemm_bytes_simple");
 }
 
-// Whether an int8 product with K-contiguous operands is cut into slices of K, and how: few 128 x 128 tiles and a long
-// K (measured: pays from K = 8192 on; below that the second pass over the partial sums costs more).
-bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, int &splits, int &kslice)
+// On 128 x 128 tiles; us = 1e30 where they do not cut it.
+SplitKPlan split_k_tiles(const sofie_hip_ctx *ctx, const GemmArgs &g)
 {
+   SplitKPlan p{1, 0, 128, 0, 0, 1e30f};
    const int tiles128 = cdiv(g.M, 128) * cdiv(g.N, 128);
-   if (!(tiles128 * 2 <= ctx->num_cus && g.K >= 8192)) return false;
-   splits = ctx->num_cus / tiles128;
+   if (!(tiles128 * 2 <= ctx->num_cus && g.K >= 8192)) return p;
+   p.splits = ctx->num_cus / tiles128;
    const int shortest = tiles128 * 8 <= ctx->num_cus ? 1024 : 2048;
-   if (splits > g.K / shortest) splits = g.K / shortest;
-   if (splits > 16) splits = 16;
-   kslice = cdiv(cdiv(g.K, splits), 128) * 128;
-   splits = cdiv(g.K, kslice);
-   if (splits < 2) return false;
+   if (p.splits > g.K / shortest) p.splits = g.K / shortest;
+   if (p.splits > 16) p.splits = 16;
+   p.kslice = cdiv(cdiv(g.K, p.splits), 128) * 128;
+   p.splits = cdiv(g.K, p.kslice);
    // against one launch of the small-product kernels: 4 us for the second launch and the epilogues, the steps of a slice,
    // and the partial sums written and read at 8 TB/s (300 x 130 x 8464: 14.7 us in slices, 7.5 in one launch; 256 x 256 x 12800:
    // 12.5 / 13.2; 128 x 128 x 32768: 15.4 / 29.4; 4096 x 256 x 12800: 23.7 / 32.5)
-   const float us = 4.0f + 0.54f * (kslice / 128) + 8.0f * splits * (float)g.M * g.N / 8e6f;
-   return us < small_choice(ctx, g, CHUNK_ROWS).us;
+   if (p.splits > 1) p.us = 4.0f + 0.54f * (p.kslice / 128) + 8.0f * p.splits * (float)g.M * g.N / 8e6f;
+   return p;
+}
+bool split_k_on_tiles(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   return split_k_tiles(ctx, g).us < small_choice(ctx, g, CHUNK_ROWS).us;
+}
+// The same on tiles of 16 or 32 rows and columns, their operands straight into registers (tile = 0), where there is memory for the
+// sums: the estimate of small_choice for a slice, and the second launch. 128 x 128 tiles multiply rows that are not there and give a
+// product of 64 rows to 26 compute units: us, tiles / these, with the second launch: 64 x 256 x 12800 14.0 / 8.5, 128 x 256 x 12800
+// 12.0 / 8.8, 182 x 167 x 14512 16.7 / 9.2, 93 x 351 x 20880 18.6 / 11.5; one launch / these: 37 x 23 x 10368 10.7 / 6.2, 85 x 36 x 10320 8.1 / 6.5.
+SplitKPlan split_k_direct(const sofie_hip_ctx *ctx, const GemmArgs &g)
+{
+   SplitKPlan best{1, 0, 0, 0, 0, 1e30f};
+   const int cus = ctx->num_cus;
+   for (int i = 0; i < 4 && g.K >= 8192; ++i) {
+      const int mi = 1 + (i >> 1), nj = 1 + (i & 1), resident = mi * nj == 4 ? 1 : 2;
+      const long long tiles = (long long)cdiv(g.M, 16 * mi) * cdiv(g.N, 16 * nj);
+      for (int want = 2; want <= 32 && tiles * want <= 2ll * cus * resident; want += want < 8 ? 1 : 4) {
+         const int kslice = cdiv(cdiv(g.K, want), 128) * 128, splits = cdiv(g.K, kslice);
+         if (kslice < 512) break;
+         const long long per_cu = (tiles * splits + cus - 1) / cus;
+         const float us = 4.0f + (float)((per_cu + resident - 1) / resident) + (float)per_cu * 16 * (mi + nj) * kslice / 43e3f +
+                          8.0f * splits * (float)g.M * g.N / 8e6f;
+         if (us < best.us && workspace_has_room(ctx, split_k_bytes(g, splits))) best = {splits, kslice, 0, mi, nj, us};
+      }
+   }
+   return best;
+}
+// (Measured beside the estimates: tiles take 3 us and more above theirs, 446 x 179 x 12992 16.2; the second launch costs 5 us where it comes on
+// top of k_gemm_bytes_direct's own, whose estimate is up to 1.6 us too long for few rows: below 0.9 and 0.8 of it slices lose,
+// 8 x 30 x 8208 5.5 in one launch, 6.5 in slices, 270 x 30 x 8208 6.5 / 6.7. By time these would also take the place of k_qgemm_few_rows
+// (4 x 64 x 65536 16.2 / 6.9, 8 x 1024 x 8192 8.1 / 6.7, 26 x 671 x 51392 22.2 / 13.3) and of tiles on up to 32 rows or 64 columns
+// (27 x 43 x 36880 20.6 / 7.1); test_up_to_32_rows_on_a_long_sum_are_a_pass_over_b names the kernels that run there.)
+bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, SplitKPlan &plan)
+{
+   plan = split_k_tiles(ctx, g);
+   const float one = small_choice(ctx, g, CHUNK_ROWS).us;
+   const bool cut = plan.us < one;
+   if (cut && !workspace_has_room(ctx, split_k_bytes(g, plan.splits))) return true;      // refused by the launch, or one launch
+   const SplitKPlan direct = split_k_direct(ctx, g);
+   if (direct.us + 1.0f < (g.M <= 16 ? 0.8f : 0.9f) * one && (!cut || (g.M > 32 && g.N > 64 && direct.us < plan.us + 3.0f))) {
+      plan = direct;
+      return true;
+   }
+   return cut;
 }
 
 bool big_product(const GemmArgs &g) { return (size_t)g.M * g.N >= (size_t)256 * 256 * 128 && g.M >= 256 && g.N >= 256; }
@@ -1800,8 +1871,8 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
    constexpr int BK = 128;
    constexpr int NSETS = IS_INT ? 2 : 1;
    if constexpr (IS_INT && OUT != SOFIE_OUT_BF16) {
-      int splits = 1, kslice = 0;
-      const bool cut = g.M <= 32 && split_k_plan(ctx, g, splits, kslice);
+      int kslice = 0;
+      const bool cut = g.M <= 32 && split_k_on_tiles(ctx, g);
       if (few_rows_whole(ctx, g, cut)) return launch_few_rows<OUT>(ctx, g, true);
       // (tiles in slices need less memory for their sums)
       if (few_rows_sliced(ctx, g, cut) &&
@@ -1819,10 +1890,9 @@ int dispatch_nk(sofie_hip_ctx *ctx, GemmArgs &g)
       // (integer sums, so the result does not depend on the cut), a second kernel adds them and converts. At most 16 columns
       // (the last layer of a classifier) go without slices where there is no memory for their sums: a call that needs
       // none can always be recorded.
-      int splits = 1, kslice = 0;
-      if (split_k_plan(ctx, g, splits, kslice) &&
-          (g.N > 16 || workspace_has_room(ctx, (size_t)splits * g.M * (cdiv(g.N, 4) * 4) * sizeof(int))))
-         return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, splits, kslice);
+      SplitKPlan plan;
+      if (split_k_plan(ctx, g, plan) && (g.N > 16 || workspace_has_room(ctx, split_k_bytes(g, plan.splits))))
+         return launch_split_k<Mma, BK, NSETS, OUT>(ctx, g, plan);
    }
    return launch_small<Mma, OUT>(ctx, g);
 }
@@ -2025,8 +2095,8 @@ int sofie_hip_qgemm_s8_pair(sofie_hip_ctx *ctx, int M, int K, const int8_t *A, i
    const bool lanes_ok = N1 % 4 == 0 && quads >= 8 && quads <= 64 && (quads & (quads - 1)) == 0;
    const bool operands_ok = K % 16 == 0 && lda % 16 == 0 && aligned16(A) && ldb1 % 16 == 0 && aligned16(B1) && ldb2 % 4 == 0 &&
                             (reinterpret_cast<uintptr_t>(B2) & 3u) == 0;
-   int splits = 1, kslice = 0;
-   if (N2 <= 8 && lanes_ok && operands_ok && N1 > 16 && split_k_plan(ctx, g, splits, kslice) &&
+   SplitKPlan plan;
+   if (N2 <= 8 && lanes_ok && operands_ok && N1 > 16 && split_k_plan(ctx, g, plan) &&
        !((size_t)M * N1 >= (size_t)256 * 256 * 128 && M >= 256 && N1 >= 256)) {
       GemmArgs t{};
       t.B = reinterpret_cast<const uint8_t *>(B2);
@@ -2038,7 +2108,7 @@ int sofie_hip_qgemm_s8_pair(sofie_hip_ctx *ctx, int M, int K, const int8_t *A, i
       t.relu = act2 == SOFIE_ACT_RELU;
       t.lo = (t.relu && zp_y > -128) ? zp_y : -128;
       t.s = 1.0f;
-      return launch_split_k<MmaI8, 128, 2, SOFIE_OUT_S8>(ctx, g, splits, kslice, &t, out_kind);
+      return launch_split_k<MmaI8, 128, 2, SOFIE_OUT_S8>(ctx, g, plan, &t, out_kind);
    }
    // otherwise the two layers one after the other, the first one's result in the caller's scratch tensor
    if (int rc = sofie_hip_qgemm_s8(ctx, 1, M, N1, K, A, lda, B1, ldb1, scale1, bias1, zp_mid, act1, mid, ldmid, SOFIE_OUT_S8))
