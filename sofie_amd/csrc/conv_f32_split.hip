@@ -13,6 +13,15 @@
 //   * W: a copy laid out as fragments of split numbers [16 channels][step][h, m, l][lane], once per tensor under the
 //     constant-weights promise, else in front of the launch. Straight into registers, a step ahead.
 //   * Pixels run over all images in one row, or, where that costs little, tiles end with an image; wide images are cut into strips.
+// Few channels and a large kernel (ROWS; the first layer of an image network): eight channels of a cell would be mostly zeros. There a cell
+// is the eight values that a row of the kernel meets at an output column, of one channel; a chunk of K is a row of the kernel, zeros up
+// to eight columns, K = (channel, kernel row, kernel column) in one slot. A value is split once per output column it
+// is read at, still shared by the kernel's rows. Loaded as two 16-byte pieces from any dword; columns outside the image are zeroed behind
+// the load. 16x3x224x224 -> 64, 7x7 s2 52.6 -> 32.6 us (k_conv_f32_any, 53 % of the fp32 instructions' rate); 53 of 90 random layers of
+// one to five channels and kernels of 4 to 7 columns, 1.3 times shorter in the mean (55x5x38x38 -> 146, 7x7 s2 35.9 -> 18.1; 126x1x66x66 ->
+// 54, 7x7 66.8 -> 57). Relative error against 64 bits 5e-8 to 9e-8 (1.1e-7 to 3.1e-7 before).
+// Strips of an image take turns: neighbouring ones write halves of the same 128-byte lines, which one behind the other meet in an
+// L2 (88x1x96x96 -> 150, 7x7 in strips of 16 columns 248 us strip by strip, 196 in turns).
 // All requests of a slot leave in one step: the fragments behind them wait for them (loads return in order), and one such wait
 // per slot is cheaper than one per step. A bias read behind the loop made the compiler wait for each store in front of the next one
 // (13000 cycles for 16 stores instead of 6800).
@@ -41,7 +50,8 @@ constexpr int CELL = 48;                       // LDS bytes of 8 channels of a c
 constexpr int THREADS = 256;
 
 // Cells x 8 channels of a slot that a thread carries, at most: registers, which decide how many workgroups share a compute unit.
-constexpr int items_of(int ti, int tj, int wo) { return wo == 1 ? 4 : ti * tj > 8 ? 3 : 2; }
+// (Rows of a kernel as cells: one slot, whose registers are free again in front of the loop.)
+constexpr int items_of(int ti, int tj, int wo, bool rows) { return rows || wo == 1 ? 4 : ti * tj > 8 ? 3 : 2; }
 // Workgroups a compute unit holds at once, by registers.
 constexpr int resident_of(int ti, int tj, int wo) { return ti * tj > 8 ? 2 : ti * tj > 4 || wo == 1 ? 3 : 4; }
 
@@ -57,7 +67,8 @@ struct SplitPhase {
    int OW;
    int oy0, oys, ox0, oxs;
    int th0, ths, tw0, tws;
-   FastDiv dPHW, dWS, dHP, dPW, dStrips, dTaps, dKW, dCells;
+   int tiles;                 // of a panel, where it is whole tiles and not the only one of its image: strips take turns; else 0
+   FastDiv dTiles, dPHW, dWS, dHP, dPW, dStrips, dTaps, dKW, dCells;
 };
 
 struct SplitArgs {
@@ -77,11 +88,11 @@ struct SplitArgs {
 
 enum { PIXELS, QUADS };
 
-template <int TI, int TJ, int WO, int STORE, bool PHASES>
+template <int TI, int TJ, int WO, int STORE, bool PHASES, bool ROWS>
 __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_split(SplitArgs g)
 {
    extern __shared__ __align__(16) unsigned char smem_raw[];
-   constexpr int BP = 4 / WO * TJ * 16, ITEMS = items_of(TI, TJ, WO);
+   constexpr int BP = 4 / WO * TJ * 16, ITEMS = items_of(TI, TJ, WO, ROWS);
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = wave % WO;
    // workgroup id -> (pixels, channels, phase): an XCD (an L2) works on consecutive ids; the phases of a tile, which read the same
@@ -102,7 +113,12 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
       for (int i = 1; i < MAX_PHASES; ++i)
          if (phase == i) q = g.phase[i];
    }
-   const int pb = fdiv(pid, g.dOB), ob = pid - pb * g.oblocks * g.groups;
+   int pb = fdiv(pid, g.dOB);
+   const int ob = pid - pb * g.oblocks * g.groups;
+   if (q.tiles > 0) {         // (n, tile, strip) -> (n, strip, tile)
+      const int n = fdiv(pb, q.dTiles), r = pb - n * q.strips * q.tiles, t = fdiv(r, q.dStrips);
+      pb = (n * q.strips + r - t * q.strips) * q.tiles + t;
+   }
    const int grp = ob / g.oblocks, tile0 = (ob - grp * g.oblocks) * TI * WO + wo * TI;
    const int p0 = pb * BP;
    if (p0 >= q.P) return;
@@ -113,12 +129,19 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
    }
    unsigned char *const patch = smem_raw + g.table_bytes;
    unsigned voff[ITEMS];
+   int column[ITEMS];         // ROWS: of the cell's first value
    const int items = q.cells * (g.CS >> 3);
 #pragma unroll
    for (int s = 0; s < ITEMS; ++s) {
       const int item = s * THREADS + tid, c8 = fdiv(item, q.dCells), cell = item - c8 * q.cells, row = fdiv(cell, q.dPW), col = cell - row * q.PW;
       const int grow = origin + row, panel = fdiv(grow, q.dHP), n = fdiv(panel, q.dStrips);
-      const int iy = grow - panel * q.HP - q.ph, ix = (panel - n * q.strips) * q.ws * g.sw + col - q.pw;
+      const int iy = grow - panel * q.HP - q.ph, ix = ((panel - n * q.strips) * q.ws + (ROWS ? col : 0)) * g.sw + (ROWS ? 0 : col) - q.pw;
+      if constexpr (ROWS) {
+         const bool row_there = item < items && panel < q.panels && (unsigned)iy < (unsigned)g.H;
+         column[s] = row_there ? ix : -(1 << 28);
+         voff[s] = row_there ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + (grp * g.icg + c8) * g.hw4) : OUTSIDE;
+         continue;
+      }
       const bool in = item < items && panel < q.panels && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
       voff[s] = in ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + c8 * 8 * g.hw4) : OUTSIDE;
    }
@@ -140,10 +163,40 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
             xr[s][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(e < left ? voff[s] : OUTSIDE), (int)(e < rem ? soff + e * (unsigned)g.hw4 : 0u), 0));
       }
    };
+   // ROWS: eight values of a row at once, those that are not there (and where a cell begins in front of the tensor or ends behind
+   // it, each by itself); put() leaves the columns of the image and of the kernel
+   auto fetch_rows = [&](float (&xr)[ITEMS][8]) {
+      bool edge = g.dw != 1;
+#pragma unroll
+      for (int s = 0; s < ITEMS; ++s) edge |= (int)voff[s] < 0 || (voff[s] != OUTSIDE && voff[s] + 32u > g.xbytes);
+      if (__builtin_amdgcn_ballot_w64(edge) != 0) {
+#pragma unroll
+         for (int s = 0; s < ITEMS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+               xr[s][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)((unsigned)(column[s] + e * g.dw) < (unsigned)g.W ? voff[s] + (unsigned)(e * g.dw * 4) : OUTSIDE), 0, 0));
+         return;
+      }
+#pragma unroll
+      for (int s = 0; s < ITEMS; ++s)
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            const v4f v = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)voff[s], 16 * h, 0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xr[s][4 * h + e] = v[e];
+         }
+   };
    auto put = [&](const float (&xr)[ITEMS][8], int s, unsigned char *buf) {
       if (s * THREADS + tid >= items) return;
       v4i v[3];
-      split8(xr[s], v);
+      if constexpr (ROWS) {
+         float there[8];
+#pragma unroll
+         for (int e = 0; e < 8; ++e) there[e] = e < q.KW && (unsigned)(column[s] + e * g.dw) < (unsigned)g.W ? xr[s][e] : 0.0f;
+         split8(there, v);
+      } else {
+         split8(xr[s], v);
+      }
       v4i *const d = reinterpret_cast<v4i *>(buf + (s * THREADS + tid) * CELL);
       d[0] = v[0];
       d[1] = v[1];
@@ -163,10 +216,14 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
    };
    // everything that comes from memory is requested first; what the loop needs besides is worked out while it travels
    float second[ITEMS][8];
+   if constexpr (ROWS) {
+      fetch_rows(xr);
+   } else {
 #pragma unroll
-   for (int s = 0; s < ITEMS; ++s)
-      if (s * THREADS < items) fetch(xr, s, 0);
-   if (g.nslots > 1) {
+      for (int s = 0; s < ITEMS; ++s)
+         if (s * THREADS < items) fetch(xr, s, 0);
+   }
+   if (!ROWS && g.nslots > 1) {
 #pragma unroll
       for (int s = 0; s < ITEMS; ++s)
          if (s * THREADS < items) fetch(second, s, 1);
@@ -188,14 +245,14 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
    // offset of every chunk of two slots (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
    // first chunks)
    for (int e = tid; e < 2 * q.chunks; e += THREADS) {
-      const int second = e >= q.chunks, k = second ? e - q.chunks : e, c8 = fdiv(k, q.dTaps), t = k - c8 * taps, a = fdiv(t, q.dKW), b = t - a * q.KW;
+      const int second = e >= q.chunks, k = second ? e - q.chunks : e, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
       table[e] = (c8 * q.cells + a * g.dh * q.PW + b * g.dw) * CELL + (g.nslots > 1 ? second * g.slot_bytes : 0);
    }
    int base[TJ];
 #pragma unroll
    for (int j = 0; j < TJ; ++j) {
       const int p = p0 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), c = r - oy * q.ws;
-      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh - origin) * q.PW + c * g.sw) * CELL : 0;
+      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh - origin) * q.PW + (ROWS ? c : c * g.sw)) * CELL : 0;
    }
    v4f acc[TI][TJ];
 #pragma unroll
@@ -205,7 +262,7 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
 #pragma unroll
    for (int s = 0; s < ITEMS; ++s)
       if (s * THREADS < items) put(xr, s, patch);
-   if (g.nslots > 1) {
+   if (!ROWS && g.nslots > 1) {
 #pragma unroll
       for (int s = 0; s < ITEMS; ++s)
          if (s * THREADS < items) put(second, s, patch + g.slot_bytes);
@@ -223,7 +280,7 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
       for (int p = 0; p < 3; ++p) x[j][p] = *reinterpret_cast<const v8b *>(patch + base[j] + off + p * 16);
    };
    for (int slot = 0; slot < g.nslots; ++slot) {
-      const bool last = slot + 1 == g.nslots, more = slot + 2 < g.nslots;
+      const bool last = ROWS || slot + 1 == g.nslots, more = !ROWS && slot + 2 < g.nslots;
       const int end_chunk = q.chunks * (slot + 1), end = last ? q.steps : (end_chunk + 3) >> 2;
       const bool across = !last && (end_chunk & 3) != 0;      // the last step takes chunks of the next slot, too
       const int begin = step;
@@ -303,8 +360,8 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
                   const int a = fdiv(t, q.dKW), b = t - a * q.KW, iy = iy0 + a * g.dh, ix = ix0 + b * g.dw;
                   const bool in = p < q.P && r < q.full && c < g.icg && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
                   const float xv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + (grp * g.icg + c) * g.hw4) : OUTSIDE), 0, 0));
-                  const int chunk = (c >> 3) * taps + t;
-                  const unsigned wat = wofs[i] + (unsigned)((chunk >> 2) * 3072 + ((chunk & 3) * 16 + r16) * 16 + (c & 7) * 2);
+                  const int chunk = ROWS ? c * q.KH + a : (c >> 3) * taps + t;
+                  const unsigned wat = wofs[i] + (unsigned)((chunk >> 2) * 3072 + ((chunk & 3) * 16 + r16) * 16 + (ROWS ? b : c & 7) * 2);
                   __bf16 part[3];
 #pragma unroll
                   for (int e = 0; e < 3; ++e)
@@ -356,7 +413,7 @@ __global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_s
 struct SplitWeightArgs {
    const float *w;
    v4i *dst;
-   int icg, ocg, octiles, KH0, KW0, transposed, total;      // total: triples of 16-byte pieces over all phases
+   int icg, ocg, octiles, KH0, KW0, transposed, rows, total;      // total: triples of 16-byte pieces over all phases
    SplitPhase phase[MAX_PHASES];
 };
 
@@ -374,15 +431,15 @@ __global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs 
    r >>= 6;
    const int step = r % q.steps, tile = r / q.steps;
    const int oc = (tile % g.octiles) * 16 + (lane & 15), grp = tile / g.octiles;
-   const int chunk = 4 * step + (lane >> 4), c8 = fdiv(chunk, q.dTaps), t = chunk - c8 * q.KH * q.KW;
-   const int ta = fdiv(t, q.dKW), a = q.th0 + ta * q.ths, b = q.tw0 + (t - ta * q.KW) * q.tws;
+   const int chunk = 4 * step + (lane >> 4), c8 = fdiv(chunk, q.dTaps), t = chunk - c8 * q.KH * (g.rows ? 1 : q.KW);
+   const int ta = g.rows ? t : fdiv(t, q.dKW), a = q.th0 + ta * q.ths, b = g.rows ? 0 : q.tw0 + (t - ta * q.KW) * q.tws;
    float v[8];
 #pragma unroll
    for (int e = 0; e < 8; ++e) {
-      const int ic = c8 * 8 + e;
-      const bool in = oc < g.ocg && ic < g.icg;
+      const int ic = g.rows ? c8 : c8 * 8 + e;
+      const bool in = oc < g.ocg && ic < g.icg && (!g.rows || e < q.KW);
       const size_t at = !in ? 0 : g.transposed ? ((size_t)(grp * g.icg + ic) * g.ocg + oc) : ((size_t)(grp * g.ocg + oc) * g.icg + ic);
-      v[e] = in ? g.w[(at * g.KH0 + a) * g.KW0 + b] : 0.0f;
+      v[e] = in ? g.w[(at * g.KH0 + a) * g.KW0 + (g.rows ? e : b)] : 0.0f;
    }
    const Split8 s = split8_exact(v);
    v4i *d = g.dst + q.wofs + ((size_t)tile * q.steps + step) * 192 + lane;
@@ -393,15 +450,16 @@ __global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs 
 
 struct Form {
    int ti, tj, wo, cs, strips;
+   bool rows;
    int pixels() const { return 64 / wo * tj; }
    int channels() const { return 16 * wo * ti; }
-   int items() const { return items_of(ti, tj, wo); }
+   int items() const { return items_of(ti, tj, wo, rows); }
    double time;
 };
 
 // Geometry of the problem for tiles of bp pixels, slots of cs channels and images in strips; false where a slot is more than the
 // threads of a workgroup carry, or than the LDS holds. pieces: 16-byte pieces of the fragments (which do not depend on cs and strips).
-bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int strips, size_t *pieces)
+bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int strips, bool rows, size_t *pieces)
 {
    g.CS = cs;
    g.nslots = cdiv(g.icg, cs);
@@ -411,7 +469,7 @@ bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int 
    for (int i = 0; i < p.nphases; ++i) {
       const ConvPhase &f = p.phase[i];
       SplitPhase &q = g.phase[i];
-      const int taps = f.KH * f.KW;
+      const int taps = f.KH * (rows ? 1 : f.KW);
       q.KH = f.KH; q.KW = f.KW; q.ph = f.ph; q.pw = f.pw;
       q.OW = f.OW;
       q.ws = cdiv(f.OW, strips);
@@ -421,7 +479,7 @@ bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int 
       // tiles that do not run on into the next panel read fewer rows: where the last one is nearly full
       const bool apart = (full + bp - 1) / bp * bp * 100 <= full * 104;
       const long pixels = apart ? (full + bp - 1) / bp * bp : full;
-      const long HP = (long)(f.OH - 1) * p.sh + (long)(f.KH - 1) * p.dh + 1, PW = (long)(q.ws - 1) * p.sw + (long)(f.KW - 1) * p.dw + 1;
+      const long HP = (long)(f.OH - 1) * p.sh + (long)(f.KH - 1) * p.dh + 1, PW = rows ? q.ws : (long)(q.ws - 1) * p.sw + (long)(f.KW - 1) * p.dw + 1;
       if (pixels > (1 << 28) || HP > (1 << 28) || PW > 4096) return false;
       const long cells = split_patch_rows(bp, q.ws, pixels, f.OH, p.sh, f.KH, p.dh, apart) * PW;
       // (a step reaches into one slot behind its first chunk's)
@@ -432,7 +490,7 @@ bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int 
       q.PW = (int)PW;
       q.cells = (int)cells;
       q.chunks = cs / 8 * taps;
-      q.steps = cdiv(cdiv(g.icg, 8) * taps, 4);
+      q.steps = cdiv((rows ? g.icg : cdiv(g.icg, 8)) * taps, 4);
       q.wofs = (int)total;
       total += (size_t)p.groups * g.octiles * q.steps * 192;
       q.oy0 = f.oy0; q.oys = f.oys; q.ox0 = f.ox0; q.oxs = f.oxs;
@@ -471,19 +529,38 @@ double estimate(const SplitArgs &g, const ConvProblem &p, int cus, const Form &f
    // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings)
    const SplitPhase &q0 = g.phase[0], &q1 = g.phase[p.nphases - 1];
    const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.35 : 1.0;
-   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
+   // (a single tile of channels: 42x59x79x62 -> 9, 3x3 58.7 on k_conv_f32_any, 66.8 here, is the one of 90 layers that came out longer)
+   const double narrow = f.wo == 1 && !f.rows ? 1.12 : 1.0;
+   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven * narrow + 3.0;
 }
 
 template <int TI, int TJ, int WO>
-int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, bool quads, long tiles)
+int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, bool quads, bool rows, long tiles)
 {
-   constexpr auto kern_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false>, kern_q = k_conv_f32_split<TI, TJ, WO, QUADS, false>, kern_t = k_conv_f32_split<TI, TJ, WO, PIXELS, true>;
+   auto start = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * nphases)), dim3(THREADS), (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), ctx->stream, g);
+      return check_launch(ctx, "k_conv_f32_split");
+   };
+   if constexpr (TI * TJ <= 8 && TI <= 2) {
+      constexpr auto rows_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false, true>, rows_q = k_conv_f32_split<TI, TJ, WO, QUADS, false, true>;
+      SOFIE_LARGE_LDS(rows_p);
+      SOFIE_LARGE_LDS(rows_q);
+      if (rows) return start(quads ? rows_q : rows_p);
+   }
+   constexpr auto kern_p = k_conv_f32_split<TI, TJ, WO, PIXELS, false, false>, kern_q = k_conv_f32_split<TI, TJ, WO, QUADS, false, false>,
+                  kern_t = k_conv_f32_split<TI, TJ, WO, PIXELS, true, false>;
    SOFIE_LARGE_LDS(kern_p);
    SOFIE_LARGE_LDS(kern_q);
    SOFIE_LARGE_LDS(kern_t);
-   hipLaunchKernelGGL(nphases > 1 ? kern_t : quads ? kern_q : kern_p, dim3((unsigned)(tiles * nphases)), dim3(THREADS),
-                      (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), ctx->stream, g);
-   return check_launch(ctx, "k_conv_f32_split");
+   return start(nphases > 1 ? kern_t : quads ? kern_q : kern_p);
+}
+
+// Few channels, a large kernel: a cell is the eight values that a row of the kernel meets at an output column, of one channel (a chunk of K:
+// a row of the kernel, zeros up to eight), where that is 0.8 of the matrix cycles of the fp32 instructions or less: 5x5 and 7x7, not 3x3
+// (three channels: 288 cycles for a tile of 16 x 16, 224 on the fp32 instructions).
+bool rows_of(const ConvProblem &p, long icg)
+{
+   return icg < 6 && p.nphases == 1 && !p.transposed && p.KW0 <= 8 && 96 * ((icg * p.KH0 + 3) / 4) * 5 < 4 * 32 * ((icg * p.KH0 * p.KW0 + 3) / 4);
 }
 
 }  // namespace
@@ -495,7 +572,8 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    // chunks of eight, and short sums, which are their stores (60x1x16x72 -> 247, 3x3 27 us on k_conv_f32_any, 34 here; the tests of the
    // other kernels name them up to 144 products: 55x16x60x60 -> 64, 3x3, 1x10x101x101 -> 64).
    const long icg = p.C / p.groups;
-   if (other_us < 7.5 + (ctx->constant_weights ? 0.0 : 4.0) || icg < 6 || (p.nphases == 1 ? icg * p.KH0 * p.KW0 <= 144 : icg * p.KH0 * p.KW0 < 48 * p.nphases)) return SOFIE_HIP_OK;
+   const bool rows = rows_of(p, icg);
+   if (other_us < 7.5 + (ctx->constant_weights ? 0.0 : 4.0) || (!rows && icg < 6) || (rows ? false : p.nphases == 1 ? icg * p.KH0 * p.KW0 <= 144 : icg * p.KH0 * p.KW0 < 48 * p.nphases)) return SOFIE_HIP_OK;
    const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
    // descriptors and OUTSIDE: 1 GiB of images per launch
    const size_t room = ((size_t)1 << 30) - ((size_t)16 << 20);
@@ -522,18 +600,19 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
       double mma = 0.0;      // matrix instructions per 16 channels and pixel
       for (int i = 0; i < p.nphases; ++i)
-         mma += (double)n * p.phase[i].OH * p.phase[i].OW * cdiv(cdiv(g.icg, 8) * p.phase[i].KH * p.phase[i].KW, 4) * p.groups * 96.0 / 16.0 / 4.0;
-      Form best{0, 0, 0, 0, 0, other_us};
+         mma += (double)n * p.phase[i].OH * p.phase[i].OW * cdiv(rows ? g.icg * p.phase[i].KH : cdiv(g.icg, 8) * p.phase[i].KH * p.phase[i].KW, 4) * p.groups * 96.0 / 16.0 / 4.0;
+      Form best{0, 0, 0, 0, 0, rows, other_us};
       for (const auto &f : forms) {
-         Form form{f[0], f[1], f[2], 16, 0, 0.0};
+         if (rows && f[0] > 2) continue;
+         Form form{f[0], f[1], f[2], rows ? 8 * g.icg : 16, 0, rows, 0.0};
          if (f[0] > 1 && f[2] * (f[0] - 1) >= g.octiles) continue;      // tiles of nothing
          // (cannot be shorter than its matrix instructions)
          if (mma * cdiv(g.octiles, f[2] * f[0]) * f[2] * f[0] * 0.889 / (2100.0 * cus) + 3.0 >= best.time) continue;
-         for (; form.cs <= 32; form.cs *= 2) {
+         for (; form.cs <= (rows ? 8 * g.icg : 32); form.cs *= 2) {
             double least = 0.0;
             form.strips = 0;
             for (int strips = 1; strips <= 16; ++strips) {
-               if (!lay_out(g, p, form.pixels(), form.items(), form.cs, strips, &pieces)) continue;
+               if (!lay_out(g, p, form.pixels(), form.items(), form.cs, strips, rows, &pieces)) continue;
                const SplitPhase &q = g.phase[0];
                if ((double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
                const double cost = (double)q.strips * q.PHW * (1.0 + 0.02 * q.cells / form.pixels());
@@ -545,7 +624,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
                }
             }
             if (form.strips == 0) continue;
-            lay_out(g, p, form.pixels(), form.items(), form.cs, form.strips, &pieces);
+            lay_out(g, p, form.pixels(), form.items(), form.cs, form.strips, rows, &pieces);
             form.time = estimate(g, p, cus, form, n, quads());
             if (form.time < best.time) best = form;
          }
@@ -557,15 +636,17 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    Form best = choose(per);
    if (best.ti == 0) return SOFIE_HIP_OK;
    auto prepare = [&] {
-      lay_out(g, p, best.pixels(), best.items(), best.cs, best.strips, &pieces);
+      lay_out(g, p, best.pixels(), best.items(), best.cs, best.strips, rows, &pieces);
       for (int i = 0; i < p.nphases; ++i) {
          SplitPhase &q = g.phase[i];
+         q.tiles = q.strips > 1 && q.PHW % best.pixels() == 0 ? q.PHW / best.pixels() : 0;
+         q.dTiles = make_fastdiv((unsigned)(q.tiles > 0 ? q.strips * q.tiles : 1));
          q.dPHW = make_fastdiv((unsigned)q.PHW);
          q.dWS = make_fastdiv((unsigned)q.ws);
          q.dHP = make_fastdiv((unsigned)q.HP);
          q.dPW = make_fastdiv((unsigned)q.PW);
          q.dStrips = make_fastdiv((unsigned)q.strips);
-         q.dTaps = make_fastdiv((unsigned)(q.KH * q.KW));
+         q.dTaps = make_fastdiv((unsigned)(q.KH * (rows ? 1 : q.KW)));
          q.dKW = make_fastdiv((unsigned)q.KW);
          q.dCells = make_fastdiv((unsigned)q.cells);
       }
@@ -578,7 +659,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    // the step behind the last one may be asked for, to no use
    const size_t wbytes = pieces * 16 + 4096;
    g.wbytes = (unsigned)wbytes;
-   int key[7 + 7 * MAX_PHASES] = {5, p.groups, g.ocg, g.icg, p.KH0 * 4096 + p.KW0, p.transposed, p.nphases};
+   int key[7 + 7 * MAX_PHASES] = {rows ? 6 : 5, p.groups, g.ocg, g.icg, p.KH0 * 4096 + p.KW0, p.transposed, p.nphases};
    for (int i = 0; i < p.nphases; ++i) {
       const SplitPhase &q = g.phase[i];
       const int v[7] = {q.KH, q.KW, q.th0, q.ths, q.tw0, q.tws, q.wofs};
@@ -592,7 +673,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       SplitWeightArgs a{};
       a.w = p.w; a.dst = static_cast<v4i *>(ws);
       a.icg = g.icg; a.ocg = g.ocg; a.octiles = g.octiles;
-      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.total = (int)(pieces / 3);
+      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.rows = rows; a.total = (int)(pieces / 3);
       for (int i = 0; i < MAX_PHASES; ++i) a.phase[i] = g.phase[i];
       hipLaunchKernelGGL(k_conv_f32_split_weights, dim3((unsigned)cdiv(a.total, 256)), dim3(256), 0, ctx->stream, a);
       if (int rc = check_launch(ctx, "k_conv_f32_split_weights")) return rc;
@@ -626,7 +707,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       }
       int rc = SOFIE_HIP_OK;
       switch (best.ti * 100 + best.tj * 10 + best.wo) {
-#define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, quads(), tiles); break
+#define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, quads(), rows, tiles); break
          SOFIE_FORM(4, 4, 2); SOFIE_FORM(3, 4, 2); SOFIE_FORM(2, 4, 2); SOFIE_FORM(4, 2, 2); SOFIE_FORM(2, 2, 2); SOFIE_FORM(1, 4, 2); SOFIE_FORM(1, 2, 2);
          SOFIE_FORM(1, 4, 1);
 #undef SOFIE_FORM
