@@ -32,4 +32,7 @@ int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool
 // the microseconds of the caller's other way.
 int conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done);
 
+// The same for k_conv_f32_short (conv_f32_short.hip).
+int conv_f32_short(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done);
+
 }  // namespace sofie

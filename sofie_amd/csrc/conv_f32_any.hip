@@ -588,12 +588,16 @@ int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_u
    };
    Form best = choose(per);
    if (best.ti == 0) return SOFIE_HIP_OK;
+   const double here_us = best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1);
+   // Shorter sums are shorter on the vector unit.
+   if (!split_only)
+      if (int rc = conv_f32_short(ctx, p, 0.9 * (here_us < other_us ? here_us : other_us), done); rc || *done) return rc;
    // Longer sums on many tiles are shorter on the bf16 matrix instructions; both estimates are off by some 10 %.
-   if (int rc = conv_f32_split(ctx, p, 0.9 * (best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1)), done); rc || *done) return rc;
+   if (int rc = conv_f32_split(ctx, p, 0.9 * here_us, done); rc || *done) return rc;
    if (split_only) return SOFIE_HIP_OK;
    // against what the caller has instead (the estimate's unit is a cycle at 2400 MHz; weights that are not kept are laid out in
    // front of the launch, 3.1 us)
-   if (other_us < 0.95 * (best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1))) return SOFIE_HIP_OK;
+   if (other_us < 0.95 * here_us) return SOFIE_HIP_OK;
 
    int key[8 + 7 * MAX_PHASES] = {quad ? 4 : 3, p.groups, g.ocg, g.icg, p.KH0, p.KW0, p.transposed, p.nphases};
    for (int i = 0; i < p.nphases; ++i) {
