@@ -27,11 +27,10 @@
 // (13000 cycles for 16 stores instead of 6800).
 //
 // Bound: the device's power under bf16 matrix instructions on large layers (256x64x56x56 -> 128: 1.65 GHz, the matrix pipe
-// busy for 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
+// busy for 60 to 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
 // smaller ones. Relative error against 64 bits a quarter of the fp32 instructions'. us against k_conv_f32_any and k_conv2d_f32_dma:
-// 256x64x56x56 -> 128, 3x3 906 -> 640 (576 for the first
-// milliseconds); 256x32x20x20 -> 64 47.4 -> 28.5; 256x64x10x10 -> 128 44.4 -> 27.5; 169x80x16x16 -> 128,
-// 5x5 220 -> 116; 16x64x32x32 -> 65, 7x7 107 -> 51; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 101 (89). Three workgroups per compute
+// 256x64x56x56 -> 128, 3x3 906 -> 583; 256x32x20x20 -> 64 47.4 -> 28.5; 256x64x10x10 -> 128 44.4 -> 29.5; 169x80x16x16 -> 128,
+// 5x5 220 -> 116; 16x64x32x32 -> 65, 7x7 107 -> 51; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 87. Three workgroups per compute
 // unit instead of two (fewer cells per thread and slot) were 12 % of the last.
 #include <cmath>
 
@@ -529,9 +528,7 @@ double estimate(const SplitArgs &g, const ConvProblem &p, int cus, const Form &f
    // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings)
    const SplitPhase &q0 = g.phase[0], &q1 = g.phase[p.nphases - 1];
    const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.35 : 1.0;
-   // (a single tile of channels: 42x59x79x62 -> 9, 3x3 58.7 on k_conv_f32_any, 66.8 here, is the one of 90 layers that came out longer)
-   const double narrow = f.wo == 1 && !f.rows ? 1.12 : 1.0;
-   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven * narrow + 3.0;
+   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
 }
 
 template <int TI, int TJ, int WO>
@@ -594,8 +591,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    auto quads = [&] { return whole && (g.phase[0].strips == 1 ? (long)p.OH0 * p.OW0 % 4 == 0 : p.OW0 % 4 == 0); };
    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
    size_t pieces = 0;
-   // the form for a launch on n images: tiles of 32 ti channels x 32 tj pixels, slots of 16 or 32 channels, the images in as many
-   // strips as read least for their pixels
+   // the form for a launch on n images: tiles of 32 ti channels x 32 tj pixels, slots of 16 or 32 channels, the images in strips
    auto choose = [&](size_t n) {
       static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
       double mma = 0.0;      // matrix instructions per 16 channels and pixel
@@ -609,23 +605,25 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
          // (cannot be shorter than its matrix instructions)
          if (mma * cdiv(g.octiles, f[2] * f[0]) * f[2] * f[0] * 0.889 / (2100.0 * cus) + 3.0 >= best.time) continue;
          for (; form.cs <= (rows ? 8 * g.icg : 32); form.cs *= 2) {
-            double least = 0.0;
+            // (as many strips as the estimate says: fewer cells for a tile's pixels against whole lines per store, 4-byte stores where strips are no
+            // whole fours, 256x64x10x10 -> 128 29.5 us in one strip, 36.2 in five of two columns; by the number of cells alone 42x59x79x62 -> 9, 3x3 66.5, now 46.9,
+            // and k_conv_f32_any 58.7)
+            double least = HUGE_VAL;
             form.strips = 0;
             for (int strips = 1; strips <= 16; ++strips) {
                if (!lay_out(g, p, form.pixels(), form.items(), form.cs, strips, rows, &pieces)) continue;
                const SplitPhase &q = g.phase[0];
                if ((double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
-               const double cost = (double)q.strips * q.PHW * (1.0 + 0.02 * q.cells / form.pixels());
-               if (form.strips == 0 || cost < least) {
-                  least = cost;
+               const double time = estimate(g, p, cus, form, n, quads()) * (strips > 1 ? 1.02 : 1.0);
+               if (time < least) {
+                  least = time;
                   form.strips = strips;
                } else if (strips > form.strips + 1) {
                   break;
                }
             }
             if (form.strips == 0) continue;
-            lay_out(g, p, form.pixels(), form.items(), form.cs, form.strips, rows, &pieces);
-            form.time = estimate(g, p, cus, form, n, quads());
+            form.time = least;
             if (form.time < best.time) best = form;
          }
       }
