@@ -1825,15 +1825,16 @@ SplitKPlan split_k_direct(const sofie_hip_ctx *ctx, const GemmArgs &g)
 // top of k_gemm_bytes_direct's own, whose estimate is up to 1.6 us too long for few rows: below 0.9 and 0.8 of it slices lose,
 // 8 x 30 x 8208 5.5 in one launch, 6.5 in slices, 270 x 30 x 8208 6.5 / 6.7. By time these would also take the place of k_qgemm_few_rows
 // (4 x 64 x 65536 16.2 / 6.9, 8 x 1024 x 8192 8.1 / 6.7, 26 x 671 x 51392 22.2 / 13.3) and of tiles on up to 32 rows or 64 columns
-// (27 x 43 x 36880 20.6 / 7.1); test_up_to_32_rows_on_a_long_sum_are_a_pass_over_b names the kernels that run there.)
-bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, SplitKPlan &plan)
+// (27 x 43 x 36880 20.6 / 7.1); test_up_to_32_rows_on_a_long_sum_are_a_pass_over_b names the kernels that run there. In a pair of layers, whose
+// finishing pass is a launch of its own anyway, they do: the int8 classifier at batch 1 29.8 -> 23.7 us, at 32 32.2 -> 26.7.)
+bool split_k_plan(const sofie_hip_ctx *ctx, const GemmArgs &g, SplitKPlan &plan, bool pair = false)
 {
    plan = split_k_tiles(ctx, g);
    const float one = small_choice(ctx, g, CHUNK_ROWS).us;
    const bool cut = plan.us < one;
    if (cut && !workspace_has_room(ctx, split_k_bytes(g, plan.splits))) return true;      // refused by the launch, or one launch
    const SplitKPlan direct = split_k_direct(ctx, g);
-   if (direct.us + 1.0f < (g.M <= 16 ? 0.8f : 0.9f) * one && (!cut || (g.M > 32 && g.N > 64 && direct.us < plan.us + 3.0f))) {
+   if (cut ? (pair || (g.M > 32 && g.N > 64)) && direct.us < one && direct.us < plan.us + 3.0f : direct.us + 1.0f < (g.M <= 16 ? 0.8f : 0.9f) * one) {
       plan = direct;
       return true;
    }
@@ -2096,7 +2097,7 @@ int sofie_hip_qgemm_s8_pair(sofie_hip_ctx *ctx, int M, int K, const int8_t *A, i
    const bool operands_ok = K % 16 == 0 && lda % 16 == 0 && aligned16(A) && ldb1 % 16 == 0 && aligned16(B1) && ldb2 % 4 == 0 &&
                             (reinterpret_cast<uintptr_t>(B2) & 3u) == 0;
    SplitKPlan plan;
-   if (N2 <= 8 && lanes_ok && operands_ok && N1 > 16 && split_k_plan(ctx, g, plan) &&
+   if (N2 <= 8 && lanes_ok && operands_ok && N1 > 16 && split_k_plan(ctx, g, plan, true) &&
        !((size_t)M * N1 >= (size_t)256 * 256 * 128 && M >= 256 && N1 >= 256)) {
       GemmArgs t{};
       t.B = reinterpret_cast<const uint8_t *>(B2);

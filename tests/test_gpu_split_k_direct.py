@@ -59,7 +59,7 @@ def test_product_in_slices(ctx, M, N, K):
         assert bool((y[0] == 77).all() and (y[M + 1] == 77).all())
 
 
-@pytest.mark.parametrize("M,N1,K,N2", [(64, 256, 12800, 5), (33, 128, 12304, 8), (130, 128, 16384, 1)])
+@pytest.mark.parametrize("M,N1,K,N2", [(64, 256, 12800, 5), (1, 256, 12800, 5), (30, 32, 24592, 8), (33, 128, 12304, 8), (130, 128, 16384, 1)])
 def test_pair_in_slices(ctx, M, N1, K, N2):
     gen = torch.Generator().manual_seed(M + K)
     a, b1, b2 = int8(gen, M, K), int8(gen, N1, K), int8(gen, N2, N1)
