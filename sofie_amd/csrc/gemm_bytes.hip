@@ -12,8 +12,6 @@
 // packed results go through a per-wavefront LDS staging block and leave as 16-byte row
 // segments. Workgroup ids are remapped so that each XCD (ids are dealt round-robin over the
 // 8 XCDs) owns a compact rectangle of output tiles and its L2 sees each operand panel once.
-#include <type_traits>
-
 #include "common.h"
 #include "gemm_tile.h"
 #include "row_chunk.h"
@@ -1065,34 +1063,44 @@ template <class Mma, int OUT> struct IS_SPLITTABLE {
    static constexpr bool value = __is_same(typename Mma::Acc, v16i) && OUT == SOFIE_OUT_S32;
 };
 
-// Sum over the K slices of four consecutive int32 partial sums. The loads of eight slices are issued together before
-// the first addition (one after the other, each waiting for the one before, they were the length of the pass).
+// Sum over the K slices of four consecutive int32 partial sums. The loads of four slices (MANY: of eight) are
+// issued together before the first addition (one after the other, each waiting for the one before, they were the length of the
+// pass). Eight where the pass is a few wavefronts' latency (many_slices); with a wavefront on every SIMD and more, four are enough.
+template <bool MANY>
 __device__ __forceinline__ v4i sum_slices(const int *__restrict__ p, size_t plane, int splits)
 {
    v4i s = {0, 0, 0, 0};
-   auto some = [&](auto count, int k) {
-      constexpr int COUNT = decltype(count)::value;
-      v4i v[COUNT];
-#pragma unroll
-      for (int i = 0; i < COUNT; ++i) v[i] = *reinterpret_cast<const v4i *>(p + (size_t)(k + i) * plane);
-#pragma unroll
-      for (int i = 0; i < COUNT; ++i)
-#pragma unroll
-         for (int e = 0; e < 4; ++e) s[e] += v[i][e];
-   };
    int k = 0;
-   for (; k + 8 <= splits; k += 8) some(std::integral_constant<int, 8>{}, k);
-   if (splits & 4) {
-      some(std::integral_constant<int, 4>{}, k);
-      k += 4;
+   if constexpr (MANY) {
+      for (; k + 8 <= splits; k += 8) {
+         v4i v[8];
+#pragma unroll
+         for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const v4i *>(p + (size_t)(k + i) * plane);
+#pragma unroll
+         for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += v[i][e];
+      }
    }
-   for (; k < splits; ++k) some(std::integral_constant<int, 1>{}, k);
+   for (; k + 4 <= splits; k += 4) {
+      const v4i a = *reinterpret_cast<const v4i *>(p + (size_t)k * plane);
+      const v4i b = *reinterpret_cast<const v4i *>(p + (size_t)(k + 1) * plane);
+      const v4i c = *reinterpret_cast<const v4i *>(p + (size_t)(k + 2) * plane);
+      const v4i d = *reinterpret_cast<const v4i *>(p + (size_t)(k + 3) * plane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += (a[e] + b[e]) + (c[e] + d[e]);
+   }
+   for (; k < splits; ++k) {
+      const v4i v = *reinterpret_cast<const v4i *>(p + (size_t)k * plane);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += v[e];
+   }
    return s;
 }
 
 // Sum of the K slices' int32 partial tiles, then bias and the output conversion of the unsplit kernel.
 // One thread per four consecutive columns of one row; P is [splits][M][ldp], ldp a multiple of 4.
-template <int OUT>
+template <int OUT, bool MANY>
 __global__ void __launch_bounds__(256) k_splitk_finish(GemmArgs g, const int *__restrict__ P, int splits, int ldp)
 {
    const int quads = ldp >> 2;
@@ -1100,7 +1108,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish(GemmArgs g, const int *__
    if (t >= (size_t)g.M * quads) return;
    const int m = (int)(t / quads), n = (int)(t % quads) * 4;
    const size_t plane = (size_t)g.M * ldp;
-   const v4i s = sum_slices(P + (size_t)m * ldp + n, plane, splits);
+   const v4i s = sum_slices<MANY>(P + (size_t)m * ldp + n, plane, splits);
    constexpr int ESZ = OutSize<OUT>::value;
    unsigned char *out = static_cast<unsigned char *>(g.Y) + ((size_t)m * g.ldy + n) * ESZ;
 #pragma unroll
@@ -1133,7 +1141,7 @@ __device__ __forceinline__ int wave_sum_in_lane63(int v)
    return v;
 }
 
-template <int OUT2, int QUADS>
+template <int OUT2, int QUADS, bool MANY>
 __global__ void __launch_bounds__(256) k_splitk_finish_pair(GemmArgs g1, const int *__restrict__ P, int splits, int ldp, GemmArgs g2)
 {
    constexpr int quads = QUADS;
@@ -1151,7 +1159,7 @@ __global__ void __launch_bounds__(256) k_splitk_finish_pair(GemmArgs g1, const i
    }
 #pragma unroll
    for (int j = 0; j < 8; ++j) w2[j] = j < g2.N ? *reinterpret_cast<const int *>(g2.B + (size_t)j * g2.ldb + n) : 0;
-   const v4i s = sum_slices(P + (size_t)m * ldp + n, plane, splits);
+   const v4i s = sum_slices<MANY>(P + (size_t)m * ldp + n, plane, splits);
    unsigned packed = 0;
 #pragma unroll
    for (int e = 0; e < 4; ++e) {
@@ -1704,7 +1712,7 @@ int launch_few_rows(sofie_hip_ctx *ctx, GemmArgs &g, bool whole)
    else hipLaunchKernelGGL(k_qgemm_few_rows<2>, grid, dim3(256), 0, ctx->stream, g, static_cast<int *>(part), ldp, kslice);
    if (int rc = check_launch(ctx, "k_qgemm_few_rows")) return rc;
    const size_t threads = (size_t)g.M * (ldp / 4);
-   hipLaunchKernelGGL((k_splitk_finish<OUT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, g,
+   hipLaunchKernelGGL((k_splitk_finish<OUT, false>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, ctx->stream, g,
                       static_cast<const int *>(part), splits, ldp);
    return check_launch(ctx, "k_splitk_finish");
 }
@@ -1717,6 +1725,8 @@ struct SplitKPlan {
    float us;
 };
 size_t split_k_bytes(const GemmArgs &g, int splits) { return (size_t)splits * g.M * (cdiv(g.N, 4) * 4) * sizeof(int); }
+
+bool many_slices(size_t threads, int splits) { return splits >= 8 && threads <= 32768; }
 
 // K cut into plan.splits slices of plan.kslice bytes (a multiple of BK): partial sums into the context's scratch
 // buffer, then k_splitk_finish writes Y.
@@ -1747,12 +1757,13 @@ int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, const SplitKPlan &plan, cons
    if (tail) {
       if constexpr (OUT == SOFIE_OUT_S8) {
          const int *pp = static_cast<const int *>(part);
+         auto finish = [&](auto few, auto many) {
+            hipLaunchKernelGGL(many_slices(threads, splits) ? many : few, fgrid, dim3(256), 0, ctx->stream, g, pp, splits, ldp, *tail);
+         };
 #define SOFIE_PAIR_LAUNCH(Q_)                                                                                              \
    do {                                                                                                                     \
-      if (tail_out == SOFIE_OUT_F32)                                                                                        \
-         hipLaunchKernelGGL((k_splitk_finish_pair<SOFIE_OUT_F32, Q_>), fgrid, dim3(256), 0, ctx->stream, g, pp, splits, ldp, *tail); \
-      else                                                                                                                  \
-         hipLaunchKernelGGL((k_splitk_finish_pair<SOFIE_OUT_S8, Q_>), fgrid, dim3(256), 0, ctx->stream, g, pp, splits, ldp, *tail);  \
+      if (tail_out == SOFIE_OUT_F32) finish(k_splitk_finish_pair<SOFIE_OUT_F32, Q_, false>, k_splitk_finish_pair<SOFIE_OUT_F32, Q_, true>); \
+      else finish(k_splitk_finish_pair<SOFIE_OUT_S8, Q_, false>, k_splitk_finish_pair<SOFIE_OUT_S8, Q_, true>);             \
    } while (0)
          switch (ldp / 4) {
          case 8: SOFIE_PAIR_LAUNCH(8); break;
@@ -1764,7 +1775,7 @@ int launch_split_k(sofie_hip_ctx *ctx, GemmArgs &g, const SplitKPlan &plan, cons
          return check_launch(ctx, "k_splitk_finish_pair");
       }
    }
-   hipLaunchKernelGGL((k_splitk_finish<OUT>), fgrid, dim3(256), 0, ctx->stream, g, static_cast<const int *>(part), splits, ldp);
+   hipLaunchKernelGGL((many_slices(threads, splits) ? k_splitk_finish<OUT, true> : k_splitk_finish<OUT, false>), fgrid, dim3(256), 0, ctx->stream, g, static_cast<const int *>(part), splits, ldp);
    return check_launch(ctx, "k_splitk_finish");
 }
 
