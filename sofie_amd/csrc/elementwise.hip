@@ -102,8 +102,8 @@ __global__ void k_maxpool2d(const T *__restrict__ x, T *__restrict__ y, int N, i
    y[idx] = best;
 }
 
-// 2 x 2 windows two cells apart without pads, rows of whole V outputs: 16-byte loads of both rows, V outputs per thread in one
-// store. Bound: memory. 256x32x40x40 18.7 -> 10.3 us (6.4 TB/s), 256x64x20x20 9.9 -> 4.2. (k_maxpool2d with its divisions as
+// 2 x 2 windows two cells apart, each of them whole inside its plane (2 OH <= H, 2 OW <= W), rows of whole V outputs: 16-byte loads of
+// both rows, V outputs per thread in one store. Bound: memory. 256x32x40x40 18.7 -> 10.3 us (6.4 TB/s), 256x64x20x20 9.9 -> 4.2. (k_maxpool2d with its divisions as
 // multiplications was no faster: 17.9 -> 17.5 on 41x41.)
 template <int V>
 __global__ void __launch_bounds__(256) k_maxpool2d_f32_pairs(const float *__restrict__ x, float *__restrict__ y, int total, int H, int W, int OH, int OW, FastDiv dOWV,
@@ -403,7 +403,9 @@ int sofie_hip_maxpool2d_f32(sofie_hip_ctx *ctx, const float *x, float *y, int NC
    SOFIE_REQUIRE(ctx, x && y, "null operand");
    int OH, OW;
    if (int rc = pool_dims(ctx, H, W, kh, kw, pt, pl, pb, pr, sh, sw, &OH, &OW)) return rc;
-   if (kh == 2 && kw == 2 && sh == 2 && sw == 2 && pt == 0 && pl == 0 && W % 4 == 0 && OW % 2 == 0 && aligned16(x) && aligned16(y)) {
+   // (pads behind the plane may give windows that reach over its end: 7 rows and one pad are four windows)
+   const bool inside = pt == 0 && pl == 0 && OH <= H / 2 && OW <= W / 2;
+   if (kh == 2 && kw == 2 && sh == 2 && sw == 2 && inside && W % 4 == 0 && OW % 2 == 0 && aligned16(x) && aligned16(y)) {
       const int v = OW % 4 == 0 ? 4 : 2;
       const size_t groups = (size_t)NC * OH * (OW / v);
       if (groups < ((size_t)1 << 31)) {

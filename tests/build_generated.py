@@ -30,6 +30,7 @@ def all_specs(with_large=True):
     specs.append(models.conv1d_spec())
     specs.append(models.conv3d_spec())
     specs.append(models.pool1d_spec())
+    specs.append(models.pool2d_spec())
     specs.append(models.pool3d_spec())
     specs.append(models.qcnn_rt_spec(oracle))
     specs.append(models.cnn_f32_rt_spec())

@@ -349,6 +349,23 @@ def pool1d_reference(oracle):
     return oracle.avgpool2d(m, (1, 4), (1, 1), (0, 2, 0, 1))[:, :, 0, :]
 
 
+def pool2d_input(seed=57):
+    return np.random.default_rng(seed).standard_normal((3, 5, 9, 16)).astype(np.float32)
+
+
+def pool2d_spec(name="pool2d_end_pads"):
+    """MaxPool on [3,5,9,16] (window 2x2, stride 2, pads only behind: one row and one column)."""
+    s = emit.ModelSpec(name)
+    s.add_input("x", "FLOAT", pool2d_input().shape)
+    s.maxpool("x", "y", (2, 2), (0, 0, 1, 1), (2, 2))
+    s.set_output("y")
+    return s
+
+
+def pool2d_reference(oracle):
+    return oracle.maxpool2d(pool2d_input(), (2, 2), (2, 2), (0, 0, 1, 1))
+
+
 def pool3d_input(seed=54):
     return np.random.default_rng(seed).standard_normal((2, 3, 8, 9, 10)).astype(np.float32)
 

@@ -188,6 +188,13 @@ def test_pooling_over_one_and_three_axes_sessions(tmp_path):
     assert y.size == ref.size and np.array_equal(y, ref.reshape(-1))
 
 
+def test_pooling_with_pads_behind_the_plane_session(tmp_path):
+    """MaxPool 2x2 of stride 2 on planes of odd height, one pad behind each axis: the last windows have one row."""
+    y = run_session("pool2d_end_pads", models.pool2d_input(), tmp_path)
+    ref = models.pool2d_reference(oracle)
+    assert y.size == ref.size and np.array_equal(y, ref.reshape(-1))
+
+
 def test_conv_batchnorm_convtranspose_session(tmp_path):
     """Conv -> BatchNormalization -> Relu (folded into the convolution at generation time) -> MaxPool ->
     BatchNormalization (its own kernel) -> ConvTranspose -> Relu against the unfused oracle steps; 1e-5 relative

@@ -21,3 +21,16 @@ def test_maxpool_pairs(nc, h, w):
     x[r.random(x.shape) < 0.5] = np.nan
     q = x[:, :, :h // 2 * 2, :w // 2 * 2].reshape(1, nc, h // 2, 2, w // 2, 2)
     assert np.array_equal(ops.maxpool2d(x, (2, 2), (2, 2)), np.where(np.isnan(q), -np.inf, q).max(axis=(3, 5)))
+
+
+@pytest.mark.parametrize("pads", [(0, 0, 1, 0), (0, 0, 0, 1), (0, 0, 1, 1), (0, 0, 2, 0), (0, 0, 0, 4), (0, 0, 3, 5), (1, 0, 0, 0), (0, 1, 0, 1)])
+@pytest.mark.parametrize("nc,h,w", [(1, 7, 8), (5, 7, 8), (5, 8, 8), (3, 41, 40), (2, 2, 4), (1, 3, 4), (9, 6, 20)])
+def test_windows_that_reach_over_the_planes_end(nc, h, w, pads):
+    """Pads behind the plane (and in front of it): cells that are not there are left out, not the next plane's or those behind the tensor.
+    Every value lies below every value of the plane behind it, so that one cell of that would be seen."""
+    from sofie_amd import ops
+    r = np.random.default_rng(h * w + sum(pads))
+    x = (r.integers(-2, 3, (1, nc, h, w)) + 10 * np.arange(nc)[None, :, None, None]).astype(np.float32)
+    x[r.random(x.shape) < 0.1] = -np.inf
+    got, ref = ops.maxpool2d(x, (2, 2), (2, 2), pads), oracle.maxpool2d(x, (2, 2), (2, 2), pads)
+    assert got.shape == ref.shape and np.array_equal(got.view(np.int32), ref.view(np.int32))
