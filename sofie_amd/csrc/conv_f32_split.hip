@@ -32,10 +32,8 @@
 // 256x64x56x56 -> 128, 3x3 906 -> 583; 256x32x20x20 -> 64 47.4 -> 28.5; 256x64x10x10 -> 128 44.4 -> 29.5; 169x80x16x16 -> 128,
 // 5x5 220 -> 116; 16x64x32x32 -> 65, 7x7 107 -> 51; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 87. Three workgroups per compute
 // unit instead of two (fewer cells per thread and slot) were 12 % of the last.
-#include <cmath>
-
 #include "conv_f32.h"
-#include "conv_f32_patch.h"
+#include "conv_f32_split_plan.h"
 #include "gemm_tile.h"
 #include "split_bf16.h"
 
@@ -44,15 +42,8 @@ using namespace sofie;
 namespace {
 
 constexpr unsigned OUTSIDE = 0x40000000u;      // no descriptor of this file reaches it
-constexpr int MAX_PHASES = 4;
-constexpr int CELL = 48;                       // LDS bytes of 8 channels of a cell: h, m, l
-constexpr int THREADS = 256;
-
-// Cells x 8 channels of a slot that a thread carries, at most: registers, which decide how many workgroups share a compute unit.
-// (Rows of a kernel as cells: one slot, whose registers are free again in front of the loop.)
-constexpr int items_of(int ti, int tj, int wo, bool rows) { return rows || wo == 1 ? 4 : ti * tj > 8 ? 3 : 2; }
-// Workgroups a compute unit holds at once, by registers.
-constexpr int resident_of(int ti, int tj, int wo) { return ti * tj > 8 ? 2 : ti * tj > 4 || wo == 1 ? 3 : 4; }
+constexpr int MAX_PHASES = SplitPlan::MAX_PHASES, CELL = SplitPlan::CELL, THREADS = SplitPlan::THREADS;
+static_assert(SplitPlan::MAX_LDS == kMaxDynamicLds, "LDS of a compute unit");
 
 struct SplitPhase {
    int P, PHW, panels;        // pixels, of a panel; panels (strips of images)
@@ -88,10 +79,10 @@ struct SplitArgs {
 enum { PIXELS, QUADS };
 
 template <int TI, int TJ, int WO, int STORE, bool PHASES, bool ROWS>
-__global__ void __launch_bounds__(THREADS, resident_of(TI, TJ, WO)) k_conv_f32_split(SplitArgs g)
+__global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k_conv_f32_split(SplitArgs g)
 {
    extern __shared__ __align__(16) unsigned char smem_raw[];
-   constexpr int BP = 4 / WO * TJ * 16, ITEMS = items_of(TI, TJ, WO, ROWS);
+   constexpr int BP = 4 / WO * TJ * 16, ITEMS = SplitPlan::items_of(TI, TJ, WO, ROWS);
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = wave % WO;
    // workgroup id -> (pixels, channels, phase): an XCD (an L2) works on consecutive ids; the phases of a tile, which read the same
@@ -447,90 +438,6 @@ __global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs 
    d[128] = __builtin_bit_cast(v4i, s.l);
 }
 
-struct Form {
-   int ti, tj, wo, cs, strips;
-   bool rows;
-   int pixels() const { return 64 / wo * tj; }
-   int channels() const { return 16 * wo * ti; }
-   int items() const { return items_of(ti, tj, wo, rows); }
-   double time;
-};
-
-// Geometry of the problem for tiles of bp pixels, slots of cs channels and images in strips; false where a slot is more than the
-// threads of a workgroup carry, or than the LDS holds. pieces: 16-byte pieces of the fragments (which do not depend on cs and strips).
-bool lay_out(SplitArgs &g, const ConvProblem &p, int bp, int items, int cs, int strips, bool rows, size_t *pieces)
-{
-   g.CS = cs;
-   g.nslots = cdiv(g.icg, cs);
-   g.slot_bytes = 0;
-   size_t total = 0;
-   int table = 0;
-   for (int i = 0; i < p.nphases; ++i) {
-      const ConvPhase &f = p.phase[i];
-      SplitPhase &q = g.phase[i];
-      const int taps = f.KH * (rows ? 1 : f.KW);
-      q.KH = f.KH; q.KW = f.KW; q.ph = f.ph; q.pw = f.pw;
-      q.OW = f.OW;
-      q.ws = cdiv(f.OW, strips);
-      if (f.OW % 4 == 0) q.ws = (q.ws + 3) & ~3;
-      q.strips = cdiv(f.OW, q.ws);
-      const long full = (long)f.OH * q.ws;
-      // tiles that do not run on into the next panel read fewer rows: where the last one is nearly full
-      const bool apart = (full + bp - 1) / bp * bp * 100 <= full * 104;
-      const long pixels = apart ? (full + bp - 1) / bp * bp : full;
-      const long HP = (long)(f.OH - 1) * p.sh + (long)(f.KH - 1) * p.dh + 1, PW = rows ? q.ws : (long)(q.ws - 1) * p.sw + (long)(f.KW - 1) * p.dw + 1;
-      if (pixels > (1 << 28) || HP > (1 << 28) || PW > 4096) return false;
-      const long cells = split_patch_rows(bp, q.ws, pixels, f.OH, p.sh, f.KH, p.dh, apart) * PW;
-      // (a step reaches into one slot behind its first chunk's)
-      if (cells * (cs / 8) > (long)items * THREADS || (g.nslots > 1 && cs / 8 * taps < 4)) return false;
-      q.full = (int)full;
-      q.PHW = (int)pixels;
-      q.HP = (int)HP;
-      q.PW = (int)PW;
-      q.cells = (int)cells;
-      q.chunks = cs / 8 * taps;
-      q.steps = cdiv((rows ? g.icg : cdiv(g.icg, 8)) * taps, 4);
-      q.wofs = (int)total;
-      total += (size_t)p.groups * g.octiles * q.steps * 192;
-      q.oy0 = f.oy0; q.oys = f.oys; q.ox0 = f.ox0; q.oxs = f.oxs;
-      q.th0 = f.th0; q.ths = f.ths; q.tw0 = f.tw0; q.tws = f.tws;
-      if (q.cells * (cs / 8) * CELL > g.slot_bytes) g.slot_bytes = q.cells * (cs / 8) * CELL;
-      if (2 * q.chunks * 4 > table) table = 2 * q.chunks * 4;
-   }
-   *pieces = total;
-   g.table_bytes = (table + 255) & ~255;
-   return total * 16 <= ((size_t)1 << 29) && g.table_bytes + (g.nslots > 1 ? 2 : 1) * g.slot_bytes <= kMaxDynamicLds;
-}
-
-// Microseconds of a form on n images, laid out in g. A workgroup that is alone on its compute unit waits for memory in front of its loop,
-// once per slot and once per step, and for its stores behind it; workgroups that share one wait for each other's matrix
-// instructions (96 cycles a tile and step), operands, stores and conversions. A fit to 1760 timings of 201 convolutions over the ranges
-// of perf/cases.py (8.4 % rms; the form it picks is 1.1 % behind the best one in the mean).
-double estimate(const SplitArgs &g, const ConvProblem &p, int cus, const Form &f, size_t n, bool quads)
-{
-   const int bp = f.pixels(), oblocks = cdiv(g.octiles, f.wo * f.ti), pieces = f.ti * f.tj;
-   const int by_registers = resident_of(f.ti, f.tj, f.wo), by_lds = kMaxDynamicLds / (g.table_bytes + (g.nslots > 1 ? 2 : 1) * g.slot_bytes);
-   const int resident = by_lds < by_registers ? by_lds : by_registers;
-   const double store_alone = p.nphases > 1 ? 280.0 : quads ? 0.0 : 292.0, store = p.nphases > 1 ? 259.0 : quads ? 0.0 : 176.0;
-   double tiles = 0.0, alone = 0.0, work = 0.0;
-   for (int i = 0; i < p.nphases; ++i) {
-      const SplitPhase &q = g.phase[i];
-      const double mma = 96.0 * q.steps * pieces, reads = (double)q.steps * (f.ti + f.tj), items = (double)q.cells * (g.CS / 8) / THREADS;
-      const double t = (double)cdiv((int)n * q.strips * q.PHW, bp) * oblocks * g.groups;
-      const double one = 3344.0 + (287.0 + store_alone) * pieces + g.nslots * (1053.0 + 785.0 * items) + 100.0 * reads + 0.579 * mma;
-      if (one > alone) alone = one;
-      work += t * (0.889 * mma + 33.5 * reads + (151.0 + store) * pieces + 598.0 * g.nslots * items + 527.0);
-      tiles += t;
-   }
-   const double per_cu = tiles / cus, rounds = per_cu / resident, whole = rounds + 0.895 * (std::ceil(rounds) - rounds);
-   const double waits = alone * (whole > 1.0 ? whole : 1.0), busy = std::ceil(per_cu) * work / tiles;
-   const double w2 = waits * waits, b2 = busy * busy;
-   // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings)
-   const SplitPhase &q0 = g.phase[0], &q1 = g.phase[p.nphases - 1];
-   const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.35 : 1.0;
-   return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
-}
-
 template <int TI, int TJ, int WO>
 int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, bool quads, bool rows, long tiles)
 {
@@ -580,63 +487,38 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       if (f.KH < 1 || f.KW < 1 || f.OH < 1 || f.OW < 1 || (long)f.KH * f.KW > 256) return SOFIE_HIP_OK;
    }
    SplitArgs g{};
-   g.icg = p.C / p.groups;
-   g.ocg = p.OC / p.groups;
+   SplitPlan plan(p, rows);
+   g.icg = plan.icg;
+   g.ocg = plan.ocg;
    g.groups = p.groups;
-   g.octiles = cdiv(g.ocg, 16);
+   g.octiles = plan.octiles;
    size_t per = room / (image > out_image ? image : out_image);
    if (per > (size_t)p.N) per = (size_t)p.N;
-   const ConvPhase &f0 = p.phase[0];
-   const bool whole = p.nphases == 1 && f0.oys == 1 && f0.oxs == 1 && f0.oy0 == 0 && f0.ox0 == 0 && f0.OW == p.OW0 && f0.OH == p.OH0;
-   auto quads = [&] { return whole && (g.phase[0].strips == 1 ? (long)p.OH0 * p.OW0 % 4 == 0 : p.OW0 % 4 == 0); };
    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-   size_t pieces = 0;
-   // the form for a launch on n images: tiles of 32 ti channels x 32 tj pixels, slots of 16 or 32 channels, the images in strips
-   auto choose = [&](size_t n) {
-      static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
-      double mma = 0.0;      // matrix instructions per 16 channels and pixel
-      for (int i = 0; i < p.nphases; ++i)
-         mma += (double)n * p.phase[i].OH * p.phase[i].OW * cdiv(rows ? g.icg * p.phase[i].KH : cdiv(g.icg, 8) * p.phase[i].KH * p.phase[i].KW, 4) * p.groups * 96.0 / 16.0 / 4.0;
-      Form best{0, 0, 0, 0, 0, rows, other_us};
-      for (const auto &f : forms) {
-         if (rows && f[0] > 2) continue;
-         Form form{f[0], f[1], f[2], rows ? 8 * g.icg : 16, 0, rows, 0.0};
-         if (f[0] > 1 && f[2] * (f[0] - 1) >= g.octiles) continue;      // tiles of nothing
-         // (cannot be shorter than its matrix instructions)
-         if (mma * cdiv(g.octiles, f[2] * f[0]) * f[2] * f[0] * 0.889 / (2100.0 * cus) + 3.0 >= best.time) continue;
-         for (; form.cs <= (rows ? 8 * g.icg : 32); form.cs *= 2) {
-            // (as many strips as the estimate says: fewer cells for a tile's pixels against whole lines per store, 4-byte stores where strips are no
-            // whole fours, 256x64x10x10 -> 128 29.5 us in one strip, 36.2 in five of two columns; by the number of cells alone 42x59x79x62 -> 9, 3x3 66.5, now 46.9,
-            // and k_conv_f32_any 58.7)
-            double least = HUGE_VAL;
-            form.strips = 0;
-            for (int strips = 1; strips <= 16; ++strips) {
-               if (!lay_out(g, p, form.pixels(), form.items(), form.cs, strips, rows, &pieces)) continue;
-               const SplitPhase &q = g.phase[0];
-               if ((double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
-               const double time = estimate(g, p, cus, form, n, quads()) * (strips > 1 ? 1.02 : 1.0);
-               if (time < least) {
-                  least = time;
-                  form.strips = strips;
-               } else if (strips > form.strips + 1) {
-                  break;
-               }
-            }
-            if (form.strips == 0) continue;
-            form.time = least;
-            if (form.time < best.time) best = form;
-         }
-      }
-      return best;
-   };
    // (weights that are not kept are laid out in front of the launch, twice the bytes of k_conv_f32_any's)
    other_us = (other_us - (ctx->constant_weights ? 0.0 : 4.0)) * ((double)per / (double)p.N);
-   Form best = choose(per);
+   SplitPlan::Form best = plan.choose(per, cus, other_us);
    if (best.ti == 0) return SOFIE_HIP_OK;
    auto prepare = [&] {
-      lay_out(g, p, best.pixels(), best.items(), best.cs, best.strips, rows, &pieces);
+      g.CS = best.cs;
+      g.nslots = plan.slots(best.cs);
+      g.table_bytes = plan.table_bytes(best.cs);
+      g.slot_bytes = 0;
       for (int i = 0; i < p.nphases; ++i) {
+         const ConvPhase &f = p.phase[i];
          SplitPhase &q = g.phase[i];
+         SplitPlan::Panels s;
+         plan.panels(s, i, best.pixels(), best.strips);
+         q.ws = s.ws; q.strips = s.strips; q.PHW = s.PHW; q.full = s.full;
+         q.HP = s.HP; q.PW = s.PW; q.cells = s.cells;
+         q.KH = f.KH; q.KW = f.KW; q.ph = f.ph; q.pw = f.pw;
+         q.OW = f.OW;
+         q.chunks = best.cs / 8 * plan.chunks[i];
+         q.steps = plan.steps[i];
+         q.wofs = (int)plan.wofs[i];
+         q.oy0 = f.oy0; q.oys = f.oys; q.ox0 = f.ox0; q.oxs = f.oxs;
+         q.th0 = f.th0; q.ths = f.ths; q.tw0 = f.tw0; q.tws = f.tws;
+         if (SplitPlan::slot_bytes(q.cells, best.cs) > g.slot_bytes) g.slot_bytes = SplitPlan::slot_bytes(q.cells, best.cs);
          q.tiles = q.strips > 1 && q.PHW % best.pixels() == 0 ? q.PHW / best.pixels() : 0;
          q.dTiles = make_fastdiv((unsigned)(q.tiles > 0 ? q.strips * q.tiles : 1));
          q.dPHW = make_fastdiv((unsigned)q.PHW);
@@ -655,7 +537,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    };
    prepare();
    // the step behind the last one may be asked for, to no use
-   const size_t wbytes = pieces * 16 + 4096;
+   const size_t wbytes = plan.pieces * 16 + 4096;
    g.wbytes = (unsigned)wbytes;
    int key[7 + 7 * MAX_PHASES] = {rows ? 6 : 5, p.groups, g.ocg, g.icg, p.KH0 * 4096 + p.KW0, p.transposed, p.nphases};
    for (int i = 0; i < p.nphases; ++i) {
@@ -671,7 +553,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       SplitWeightArgs a{};
       a.w = p.w; a.dst = static_cast<v4i *>(ws);
       a.icg = g.icg; a.ocg = g.ocg; a.octiles = g.octiles;
-      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.rows = rows; a.total = (int)(pieces / 3);
+      a.KH0 = p.KH0; a.KW0 = p.KW0; a.transposed = p.transposed; a.rows = rows; a.total = (int)(plan.pieces / 3);
       for (int i = 0; i < MAX_PHASES; ++i) a.phase[i] = g.phase[i];
       hipLaunchKernelGGL(k_conv_f32_split_weights, dim3((unsigned)cdiv(a.total, 256)), dim3(256), 0, ctx->stream, a);
       if (int rc = check_launch(ctx, "k_conv_f32_split_weights")) return rc;
@@ -687,8 +569,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
       const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
       if (n != per) {
-         other_us = HUGE_VAL;
-         best = choose(n);
+         best = plan.choose(n, cus, HUGE_VAL);
          prepare();
       }
       g.x = p.x + n0 * (image / 4);
@@ -705,7 +586,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       }
       int rc = SOFIE_HIP_OK;
       switch (best.ti * 100 + best.tj * 10 + best.wo) {
-#define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, quads(), rows, tiles); break
+#define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, plan.quads(g.phase[0].strips), rows, tiles); break
          SOFIE_FORM(4, 4, 2); SOFIE_FORM(3, 4, 2); SOFIE_FORM(2, 4, 2); SOFIE_FORM(4, 2, 2); SOFIE_FORM(2, 2, 2); SOFIE_FORM(1, 4, 2); SOFIE_FORM(1, 2, 2);
          SOFIE_FORM(1, 4, 1);
 #undef SOFIE_FORM

@@ -1,0 +1,92 @@
+"""How k_conv_f32_split chooses tiles, slots and strips (sofie_amd/csrc/conv_f32_split_plan.h), on the host: the same choice as a search that
+leaves no form out, and few estimates on the way (each call makes them, in front of launches that may take 6 us)."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "conv_f32_split_plan.h"
+using namespace sofie;
+
+// every form and slot, no bound in front of the strips
+static double search(SplitPlan &plan, size_t n, double other_us, int icg, int octiles)
+{
+   static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
+   double best = other_us;
+   for (const auto &f : forms) {
+      if ((plan.rows && f[0] > 2) || (f[0] > 1 && f[2] * (f[0] - 1) >= octiles)) continue;
+      for (int cs = plan.rows ? 8 * icg : 16; cs <= (plan.rows ? 8 * icg : 32); cs *= 2) {
+         SplitPlan::Form form{f[0], f[1], f[2], cs, 0, 0.0};
+         double least = HUGE_VAL;
+         for (int strips = 1; strips <= 16; ++strips) {
+            SplitPlan::Panels q[4], kinds[4];
+            int cells = 0;
+            bool fits = true;
+            for (int i = 0; i < plan.nphases; ++i) {
+               fits = fits && plan.panels(q[i], i, form.pixels(), strips) && (plan.slots(cs) == 1 || cs / 8 * plan.chunks[i] >= 4);
+               if (fits && q[i].cells > cells) cells = q[i].cells;
+            }
+            if (!fits || cells * (cs / 8) > SplitPlan::items_of(f[0], f[1], f[2], plan.rows) * SplitPlan::THREADS) continue;
+            if (plan.table_bytes(cs) + (plan.slots(cs) > 1 ? 2 : 1) * SplitPlan::slot_bytes(cells, cs) > SplitPlan::MAX_LDS) continue;
+            if ((double)n * q[0].strips * q[0].PHW > (double)(1 << 30)) continue;
+            for (int k = 0; k < plan.kinds; ++k) kinds[k] = q[plan.kind[k]];
+            const double time = plan.estimate(form, kinds, n, 256) * (strips > 1 ? 1.02 : 1.0);
+            if (time < least) least = time, form.strips = strips;
+            else if (strips > form.strips + 1) break;
+         }
+         if (least < best) best = least;
+      }
+   }
+   return best;
+}
+
+int main()
+{
+   srand(7);
+   auto pick = [](int lo, int hi) { return lo + rand() % (hi - lo + 1); };
+   long layers = 0, taken = 0, estimates = 0, without = 0, most = 0;
+   while (layers < 3000) {
+      ConvProblem p{};
+      const int kind = rand() % 4;      // convolution, few channels, transposed 4x4 and 3x3 of stride 2
+      const int k = kind == 1 ? pick(4, 8) : kind == 2 ? 4 : kind == 3 ? 3 : 2 * pick(0, 3) + 1, s = kind >= 2 ? 2 : pick(1, 2), pad = (k - 1) / 2;
+      p.N = 1 << pick(0, 8), p.C = kind == 1 ? pick(1, 5) : pick(6, 260), p.OC = pick(8, 260), p.groups = 1;
+      p.H = pick(5, 150), p.W = rand() % 2 ? p.H : pick(5, 224);
+      p.dh = p.dw = 1, p.KH0 = p.KW0 = k, p.transposed = kind >= 2, p.nphases = kind >= 2 ? 4 : 1;
+      p.sh = p.sw = kind >= 2 ? 1 : s;
+      p.OH0 = kind >= 2 ? s * (p.H - 1) + k - 2 * pad : (p.H + 2 * pad - k) / s + 1;
+      p.OW0 = kind >= 2 ? s * (p.W - 1) + k - 2 * pad : (p.W + 2 * pad - k) / s + 1;
+      if ((double)p.N * p.C * p.H * p.W > (1 << 27) || (double)p.N * p.OC * p.OH0 * p.OW0 > (1 << 27)) continue;
+      for (int i = 0; i < p.nphases; ++i) {
+         ConvPhase &f = p.phase[i];
+         if (kind < 2) f = {p.OH0, p.OW0, k, k, pad, pad, 0, 1, 0, 1, 0, 1, 0, 1};
+         else f = {(p.OH0 + 1 - i / 2) / 2, (p.OW0 + 1 - i % 2) / 2, k == 4 ? 2 : 1 + i / 2, k == 4 ? 2 : 1 + i % 2, 1 - i / 2, 1 - i % 2, 0, 2, 0, 2, i / 2, 2, i % 2, 2};
+      }
+      const bool rows = kind == 1;
+      const double other = rand() % 2 ? HUGE_VAL : 7.5 + rand() % 40;
+      SplitPlan plan(p, rows), all(p, rows);
+      const SplitPlan::Form form = plan.choose(p.N, 256, other);
+      const double best = search(all, p.N, other, p.C, plan.octiles);
+      if (form.time != best) return printf("layer %ld: %.17g, searched %.17g\n", layers, form.time, best), 1;
+      ++layers;
+      taken += form.ti > 0;
+      estimates += plan.evaluated;
+      without += all.evaluated;      // (its end of a row of strips that only get longer is the same)
+      most = plan.evaluated > most ? plan.evaluated : most;
+   }
+   printf("%ld %ld %ld %ld %ld\n", layers, taken, estimates, without, most);
+}
+"""
+
+
+def test_the_choice_of_a_full_search_with_few_estimates(tmp_path):
+    src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "sofie_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    layers, taken, estimates, without, most = map(int, out.stdout.split())
+    assert layers == 3000 and taken > 1000
+    assert estimates <= 7 * layers and most <= 70 and without >= 4 * estimates, out.stdout
