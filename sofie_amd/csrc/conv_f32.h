@@ -5,8 +5,9 @@
 
 namespace sofie {
 
-// Runs the problem on k_conv_f32_any (conv_f32_any.hip) or k_conv_f32_split; *done stays false where they do not take it, or where
-// the former's estimate is above the microseconds of the caller's other way. split_only: not on the former.
+// Runs the problem on k_conv_f32_any (conv_f32_any.hip), k_conv_f32_split or k_conv_f32_short; *done stays false where they do not take it,
+// or where their estimates are above the microseconds of the caller's other way (HUGE_VAL: it has no estimate of that). split_only: on
+// k_conv_f32_split, if that is shorter than k_conv_f32_any by their estimates.
 int conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done, bool split_only = false);
 
 // Runs the problem on k_conv_f32_split (conv_f32_split.hip); *done stays false where it does not take it, or where its estimate is above

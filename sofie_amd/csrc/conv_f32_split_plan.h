@@ -161,6 +161,9 @@ struct SplitPlan {
             if (s.cells[strips - 1] == 0 || s.cells[strips - 1] > room) continue;
             if (table_bytes(cs) + (slots(cs) > 1 ? 2 : 1) * (long)slot_bytes(s.cells[strips - 1], cs) > MAX_LDS) continue;
             if ((double)n * q[0].strips * q[0].PHW > (double)(1 << 30)) continue;
+            // (128 channels x 64 pixels with 4-byte stores take up to 1.8 times what the estimate says, and more than the next form: transposed
+            // 23x110x51x10 -> 256, 3x3 s2 108 us, 64 without it, 83 on k_conv_f32_any; 118x20x29x34 -> 225, 3x3 115, on k_conv2d_f32_dma 106)
+            if (form.ti == 4 && form.tj == 2 && !quads(q[0].strips)) continue;
             const double time = estimate(form, q, n, cus) * (strips > 1 ? 1.02 : 1.0);
             if (time < form.time) {
                form.time = time;
@@ -251,9 +254,10 @@ private:
          const double per_cu = tiles / cus, rounds = per_cu / resident, whole = rounds + 0.895 * (up(rounds) - rounds);
          const double waits = alone * (whole > 1.0 ? whole : 1.0), busy = up(per_cu) * work / tiles;
          const double w2 = waits * waits, b2 = busy * busy;
-         // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings)
+         // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings; with 1.4 the layers it takes of 190
+         // random ones are 0.96 to 1.75 times k_conv_f32_any's time, with 1.35 0.94)
          const ConvPhase &q0 = l.p.phase[0], &q1 = l.p.phase[l.nphases - 1];
-         const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.35 : 1.0;
+         const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.4 : 1.0;
          return std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
       }
    };

@@ -1,5 +1,6 @@
 """How k_conv_f32_split chooses tiles, slots and strips (sofie_amd/csrc/conv_f32_split_plan.h), on the host: the same choice as a search that
-leaves no form out, and few estimates on the way (each call makes them, in front of launches that may take 6 us)."""
+leaves no form out, and few estimates on the way (each call makes them, in front of launches that may take 6 us). No tile of 128 channels x
+64 pixels where stores are four bytes, which takes up to 1.8 times its estimate."""
 import os
 import subprocess
 
@@ -32,6 +33,7 @@ static double search(SplitPlan &plan, size_t n, double other_us, int icg, int oc
             if (!fits || cells * (cs / 8) > SplitPlan::items_of(f[0], f[1], f[2], plan.rows) * SplitPlan::THREADS) continue;
             if (plan.table_bytes(cs) + (plan.slots(cs) > 1 ? 2 : 1) * SplitPlan::slot_bytes(cells, cs) > SplitPlan::MAX_LDS) continue;
             if ((double)n * q[0].strips * q[0].PHW > (double)(1 << 30)) continue;
+            if (f[0] == 4 && f[1] == 2 && !plan.quads(q[0].strips)) continue;
             for (int k = 0; k < plan.kinds; ++k) kinds[k] = q[plan.kind[k]];
             const double time = plan.estimate(form, kinds, n, 256) * (strips > 1 ? 1.02 : 1.0);
             if (time < least) least = time, form.strips = strips;
@@ -70,6 +72,7 @@ int main()
       const SplitPlan::Form form = plan.choose(p.N, 256, other);
       const double best = search(all, p.N, other, p.C, plan.octiles);
       if (form.time != best) return printf("layer %ld: %.17g, searched %.17g\n", layers, form.time, best), 1;
+      if (form.ti == 4 && form.tj == 2 && !plan.quads(form.strips)) return printf("layer %ld: 128 channels x 64 pixels with 4-byte stores\n", layers), 1;
       ++layers;
       taken += form.ti > 0;
       estimates += plan.evaluated;
