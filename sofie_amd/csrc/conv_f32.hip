@@ -659,8 +659,8 @@ ConvProblem problem_of(const ConvArgs &g)
 }
 
 // The whole of g (its one phase, or all of them) on k_conv_f32_any; *done stays false where it does not take it, or where
-// other_us is the shorter way. split_only: on k_conv_f32_split or not at all.
-int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us = HUGE_VAL, bool split_only = false)
+// other_us is the shorter way.
+int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us = HUGE_VAL, ConvWays ways = ALL_WAYS)
 {
    ConvProblem p = problem_of(g);
    p.nphases = g.nphases > 1 ? g.nphases : 1;
@@ -669,7 +669,7 @@ int run_any(sofie_hip_ctx *ctx, const ConvArgs &g, bool *done, double other_us =
       const PhaseArgs &f = g.phase[i];
       p.phase[i] = {f.OH, f.OW, f.KH, f.KW, f.ph, f.pw, f.th0, g.ths, f.tw0, g.tws, f.oy0, g.oys, f.ox0, g.oxs};
    }
-   return conv_f32_any(ctx, p, other_us, done, split_only);
+   return conv_f32_any(ctx, p, other_us, done, ways);
 }
 
 // Whether a layer that k_conv2d_f32_dma takes (full channel blocks of an even K) runs on k_conv_f32_any all the same.
@@ -895,13 +895,13 @@ int launch(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
 // the channel block and patch geometry a launch of its own would get; the grid is as wide as the phase with most
 // pixel tiles. *done stays false if a phase does not fit (the caller then launches the phases one by one).
 template <int TI, int TJ>
-int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
+int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done, ConvWays ways)
 {
    constexpr int BOC = 2 * TI * 32, BP = 2 * TJ * 32, LDW = BOC + 1;
    const size_t budget = 52 * 1024;
    *done = false;
    const int octiles = cdiv(g.ocg, BOC);
-   if ((size_t)g.groups * octiles > 65535 || (size_t)g.N * g.nphases > 65535) return run_any(ctx, g, done);
+   if ((size_t)g.groups * octiles > 65535 || (size_t)g.N * g.nphases > 65535) return run_any(ctx, g, done, HUGE_VAL, ways);
    size_t lds_max = 0;
    int tiles_max = 0;
    // First choice: operands by LDS-DMA under the matrix loop, on sub-kernels gathered into the [K][channel] order (a
@@ -1028,7 +1028,7 @@ int launch_phases(sofie_hip_ctx *ctx, ConvArgs &g, bool *done)
          cells += tiles * cut;
       }
       const double other = staged ? staged_us(true, K, patch, all_tiles, work, cells, (double)g.N * g.OC * g.OH0 * g.OW0) : HUGE_VAL;
-      if (int rc = run_any(ctx, g, done, other)) return rc;
+      if (int rc = run_any(ctx, g, done, other, ways)) return rc;
       if (*done) return SOFIE_HIP_OK;
    }
    for (int i = 0; i < g.nphases; ++i) {
@@ -1083,7 +1083,7 @@ int run_conv(sofie_hip_ctx *ctx, ConvArgs &g)
    int rc;
    const Beyond beyond = beyond_dma(ctx, g);
    if (beyond && (!g.transposed || (g.uh == 1 && g.uw == 1))) {
-      rc = run_any(ctx, g, &done, dma_us(ctx, g), beyond == SPLIT);
+      rc = run_any(ctx, g, &done, dma_us(ctx, g), beyond == SPLIT ? SPLIT_ONLY : ALL_WAYS);
       if (rc || done) return rc;
    }
    const Tiling t = tiling_of(ctx, g);
@@ -1276,8 +1276,10 @@ extern "C" int sofie_hip_conv_transpose2d_f32(sofie_hip_ctx *ctx, const float *x
       if (ok && all.nphases > 1) {
          all.dUH = make_fastdiv(1u); all.dUW = make_fastdiv(1u); all.dOW = make_fastdiv(1u);
          bool done = false;
-         if (const Beyond beyond = beyond_dma(ctx, all)) {
-            if (int rc = run_any(ctx, all, &done, HUGE_VAL, beyond == SPLIT)) return rc;
+         const Beyond beyond = beyond_dma(ctx, all);
+         const ConvWays left = beyond == SPLIT ? SPLIT_DECLINED : ALL_WAYS;
+         if (beyond) {
+            if (int rc = run_any(ctx, all, &done, HUGE_VAL, beyond == SPLIT ? SPLIT_ONLY : ALL_WAYS)) return rc;
             if (done) return SOFIE_HIP_OK;
          }
          // tiles as for the plain convolution: the largest that still give every compute unit one
@@ -1287,9 +1289,9 @@ extern "C" int sofie_hip_conv_transpose2d_f32(sofie_hip_ctx *ctx, const float *x
             return t * all.groups * cdiv(all.ocg, boc) * all.N;
          };
          int rc;
-         if (all.ocg > 64 && tiles(128, 128) >= (size_t)ctx->num_cus) rc = launch_phases<2, 2>(ctx, all, &done);
-         else if (tiles(64, 128) >= (size_t)ctx->num_cus) rc = launch_phases<1, 2>(ctx, all, &done);
-         else rc = launch_phases<1, 1>(ctx, all, &done);
+         if (all.ocg > 64 && tiles(128, 128) >= (size_t)ctx->num_cus) rc = launch_phases<2, 2>(ctx, all, &done, left);
+         else if (tiles(64, 128) >= (size_t)ctx->num_cus) rc = launch_phases<1, 2>(ctx, all, &done, left);
+         else rc = launch_phases<1, 1>(ctx, all, &done, left);
          if (rc || done) return rc;
       }
    }

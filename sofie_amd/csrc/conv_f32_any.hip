@@ -455,7 +455,7 @@ int launch(sofie_hip_ctx *ctx, const AnyArgs &g, int nphases, int mode, int stor
 
 }  // namespace
 
-int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done, bool split_only)
+int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_us, bool *done, ConvWays ways)
 {
    *done = false;
    const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
@@ -590,12 +590,13 @@ int sofie::conv_f32_any(sofie_hip_ctx *ctx, const ConvProblem &p, double other_u
    if (best.ti == 0) return SOFIE_HIP_OK;
    const double here_us = best.time / 2400.0 * ((double)p.N / (double)per) + (ctx->constant_weights ? 0.0 : 3.1);
    // Shorter sums are shorter on the vector unit.
-   if (!split_only)
+   if (ways != SPLIT_ONLY)
       if (int rc = conv_f32_short(ctx, p, 0.9 * (here_us < other_us ? here_us : other_us), done); rc || *done) return rc;
    // Longer sums on many tiles are shorter on the bf16 matrix instructions. The estimates are off by some 10 %; of 42 random 3x3 layers of 18 to
    // 26 channels that it takes none is longer than on the kernel it takes the place of.
-   if (int rc = conv_f32_split(ctx, p, 0.9 * here_us < 0.95 * other_us ? 0.9 * here_us : 0.95 * other_us, done); rc || *done) return rc;
-   if (split_only) return SOFIE_HIP_OK;
+   if (ways != SPLIT_DECLINED)
+      if (int rc = conv_f32_split(ctx, p, 0.9 * here_us < 0.95 * other_us ? 0.9 * here_us : 0.95 * other_us, done); rc || *done) return rc;
+   if (ways == SPLIT_ONLY) return SOFIE_HIP_OK;
    // against what the caller has instead (the estimate's unit is a cycle at 2400 MHz; weights that are not kept are laid out in
    // front of the launch, 3.1 us)
    if (other_us < 0.95 * here_us) return SOFIE_HIP_OK;

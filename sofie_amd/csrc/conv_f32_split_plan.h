@@ -2,11 +2,12 @@
 // alone, also for a host program that checks it against a search through everything.
 //
 // Every call works this out anew, in front of a launch that may take 6 us: forms (tile and slot) come in the order of what they take at
-// least, those that cannot be shorter than the best so far are left before their strips are looked at, and what strips of an image
-// need depends on the tile's pixels alone and is worked out once for all forms and for phases of the same sizes. us of a call on the host
-// without its launches, every form laid out for up to 16 strips / now / without this kernel (2.7 GHz): 256x64x56x56 -> 128, 3x3 6.4 / 2.8 / 0.8;
-// 1x128x56x56 -> 128, 3x3, which k_conv_f32_any takes, 5.9 / 1.5 / 0.8; transposed 1x111x25x25 -> 192, 4x4 s2, taken by it, too, 26 / 4.0 / 1.3, and
-// 17.6 us a call on the device for 11.0 of the kernel; 300 random layers 1.46 / 0.84 / 0.50 in the mean, 15 / 3.6 / 1.3 at most.
+// least, by a bound on the cells that any strips need; those that cannot be shorter than the best so far are left before their strips are
+// looked at, and what strips of an image need depends on the tile's pixels alone and is worked out once for all forms and for phases of the
+// same sizes. us of a call on the host without its launches, every form laid out for up to 16 strips / now / without this kernel (2.7 GHz):
+// 256x64x56x56 -> 128, 3x3 6.4 / 2.4 / 0.7; 1x128x56x56 -> 128, 3x3, which k_conv_f32_any takes, 5.9 / 1.3 / 0.7; transposed 1x111x25x25 -> 192,
+// 4x4 s2, taken by it, too, 26 / 2.8 / 1.2, and 17.6 us a call on the device for 11.0 of the kernel; 300 random layers 1.5 / 0.73 / 0.50 in the
+// mean, 17 / 3.2 / 1.3 at most.
 #pragma once
 #include <cmath>
 
@@ -124,6 +125,8 @@ struct SplitPlan {
       Form best{0, 0, 0, 0, 0, other_us};
       if (pieces * 16 > ((size_t)1 << 29)) return best;
       for (Strips &s : strips_seen) s.seen = 0;
+      for (int k = 0; k < kinds; ++k)
+         for (int t = 0; t < 3; ++t) least_cells[t][k] = cells_at_least(p.phase[kind[k]], 64 << t);
       // what may be the shortest first
       struct Candidate {
          Form form;
@@ -135,12 +138,12 @@ struct SplitPlan {
          if (f[0] > 1 && f[2] * (f[0] - 1) >= octiles) continue;      // tiles of nothing
          for (int cs = rows ? 8 * icg : 16; cs <= (rows ? 8 * icg : 32); cs *= 2) {
             Form form{f[0], f[1], f[2], cs, 0, 0.0};
-            // (a tile's patch has a cell for each of its pixels and more)
-            if (form.pixels() > cells_of(form)) continue;
-            bool enough = true;       // a step reaches into one slot behind its first chunk's
-            for (int k = 0; k < kinds; ++k) enough = enough && (slots(cs) == 1 || cs / 8 * chunks[kind[k]] >= 4);
+            // (a step reaches into one slot behind its first chunk's)
+            bool enough = true;
+            for (int k = 0; k < kinds; ++k) enough = enough && least_cells[tile_of(form)][k] <= cells_of(form) && (slots(cs) == 1 || cs / 8 * chunks[kind[k]] >= 4);
+            if (!enough) continue;
             form.time = least_time(form, n, cus);
-            if (!enough || form.time >= best.time) continue;
+            if (form.time >= best.time) continue;
             int at = count++;
             for (; at > 0 && candidates[at - 1].form.time > form.time; --at) candidates[at] = candidates[at - 1];
             candidates[at] = {form, (int)(&f - forms) * 2 + (cs == 32)};
@@ -151,7 +154,7 @@ struct SplitPlan {
          Form form = candidates[c].form;
          form.time = HUGE_VAL;
          const int cs = form.cs, bp = form.pixels(), room = cells_of(form);
-         Strips &s = strips_seen[bp == 64 ? 0 : bp == 128 ? 1 : 2];
+         Strips &s = strips_seen[tile_of(form)];
          // (as many strips as the estimate says: fewer cells for a tile's pixels against whole lines per store, 4-byte stores where strips are no
          // whole fours, 256x64x10x10 -> 128 29.5 us in one strip, 36.2 in five of two columns; by the number of cells alone 42x59x79x62 -> 9, 3x3 66.5,
          // now 46.9, and k_conv_f32_any 58.7)
@@ -205,6 +208,17 @@ private:
       Panels panels[MAX_STRIPS][MAX_PHASES];      // of each kind of phases
    };
    Strips strips_seen[3];                  // tiles of 64, 128 and 256 pixels
+   int least_cells[3][MAX_PHASES];         // of each kind of phases
+   static int tile_of(const Form &f) { return f.pixels() == 64 ? 0 : f.pixels() == 128 ? 1 : 2; }
+
+   // Cells of the patch of bp pixels, whatever the strips: r rows of pixels of bp / r columns read ((r - 1) sh + h) x ((bp / r - 1) sw + w)
+   // cells, h x w under one pixel; the smallest product over all real r (rounded down, and by 1 for the square roots).
+   int cells_at_least(const ConvPhase &f, int bp) const
+   {
+      const double h = (double)(f.KH - 1) * p.dh + 1, w = rows ? 1.0 : (double)(f.KW - 1) * p.dw + 1, sh = p.sh < h ? p.sh : h, sw = rows ? 1.0 : p.sw < w ? p.sw : w;
+      const double root = std::sqrt((h - sh) * (w - sw)) + std::sqrt(bp * sh * sw), cells = root * root;
+      return cells < 1e6 ? (int)cells - 1 : 1000000;
+   }
 
    void look_at(Strips &s, int bp, int strips)
    {
@@ -262,11 +276,11 @@ private:
       }
    };
 
-   // What the estimate cannot be below, whatever the strips: every pixel once, a cell for each pixel of a tile, the better kind of stores.
+   // What the estimate cannot be below, whatever the strips: every pixel once, the fewest cells, the better kind of stores.
    double least_time(const Form &f, size_t n, int cus) const
    {
       Sum s(*this, f, cus, resident_of(f.ti, f.tj, f.wo), quads(1) || quads(2));
-      for (int k = 0; k < kinds; ++k) s.add(k, (int)(((double)n * p.phase[kind[k]].OH * p.phase[kind[k]].OW + f.pixels() - 1) / f.pixels()), f.pixels());
+      for (int k = 0; k < kinds; ++k) s.add(k, (int)(((double)n * p.phase[kind[k]].OH * p.phase[kind[k]].OW + f.pixels() - 1) / f.pixels()), least_cells[tile_of(f)][k]);
       return s.time();
    }
 };

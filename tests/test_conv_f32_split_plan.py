@@ -92,4 +92,4 @@ def test_the_choice_of_a_full_search_with_few_estimates(tmp_path):
     assert out.returncode == 0, out.stdout
     layers, taken, estimates, without, most = map(int, out.stdout.split())
     assert layers == 3000 and taken > 1000
-    assert estimates <= 7 * layers and most <= 70 and without >= 4 * estimates, out.stdout
+    assert estimates <= 6 * layers and most <= 50 and without >= 4 * estimates, out.stdout
