@@ -223,14 +223,18 @@ __global__ void __launch_bounds__(WAVES * 64, 2) k_gemm_f32_split(GemmF32Args g)
    }
    wait_lds_reads();
 
-   // sums that are not finite: again, with fp32 instructions on the operands as they are
+   // sums that are not finite: again, with fp32 instructions on the operands as they are (1500 x 1001 x 1111, 29 us: 14 more with one
+   // infinity, 28 with one in a hundred)
    v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
-         for (int e = 0; e < 4; ++e) none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
+         for (int e = 0; e < 4; ++e) {
+            acc[i][j][e] = unscaled(acc[i][j][e]);
+            none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
+         }
    if (__builtin_amdgcn_ballot_w64((none[0] + none[1]) + (none[2] + none[3]) != 0.0f) != 0) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)

@@ -45,7 +45,7 @@ CONV = [
 
 @pytest.mark.parametrize("shape", CONV)
 def test_rows_as_cells(ops, kept, shape):
-    """Products of split numbers lose less than 2^-26 each, sums are rounded once per 32 k: 1e-5 of the largest output as for the other fp32
+    """Products of split numbers lose at most 2^-24 each (2^-27 in the mean), sums are rounded once per 32 k: 1e-5 of the largest output as for the other fp32
     kernels, 3e-7 in the 2-norm."""
     n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
     t, l, b, r = pads

@@ -59,8 +59,8 @@ def reference(x, w, bias, s, pads, d, groups):
 
 @pytest.mark.parametrize("shape", CONV)
 def test_conv_in_three_parts(ops, kept, shape):
-    """Products of split numbers lose less than 2^-26 each and sums are rounded once per 32 k at their own size, where fp32 products
-    in a row are rounded K times: 1e-5 of the largest output, as for the other fp32 kernels, and 3e-7 in the 2-norm (they show up to
+    """Products of split numbers lose at most 2^-24 each (2^-27 in the mean) and sums are rounded once per 32 k at their own size, where fp32
+    products in a row are rounded K times: 1e-5 of the largest output, as for the other fp32 kernels, and 3e-7 in the 2-norm (they show up to
     1e-6 at these K)."""
     n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
     g = torch.Generator(device="cuda").manual_seed(n + c + oc)
@@ -120,8 +120,7 @@ def test_values_that_are_not_finite_stay_in_their_windows(ops, kept, c, relu):
 
 
 def test_small_and_mixed_magnitudes_keep_their_bits(ops, kept):
-    """Every cell is split by itself: rows 2^60 apart in one tile, and weights near the smallest normal numbers of bf16's lowest part, are
-    as exact as rows of ones."""
+    """Every cell is split by itself: rows 2^60 apart in one tile, and channels of weights 2^100 apart, are as exact as rows of ones."""
     g = torch.Generator(device="cuda").manual_seed(5)
     x = torch.randn(64, 64, 28, 28, device="cuda", generator=g) * torch.exp2(torch.randint(-30, 31, (64, 1, 28, 1), device="cuda", generator=g).float())
     w = torch.randn(96, 64, 3, 1, device="cuda", generator=g) * torch.exp2(torch.randint(-60, 40, (96, 1, 1, 1), device="cuda", generator=g).float())
@@ -131,7 +130,42 @@ def test_small_and_mixed_magnitudes_keep_their_bits(ops, kept):
     assert names[-1] == "k_conv_f32_split"
     ref = torch.nn.functional.conv2d(x.double(), w.double(), None, 1, (1, 0)).cpu()
     size = torch.nn.functional.conv2d(x.double().abs(), w.double().abs(), None, 1, (1, 0)).cpu()
-    assert bool(((y.cpu().double() - ref).abs() <= 2.0 ** -21 * size).all())      # two roundings of 2^-24 per 32 k and 2^-26 per product
+    assert bool(((y.cpu().double() - ref).abs() <= 2.0 ** -21 * size).all())      # two roundings of 2^-24 per 32 k and 2^-24 per product
+
+
+# exponents of cells and weights: the smallest numbers of fp32 (2^-149) against large ones, products near 2^-126, sums above 2^95 (which
+# are repeated with fp32 instructions), and all of them next to each other (None)
+EXPONENTS = [(-114, 100), (-126, 110), (-140, 108), (110, -126), (100, -140), (-60, -60), (60, 60), (112, 0), (None, 0), (0, None)]
+
+
+@pytest.mark.parametrize("e,f", EXPONENTS)
+@pytest.mark.parametrize("kind", ["3x3", "rows", "phases"])
+def test_magnitudes_of_all_sizes_keep_their_bits(ops, kept, kind, e, f):
+    """Whatever the exponents: each output as near to float64 as with operands of one size, where the lowest bits of cells and weights are
+    below those of bf16's smallest number, too. 2^-21 of the sum of the products' sizes: a rounding of 2^-24 per 32 k (at most 32 here, and they
+    add as their square root) and 2^-24 per product. Where all exponents meet, sums above 2^95 among them are repeated, a rounding of 2^-24 for
+    each of K products, of the size of the largest: K^1/2 2^-24."""
+    c, k = {"3x3": (64, 3), "rows": (3, 7), "phases": (64, 4)}[kind]
+    g = torch.Generator().manual_seed(5)
+
+    def scaled(t, exponent):
+        s = torch.randint(-140, 120, t.shape, generator=g).double() if exponent is None else torch.full((), float(exponent), dtype=torch.float64)
+        return (t.double() * torch.exp2(s)).float()
+    x = scaled(torch.randn(48, c, 40, 40, generator=g), e)
+    w = scaled(torch.randn((c, 64, k, k) if kind == "phases" else (96, c, k, k), generator=g) * (c * k * k) ** -0.5, f)
+    xd, wd = x.cuda(), w.cuda()
+    torch.cuda.synchronize()
+    if kind == "phases":
+        y, names = names_of(kept, lambda: ops.conv_transpose2d_f32(xd, wd, None, (1, 1, 1, 1), (2, 2), (1, 1), 1, (0, 0), ctx=kept))
+        conv = lambda a, b: torch.nn.functional.conv_transpose2d(a, b, None, 2, 1)
+    else:
+        y, names = names_of(kept, lambda: ops.conv2d_f32(xd, wd, None, (k // 2, k // 2), ctx=kept))
+        conv = lambda a, b: torch.nn.functional.conv2d(a, b, None, 1, k // 2)
+    assert names[-1] == "k_conv_f32_split"
+    bound = 2.0 ** -21 if None not in (e, f) else (c * k * k) ** 0.5 * 2.0 ** -24
+    for i in (0, 20, 47):
+        xi, wi = x[i:i + 1].double(), w.double()
+        assert bool(((y[i:i + 1].cpu().double() - conv(xi, wi)).abs() <= bound * conv(xi.abs(), wi.abs()) + c * k * k * 2.0 ** -149).all()), i
 
 
 def test_whole_numbers_are_exact(ops, kept):

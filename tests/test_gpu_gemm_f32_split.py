@@ -47,7 +47,7 @@ SHAPES = [(64, 6208, 1106), (65, 6209, 1105), (112, 7656, 1284), (97, 6301, 1283
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_gemm_in_three_parts(ops, shape, tA, tB):
-    """Products of split numbers lose less than 2^-26 each and sums are rounded once per 32 k at their own size, where fp32 products in a
+    """Products of split numbers lose at most 2^-24 each (2^-27 in the mean) and sums are rounded once per 32 k at their own size, where fp32 products in a
     row are rounded K times: 3e-7 in the 2-norm and 1e-6 of the largest output (fp32 instructions show up to 1.2e-6 at these K).
     The same bits on a second call."""
     M, N, K = shape
@@ -100,4 +100,25 @@ def test_gemm_in_three_parts_of_values_that_are_not_finite(ops, tB):
         fin = ref32[i].isfinite()
         if bool(fin.any()):
             assert float((got[i][fin].double() - ref32[i][fin]).abs().max()) <= 1e-5 * float(ref32[i][fin].abs().max()), r
+    ctx.close()
+
+
+@pytest.mark.parametrize("e,f", [(-114, 100), (-126, 110), (-140, 108), (100, -140), (-60, -60), (60, 60), (112, 0), (None, 0), (0, None)])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0)])
+def test_magnitudes_of_all_sizes_keep_their_bits(ops, tA, tB, e, f):
+    """Whatever the exponents of a and b (None: all of them next to each other): each output as near to float64 as with operands of one size,
+    where their lowest bits are below those of bf16's smallest number, too. 2^-21 of the sum of the products' sizes: a rounding of 2^-24 per
+    32 k of a wavefront and for the wavefronts' sums, and 2^-24 per product."""
+    M, N, K = (1500, 1001, 1111) if not tA else (4624, 640, 1111)
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def scaled(shape, exponent):
+        s = torch.randint(-140, 120, shape, device="cuda", generator=g).double() if exponent is None else torch.full((), float(exponent), dtype=torch.float64, device="cuda")
+        return (torch.randn(shape, device="cuda", generator=g).double() * torch.exp2(s)).float()
+    a, b = scaled((K, M) if tA else (M, K), e), scaled((N, K) if tB else (K, N), f)
+    ctx = ops.Context(0)
+    y, names = product(ctx, a, b, tA, tB, None)
+    assert "k_gemm_f32_split" in names, names
+    a, b = (a.t() if tA else a).double().contiguous(), (b.t() if tB else b).double().contiguous()
+    assert bool(((y.double() - a @ b).abs() <= 2.0 ** -21 * (a.abs() @ b.abs()) + K * 2.0 ** -149).all())
     ctx.close()
