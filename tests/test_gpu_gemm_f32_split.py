@@ -1,5 +1,6 @@
-"""fp32 products on k_gemm_f32_split (operands as three bf16 numbers): every storage, 32, 64 and 96 rows per workgroup, K in slices, a K of
-one chunk per wavefront and less, rows, columns and K that are no whole fours, against float64; values that are not finite."""
+"""fp32 products on k_gemm_f32_split (operands as three bf16 numbers): every storage, 32, 64 and 96 rows per workgroup, K in slices, the
+shortest K it is chosen for (two chunks per wavefront, one k in the last), rows, columns and K that are no whole fours, against float64;
+values that are not finite."""
 import ctypes as C
 
 import pytest
@@ -39,14 +40,16 @@ def product(ctx, a, b, tA, tB, bias, alpha=1.0, beta=1.0, relu=False, pad=0):
     return y[1:M + 1, :N], [line.split()[0] for line in buf.value.decode().splitlines()]
 
 
-# M, N, K; 32 rows per workgroup, 64, 96, K in slices; every storage
-SHAPES = [(64, 6208, 1106), (65, 6209, 1105), (112, 7656, 1284), (97, 6301, 1283), (1500, 1001, 1111), (1501, 1003, 1024), (1441, 1089, 258),
-          (1537, 1023, 257), (4624, 133, 5187), (130, 3633, 4279), (2447, 107, 5990)]
+# M, N, K: whether A stored along M takes the kernel, too (64 rows per workgroup or none); slices of K
+SHAPES = [((64, 6208, 1106), False, 1), ((65, 6209, 1105), True, 1), ((112, 7656, 1284), True, 1), ((97, 6301, 1283), True, 1),
+          ((1500, 1001, 1111), False, 1), ((1501, 1003, 1024), False, 1), ((1441, 1089, 1538), True, 1), ((1537, 1023, 2049), True, 1),
+          ((1195, 1160, 481), False, 1), ((1757, 2409, 486), False, 1), ((4624, 133, 5187), True, 1), ((130, 3633, 4279), False, 2),
+          ((2447, 107, 5990), True, 3), ((3001, 1001, 1113), True, 1)]
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape,along_m,slices", SHAPES)
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-def test_gemm_in_three_parts(ops, shape, tA, tB):
+def test_gemm_in_three_parts(ops, shape, along_m, slices, tA, tB):
     """Products of split numbers lose at most 2^-24 each (2^-27 in the mean) and sums are rounded once per 32 k at their own size, where fp32 products in a
     row are rounded K times: 3e-7 in the 2-norm and 1e-6 of the largest output (fp32 instructions show up to 1.2e-6 at these K).
     The same bits on a second call."""
@@ -59,11 +62,12 @@ def test_gemm_in_three_parts(ops, shape, tA, tB):
     ctx = ops.Context(0)
     y, names = product(ctx, a, b, tA, tB, bias)
     want = ref + bias.double()
-    if "k_gemm_f32_split" in names:
+    if not tA or along_m:
+        assert names == ["k_gemm_f32_split"] + ["k_gemm_f32_skinny_finish"] * (slices > 1), names
         err = y.double() - want
         assert float(err.norm()) <= 3e-7 * float(want.norm()) and float(err.abs().max()) <= 1e-6 * float(want.abs().max())
-    else:      # (operands stored along M take 64 rows or nothing)
-        assert tA or K < 300, names
+    else:
+        assert "k_gemm_f32_split" not in names, names
     assert torch.equal(y, product(ctx, a, b, tA, tB, bias)[0])
     y, _ = product(ctx, a, b, tA, tB, bias, alpha=-0.5, beta=2.0, relu=True, pad=3)
     want = (-0.5 * ref + 2.0 * bias.double()).clamp(min=0)
@@ -71,20 +75,21 @@ def test_gemm_in_three_parts(ops, shape, tA, tB):
     ctx.close()
 
 
-@pytest.mark.parametrize("tB", [0, 1])
-def test_gemm_in_three_parts_of_values_that_are_not_finite(ops, tB):
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_in_three_parts_of_values_that_are_not_finite(ops, tA, tB):
     """Infinities, NaN and sums that overflow stay where fp32 products put them, and finite ones next to them stay right; numbers that
     bf16 would round up to infinity are finite."""
-    M, N, K = 1500, 1001, 1111
+    M, N, K = 3001 if tA else 1500, 1001, 1111
     g = torch.Generator(device="cuda").manual_seed(5)
     a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g)
     a[3, 7], a[700, 1110], a[1499, 0], a[900, 50], b[50, 1000] = float("inf"), float("nan"), float("-inf"), 3.4e38, 0.25
+    a[[3, 700, 900, 1499], 9] = 0.0      # (b[9, 33] below: two products that overflow with opposite signs are NaN in fp32)
     a[40, :] = 0.0
     a[40, 9], b[9, 33] = 1.0, 3.4028234e38
     a[41, :] = 3e38
     b[:, 500] = 1.0
     ctx = ops.Context(0)
-    y, names = product(ctx, a, b.t().contiguous() if tB else b, 0, tB, None)
+    y, names = product(ctx, a.t().contiguous() if tA else a, b.t().contiguous() if tB else b, tA, tB, None)
     assert "k_gemm_f32_split" in names, names
     rows = [3, 40, 41, 700, 900, 1499, 0, 1, 64, 1498]
     ref = a[rows].cpu().double() @ b.cpu().double()
