@@ -80,10 +80,10 @@ enum { PIXELS, QUADS };
 
 // Where the caller's weight of a phase's tap (a, b) lies.
 template <class Args>
-__device__ __forceinline__ size_t weight_at(const Args &g, const SplitPhase &q, int grp, int oc, int ic, int a, int b, bool rows)
+__device__ __forceinline__ unsigned weight_at(const Args &g, const SplitPhase &q, int grp, int oc, int ic, int a, int b, bool rows)
 {
-   const size_t at = g.transposed ? (size_t)(grp * g.icg + ic) * g.ocg + oc : (size_t)(grp * g.ocg + oc) * g.icg + ic;
-   return (at * g.KH0 + q.th0 + a * q.ths) * g.KW0 + (rows ? b : q.tw0 + b * q.tws);
+   const int at = g.transposed ? (grp * g.icg + ic) * g.ocg + oc : (grp * g.ocg + oc) * g.icg + ic;
+   return (unsigned)((at * g.KH0 + q.th0 + a * q.ths) * g.KW0 + (rows ? b : q.tw0 + b * q.tws));
 }
 
 template <int TI, int TJ, int WO, int STORE, bool PHASES, bool ROWS>
@@ -333,6 +333,8 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       }
    }
 
+   // (what was requested behind the last step is let in here: the compiler would wait for it between stores, and so for stores)
+   __builtin_amdgcn_s_waitcnt(0);
    // sums that are not finite: again, with fp32 instructions on the operands as they were given. 256x64x56x56 -> 128, 3x3, 0.6 ms: 0.1 ms more
    // with one infinity, 0.5 with one in every image, 5 with an infinite weight or one infinity in a hundred cells, where every tile is repeated
    v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -341,44 +343,55 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
       for (int j = 0; j < TJ; ++j)
 #pragma unroll
-         for (int e = 0; e < 4; ++e) {
-            acc[i][j][e] = unscaled(acc[i][j][e]);
-            none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
-         }
+         for (int e = 0; e < 4; ++e) none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
    const float any = (none[0] + none[1]) + (none[2] + none[3]);
+   float factor = UNSCALE;
    int p1 = p0;      // (so that nothing of the pixels' places is kept in registers through the loop)
    asm volatile("" : "+s"(p1));
    if (__builtin_amdgcn_ballot_w64(any != 0.0f) != 0) {
-      // (arguments of this branch alone, once more from memory: kept in registers through the loop they cost 3 % of every call)
+      // (the arguments once more, from memory, and one tile after the other: in registers through the loop, for this branch, they cost 3 %
+      // of every call and up to 13 with few channels. 32 channels x 128 pixels read the weights' alone again: with all of them the
+      // compiler spills fragments in the loop.)
+      constexpr bool ALL = TI * TJ != 4 || WO == 1 || TI == 2;
       auto again = __builtin_amdgcn_kernarg_segment_ptr();
       asm volatile("" : "+s"(again));
-      const SplitArgs &late = *(const SplitArgs *)again;
-      const SplitPhase &late_phase = late.phase[PHASES ? phase : 0];
-#pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-         for (int j = 0; j < TJ; ++j) {
-            const int p = p1 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), n = fdiv(panel, q.dStrips);
-            const int iy0 = oy * g.sh - q.ph, ix0 = ((panel - n * q.strips) * q.ws + r - oy * q.ws) * g.sw - q.pw;
-            const int oc = (tile0 + i) * 16 + r16;
-            v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int c0 = 0; c0 < g.icg; c0 += 4) {
-               const int c = c0 + kg;
-               for (int t = 0; t < taps; ++t) {
-                  const int a = fdiv(t, q.dKW), b = t - a * q.KW, iy = iy0 + a * g.dh, ix = ix0 + b * g.dw;
-                  const bool in = p < q.P && r < q.full && c < g.icg && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
-                  const float xv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * g.chw4 + (iy * g.W + ix) * 4 + (grp * g.icg + c) * g.hw4) : OUTSIDE), 0, 0));
-                  const float wv = c < g.icg && oc < g.ocg ? late.w0[weight_at(late, late_phase, grp, oc, c, a, b, ROWS)] : 0.0f;
-                  sum = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wv, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, sum, 0, 0, 0);
-               }
+      const SplitArgs &late = *(const SplitArgs *)again, &h = ALL ? late : g;
+      const SplitPhase &weights = late.phase[PHASES ? phase : 0], &f = ALL ? weights : q;
+      const int ftaps = f.KH * f.KW;
+      const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(h.x), 0, (int)h.xbytes, 0x00020000);
+      const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(late.w0), 0, (int)OUTSIDE, 0x00020000);
+#pragma unroll 1
+      for (int tile = 0; tile < TI * TJ; ++tile) {
+         const int p = p1 + (wp * TJ + tile % TJ) * 16 + r16, panel = fdiv(p, f.dPHW), r = p - panel * f.PHW, oy = fdiv(r, f.dWS), n = fdiv(panel, f.dStrips);
+         const int iy0 = oy * h.sh - f.ph, ix0 = ((panel - n * f.strips) * f.ws + r - oy * f.ws) * h.sw - f.pw;
+         const int oc = (tile0 + tile / TJ) * 16 + r16;
+         v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+         for (int c0 = 0; c0 < h.icg; c0 += 4) {
+            const int c = c0 + kg;
+#pragma unroll 1
+            for (int t = 0; t < ftaps; ++t) {
+               const int a = fdiv(t, f.dKW), b = t - a * f.KW, iy = iy0 + a * h.dh, ix = ix0 + b * h.dw;
+               const bool in = p < f.P && r < f.full && c < h.icg && (unsigned)iy < (unsigned)h.H && (unsigned)ix < (unsigned)h.W;
+               const float xv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * h.chw4 + (iy * h.W + ix) * 4 + (grp * h.icg + c) * h.hw4) : OUTSIDE), 0, 0));
+               const float wv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ors, (int)(c < h.icg && oc < h.ocg ? 4u * weight_at(late, weights, grp, oc, c, a, b, ROWS) : OUTSIDE), 0, 0));
+               sum = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wv, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, sum, 0, 0, 0);
             }
-            acc[i][j] = sum;
          }
+#pragma unroll
+         for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+#pragma unroll
+               for (int e = 0; e < 4; ++e) acc[i][j][e] = tile == i * TJ + j ? sum[e] : acc[i][j][e];
+      }
+      factor = 1.0f;
    }
 
    const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(g.y, 0, (int)g.ybytes, 0x00020000);
    const rsrc_t yrs4 = make_rsrc(g.y, g.ybytes);
    auto finish = [&](float v, float b) {
+      v = __fmul_rn(v, factor);
       if (g.bias) v = __fadd_rn(v, b);
       return g.relu ? (v > 0.0f ? v : 0.0f) : v;
    };

@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(WAVES * 64, 2) k_gemm_f32_split(GemmF32Args g)
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
          for (int e = 0; e < 4; ++e) {
-            acc[i][j][e] = unscaled(acc[i][j][e]);
+            acc[i][j][e] = __fmul_rn(acc[i][j][e], UNSCALE);
             none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
          }
    if (__builtin_amdgcn_ballot_w64((none[0] + none[1]) + (none[2] + none[3]) != 0.0f) != 0) {

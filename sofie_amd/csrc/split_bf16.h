@@ -3,8 +3,8 @@
 // 2^16 x = h + m + l with h = bf16(2^16 x), m = bf16(2^16 x - h), l = bf16(2^16 x - h - m), all rounded to nearest even: both subtractions
 // are exact, h takes eight of the 24 bits, m eight of the at most 16 that are left, and l the rest, so the sum is 2^16 x itself. The
 // factor puts the last bit of the smallest fp32 number, 2^-149, on the last bit of the smallest bf16, 2^-133 (without it numbers below
-// 2^-110 lost bits: relative error 5.6e-7 at 2^-114, 2.3e-3 at 2^-126); sums are 2^32 times too large and are set right behind the
-// loop (unscaled, exact). The factor costs a multiplication per number split: 1500 x 1001 x 1111 28.7 -> 29.5 us, 256x64x56x56 -> 128, 3x3
+// 2^-110 lost bits: relative error 5.6e-7 at 2^-114, 2.3e-3 at 2^-126); sums are 2^32 times too large and are multiplied by
+// 2^-32 behind the loop (UNSCALE). The factor costs a multiplication per number split: 1500 x 1001 x 1111 28.7 -> 29.5 us, 256x64x56x56 -> 128, 3x3
 // 597 -> 606, transposed 64x128x28x28 -> 64, 4x4 s2 88.3 -> 92.0, 16x3x224x224 -> 64, 7x7 s2 32.7 -> 33.1.
 //
 // Of the nine products of two such numbers six are summed; the others (m l, l m, l l) are together at most 2^-24 of the whole product
@@ -53,7 +53,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], v4i (&d)[3])
    }
 }
 
-// The sum of such products as the sum of the products themselves.
-__device__ __forceinline__ float unscaled(float sum) { return __fmul_rn(sum, 0x1p-32f); }
+// What a sum of such products is multiplied by.
+constexpr float UNSCALE = 0x1p-32f;
 
 }  // namespace sofie
