@@ -17,11 +17,11 @@
 // is the eight values that a row of the kernel meets at an output column, of one channel; a chunk of K is a row of the kernel, zeros up
 // to eight columns, K = (channel, kernel row, kernel column) in one slot. A value is split once per output column it
 // is read at, still shared by the kernel's rows. Loaded as two 16-byte pieces from any dword; columns outside the image are zeroed behind
-// the load. 16x3x224x224 -> 64, 7x7 s2 52.6 -> 32.6 us (k_conv_f32_any, 53 % of the fp32 instructions' rate); 53 of 90 random layers of
-// one to five channels and kernels of 4 to 7 columns, 1.3 times shorter in the mean (55x5x38x38 -> 146, 7x7 s2 35.9 -> 18.1; 126x1x66x66 ->
-// 54, 7x7 66.8 -> 57). Relative error against 64 bits 5e-8 to 9e-8 (1.1e-7 to 3.1e-7 before).
+// the load. 16x3x224x224 -> 64, 7x7 s2 52.6 -> 33.2 us (k_conv_f32_any, 53 % of the fp32 instructions' rate); 53 of 90 random layers of
+// one to five channels and kernels of 4 to 7 columns, 1.3 times shorter in the mean (55x5x38x38 -> 146, 7x7 s2 35.9 -> 16.9; 126x1x66x66 ->
+// 54, 7x7 66.8 -> 43.4). Relative error against 64 bits 5e-8 to 9e-8 (1.1e-7 to 3.1e-7 before).
 // Strips of an image take turns: neighbouring ones write halves of the same 128-byte lines, which one behind the other meet in an
-// L2 (88x1x96x96 -> 150, 7x7 in strips of 16 columns 248 us strip by strip, 196 in turns).
+// L2 (88x1x96x96 -> 150, 7x7 in strips of 16 columns 248 us strip by strip, 192 in turns).
 // All requests of a slot leave in one step: the fragments behind them wait for them (loads return in order), and one such wait
 // per slot is cheaper than one per step. A bias read behind the loop made the compiler wait for each store in front of the next one
 // (13000 cycles for 16 stores instead of 6800).
@@ -29,8 +29,8 @@
 // Bound: the device's power under bf16 matrix instructions on large layers (256x64x56x56 -> 128: 1.65 GHz, the matrix pipe
 // busy for 60 to 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
 // smaller ones. Relative error against 64 bits a quarter of the fp32 instructions'. us against k_conv_f32_any and k_conv2d_f32_dma:
-// 256x64x56x56 -> 128, 3x3 906 -> 583; 256x32x20x20 -> 64 47.4 -> 28.5; 256x64x10x10 -> 128 44.4 -> 29.5; 169x80x16x16 -> 128,
-// 5x5 220 -> 116; 16x64x32x32 -> 65, 7x7 107 -> 51; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 87. Three workgroups per compute
+// 256x64x56x56 -> 128, 3x3 906 -> 605; 256x32x20x20 -> 64 47.4 -> 29.4; 256x64x10x10 -> 128 44.4 -> 27.2; 169x80x16x16 -> 128,
+// 5x5 220 -> 102; 16x64x32x32 -> 65, 7x7 107 -> 49.5; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 92. Three workgroups per compute
 // unit instead of two (fewer cells per thread and slot) were 12 % of the last.
 #include "conv_f32.h"
 #include "conv_f32_split_plan.h"
@@ -335,8 +335,9 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 
    // (what was requested behind the last step is let in here: the compiler would wait for it between stores, and so for stores)
    __builtin_amdgcn_s_waitcnt(0);
-   // sums that are not finite: again, with fp32 instructions on the operands as they were given. 256x64x56x56 -> 128, 3x3, 0.6 ms: 0.1 ms more
-   // with one infinity, 0.5 with one in every image, 5 with an infinite weight or one infinity in a hundred cells, where every tile is repeated
+   // sums that are not finite: again, with fp32 instructions on the operands as they were given. 256x64x56x56 -> 128, 3x3, 0.6 ms: 0.16 ms more
+   // with one infinity, 0.46 with one in every image, 6 to 8 with an infinite weight or one infinity in a hundred cells (every tile repeated);
+   // 16x3x224x224 -> 64, 7x7 s2, 33 us: 0.13, 0.42 and 0.44 ms more
    v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
    for (int i = 0; i < TI; ++i)

@@ -157,7 +157,7 @@ struct SplitPlan {
          Strips &s = strips_seen[tile_of(form)];
          // (as many strips as the estimate says: fewer cells for a tile's pixels against whole lines per store, 4-byte stores where strips are no
          // whole fours, 256x64x10x10 -> 128 29.5 us in one strip, 36.2 in five of two columns; by the number of cells alone 42x59x79x62 -> 9, 3x3 66.5,
-         // now 46.9, and k_conv_f32_any 58.7)
+         // now 44.5, and k_conv_f32_any 58.7)
          for (int strips = 1; strips <= MAX_STRIPS; ++strips) {
             if (strips > s.seen) look_at(s, bp, strips);
             const Panels *q = s.panels[strips - 1];

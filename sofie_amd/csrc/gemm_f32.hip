@@ -774,7 +774,7 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
          consider(TILES, t.mi, t.nj, s, 2.0f + step * cdiv(steps, s) + (s > 1 ? 5.0f + 8.0f * s * (float)g.M * g.N / 6e6f : 0.0f));
       }
    }
-   // (operands as three bf16 numbers on the bf16 matrix instructions: 1500 x 1001 x 1111 27 us, 33 on 32 x 64 tiles)
+   // (operands as three bf16 numbers on the bf16 matrix instructions: 1500 x 1001 x 1111 29 us, 33 on 32 x 64 tiles)
    const SplitChoice split = gemm_f32_split_choice(ctx, g, nz, one_launch);
    consider(SPLIT, split.mi, 4, split.splits, split.us);
    if (g.K >= 4 && best.us >= 1e30f) consider_direct();
@@ -879,7 +879,7 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
    const int tiles = dma ? cdiv(M, tile) * cdiv(N, tile) : 0, steps = K / 32;
    const bool sliced = small && tiles * 2 <= ctx->num_cus && steps >= 16;
    // k_gemm_f32_split instead of whole tiles of 24 us and more (by kTileCosts; below that it gains little, and test_gemm_f32_large
-   // names the kernels): us 2048^3 137 / 110, 4096 x 4096 x 3000 700 / 604; 1024^3 here
+   // names the kernels): us 2048^3 137 / 124, 4096 x 4096 x 3000 700 / 636; 1024^3 here, 22
    bool split = false;
    if (dma && !sliced) {
       const int per_cu = cdiv(tiles, ctx->num_cus);

@@ -13,8 +13,9 @@
 //
 // Bound: vector instructions (eleven for two numbers to split, four a tile to add) beside the matrix instructions, which
 // run under them only in part: 1.3 us a chunk of 64 rows and SIMD, 0.64 of it matrix instructions. Relative error against 64 bits 7e-8 to
-// 1.2e-7 (k_gemm_f32 3e-7 to 1.2e-6). us against k_gemm_f32 and k_gemm_f32_dma: 1500 x 1001 x 1111 33 -> 27; 256 x 256 x 12800 25 -> 22;
-// 2048^3 137 -> 110; 4096 x 4096 x 3000 700 -> 604; 172 random products it takes 1.17 times shorter in the median. Operands straight into
+// 1.2e-7 (k_gemm_f32 3e-7 to 1.2e-6). us against k_gemm_f32 and k_gemm_f32_dma: 1500 x 1001 x 1111 33 -> 29; 2048^3 137 -> 124;
+// 4096 x 4096 x 3000 700 -> 636; 172 random products it takes 1.17 times shorter in the median, before the factor that split_bf16.h
+// multiplies with (3 to 5 % of these). Operands straight into
 // registers were no faster at 2048^3 (119; 35 bytes per ns and compute unit), two buffers for each of four wavefronts neither (125).
 #include "gemm_f32.h"
 #include "gemm_tile.h"

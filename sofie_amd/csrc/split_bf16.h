@@ -4,8 +4,8 @@
 // are exact, h takes eight of the 24 bits, m eight of the at most 16 that are left, and l the rest, so the sum is 2^16 x itself. The
 // factor puts the last bit of the smallest fp32 number, 2^-149, on the last bit of the smallest bf16, 2^-133 (without it numbers below
 // 2^-110 lost bits: relative error 5.6e-7 at 2^-114, 2.3e-3 at 2^-126); sums are 2^32 times too large and are multiplied by
-// 2^-32 behind the loop (UNSCALE). The factor costs a multiplication per number split: 1500 x 1001 x 1111 28.7 -> 29.5 us, 256x64x56x56 -> 128, 3x3
-// 597 -> 606, transposed 64x128x28x28 -> 64, 4x4 s2 88.3 -> 92.0, 16x3x224x224 -> 64, 7x7 s2 32.7 -> 33.1.
+// 2^-32 behind the loop (UNSCALE). The factor costs a multiplication per number split: 1500 x 1001 x 1111 28.4 -> 29.2 us, 4096^3 792 -> 820,
+// 256x64x56x56 -> 128, 3x3 597 -> 605, transposed 64x128x28x28 -> 64, 4x4 s2 90.3 -> 93.3; 66 random convolutions 0.8 % in the median.
 //
 // Of the nine products of two such numbers six are summed; the others (m l, l m, l l) are together at most 2^-24 of the whole product
 // (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|; 1 + 2^-8 - 2^-17 by itself), and 2^-27 of it in the root mean square over random operands. A product
@@ -28,7 +28,7 @@ namespace sofie {
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
 // Eight numbers as h, m and l, two at a time: v_cvt_pk_bf16_f32, the two bf16 as fp32 by a shift and a mask, subtractions: eleven
-// instructions a pair (18 where the compiler converted each number by itself). x - h as a sum of products of bf16 (v_dot2c_f32_bf16, seven
+// instructions a pair behind the two multiplications (18 where the compiler converted each number by itself). x - h as a sum of products of bf16 (v_dot2c_f32_bf16, seven
 // a pair) waits for the matrix pipe: ns for each v_mfma_f32_16x16x32_bf16, two wavefronts on a SIMD: 7.4 alone, 7.5 with two
 // conversions or subtractions behind it, 9.1 with three; 14.6 with two dot products.
 __device__ __forceinline__ void split8(const float (&x)[8], v4i (&d)[3])
