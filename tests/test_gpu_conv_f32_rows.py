@@ -65,6 +65,25 @@ def test_rows_as_cells(ops, kept, shape):
             assert "k_conv_f32_split" not in names or float(err.norm()) <= 3e-7 * float(ref.norm()), i
 
 
+@pytest.mark.parametrize("shape", CONV)
+def test_sums_that_are_repeated(ops, kept, shape):
+    """Operands of 2^60: every sum passes 2^95 on the way and is formed again with fp32 instructions from the operands as they were given. A
+    rounding of 2^-24 for each of K products, which add as their square root."""
+    n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
+    t, l, b, r = pads
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    products = c // groups * kh * kw
+    x = torch.randn(n, c, h, w, device="cuda", generator=g) * 2.0 ** 60
+    wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * products ** -0.5 * 2.0 ** 60
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv2d_f32(x, wt, None, pads, s, d, groups, ctx=kept))
+    assert "k_conv_f32_split" in names, names
+    for i in sorted({0, n // 2, n - 1}):
+        conv = lambda a, v: torch.nn.functional.conv2d(torch.nn.functional.pad(a, (l, r, t, b)), v, None, s, 0, d, groups)
+        xi, wi = x[i:i + 1].cpu().double(), wt.cpu().double()
+        assert bool(((y[i:i + 1].cpu().double() - conv(xi, wi)).abs() <= products ** 0.5 * 2.0 ** -24 * conv(xi.abs(), wi.abs())).all()), i
+
+
 def test_values_that_are_not_finite_stay_in_their_windows(ops, kept):
     """The eighth value of a cell, a column the kernel does not have, is no factor: an infinity there leaves the pixel alone."""
     g = torch.Generator().manual_seed(3)

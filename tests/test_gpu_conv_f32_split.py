@@ -94,6 +94,35 @@ def test_transposed_conv_in_three_parts(ops, kept, n, c, h, w, oc, k, s):
         assert float((y[i:i + 1].cpu().double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
 
 
+@pytest.mark.parametrize("shape", CONV + [
+    (64, 128, 28, 28, 64, 4, 2), (30, 143, 32, 34, 181, 4, 2), (120, 87, 19, 21, 256, 3, 2), (64, 120, 20, 20, 90, 3, 1)])      # transposed: k, stride
+def test_sums_that_are_repeated_in_every_form(ops, kept, shape):
+    """Operands of 2^60: every sum passes 2^95 on the way and is formed again with fp32 instructions from the operands as they were given, flipped
+    and strided kernels of transposed layers among them. A rounding of 2^-24 for each of K products, which add as their square root."""
+    transposed = len(shape) == 7
+    n, c, h, w, oc = shape[:5]
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    x = torch.randn(n, c, h, w, device="cuda", generator=g) * 2.0 ** 60
+    if transposed:
+        k, s = shape[5:]
+        wt = torch.randn(c, oc, k, k, device="cuda", generator=g) * (c * k * k) ** -0.5 * 2.0 ** 60
+        products = c * k * k
+        conv = lambda a, b: torch.nn.functional.conv_transpose2d(a, b, None, s, 1)
+        call = lambda: ops.conv_transpose2d_f32(x, wt, None, (1, 1, 1, 1), (s, s), (1, 1), 1, (0, 0), ctx=kept)
+    else:
+        kh, kw, s, (t, l, b, r), d, groups = shape[5:]
+        products = c // groups * kh * kw
+        wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * products ** -0.5 * 2.0 ** 60
+        conv = lambda a, v: torch.nn.functional.conv2d(torch.nn.functional.pad(a, (l, r, t, b)), v, None, s, 0, d, groups)
+        call = lambda: ops.conv2d_f32(x, wt, None, (t, l, b, r), s, d, groups, ctx=kept)
+    torch.cuda.synchronize()
+    y, names = names_of(kept, call)
+    assert "k_conv_f32_split" in names or (transposed and k == 3 and s == 2), names
+    for i in sorted({0, n // 2, n - 1}):
+        xi, wi = x[i:i + 1].cpu().double(), wt.cpu().double()
+        assert bool(((y[i:i + 1].cpu().double() - conv(xi, wi)).abs() <= products ** 0.5 * 2.0 ** -24 * conv(xi.abs(), wi.abs())).all()), i
+
+
 @pytest.mark.parametrize("c,relu", [(72, False), (16, True)])
 def test_values_that_are_not_finite_stay_in_their_windows(ops, kept, c, relu):
     """Infinities and NaN in cells, weights and products: the parts of a split infinity are no numbers, but its sums are the fp32
