@@ -957,23 +957,28 @@ extern "C" int sofie_hip_gemm_f32_stacked(sofie_hip_ctx *ctx, int transA, int tr
 // dword: a piece is 64 rows of k x 16 columns, 16 loads. A wavefront's pieces form one list over all column tiles, parts of K and
 // layers, and the loads of the next piece are always under way while one is multiplied: the first weights (and biases) of a layer
 // arrive under the layer before it. Against one thread per output and 1, 4 or 8 rows per workgroup (us): 64-128-64-8 on 256 rows
-// 7.5 -> 6.6, on 16384 27.4 -> 12.5; 20-32-32-1 on 4096 15.5 -> 5.3; 100-487-13 on 8192 34.8 -> 16.7. What bounds it: launch and
+// 7.5 -> 6.6, on 16384 27.4 -> 12.5; 20-32-32-1 on 4096 15.5 -> 5.3; 100-487-13 on 8192 34.8 -> 16.7. The arguments of a layer in one scalar
+// load, those of the first four layers fetched at the start, x ahead of the weights: 64-128-64-8 on 256 rows 6.6 -> 5.9, 60 random
+// chains (k_mlp_f32_row's, too) 1.065 times shorter in the mean, none longer (with units dealt on from layer to layer, so that idle
+// wavefronts ask for the next layer's weights, 6.05). What bounds it: launch and
 // memory latency for a small network on a few rows; a compute unit's share of the L2 (43 B/ns measured, every workgroup reads all
 // weights) up to 16 rows for each of them; the matrix instructions above.
 // A layer with fewer column tiles than the workgroup has wavefronts deals the pieces of K to parts, added in LDS in order.
 namespace {
 
+struct MlpLayer {      // 32 bytes: one scalar load
+   const float *W, *bias;
+   int K, N, relu;
+   int psh;      // k_mlp_f32: the pieces of K are dealt to 1 << psh parts
+};
+
 struct MlpArgs {
-   const float *W[SOFIE_MLP_MAX_LAYERS];
-   const float *bias[SOFIE_MLP_MAX_LAYERS];
-   int dims[SOFIE_MLP_MAX_LAYERS + 1];
-   int relu[SOFIE_MLP_MAX_LAYERS];
    const float *x;
    float *y;
    int n_layers, M, ldx, ldy;
    int ld[2];   // floats per row of the two activation buffers: the inputs of even and of odd layers
    int maxd;    // k_mlp_f32_row: the widest layer
-   int psh[SOFIE_MLP_MAX_LAYERS];   // the pieces of a layer's K are dealt to 1 << psh parts
+   alignas(64) MlpLayer layer[SOFIE_MLP_MAX_LAYERS];
 };
 
 template <int RT, int NW>
@@ -988,6 +993,15 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int c = lane & 15, kg = lane >> 4;
    const int row0 = blockIdx.x * ROWS;
+   {  // the arguments up to the fourth layer are asked for at once: read where a layer needs them they are a trip to memory each
+      constexpr int LINES = 3;
+      const int *const args = (const int *)__builtin_amdgcn_kernarg_segment_ptr();
+      int line[LINES];
+#pragma unroll
+      for (int i = 0; i < LINES; ++i) line[i] = args[16 * i];
+#pragma unroll
+      for (int i = 0; i < LINES; ++i) asm volatile("" : : "s"(line[i]));
+   }
 
    // the next piece whose weights are requested: layer, unit (column tile and part), piece of K; and what its layer's pieces share
    int fl = -1, fu = 0, fp = 0, fK = 0, fN = 0, fsh = 0, funits = 0;
@@ -995,15 +1009,16 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
    auto settle = [&] {       // onto the first piece of this wavefront at or behind unit fu
       while (fu >= funits) {
          if (++fl >= a.n_layers) return;
-         fK = a.dims[fl];
-         fN = a.dims[fl + 1];
-         fsh = a.psh[fl];
+         const MlpLayer f = a.layer[fl];
+         fK = f.K;
+         fN = f.N;
+         fsh = f.psh;
          funits = ((fN + 15) >> 4) << fsh;
          fu = wave;
          // rows behind K lie outside the descriptor and arrive as zeros; columns behind N hold other weights and end in
          // columns of the result that are dropped
-         fw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.W[fl]), 0, fK * fN * 4, 0x00020000);
-         fb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.bias[fl]), 0, a.bias[fl] ? fN * 4 : 0, 0x00020000);
+         fw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(f.W), 0, fK * fN * 4, 0x00020000);
+         fb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(f.bias), 0, f.bias ? fN * 4 : 0, 0x00020000);
       }
       fp = fu & ((1 << fsh) - 1);
    };
@@ -1026,30 +1041,33 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
          settle();
       }
    };
+   // the rows of x, with zeros up to a whole 16 of K and for rows behind M; the first 64 columns are requested ahead of the weights
+   const int K0 = a.layer[0].K;
+   float v[ROWS / NW];
+   auto request_x = [&](int k) {
+#pragma unroll
+      for (int i = 0; i < ROWS / NW; ++i) {
+         const int row = row0 + i * NW + wave;
+         v[i] = row < a.M && k < K0 ? a.x[(size_t)row * a.ldx + k] : 0.0f;
+      }
+   };
+   request_x(lane);
    settle();
    fetch();
-
-   {  // the rows of x, with zeros up to a whole 16 of K and for rows behind M
-      const int K = a.dims[0], KP = (K + 15) & ~15;
-      for (int k = lane; k < KP; k += 64) {
-         float v[ROWS / NW];
+   for (int k = lane, KP = (K0 + 15) & ~15; k < KP; k += 64) {
+      if (k >= 64) request_x(k);
 #pragma unroll
-         for (int i = 0; i < ROWS / NW; ++i) {
-            const int row = row0 + i * NW + wave;
-            v[i] = row < a.M && k < K ? a.x[(size_t)row * a.ldx + k] : 0.0f;
-         }
-#pragma unroll
-         for (int i = 0; i < ROWS / NW; ++i) buf[0][(i * NW + wave) * a.ld[0] + k] = v[i];
-      }
+      for (int i = 0; i < ROWS / NW; ++i) buf[0][(i * NW + wave) * a.ld[0] + k] = v[i];
    }
    __syncthreads();
 
    for (int l = 0; l < a.n_layers; ++l) {
-      const int K = a.dims[l], N = a.dims[l + 1], ldi = a.ld[l & 1], ldo = a.ld[(l + 1) & 1];
+      const MlpLayer f = a.layer[l];
+      const int K = f.K, N = f.N, ldi = a.ld[l & 1], ldo = a.ld[(l + 1) & 1];
       const float *in = l & 1 ? buf[1] : buf[0];
       float *out = l & 1 ? buf[0] : buf[1];
-      const bool last = l + 1 == a.n_layers, relu = a.relu[l];
-      const int sh = a.psh[l], parts = 1 << sh, tiles = (N + 15) >> 4, pieces = (K + 63) >> 6;
+      const bool last = l + 1 == a.n_layers, relu = f.relu;
+      const int sh = f.psh, parts = 1 << sh, tiles = (N + 15) >> 4, pieces = (K + 63) >> 6;
       // columns behind N become the zeros up to a whole 16 of the next layer's K
       auto finish = [&](int r, int n, float v) {
          if (relu) v = fmaxf(v, 0.0f);
@@ -1110,7 +1128,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
 // One row per workgroup and one output per thread, plain fused multiply-adds: a layer of fewer than 256 outputs is cut into parts of
 // K whose sums meet in LDS. For up to two rows per compute unit, where it is the shorter chain of waits (us, against k_mlp_f32):
 // 144-128-41 on 256 rows 6.1 / 7.2, 147-112-128-32-95-23 10.8 / 12.2, 8-500-9 6.1 / 6.6; not with a layer of 8 outputs or fewer
-// (32 parts and more, added one after the other): 64-128-64-8 7.5 / 6.6, 20-32-32-1 16.0 / 5.3.
+// (32 parts and more, added one after the other): 64-128-64-8 7.5 / 5.9, 20-32-32-1 16.0 / 5.3.
 __global__ void __launch_bounds__(256) k_mlp_f32_row(MlpArgs a)
 {
    constexpr int R = 1;
@@ -1120,7 +1138,7 @@ __global__ void __launch_bounds__(256) k_mlp_f32_row(MlpArgs a)
    const int tid = threadIdx.x;
    const int row0 = blockIdx.x * R;
    {
-      const int K0 = a.dims[0];
+      const int K0 = a.layer[0].K;
       for (int idx = tid; idx < R * K0; idx += 256) {
          const int r = idx / K0, k = idx - r * K0;
          buf_in[r * a.maxd + k] = row0 + r < a.M ? a.x[(size_t)(row0 + r) * a.ldx + k] : 0.0f;
@@ -1128,8 +1146,9 @@ __global__ void __launch_bounds__(256) k_mlp_f32_row(MlpArgs a)
    }
    __syncthreads();
    for (int l = 0; l < a.n_layers; ++l) {
-      const int K = a.dims[l], N = a.dims[l + 1];
-      const float *__restrict__ W = a.W[l];
+      const MlpLayer f = a.layer[l];
+      const int K = f.K, N = f.N;
+      const float *__restrict__ W = f.W;
       const bool last = l + 1 == a.n_layers;
       // columns per pass (a power of two, at most 256) and the parts K is cut into
       int n2 = 1;
@@ -1154,8 +1173,8 @@ __global__ void __launch_bounds__(256) k_mlp_f32_row(MlpArgs a)
             }
          }
          auto finish = [&](int r, int oo, float v) {
-            if (a.bias[l]) v += a.bias[l][oo];
-            if (a.relu[l]) v = fmaxf(v, 0.0f);
+            if (f.bias) v += f.bias[oo];
+            if (f.relu) v = fmaxf(v, 0.0f);
             if (last) {
                if (row0 + r < a.M) a.y[(size_t)(row0 + r) * a.ldy + oo] = v;
             } else {
@@ -1193,8 +1212,9 @@ int launch_mlp(sofie_hip_ctx *ctx, MlpArgs &a, size_t lds)
 {
    SOFIE_LARGE_LDS((k_mlp_f32<RT, NW>));
    for (int l = 0; l < a.n_layers; ++l) {
-      const int tiles = cdiv(a.dims[l + 1], 16), pieces = cdiv(a.dims[l], 64);
-      for (a.psh[l] = 0; (2 * tiles << a.psh[l]) <= NW && (2 << a.psh[l]) <= pieces;) ++a.psh[l];
+      MlpLayer &f = a.layer[l];
+      const int tiles = cdiv(f.N, 16), pieces = cdiv(f.K, 64);
+      for (f.psh = 0; (2 * tiles << f.psh) <= NW && (2 << f.psh) <= pieces;) ++f.psh;
    }
    // a launch holds fewer than 2^32 threads: 67 million rows at 16 per workgroup of 1024
    const int M = a.M, most = (1 << 21) * 16 * RT;
@@ -1211,13 +1231,14 @@ int launch_mlp(sofie_hip_ctx *ctx, MlpArgs &a, size_t lds)
 // A layer as a product of its own (lda and ldy: of x and y for the first and the last, else of the scratch buffer).
 GemmF32Args mlp_layer(const MlpArgs &a, int l, const float *in, int lda, float *out, int ldy)
 {
+   const MlpLayer &f = a.layer[l];
    GemmF32Args g{};
-   g.A = in; g.B = a.W[l]; g.bias = a.bias[l]; g.Y = out;
-   g.M = a.M; g.N = a.dims[l + 1]; g.K = a.dims[l];
+   g.A = in; g.B = f.W; g.bias = f.bias; g.Y = out;
+   g.M = a.M; g.N = f.N; g.K = f.K;
    g.lda = lda; g.ldb = g.N; g.ldy = ldy;
-   g.alpha = 1.0f; g.beta = a.bias[l] ? 1.0f : 0.0f;
-   g.bias_kind = a.bias[l] ? SOFIE_BIAS_ROW : SOFIE_BIAS_NONE;
-   g.relu = a.relu[l];
+   g.alpha = 1.0f; g.beta = f.bias ? 1.0f : 0.0f;
+   g.bias_kind = f.bias ? SOFIE_BIAS_ROW : SOFIE_BIAS_NONE;
+   g.relu = f.relu;
    return g;
 }
 
@@ -1233,14 +1254,15 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    MlpArgs a{};
    for (int l = 0; l <= n_layers; ++l) {
       SOFIE_REQUIRE(ctx, dims[l] >= 1 && dims[l] <= SOFIE_MLP_MAX_WIDTH, "layer width out of range");
-      a.dims[l] = dims[l];
+      if (l < n_layers) a.layer[l].K = dims[l];
+      if (l > 0) a.layer[l - 1].N = dims[l];
    }
    for (int l = 0; l < n_layers; ++l) {
       SOFIE_REQUIRE(ctx, W[l], "null weight matrix");
       SOFIE_REQUIRE(ctx, act[l] == SOFIE_ACT_NONE || act[l] == SOFIE_ACT_RELU, "unknown activation");
-      a.W[l] = W[l];
-      a.bias[l] = bias ? bias[l] : nullptr;
-      a.relu[l] = act[l] == SOFIE_ACT_RELU;
+      a.layer[l].W = W[l];
+      a.layer[l].bias = bias ? bias[l] : nullptr;
+      a.layer[l].relu = act[l] == SOFIE_ACT_RELU;
    }
    if (M == 0) return SOFIE_HIP_OK;
    SOFIE_REQUIRE(ctx, x && y, "null operand");
@@ -1258,7 +1280,7 @@ extern "C" int sofie_hip_mlp_f32(sofie_hip_ctx *ctx, int n_layers, const int *di
    const int rt = M > 64 * cus && lds(4, 8) <= (size_t)kMaxDynamicLds ? 4 : M > 16 * cus && lds(2, 8) <= (size_t)kMaxDynamicLds ? 2 : 1;
    // In one launch every workgroup takes in all weights, 43 bytes per ns and compute unit, which a launch per layer (2.8 us each)
    // shares out: the shorter estimate, and a single layer is a product in any case. One launch against a launch per layer:
-   // 64-128-64-8 on 256 rows 6.6 / 13.4 us, 256-256-256-16 on 512 rows 18.5 / 12.8, 1024-1024-1024 on 256 rows 199 / 22.5.
+   // 64-128-64-8 on 256 rows 5.9 / 13.4 us, 256-256-256-16 on 512 rows 18.5 / 12.8, 1024-1024-1024 on 256 rows 199 / 22.5.
    // (k_mlp_f32_row: the weights as often as a compute unit has rows; 8-16-768 on 8 rows 6.0 us, 6.9 in two launches.)
    const int per_cu = cdiv(cdiv(M, 16 * rt), cus);
    int narrowest = dims[1];
