@@ -86,22 +86,34 @@ __global__ void __launch_bounds__(NW * 64) k_qconv_any(AnyArgs a)
       const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char *)big;
       for (int f = wave; f < NB * a.S; f += NW) dma16(rs, lds0 + f * 1024, lane * 16, (ob * NB * a.S + f) * 1024);
    }
-   for (int q = tid; q < a.S * 4; q += NW * 64) {
-      const int kh = fdiv(q, a.dRun), r = q - kh * a.run16;
-      const int kw = BOUNDS ? fdiv(r, a.dC16) : 0;
-      // chunks behind the last kernel row carry zero weights: they read the first chunk again
-      tab[q] = q < a.chunks ? v2i{kh * a.row + r * 16, kh << 16 | kw} : v2i{0, 0};
-   }
-   if (tid < OCT) {
-      const int n = n0 + tid;
-      s_scale[tid] = n < a.OC ? a.scale[n] : 0.0f;
-      s_bias[tid] = a.bias && n < a.OC ? a.bias[n] : 0;
-   }
-   if constexpr (BLDS) wait_vmcnt<0>();
-   __syncthreads();
-
    const int s_per = (a.S + WK - 1) / WK;
    const int s0 = wk * s_per, s1 = min(s0 + s_per, a.S);
+   // offset and (row << 16 | column) of a chunk; chunks behind the last kernel row carry zero weights: they read the first chunk again
+   auto chunk = [&](int q) {
+      const int kh = fdiv(q, a.dRun), r = q - kh * a.run16;
+      const int kw = BOUNDS ? fdiv(r, a.dC16) : 0;
+      return q < a.chunks ? v2i{kh * a.row + r * 16, kh << 16 | kw} : v2i{0, 0};
+   };
+   float scale = 0.0f;
+   int bias = 0;
+   if (tid < OCT && n0 + tid < a.OC) {
+      scale = a.scale[n0 + tid];
+      if (a.bias) bias = a.bias[n0 + tid];
+   }
+   auto tables = [&](bool offsets) {
+      if (offsets)
+         for (int q = tid; q < a.S * 4; q += NW * 64) tab[q] = chunk(q);
+      if (tid < OCT) {
+         s_scale[tid] = scale;
+         s_bias[tid] = bias;
+      }
+   };
+   if constexpr (BLDS) {
+      tables(true);
+      wait_vmcnt<0>();
+      __syncthreads();
+   }
+
    const float zpo = (float)(a.zp + 128), lof = (float)(a.lo + 128);
 
    // sums of a tile (POOL: of the four positions) -> requantised bytes of pixel m, channels n0 + 16 i + 4 kg ..
@@ -155,8 +167,7 @@ __global__ void __launch_bounds__(NW * 64) k_qconv_any(AnyArgs a)
 
       v4i fa[D][MB], fb[BLDS ? 1 : D][NB];
       int pad[D][MB];      // BOUNDS: the zero-point where the chunk lies outside the image (its load returns 0), else 0
-      auto load = [&](int buf, int s) {
-         const v2i e = tab[s * 4 + kg];
+      auto load = [&](int buf, int s, v2i e) {
 #pragma unroll
          for (int j = 0; j < MB; ++j) {
             unsigned off = (unsigned)(base[j] + e[0]);
@@ -191,15 +202,29 @@ __global__ void __launch_bounds__(NW * 64) k_qconv_any(AnyArgs a)
             for (int i = 0; i < NB; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b[i], f, acc[i][j], 0, 0, 0);
          }
       };
+      // Weights from memory (one tile): the first requests leave with chunks that the wavefront works out by itself, and only steps
+      // behind them need the table, which is written while they travel. Behind the barrier of the table and the scales, 16x48x35x29 -> 80,
+      // 3x3 s2 took 6.5 us instead of 6.15.
       if (s0 < s1) {
 #pragma unroll
-         for (int u = 0; u < D; ++u) load(u, min(s0 + u, s1 - 1));
+         for (int u = 0; u < D; ++u) {
+            if (!BLDS && s0 + u >= s1) break;
+            const int s = min(s0 + u, s1 - 1);
+            load(u, s, BLDS ? tab[s * 4 + kg] : chunk(s * 4 + kg));
+         }
+      }
+      if constexpr (!BLDS) {
+         tables(s_per > D);
+         if (WK == 1 || s_per > D) __syncthreads();
+      }
+      if (s0 < s1) {
          int s = s0;
          for (; s + D < s1; s += D) {
 #pragma unroll
             for (int u = 0; u < D; ++u) {
                mma(u, s + u);
-               load(u, min(s + u + D, s1 - 1));
+               const int next = min(s + u + D, s1 - 1);
+               load(u, next, tab[next * 4 + kg]);
             }
          }
 #pragma unroll
@@ -460,20 +485,13 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       SOFIE_LARGE_LDS(kb); SOFIE_LARGE_LDS(kn); SOFIE_LARGE_LDS(pb); SOFIE_LARGE_LDS(pn);                                    \
       return go(pool ? (bounds ? pb : pn) : (bounds ? kb : kn), NB_, NW_, WK_, pool ? 1 : MB_, big_, resident_);             \
    } while (0)
-   // The form, by the number of workgroups it gives and by what the LDS holds. Timed in every form on 356 layers of 3 to 256 channels,
-   // 1x1 to 7x7, stride 1 and 2, a quarter of them pooled (kept weights; us in the order A B C D E):
+   // The form, by the number of workgroups it gives and by what the LDS holds.
    //   A, B  64 pixels x up to 64 channels per wavefront, weights in LDS, as many workgroups as are resident at once walk over the
    //         tiles: for a tile per compute unit and more. A: four wavefronts, up to three workgroups in a compute unit, for weights
    //         of up to 50 KB or fewer than two rounds of tiles; B: eight wavefronts, one workgroup, for larger weights (up to
-   //         144 KB). 81x16x83x83 -> 54, 3x3 42 30 38 239 378; 43x16x100x100 -> 124, 5x5 s2 26 19 23 119 172.
-   //   C     32 pixels x up to 64 channels, weights from memory: for fewer tiles, and for fewer than four K-steps, which are not
-   //         worth dealing out (16 channels at a time where that leaves compute units without a workgroup).
-   //   D, E  16 pixels x 32 or 16 channels, the K-steps dealt to eight wavefronts: for the fewest. 114x32x21x21 -> 24, 3x3 s2, pooled
-   //         7.0 9.3 6.3 5.8 9.0.
-   // What the rule picks is 8 % behind the best of them in the mean. Where it picks C or E no other form is ahead in the mean (the
-   // next one: A 1.02, D 0.99 times its time). It is off in two places: of 47 layers in A 23 are 5 % and more faster in B and none
-   // is slower; of 72 in D 30 are faster in C, pooled 5x5 and 7x7 ones on 16 channels by up to 4.6 times (12x16x73x73 -> 38, 5x5,
-   // pooled 6.1 6.7 6.2 28.5 33.7).
+   //         144 KB). us in A, B, C: 81x16x83x83 -> 54, 3x3 42 30 38; 43x16x100x100 -> 124, 5x5 s2 26 19 23.
+   //         Of 47 layers in A 23 are 5 % and more faster in B and none is slower.
+   //   C, D, E  weights from memory, below.
    // Channels per workgroup: up to four tiles of 16, as few idle ones as possible.
    auto even = [&](int most) { return cdiv(p.nt, cdiv(p.nt, most)); };
    const int mb = pool ? 1 : 4;
@@ -494,18 +512,41 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       if (nb == 3) SOFIE_ANY(4, 4, 3, 8, 1, 3, true, wlds, 1);
       SOFIE_ANY(4, 4, 4, 8, 1, 3, true, wlds, 1);
    }
-   // fewer tiles: smaller ones, weights from memory; few K-steps are not worth dealing out
-   const long long mid_tiles = (long long)cdiv(a.M, 4 * (pool ? 1 : 2) * 16) * cdiv(p.nt, even(4));
-   if (mid_tiles >= cus || p.S < 4) {
-      nb = mid_tiles >= cus ? even(4) : 1;
-      if (nb == 1) SOFIE_ANY(2, 4, 1, 4, 1, 4, false, 0, 0);
-      if (nb == 2) SOFIE_ANY(2, 4, 2, 4, 1, 3, false, 0, 0);
-      if (nb == 3) SOFIE_ANY(2, 4, 3, 4, 1, 3, false, 0, 0);
-      SOFIE_ANY(2, 4, 4, 4, 1, 3, false, 0, 0);
+   // Fewer tiles: weights from memory. C: 32 pixels (pooled 16) x up to four or two tiles of channels, a wavefront has all of K; else
+   // the K-steps dealt to four wavefronts (D: 16 or 32 pixels x 32 channels, E: 16 x 16) or eight (E). Microseconds: a launch and
+   // the requests one behind the other, and per workgroup of a compute unit its wavefronts' starts, operands (more by the ones requested
+   // in vain behind a short K), sums and conversions. A fit to 457 random layers of 16 to 256 channels with kept weights, a third of them
+   // pooled, on which the forms differ: what it picks is 1.7 % behind the best of ten forms in the mean and 1.14 times faster than
+   // a rule by tiles alone with eight wavefronts in every dealt form (16x48x35x29 -> 80, 3x3 s2 6.2 -> 4.1 us; 14792 pooled pixels -> 48
+   // on 7 K-steps 26.9 -> 6.3; 14x14x512 -> 512, 3x3 9.2 -> 6.3).
+   struct Few {
+      int mb, nb, nw, wk, d;
+   };
+   const Few few[] = {{2, even(4), 4, 1, even(4) == 1 ? 4 : 3}, {2, even(2), 4, 1, even(2) == 1 ? 4 : 3}, {1, 2, 4, 4, 4}, {2, 2, 4, 4, 4}, {1, 1, 4, 4, 4}, {1, 1, 8, 8, 4}};
+   int pick = 0;
+   float least = 1e30f;
+   for (int f = 0; f < 6; ++f) {
+      const Few &q = few[f];
+      const float workgroups = (float)cdiv(a.M, q.nw / q.wk * (pool ? 1 : q.mb) * 16) * (float)cdiv(p.nt, q.nb), per_cu = workgroups > (float)cus ? workgroups / (float)cus : 1.0f;
+      const int steps = cdiv(p.S, q.wk), mbs = pool ? 4 : q.mb, pieces = mbs * q.nb;
+      const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? 0.353f + 0.153f * (float)(steps - q.d) / (float)q.d : 0.0f);
+      const float work = (float)q.nw * (0.0379f + ((float)steps + 0.211f * (float)q.d) * (0.0126f * (float)mbs + 0.0059f * (float)q.nb)) +
+                         (0.022f * (float)(q.nw / q.wk) + (q.wk > 1 ? 0.0086f * (float)q.nw : 0.0f)) * (float)pieces;
+      if (waits + per_cu * work < least) {
+         least = waits + per_cu * work;
+         pick = f;
+      }
    }
-   if ((long long)cdiv(a.M, 16) * cdiv(p.nt, 2) >= cus && p.nt > 1)
-      SOFIE_ANY(1, 4, 2, 8, 8, 4, false, (size_t)8 * 2 * (pool ? 4 : 1) * 1024, 0);
-   SOFIE_ANY(1, 4, 1, 8, 8, 4, false, (size_t)8 * 1 * (pool ? 4 : 1) * 1024, 0);
+   nb = few[pick].nb;
+   const auto sums = [&](int waves, int m, int n) { return (size_t)waves * n * (pool ? 4 : m) * 1024; };
+   if (pick == 2) SOFIE_ANY(1, 4, 2, 4, 4, 4, false, sums(4, 1, 2), 0);
+   if (pick == 3) SOFIE_ANY(2, 4, 2, 4, 4, 4, false, sums(4, 2, 2), 0);
+   if (pick == 4) SOFIE_ANY(1, 4, 1, 4, 4, 4, false, sums(4, 1, 1), 0);
+   if (pick == 5) SOFIE_ANY(1, 4, 1, 8, 8, 4, false, sums(8, 1, 1), 0);
+   if (nb == 1) SOFIE_ANY(2, 4, 1, 4, 1, 4, false, 0, 0);
+   if (nb == 2) SOFIE_ANY(2, 4, 2, 4, 1, 3, false, 0, 0);
+   if (nb == 3) SOFIE_ANY(2, 4, 3, 4, 1, 3, false, 0, 0);
+   SOFIE_ANY(2, 4, 4, 4, 1, 3, false, 0, 0);
 #undef SOFIE_ANY
 }
 

@@ -2,7 +2,7 @@
 
 The shapes cover the input read in place (channels-last, C a multiple of 16) with and without pads, the padded copy from
 channels-last, channel-plane and float input, the three sizes of workgroup (whole tiles with the weights in LDS, small tiles, K
-dealt to eight wavefronts), one to four tiles of 16 channels per workgroup and remainders of all of them, and the fused 2x2
+dealt to four or eight wavefronts), one to four tiles of 16 channels per workgroup and remainders of all of them, and the fused 2x2
 pooling with scales of both signs."""
 import ctypes as C
 
@@ -158,3 +158,22 @@ def test_recorded_calls(ops, promise, warm):
         assert np.array_equal(y.cpu().numpy(), want)
     ctx.check(ctx.lib.sofie_hip_graph_destroy(ctx.h, graph))
     ctx.close()
+
+
+@pytest.mark.parametrize("steps", [1, 3, 4, 5, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("n,h,w,oc", [(1, 5, 9, 7), (3, 20, 23, 40), (9, 22, 25, 72)])
+@pytest.mark.parametrize("pool", [False, True])
+def test_few_tiles_by_steps_of_k(ops, steps, n, h, w, oc, pool):
+    """Weights from memory: K of up to as many steps as a wavefront requests at once, and of one more, dealt to one, four and eight."""
+    c = 64 * steps - 16 * (steps % 2)
+    x, wt, scale, bias = make(np.random.default_rng(steps + oc), n, c, h, w, oc, 1, 1, pool)
+    want = oracle.qconv2d_s8(x, wt, scale, bias, (0, 0), (1, 1), 1, 7, -9, False)
+    xl, wl = np.ascontiguousarray(x.transpose(0, 2, 3, 1)), np.ascontiguousarray(wt.transpose(0, 2, 3, 1))
+    if pool:
+        oh, ow = h // 2, w // 2
+        want = np.max([want[:, :, i:2 * oh:2, j:2 * ow:2] for i in (0, 1) for j in (0, 1)], 0)
+        got = ops.qconv2d_pool_s8(xl, wt, scale, bias, (0, 0), (1, 1), 1, 7, -9, False, (2, 2), (2, 2), x_layout=L.LAYOUT_NHWC, y_layout=L.LAYOUT_NHWC)
+    else:
+        got = ops.qconv2d_s8(xl, wl, x_layout=L.LAYOUT_NHWC, w_layout=L.LAYOUT_NHWC, y_layout=L.LAYOUT_NHWC, scale=scale, bias=bias,
+                             pads=(0, 0), strides=(1, 1), zpx=7, zpy=-9, relu=False)
+    assert np.array_equal(got.transpose(0, 3, 1, 2), want)
