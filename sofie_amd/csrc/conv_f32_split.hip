@@ -29,7 +29,7 @@
 // Bound: the device's power under bf16 matrix instructions on large layers (256x64x56x56 -> 128: 1.65 GHz, the matrix pipe
 // busy for 60 to 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
 // smaller ones. Relative error against 64 bits a quarter of the fp32 instructions'. us against k_conv_f32_any and k_conv2d_f32_dma:
-// 256x64x56x56 -> 128, 3x3 906 -> 605; 256x32x20x20 -> 64 47.4 -> 29.4; 256x64x10x10 -> 128 44.4 -> 27.2; 169x80x16x16 -> 128,
+// 256x64x56x56 -> 128, 3x3 906 -> 568; 256x32x20x20 -> 64 47.4 -> 29.4; 256x64x10x10 -> 128 44.4 -> 27.2; 169x80x16x16 -> 128,
 // 5x5 220 -> 102; 16x64x32x32 -> 65, 7x7 107 -> 49.5; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 92. Three workgroups per compute
 // unit instead of two (fewer cells per thread and slot) were 12 % of the last.
 #include "conv_f32.h"
