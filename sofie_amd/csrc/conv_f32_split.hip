@@ -22,6 +22,11 @@
 // 54, 7x7 66.8 -> 43.4). Relative error against 64 bits 5e-8 to 9e-8 (1.1e-7 to 3.1e-7 before).
 // Strips of an image take turns: neighbouring ones write halves of the same 128-byte lines, which one behind the other meet in an
 // L2 (88x1x96x96 -> 150, 7x7 in strips of 16 columns 248 us strip by strip, 192 in turns).
+// The four phases of a transposed layer of stride 2 x 2 (TOGETHER): a workgroup for each of them reads and splits the same cells and
+// stores every other column. Here a workgroup has a wavefront for each phase on 16 TJ places of one patch; where rows are whole fours two phases
+// exchange half of their columns in LDS and store 16 bytes each. What bounds it then are the weights, 12 KB a step and wavefront from
+// the L2 where four wavefronts share them otherwise. Transposed 64x128x28x28 -> 64, 4x4 s2 89.5 -> 81; 140 random layers of stride 2 1.1 times
+// shorter in the mean, 1.2 to 1.6 times where the route changed (3x3, 56x107x56x56 -> 16 97 -> 68.5; 2x2, 114x231x48x35 -> 16 136 -> 104).
 // All requests of a slot leave in one step: the fragments behind them wait for them (loads return in order), and one such wait
 // per slot is cheaper than one per step. A bias read behind the loop made the compiler wait for each store in front of the next one
 // (13000 cycles for 16 stores instead of 6800).
@@ -30,7 +35,7 @@
 // busy for 60 to 70 % of the cycles; without any loads in the loop 458 us), prologue, slots' waits and stores on
 // smaller ones. Relative error against 64 bits a quarter of the fp32 instructions'. us against k_conv_f32_any and k_conv2d_f32_dma:
 // 256x64x56x56 -> 128, 3x3 906 -> 568; 256x32x20x20 -> 64 47.4 -> 29.4; 256x64x10x10 -> 128 44.4 -> 27.2; 169x80x16x16 -> 128,
-// 5x5 220 -> 102; 16x64x32x32 -> 65, 7x7 107 -> 49.5; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 92. Three workgroups per compute
+// 5x5 220 -> 102; 16x64x32x32 -> 65, 7x7 107 -> 49.5; transposed 64x128x28x28 -> 64, 4x4 s2 123 -> 81. Three workgroups per compute
 // unit instead of two (fewer cells per thread and slot) were 12 % of the last.
 #include "conv_f32.h"
 #include "conv_f32_split_plan.h"
@@ -49,6 +54,8 @@ struct SplitPhase {
    int P, PHW, panels;        // pixels, of a panel; panels (strips of images)
    int ws, strips;            // columns of a strip, strips of an image
    int KH, KW, ph, pw;
+   int down, right;           // where its taps begin in the patch, whose pads are ph and pw (a patch of several phases)
+   int OH;
    int HP, PW, cells;         // rows of a panel's input, cells of a row, of a tile's patch
    int full;                  // pixels of a panel that exist (PHW: up to whole tiles where tiles do not run on into the next panel)
    int chunks;                // of a slot: 8 channels of a tap each
@@ -71,12 +78,14 @@ struct SplitArgs {
    int octiles, oblocks;
    int chw4, hw4, ocplane4, plane4, OW0;
    int table_bytes, slot_bytes;      // LDS: table of offsets, two slots
+   int table_ints;            // TOGETHER: from one phase's table to the next one's
    int nphases;
    FastDiv dOB, dPhases;
    SplitPhase phase[MAX_PHASES];
 };
 
 enum { PIXELS, QUADS };
+typedef float v2f __attribute__((ext_vector_type(2)));
 
 // Where the caller's weight of a phase's tap (a, b) lies.
 template <class Args>
@@ -86,13 +95,15 @@ __device__ __forceinline__ unsigned weight_at(const Args &g, const SplitPhase &q
    return (unsigned)((at * g.KH0 + q.th0 + a * q.ths) * g.KW0 + (rows ? b : q.tw0 + b * q.tws));
 }
 
+// WO: wavefronts along the channels; TOGETHER: all have the same channels and pixels, of a phase each
 template <int TI, int TJ, int WO, int STORE, bool PHASES, bool ROWS>
 __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k_conv_f32_split(SplitArgs g)
 {
    extern __shared__ __align__(16) unsigned char smem_raw[];
+   constexpr bool TOGETHER = WO == SplitPlan::TOGETHER;
    constexpr int BP = 4 / WO * TJ * 16, ITEMS = SplitPlan::items_of(TI, TJ, WO, ROWS);
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-   const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = wave % WO;
+   const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = TOGETHER ? 0 : wave % WO;
    // workgroup id -> (pixels, channels, phase): an XCD (an L2) works on consecutive ids; the phases of a tile, which read the same
    // input and write every other pixel of the same lines, are next to each other, and so are the channel blocks of a pixel block
    int pid = blockIdx.x, phase = 0;
@@ -100,13 +111,15 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       const int tiles = gridDim.x, xcd = pid & 7, base = tiles >> 3, rem = tiles & 7;
       pid = (pid >> 3) + xcd * base + (xcd < rem ? xcd : rem);
    }
-   if constexpr (PHASES) {
+   if constexpr (TOGETHER) {
+      phase = wave ^ (pid & 3);      // (phases of unequal length on every SIMD)
+   } else if constexpr (PHASES) {
       const int all = pid;
       pid = fdiv(all, g.dPhases);
       phase = all - pid * g.nphases;
    }
    SplitPhase q = g.phase[0];
-   if constexpr (PHASES) {
+   if constexpr (PHASES || TOGETHER) {
 #pragma unroll
       for (int i = 1; i < MAX_PHASES; ++i)
          if (phase == i) q = g.phase[i];
@@ -117,7 +130,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       const int n = fdiv(pb, q.dTiles), r = pb - n * q.strips * q.tiles, t = fdiv(r, q.dStrips);
       pb = (n * q.strips + r - t * q.strips) * q.tiles + t;
    }
-   const int grp = ob / g.oblocks, tile0 = (ob - grp * g.oblocks) * TI * WO + wo * TI;
+   const int grp = ob / g.oblocks, tile0 = (ob - grp * g.oblocks) * TI * (TOGETHER ? 1 : WO) + wo * TI;
    const int p0 = pb * BP;
    if (p0 >= q.P) return;
    int origin;      // the tile's first row of the panels' inputs
@@ -239,10 +252,10 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       }
    __builtin_amdgcn_sched_barrier(0);
    const int taps = q.KH * q.KW;
-   int *const table = reinterpret_cast<int *>(smem_raw);
+   int *const table = reinterpret_cast<int *>(smem_raw) + (TOGETHER ? phase * g.table_ints : 0);
    // offset of every chunk of two slots (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
    // first chunks)
-   for (int e = tid; e < 2 * q.chunks; e += THREADS) {
+   for (int e = TOGETHER ? lane : tid; e < 2 * q.chunks; e += TOGETHER ? 64 : THREADS) {
       const int second = e >= q.chunks, k = second ? e - q.chunks : e, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
       table[e] = (c8 * q.cells + a * g.dh * q.PW + b * g.dw) * CELL + (g.nslots > 1 ? second * g.slot_bytes : 0);
    }
@@ -250,7 +263,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
    for (int j = 0; j < TJ; ++j) {
       const int p = p0 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), c = r - oy * q.ws;
-      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh - origin) * q.PW + (ROWS ? c : c * g.sw)) * CELL : 0;
+      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh + q.down - origin) * q.PW + (ROWS ? c : c * g.sw) + q.right) * CELL : 0;
    }
    v4f acc[TI][TJ];
 #pragma unroll
@@ -357,14 +370,14 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       auto again = __builtin_amdgcn_kernarg_segment_ptr();
       asm volatile("" : "+s"(again));
       const SplitArgs &late = *(const SplitArgs *)again, &h = ALL ? late : g;
-      const SplitPhase &weights = late.phase[PHASES ? phase : 0], &f = ALL ? weights : q;
+      const SplitPhase &weights = late.phase[PHASES || TOGETHER ? phase : 0], &f = ALL ? weights : q;
       const int ftaps = f.KH * f.KW;
       const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(h.x), 0, (int)h.xbytes, 0x00020000);
       const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(late.w0), 0, (int)OUTSIDE, 0x00020000);
 #pragma unroll 1
       for (int tile = 0; tile < TI * TJ; ++tile) {
          const int p = p1 + (wp * TJ + tile % TJ) * 16 + r16, panel = fdiv(p, f.dPHW), r = p - panel * f.PHW, oy = fdiv(r, f.dWS), n = fdiv(panel, f.dStrips);
-         const int iy0 = oy * h.sh - f.ph, ix0 = ((panel - n * f.strips) * f.ws + r - oy * f.ws) * h.sw - f.pw;
+         const int iy0 = oy * h.sh + f.down - f.ph, ix0 = ((panel - n * f.strips) * f.ws + r - oy * f.ws) * h.sw + f.right - f.pw;
          const int oc = (tile0 + tile / TJ) * 16 + r16;
          v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
@@ -396,13 +409,34 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       if (g.bias) v = __fadd_rn(v, b);
       return g.relu ? (v > 0.0f ? v : 0.0f) : v;
    };
+   // TOGETHER, two phases of neighbouring columns: each takes two of the other's four pixels and stores four columns next to each other
+   v2f other[TOGETHER && STORE == QUADS ? TI : 1][TOGETHER && STORE == QUADS ? TJ : 1];
+   if constexpr (TOGETHER && STORE == QUADS) {
+      __syncthreads();      // the patch is read
+      v2f *const swap = reinterpret_cast<v2f *>(smem_raw);
+      const bool odd = q.ox0 != 0;
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+         for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = finish(acc[i][j][e], bias[i][0]);
+            swap[((wave * TI + i) * TJ + j) * 64 + lane] = odd ? v2f{acc[i][j][0], acc[i][j][1]} : v2f{acc[i][j][2], acc[i][j][3]};
+         }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+         for (int j = 0; j < TJ; ++j) other[i][j] = swap[(((wave ^ 1) * TI + i) * TJ + j) * 64 + lane];
+   }
 #pragma unroll
    for (int j = 0; j < TJ; ++j) {
       const int p = p1 + (wp * TJ + j) * 16 + (STORE == QUADS ? 4 * kg : r16);
       const int panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), n = fdiv(panel, q.dStrips);
       const int ox = (panel - n * q.strips) * q.ws + r - oy * q.ws;
-      const bool pixel = p < q.P && r < q.full && ox < q.OW;
-      const unsigned at_pixel = (unsigned)(n * g.ocplane4 + ((q.oy0 + oy * q.oys) * g.OW0 + q.ox0 + ox * q.oxs) * 4);
+      const bool pixel = p < q.P && r < q.full && ox < q.OW && (!TOGETHER || oy < q.OH);
+      const int column = TOGETHER && STORE == QUADS ? 2 * ox + 4 * q.ox0 : q.ox0 + ox * q.oxs;
+      const unsigned at_pixel = (unsigned)(n * g.ocplane4 + ((q.oy0 + oy * q.oys) * g.OW0 + column) * 4);
 #pragma unroll
       for (int i = 0; i < TI; ++i) {
          const int oc = (tile0 + i) * 16;
@@ -410,8 +444,13 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
          v4f v = acc[i][j];
          if constexpr (STORE == QUADS) {
             const bool there = pixel && oc + r16 < g.ocg;
+            if constexpr (TOGETHER) {
+               const v2f o = other[i][j];
+               v = q.ox0 != 0 ? v4f{o[0], v[2], o[1], v[3]} : v4f{v[0], o[0], v[1], o[1]};
+            } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = finish(v[e], bias[i][0]);
+               for (int e = 0; e < 4; ++e) v[e] = finish(v[e], bias[i][0]);
+            }
             store16_buf(yrs4, v, there ? at_pixel + (unsigned)(r16 * g.plane4) : OUTSIDE, (unsigned)(grp * g.ocg + oc) * (unsigned)g.plane4);
          } else {
 #pragma unroll
@@ -464,6 +503,18 @@ __global__ void __launch_bounds__(256) k_conv_f32_split_weights(SplitWeightArgs 
    d[128] = s[2];
 }
 
+template <int TI, int TJ>
+int launch_together(sofie_hip_ctx *ctx, const SplitArgs &g, bool quads, long tiles)
+{
+   constexpr auto kern_p = k_conv_f32_split<TI, TJ, SplitPlan::TOGETHER, PIXELS, false, false>, kern_q = k_conv_f32_split<TI, TJ, SplitPlan::TOGETHER, QUADS, false, false>;
+   SOFIE_LARGE_LDS(kern_p);
+   SOFIE_LARGE_LDS(kern_q);
+   const size_t patch = (size_t)(g.table_bytes + g.slot_bytes * (g.nslots > 1 ? 2 : 1)), swap = (size_t)4 * TI * TJ * 64 * 8;
+   if (quads) hipLaunchKernelGGL(kern_q, dim3((unsigned)tiles), dim3(THREADS), patch > swap ? patch : swap, ctx->stream, g);
+   else hipLaunchKernelGGL(kern_p, dim3((unsigned)tiles), dim3(THREADS), patch, ctx->stream, g);
+   return check_launch(ctx, "k_conv_f32_split");
+}
+
 template <int TI, int TJ, int WO>
 int launch(sofie_hip_ctx *ctx, const SplitArgs &g, int nphases, bool quads, bool rows, long tiles)
 {
@@ -503,7 +554,13 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    // other kernels name them up to 144 products: 55x16x60x60 -> 64, 3x3, 1x10x101x101 -> 64).
    const long icg = p.C / p.groups;
    const bool rows = rows_of(p, icg);
-   if (other_us < 7.5 + (ctx->constant_weights ? 0.0 : 4.0) || (!rows && icg < 6) || (rows ? false : p.nphases == 1 ? icg * p.KH0 * p.KW0 <= 144 : icg * p.KH0 * p.KW0 < 48 * p.nphases)) return SOFIE_HIP_OK;
+   if (other_us < 7.5 + (ctx->constant_weights ? 0.0 : 4.0) || (!rows && icg < 6)) return SOFIE_HIP_OK;
+   // (phases of short sums: all of them by one workgroup, with whole stores. 81x49x22x22 -> 47, 2x2 s2 33 us there with 4-byte stores, 28 on
+   // k_conv_f32_any; 97x73x16x16 -> 27 13 and 17.5 with 16 bytes)
+   ConvProblem united;
+   const bool unites = SplitPlan::together(p, united);
+   const bool brief = rows ? false : p.nphases == 1 ? icg * p.KH0 * p.KW0 <= 144 : icg * p.KH0 * p.KW0 < 48 * p.nphases;
+   if (brief && !(unites && icg * p.KH0 * p.KW0 >= 64 && united.phase[0].OW % 4 == 0 && p.OW0 == 2 * united.phase[0].OW)) return SOFIE_HIP_OK;
    const size_t image = (size_t)p.C * p.H * p.W * 4, out_image = (size_t)p.OC * p.OH0 * p.OW0 * 4;
    // descriptors and OUTSIDE: 1 GiB of images per launch
    const size_t room = ((size_t)1 << 30) - ((size_t)16 << 20);
@@ -523,22 +580,36 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
    // (weights that are not kept are laid out in front of the launch, twice the bytes of k_conv_f32_any's)
    other_us = (other_us - (ctx->constant_weights ? 0.0 : 4.0)) * ((double)per / (double)p.N);
-   SplitPlan::Form best = plan.choose(per, cus, other_us);
+   SplitPlan::Form best{0, 0, 0, 0, 0, other_us};
+   if (!brief) best = plan.choose(per, cus, other_us);
+   SplitPlan one(unites ? united : p, false);
+   if (unites) {
+      // (k_conv_f32_any takes longer than its estimate under phases of unequal length: of 15 layers, 3x3 s2, this was the shorter way in all, by 1.07 to
+      // 1.7 times; short sums stay there unless they are well ahead: 51x31x40x40 -> 185, 2x2 s2 88 us there, 92 here)
+      const bool uneven = united.KH0 * united.KW0 % 4 != 0;
+      const SplitPlan::Form form = one.choose_together(plan, per, cus, best.ti > 0 ? best.time : (uneven ? 1.2 : brief ? 0.85 : 1.0) * other_us);
+      if (form.ti > 0) best = form;
+   }
    if (best.ti == 0) return SOFIE_HIP_OK;
    auto prepare = [&] {
+      const bool all = best.wo == SplitPlan::TOGETHER;
       g.CS = best.cs;
       g.nslots = plan.slots(best.cs);
-      g.table_bytes = plan.table_bytes(best.cs);
+      g.table_bytes = (all ? one : plan).table_bytes(best.cs);
+      g.table_ints = all ? g.table_bytes / 16 : 0;
       g.slot_bytes = 0;
       for (int i = 0; i < p.nphases; ++i) {
          const ConvPhase &f = p.phase[i];
          SplitPhase &q = g.phase[i];
          SplitPlan::Panels s;
-         plan.panels(s, i, best.pixels(), best.strips);
+         if (all) one.panels(s, 0, best.pixels(), best.strips);
+         else plan.panels(s, i, best.pixels(), best.strips);
+         const ConvPhase &patch = all ? united.phase[0] : f;
          q.ws = s.ws; q.strips = s.strips; q.PHW = s.PHW; q.full = s.full;
          q.HP = s.HP; q.PW = s.PW; q.cells = s.cells;
-         q.KH = f.KH; q.KW = f.KW; q.ph = f.ph; q.pw = f.pw;
-         q.OW = f.OW;
+         q.KH = f.KH; q.KW = f.KW; q.ph = patch.ph; q.pw = patch.pw;
+         q.down = patch.ph - f.ph; q.right = patch.pw - f.pw;
+         q.OH = f.OH; q.OW = f.OW;
          q.chunks = best.cs / 8 * plan.chunks[i];
          q.steps = plan.steps[i];
          q.wofs = (int)plan.wofs[i];
@@ -558,7 +629,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       }
       g.nphases = p.nphases;
       g.dPhases = make_fastdiv((unsigned)p.nphases);
-      g.oblocks = cdiv(g.octiles, best.wo * best.ti);
+      g.oblocks = cdiv(g.octiles, best.beside() * best.ti);
       g.dOB = make_fastdiv((unsigned)(g.oblocks * g.groups));
    };
    prepare();
@@ -597,7 +668,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
       const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
       if (n != per) {
-         best = plan.choose(n, cus, HUGE_VAL);
+         best = best.wo == SplitPlan::TOGETHER ? one.choose_together(plan, n, cus, HUGE_VAL) : plan.choose(n, cus, HUGE_VAL);
          prepare();
       }
       g.x = p.x + n0 * (image / 4);
@@ -617,6 +688,10 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
 #define SOFIE_FORM(i, j, o) case i * 100 + j * 10 + o: rc = launch<i, j, o>(ctx, g, p.nphases, plan.quads(g.phase[0].strips), rows, tiles); break
          SOFIE_FORM(4, 4, 2); SOFIE_FORM(3, 4, 2); SOFIE_FORM(2, 4, 2); SOFIE_FORM(4, 2, 2); SOFIE_FORM(2, 2, 2); SOFIE_FORM(1, 4, 2); SOFIE_FORM(1, 2, 2);
          SOFIE_FORM(1, 4, 1);
+      case 444: rc = launch_together<4, 4>(ctx, g, one.pairs(), tiles); break;
+      case 344: rc = launch_together<3, 4>(ctx, g, one.pairs(), tiles); break;
+      case 244: rc = launch_together<2, 4>(ctx, g, one.pairs(), tiles); break;
+      case 144: rc = launch_together<1, 4>(ctx, g, one.pairs(), tiles); break;
 #undef SOFIE_FORM
       }
       if (rc) return rc;

@@ -29,12 +29,14 @@ struct SplitPlan {
    // Workgroups a compute unit holds at once, by registers.
    static constexpr int resident_of(int ti, int tj, int wo) { return ti * tj > 8 ? 2 : ti * tj > 4 || wo == 1 ? 3 : 4; }
 
-   // 16 wo ti channels x 64 / wo tj pixels per workgroup, slots of cs channels, an image in strips; rows: a row of the kernel as a cell
+   // 16 wo ti channels x 64 / wo tj pixels per workgroup, slots of cs channels, an image in strips; rows: a row of the kernel as a cell.
+   // wo = TOGETHER: a wavefront for each of four phases, 16 ti channels x 16 tj places of them.
+   static constexpr int TOGETHER = 4;
    struct Form {
       int ti, tj, wo, cs, strips;
       double time;
       int pixels() const { return 64 / wo * tj; }
-      int channels() const { return 16 * wo * ti; }
+      int beside() const { return wo == TOGETHER ? 1 : wo; }      // wavefronts side by side along the channels
    };
 
    // Panels (strips of images) of one phase under tiles of some pixels
@@ -47,6 +49,7 @@ struct SplitPlan {
    // of the layer
    int icg, ocg, octiles, nphases;
    bool rows, whole;          // whole: pixels next to each other are stored next to each other
+   bool one_for_all = false;     // one workgroup for all phases
    int steps[MAX_PHASES];     // of four chunks of eight, all of K
    int chunks[MAX_PHASES];    // of eight channels of a slot
    size_t wofs[MAX_PHASES], pieces;      // first 16-byte piece of a phase's fragments; all of them
@@ -81,7 +84,7 @@ struct SplitPlan {
    }
 
    // Whether four pixels are stored at once.
-   bool quads(int strips) const { return whole && (strips == 1 ? (long)p.OH0 * p.OW0 % 4 == 0 : p.OW0 % 4 == 0); }
+   bool quads(int strips) const { return one_for_all ? pairs() : whole && (strips == 1 ? (long)p.OH0 * p.OW0 % 4 == 0 : p.OW0 % 4 == 0); }
 
    // Strips of phase i for tiles of bp pixels; false where numbers leave their range.
    bool panels(Panels &q, int i, int bp, int strips) const
@@ -199,6 +202,70 @@ struct SplitPlan {
       return s.time();
    }
 
+   // All phases of a stride of 2 x 2 by one workgroup: the layer as a single phase whose patch is what the four read. False where
+   // that is not possible.
+   static bool together(const ConvProblem &p, ConvProblem &u)
+   {
+      if (p.nphases != 4 || p.sh != 1 || p.sw != 1) return false;
+      u = p;
+      u.nphases = 1;
+      ConvPhase &f = u.phase[0];
+      int below = 0, right = 0;
+      for (int i = 0; i < 4; ++i) {
+         const ConvPhase &q = p.phase[i];
+         if (q.oys != 2 || q.oxs != 2 || q.oy0 != i / 2 || q.ox0 != i % 2) return false;
+         if (q.OH > f.OH) f.OH = q.OH;
+         if (q.OW > f.OW) f.OW = q.OW;
+         if (q.ph > f.ph) f.ph = q.ph;
+         if (q.pw > f.pw) f.pw = q.pw;
+         if ((q.KH - 1) * p.dh - q.ph > below || i == 0) below = (q.KH - 1) * p.dh - q.ph;
+         if ((q.KW - 1) * p.dw - q.pw > right || i == 0) right = (q.KW - 1) * p.dw - q.pw;
+      }
+      // (rows and columns of the patch as a kernel without dilation)
+      f.KH = f.ph + below + 1;
+      f.KW = f.pw + right + 1;
+      u.dh = u.dw = 1;
+      return f.KH >= 1 && f.KW >= 1;
+   }
+
+   // The best form with a phase per wavefront, below other_us; this: the plan of together()'s layer, apart: the one of the four phases.
+   Form choose_together(const SplitPlan &apart, size_t n, int cus, double other_us)
+   {
+      static const int forms[][2] = {{4, 4}, {2, 4}, {3, 4}, {1, 4}};
+      Form best{0, 0, 0, 0, 0, other_us};
+      if (apart.pieces * 16 > ((size_t)1 << 29)) return best;
+      bool even = true;
+      int most = 0, all = 0;
+      for (int i = 0; i < 4; ++i) {
+         even = even && apart.chunks[i] == apart.chunks[0];
+         most = apart.chunks[i] > most ? apart.chunks[i] : most;
+         all += apart.steps[i];
+      }
+      one_for_all = true;
+      chunks[0] = 4 * most;      // (of the tables of offsets, one for each phase)
+      steps[0] = (all + 3) / 4;
+      for (const auto &f : forms) {
+         if (f[0] > 1 && f[0] - 1 >= octiles) continue;      // tiles of nothing
+         for (int cs = 16; cs <= 32; cs *= 2) {
+            // every wavefront comes to the same barriers: steps end with slots, or all alike
+            bool fits = true;
+            for (int i = 0; i < 4; ++i) fits = fits && (slots(cs) == 1 || (cs / 8 * apart.chunks[i] >= 4 && (even || cs / 8 * apart.chunks[i] % 4 == 0)));
+            for (int strips = 1; fits && strips <= MAX_STRIPS; ++strips) {
+               Form form{f[0], f[1], TOGETHER, cs, strips, 0.0};
+               Panels q;
+               // (strips of a few columns: 192x224x13x13 -> 170, 2x2 s2 on strips of one 141 us, 106 apart)
+               if (!panels(q, 0, form.pixels(), strips) || q.cells > cells_of(form) || (strips > 1 && q.ws < 8)) continue;
+               if (table_bytes(cs) + (slots(cs) > 1 ? 2 : 1) * (long)slot_bytes(q.cells, cs) > MAX_LDS || (double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
+               form.time = estimate(form, &q, n, cus) * (strips > 1 ? 1.02 : 1.0);
+               if (form.time < best.time) best = form;
+            }
+         }
+      }
+      return best;
+   }
+   // Whether four pixels of two phases are stored at once: two neighbouring columns of each.
+   bool pairs() const { return p.phase[0].OW % 4 == 0 && p.OW0 == 2 * p.phase[0].OW; }
+
 private:
    const ConvProblem &p;
 
@@ -243,10 +310,10 @@ private:
       Sum(const SplitPlan &l, const Form &f, int cus, int resident, bool quads) : l(l), f(f), cus(cus), resident(resident)
       {
          pieces = f.ti * f.tj;
-         blocks = (l.octiles + f.wo * f.ti - 1) / (f.wo * f.ti) * l.p.groups;
+         blocks = (l.octiles + f.beside() * f.ti - 1) / (f.beside() * f.ti) * l.p.groups;
          nslots = l.slots(f.cs);
-         store_alone = l.nphases > 1 ? 280.0 : quads ? 0.0 : 292.0;
-         store = l.nphases > 1 ? 259.0 : quads ? 0.0 : 176.0;
+         store_alone = l.nphases > 1 || (l.one_for_all && !quads) ? 280.0 : quads ? 0.0 : 292.0;
+         store = l.nphases > 1 ? 259.0 : quads ? 0.0 : l.one_for_all ? 259.0 : 176.0;
       }
       void add(int k, int pixel_tiles, int cells)
       {
@@ -271,12 +338,14 @@ private:
          // (phases of unequal length, 3x3 s2: the same estimate was 1.25 to 1.5 times too short on 94 timings; with 1.4 the layers it takes of 190
          // random ones are 0.96 to 1.75 times k_conv_f32_any's time, with 1.35 0.94)
          const ConvPhase &q0 = l.p.phase[0], &q1 = l.p.phase[l.nphases - 1];
-         const double uneven = q0.KH * q0.KW != q1.KH * q1.KW ? 1.4 : 1.0;
+         // A phase per wavefront: 1.24 times what is estimated in the mean over 290 timings of 47 layers, even phases or not (14 % rms; what is
+         // picked is 2.2 % behind the best of these forms in the mean): each wavefront takes in weights of its own.
+         const double uneven = l.one_for_all ? 1.25 : q0.KH * q0.KW != q1.KH * q1.KW ? 1.4 : 1.0;
          const double us = std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
          // (Under the device's power limit the form with the fewest requests for weights per matrix instruction comes out ahead of what is
          // estimated: 256x64x56x56 -> 128, 3x3 604 us on 128 channels x 64 pixels, 568 on 128 x 128. Of 50 random layers of 15 GFLOP
          // and more none changes by more than 1.3 %, what two runs of one side differ by.)
-         return pieces == 16 && us > 150.0 ? 150.0 + 0.93 * (us - 150.0) : us;
+         return pieces == 16 && us > 150.0 && !l.one_for_all ? 150.0 + 0.93 * (us - 150.0) : us;
       }
    };
 

@@ -94,6 +94,39 @@ def test_transposed_conv_in_three_parts(ops, kept, n, c, h, w, oc, k, s):
         assert float((y[i:i + 1].cpu().double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
 
 
+# N, C, H, W, OC, k, (pad, right and bottom pad less), groups: all four phases by one workgroup; 16-byte stores where W is whole fours and the output
+# twice as wide; phases of equal and of unequal length and extent; one slot and several, the last one in part; blocks of 16 to 64 channels
+TOGETHER = [
+    (64, 128, 28, 28, 64, 4, (1, 1), 1), (48, 54, 31, 29, 64, 4, (1, 1), 1), (40, 33, 24, 20, 48, 4, (0, 0), 1), (128, 32, 24, 24, 17, 2, (0, 0), 1),
+    (30, 70, 31, 33, 60, 2, (0, 0), 1), (60, 46, 24, 23, 64, 3, (1, 0), 1), (60, 46, 20, 24, 70, 3, (1, 1), 1), (24, 40, 23, 26, 96, 5, (2, 1), 1),
+    (30, 96, 20, 20, 128, 4, (1, 1), 2), (200, 24, 9, 8, 130, 3, (1, 0), 1), (16, 20, 70, 72, 16, 6, (2, 2), 1)]
+
+
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("shape", TOGETHER)
+def test_phases_of_one_workgroup(ops, kept, shape, large):
+    """Bounds as above: 1e-5 of the largest output and 3e-7 in the 2-norm; operands of 2^60, whose sums are formed again in fp32, a rounding for each
+    product."""
+    n, c, h, w, oc, k, (before, behind), groups = shape
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    big = 2.0 ** 60 if large else 1.0
+    x, wt = torch.randn(n, c, h, w, device="cuda", generator=g) * big, torch.randn(c, oc // groups, k, k, device="cuda", generator=g) * (c * k * k) ** -0.5 * big
+    torch.cuda.synchronize()
+    pads = (before, before, behind, behind)
+    y, names = names_of(kept, lambda: ops.conv_transpose2d_f32(x, wt, None, pads, (2, 2), (1, 1), groups, (0, 0), ctx=kept))
+    assert "k_conv_f32_split" in names, names
+    H, W = y.shape[2:]
+    conv = lambda a, b: torch.nn.functional.conv_transpose2d(a, b, None, 2, 0, 0, groups)[:, :, before:before + H, before:before + W]
+    for i in sorted({0, n // 2, n - 1}):
+        xi, wi = x[i:i + 1].cpu().double(), wt.cpu().double()
+        ref = conv(xi, wi)
+        err = y[i:i + 1].cpu().double() - ref
+        if large:
+            assert bool((err.abs() <= (c * k * k) ** 0.5 * 2.0 ** -24 * conv(xi.abs(), wi.abs())).all()), i
+        else:
+            assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())) and float(err.norm()) <= 3e-7 * float(ref.norm()), i
+
+
 @pytest.mark.parametrize("shape", CONV + [
     (64, 128, 28, 28, 64, 4, 2), (30, 143, 32, 34, 181, 4, 2), (120, 87, 19, 21, 256, 3, 2), (64, 120, 20, 20, 90, 3, 1)])      # transposed: k, stride
 def test_sums_that_are_repeated_in_every_form(ops, kept, shape):
