@@ -53,8 +53,11 @@ constexpr unsigned OUTSIDE = 0x80000000u;
 // MB x NB tiles of 16 pixels x 16 channels per wavefront; NW wavefronts, groups of WK of them share their pixels and deal
 // the K-steps among themselves; D fragments of every pixel tile in flight. POOL: the four pixel tiles are the positions of
 // a 2x2 window with stride 2. BLDS: the weights of the workgroup's channels stay in LDS while it walks over its tiles.
+// (Two wavefronts to a SIMD said so: left to itself the compiler took more than 256 registers with the accumulators for four wavefronts on four tiles
+// of channels, one to a SIMD: 121x16x32x32 -> 128, 5x5 27.9 -> 21 us, 16x70x59x31 -> 97, 3x3 pooled 27.7 -> 12. Three on up to two tiles of channels: 1.2
+// times longer with two.)
 template <int MB, int NB, int NW, int WK, int D, bool BOUNDS, bool POOL, bool BLDS>
-__global__ void __launch_bounds__(NW * 64) k_qconv_any(AnyArgs a)
+__global__ void __launch_bounds__(NW * 64, BLDS ? 2 : 1) k_qconv_any(AnyArgs a)
 {
    static_assert(!POOL || MB == 4, "the four window positions are the four pixel tiles");
    static_assert(!BLDS || WK == 1, "the dealt K-steps read their weights from memory");
@@ -289,66 +292,94 @@ __global__ void __launch_bounds__(256) k_qconv_any_weights(const int8_t *w, v4i 
    dst[id] = o;
 }
 
-// The padded copy of the input, one thread per dword. FROM: 0 channels-last int8, 1 int8 planes, 2 float planes (quantized).
-template <int FROM>
-__global__ void __launch_bounds__(256) k_qconv_any_input(QConvArgs g, unsigned *dst, int total, int HP, int WP, int cd, FastDiv dcd,
-                                                         FastDiv dWP, FastDiv dHP)
+// The padded copy of the input from channels-last int8: 16 bytes of the copy per thread. What lies behind a pixel's last channel meets zero
+// weights: it is what follows in the tensor. WHOLE: pixels of the copy are whole 16 bytes. Bound: the chain of divisions (one per thread and
+// extent) and memory. With a thread per dword
+// and now, us of both launches: 192x131x51x51 -> 12, 3x3 s2 88 / 51; 128x33x80x80 -> 13, 5x5 58 / 50; 60 random layers 1.1 times shorter in the mean, with the
+// forms below 1.16.
+template <bool WHOLE>
+__global__ void __launch_bounds__(256) k_qconv_any_input(QConvArgs g, v4i *dst, int total, int HP, int WP, int cd, FastDiv dcd, FastDiv dWP, FastDiv dHP)
 {
    const int id = blockIdx.x * 256 + threadIdx.x;
    if (id >= total) return;
-   // dword of a pixel fastest where the source is channels-last (contiguous reads); the column fastest where it is planes
-   int n, r, c, k;
-   if constexpr (FROM == 0) {
-      const int p = fdiv(id, dcd), R = fdiv(p, dWP);
-      k = id - p * cd;
-      c = p - R * WP;
-      n = fdiv(R, dHP);
-      r = R - n * HP;
+   const int p = fdiv(4 * id, dcd), R = fdiv(p, dWP), n = fdiv(R, dHP);
+   int k = 4 * id - p * cd, c = p - R * WP - g.pw, r = R - n * HP - g.ph;
+   const size_t bytes = (size_t)g.N * g.H * g.W * g.C;
+   size_t row = ((size_t)n * g.H + r) * g.W;      // (of a row that is there)
+   // (the last bytes of the tensor by themselves)
+   auto load4 = [&](size_t at) {
+      unsigned v = 0;
+      if (at + 4 <= bytes) __builtin_memcpy(&v, g.x + at, 4);
+      else
+#pragma unroll
+         for (int b = 0; b < 4; ++b)
+            if (at + b < bytes) v |= (unsigned)(uint8_t)g.x[at + b] << (8 * b);
+      return (int)v;
+   };
+   const int fill = (int)(0x01010101u * (unsigned)(g.zpx & 0xff));
+   v4i v = {fill, fill, fill, fill};
+   if constexpr (WHOLE) {
+      if ((unsigned)r < (unsigned)g.H && (unsigned)c < (unsigned)g.W) {
+         const size_t at = (row + c) * g.C + 4 * k;
+         if (at + 16 <= bytes) __builtin_memcpy(&v, g.x + at, 16);
+         else
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = load4(at + 4 * u);
+      }
    } else {
-      const int p = fdiv(id, dWP), R = fdiv(p, dcd);
-      c = id - p * WP;
-      k = p - R * cd;
-      n = fdiv(R, dHP);
-      r = R - n * HP;
-   }
-   const int ih = r - g.ph, iw = c - g.pw;
-   unsigned v = 0x01010101u * (unsigned)(g.zpx & 0xff);
-   if (ih >= 0 && ih < g.H && iw >= 0 && iw < g.W) {
-      const int left = g.C - 4 * k;      // channels of this dword that exist (the others meet zero weights)
-      if constexpr (FROM == 0) {
-         const int8_t *p = g.x + (((size_t)n * g.H + ih) * g.W + iw) * g.C + 4 * k;
-         if (left >= 4) __builtin_memcpy(&v, p, 4);
-         else {
-            v = 0;
-            for (int t = 0; t < left; ++t) v |= (unsigned)(uint8_t)p[t] << (8 * t);
-         }
-      } else if (left <= 0) {
-         v = 0;
-      } else {
-         const size_t plane = (size_t)g.H * g.W;
-         const size_t off = ((size_t)n * g.C + 4 * k) * plane + (size_t)ih * g.W + iw;
-         v = 0;
-         if constexpr (FROM == 1) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-               const unsigned e = (uint8_t)g.x[off + (t < left ? t : 0) * plane];
-               v |= t < left ? e << (8 * t) : 0u;
-            }
-         } else {
-            float f[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) f[t] = g.xf[off + (t < left ? t : 0) * plane];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-               float q = rintf(__fdiv_rn(f[t], g.xscale));
-               q = fminf(fmaxf(q, -1024.0f), 1024.0f);
-               const int e = min(127, max(-128, (int)q + g.zpx));
-               v |= t < left ? (unsigned)(e & 0xff) << (8 * t) : 0u;
+      for (int u = 0; u < 4; ++u) {
+         int e = fill;
+         if ((unsigned)r < (unsigned)g.H && (unsigned)c < (unsigned)g.W) e = load4((row + c) * g.C + 4 * k);
+         v[u] = e;
+         if (++k == cd) {
+            k = 0;
+            if (++c == WP - g.pw) {
+               c = -g.pw;
+               if (++r == HP - g.ph) r = -g.ph, row += (size_t)(g.H - HP) * g.W;      // (the next image's first row)
+               row += g.W;
             }
          }
       }
    }
-   dst[FROM == 0 ? id : (((size_t)n * HP + r) * WP + c) * cd + k] = v;
+   dst[id] = v;
+}
+
+// The same from planes, int8 (FLOAT: the float tensor, quantized): a dword, four channels of a pixel, per thread; channels that no pixel has are
+// not asked for or divided. 176x1x146x146 -> 16, 3x3 s2 33.5 -> 28 us (with four pixels per thread the same, and 202 -> 208 where it is 16 more
+// divisions one behind the other: 185x3x160x96 -> 55, 7x7).
+template <bool FLOAT>
+__global__ void __launch_bounds__(256) k_qconv_any_planes(QConvArgs g, unsigned *dst, int pixels, int HP, int WP, int cd, FastDiv dPixels, FastDiv dWP, FastDiv dHP)
+{
+   const int id = blockIdx.x * 256 + threadIdx.x, k = fdiv(id, dPixels);
+   if (k >= cd) return;
+   const int p = id - k * pixels, R = fdiv(p, dWP), n = fdiv(R, dHP), c = p - R * WP - g.pw, r = R - n * HP - g.ph;
+   const int left = g.C - 4 * k;      // channels of this dword and behind it (what is not there meets zero weights)
+   const size_t plane = (size_t)g.H * g.W;
+   unsigned v = 0x01010101u * (unsigned)(g.zpx & 0xff);
+   if ((unsigned)r < (unsigned)g.H && (unsigned)c < (unsigned)g.W) {
+      const size_t off = ((size_t)n * g.C + (left > 0 ? 4 * k : 0)) * plane + (size_t)r * g.W + c;
+      float f[4] = {};
+      int q[4] = {};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+         if (t > 0 && t >= g.C) continue;
+         const size_t at = off + (t < left ? t : 0) * plane;
+         if constexpr (FLOAT) f[t] = g.xf[at];
+         else q[t] = g.x[at];
+      }
+      v = 0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+         if (t > 0 && t >= g.C) continue;
+         if constexpr (FLOAT) {
+            const float z = fminf(fmaxf(rintf(__fdiv_rn(f[t], g.xscale)), -1024.0f), 1024.0f);
+            q[t] = min(127, max(-128, (int)z + g.zpx));
+         }
+         v |= t < left ? (unsigned)(q[t] & 0xff) << (8 * t) : 0u;
+      }
+   }
+   dst[(size_t)p * cd + k] = v;
 }
 
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -432,13 +463,15 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       if (int rc = check_launch(ctx, "k_qconv_any_weights")) return rc;
    }
    if (p.copy) {
-      const int cd = p.pix / 4, total = g.N * p.HP * p.WP * cd;
-      const dim3 grid((unsigned)cdiv(total, 256)), block(256);
+      const int cd = p.pix / 4, pixels = g.N * p.HP * p.WP, total = cdiv(pixels * cd, 4);
+      const FastDiv dcd = make_fastdiv(cd), dWP = make_fastdiv(p.WP), dHP = make_fastdiv(p.HP), dPixels = make_fastdiv(pixels);
+      const dim3 block(256), grid((unsigned)cdiv(g.xf || !g.x_nhwc ? pixels * cd : total, 256));
       unsigned *const dst = reinterpret_cast<unsigned *>(xs);
-      const FastDiv dcd = make_fastdiv(cd), dWP = make_fastdiv(p.WP), dHP = make_fastdiv(p.HP);
-      if (g.xf) hipLaunchKernelGGL(k_qconv_any_input<2>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
-      else if (!g.x_nhwc) hipLaunchKernelGGL(k_qconv_any_input<1>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
-      else hipLaunchKernelGGL(k_qconv_any_input<0>, grid, block, 0, ctx->stream, g, dst, total, p.HP, p.WP, cd, dcd, dWP, dHP);
+      v4i *const dst4 = reinterpret_cast<v4i *>(xs);
+      if (g.xf) hipLaunchKernelGGL(k_qconv_any_planes<true>, grid, block, 0, ctx->stream, g, dst, pixels, p.HP, p.WP, cd, dPixels, dWP, dHP);
+      else if (!g.x_nhwc) hipLaunchKernelGGL(k_qconv_any_planes<false>, grid, block, 0, ctx->stream, g, dst, pixels, p.HP, p.WP, cd, dPixels, dWP, dHP);
+      else if (cd % 4 == 0) hipLaunchKernelGGL(k_qconv_any_input<true>, grid, block, 0, ctx->stream, g, dst4, total, p.HP, p.WP, cd, dcd, dWP, dHP);
+      else hipLaunchKernelGGL(k_qconv_any_input<false>, grid, block, 0, ctx->stream, g, dst4, total, p.HP, p.WP, cd, dcd, dWP, dHP);
       if (int rc = check_launch(ctx, "k_qconv_any_input")) return rc;
    }
    AnyArgs a{};
@@ -487,10 +520,10 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    } while (0)
    // The form, by the number of workgroups it gives and by what the LDS holds.
    //   A, B  64 pixels x up to 64 channels per wavefront, weights in LDS, as many workgroups as are resident at once walk over the
-   //         tiles: for a tile per compute unit and more. A: four wavefronts, up to three workgroups in a compute unit, for weights
-   //         of up to 50 KB or fewer than two rounds of tiles; B: eight wavefronts, one workgroup, for larger weights (up to
-   //         144 KB). us in A, B, C: 81x16x83x83 -> 54, 3x3 42 30 38; 43x16x100x100 -> 124, 5x5 s2 26 19 23.
-   //         Of 47 layers in A 23 are 5 % and more faster in B and none is slower.
+   //         tiles: for a tile per compute unit and more, with 16 KB of weights and more from half of that. A: four wavefronts, two or three
+   //         workgroups in a compute unit; B: eight wavefronts, one workgroup, from four rounds of tiles and, with more than 75 KB of
+   //         weights, from two on. Both timed on 220 layers: B takes 0.87 to 0.92 times A's time from four rounds on, 1.02 to 1.13 with
+   //         two to four, 0.96 to 1.02 below; C, D or E 1.07 to 1.2 times A's from half a round on 16 KB of weights.
    //   C, D, E  weights from memory, below.
    // Channels per workgroup: up to four tiles of 16, as few idle ones as possible.
    auto even = [&](int most) { return cdiv(p.nt, cdiv(p.nt, most)); };
@@ -499,8 +532,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    while (nb > 1 && (size_t)nb * p.S * 1024 > (size_t)144 * 1024) nb = even(nb - 1);
    const size_t wlds = (size_t)nb * p.S * 1024;
    const long long big_tiles = (long long)cdiv(a.M, 4 * mb * 16) * cdiv(p.nt, nb);
-   if (big_tiles >= cus && wlds <= (size_t)144 * 1024) {
-      if (wlds + tab_bytes <= (size_t)50 * 1024 || big_tiles < 2 * cus) {
+   if ((big_tiles >= cus || (2 * big_tiles >= cus && wlds >= (size_t)16 * 1024)) && wlds <= (size_t)144 * 1024) {
+      if (big_tiles < 2 * cus || (big_tiles < 4 * cus && wlds + tab_bytes <= (size_t)75 * 1024)) {
          const int resident = (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024)) > 3 ? 3 : (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024));
          if (nb == 1) SOFIE_ANY(4, 4, 1, 4, 1, 4, true, wlds, resident);
          if (nb == 2) SOFIE_ANY(4, 4, 2, 4, 1, 4, true, wlds, resident);
@@ -527,6 +560,7 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    float least = 1e30f;
    for (int f = 0; f < 6; ++f) {
       const Few &q = few[f];
+      if (q.nb > p.nt) continue;      // tiles of nothing
       const float workgroups = (float)cdiv(a.M, q.nw / q.wk * (pool ? 1 : q.mb) * 16) * (float)cdiv(p.nt, q.nb), per_cu = workgroups > (float)cus ? workgroups / (float)cus : 1.0f;
       const int steps = cdiv(p.S, q.wk), mbs = pool ? 4 : q.mb, pieces = mbs * q.nb;
       const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? 0.353f + 0.153f * (float)(steps - q.d) / (float)q.d : 0.0f);
