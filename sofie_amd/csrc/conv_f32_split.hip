@@ -27,6 +27,9 @@
 // exchange half of their columns in LDS and store 16 bytes each. What bounds it then are the weights, 12 KB a step and wavefront from
 // the L2 where four wavefronts share them otherwise. Transposed 64x128x28x28 -> 64, 4x4 s2 89.5 -> 81; 140 random layers of stride 2 1.1 times
 // shorter in the mean, 1.2 to 1.6 times where the route changed (3x3, 56x107x56x56 -> 16 97 -> 68.5; 2x2, 114x231x48x35 -> 16 136 -> 104).
+// A layer of stride 2 reads four cells a pixel: slots of eight channels (choose_eights), whose odd number of chunks makes whole steps over four slots.
+// 33x128x99x99 -> 128, 3x3 s2 244 us on k_conv_f32_any, 170 here; 48x80x144x11 -> 192, 7x7 s2 331, 167; 45 of 100 random layers of stride 2 1.1 to 2 times shorter,
+// the others unchanged.
 // All requests of a slot leave in one step: the fragments behind them wait for them (loads return in order), and one such wait
 // per slot is cheaper than one per step. A bias read behind the loop made the compiler wait for each store in front of the next one
 // (13000 cycles for 16 stores instead of 6800).
@@ -59,6 +62,7 @@ struct SplitPhase {
    int HP, PW, cells;         // rows of a panel's input, cells of a row, of a tile's patch
    int full;                  // pixels of a panel that exist (PHW: up to whole tiles where tiles do not run on into the next panel)
    int chunks;                // of a slot: 8 channels of a tap each
+   int ring;                  // of two slots, or of four (an odd number of chunks): whole steps
    int steps;                 // of four chunks, all of K
    int wofs;                  // first 16-byte piece of the phase's fragments
    int OW;
@@ -253,10 +257,10 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
    __builtin_amdgcn_sched_barrier(0);
    const int taps = q.KH * q.KW;
    int *const table = reinterpret_cast<int *>(smem_raw) + (TOGETHER ? phase * g.table_ints : 0);
-   // offset of every chunk of two slots (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
+   // offset of every chunk of two slots, or of four (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
    // first chunks)
-   for (int e = TOGETHER ? lane : tid; e < 2 * q.chunks; e += TOGETHER ? 64 : THREADS) {
-      const int second = e >= q.chunks, k = second ? e - q.chunks : e, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
+   for (int e = TOGETHER ? lane : tid; e < q.ring; e += TOGETHER ? 64 : THREADS) {
+      const int slot = (e >= q.chunks) + (e >= 2 * q.chunks) + (e >= 3 * q.chunks), second = slot & 1, k = e - slot * q.chunks, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
       table[e] = (c8 * q.cells + a * g.dh * q.PW + b * g.dw) * CELL + (g.nslots > 1 ? second * g.slot_bytes : 0);
    }
    int base[TJ];
@@ -306,7 +310,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
             for (int j = 0; j < TJ; ++j) read_x(j, off);
          }
-         place = place + 4 == 2 * q.chunks ? 0 : place + 4;
+         place = place + 4 == q.ring ? 0 : place + 4;
          const int ahead = across ? end - 2 : end - 1;
          fresh = step >= ahead;
          const int off = table[(fresh ? 0 : place) + kg];
@@ -582,6 +586,12 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    other_us = (other_us - (ctx->constant_weights ? 0.0 : 4.0)) * ((double)per / (double)p.N);
    SplitPlan::Form best{0, 0, 0, 0, 0, other_us};
    if (!brief) best = plan.choose(per, cus, other_us);
+   const bool strided = !brief && p.nphases == 1 && (p.sh > 1 || p.sw > 1);
+   if (strided) {
+      // (slots of eight channels; estimates are off by some 8 %: 146x145x176x64 -> 40, 3x3 s2 529 us on k_conv_f32_any, 542 here)
+      const SplitPlan::Form form = plan.choose_eights(per, cus, 0.95 * best.time);
+      if (form.ti > 0) best = form;
+   }
    SplitPlan one(unites ? united : p, false);
    if (unites) {
       // (k_conv_f32_any takes longer than its estimate under phases of unequal length: of 15 layers, 3x3 s2, this was the shorter way in all, by 1.07 to
@@ -611,6 +621,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
          q.down = patch.ph - f.ph; q.right = patch.pw - f.pw;
          q.OH = f.OH; q.OW = f.OW;
          q.chunks = best.cs / 8 * plan.chunks[i];
+         q.ring = (rows || q.chunks % 2 == 0 ? 2 : 4) * q.chunks;
          q.steps = plan.steps[i];
          q.wofs = (int)plan.wofs[i];
          q.oy0 = f.oy0; q.oys = f.oys; q.ox0 = f.ox0; q.oxs = f.oxs;
@@ -668,7 +679,7 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
       const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
       if (n != per) {
-         best = best.wo == SplitPlan::TOGETHER ? one.choose_together(plan, n, cus, HUGE_VAL) : plan.choose(n, cus, HUGE_VAL);
+         best = best.wo == SplitPlan::TOGETHER ? one.choose_together(plan, n, cus, HUGE_VAL) : best.cs == 8 ? plan.choose_eights(n, cus, HUGE_VAL) : plan.choose(n, cus, HUGE_VAL);
          prepare();
       }
       g.x = p.x + n0 * (image / 4);

@@ -115,7 +115,7 @@ struct SplitPlan {
    {
       int most = 0;
       for (int i = 0; i < nphases; ++i) most = chunks[i] > most ? chunks[i] : most;
-      return (2 * (cs / 8) * most * 4 + 255) & ~255;
+      return (2 * (cs > 8 ? cs / 8 : 2) * most * 4 + 255) & ~255;      // (8 channels: four slots, whose chunks are whole steps)
    }
    // Cells a workgroup of this form can hold, by what its threads carry.
    int cells_of(const Form &f) const { return items_of(f.ti, f.tj, f.wo, rows) * THREADS / (f.cs / 8); }
@@ -200,6 +200,37 @@ struct SplitPlan {
       Sum s(*this, f, cus, by_lds < by_registers ? by_lds : by_registers, quads(q[0].strips));
       for (int k = 0; k < kinds; ++k) s.add(k, ((int)n * q[k].strips * q[k].PHW + f.pixels() - 1) / f.pixels(), q[k].cells);
       return s.time();
+   }
+
+   // The best form with slots of 8 channels, below other_us: strided layers, whose patches are too large for more (16x16x... pixels under a stride of 2
+   // read 33x33 cells).
+   Form choose_eights(size_t n, int cus, double other_us)
+   {
+      static const int forms[][3] = {{2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 2, 2}, {2, 4, 2}, {1, 4, 2}};
+      Form best{0, 0, 0, 0, 0, other_us};
+      if (pieces * 16 > ((size_t)1 << 29) || rows || nphases != 1 || chunks[0] < 4) return best;
+      for (int t = 0; t < 3; ++t) least_cells[t][0] = cells_at_least(p.phase[0], 64 << t);
+      for (const auto &f : forms) {
+         if (f[0] > 1 && f[2] * (f[0] - 1) >= octiles) continue;      // tiles of nothing
+         Form form{f[0], f[1], f[2], 8, 0, 0.0};
+         if (least_cells[tile_of(form)][0] > cells_of(form) || least_time(form, n, cus) >= best.time) continue;
+         form.time = HUGE_VAL;
+         for (int strips = 1; strips <= MAX_STRIPS; ++strips) {
+            Panels q;
+            if (!panels(q, 0, form.pixels(), strips) || q.cells > cells_of(form)) continue;
+            if (table_bytes(8) + 2 * (long)slot_bytes(q.cells, 8) > MAX_LDS || (double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
+            if (form.ti == 4 && form.tj == 2 && !quads(q.strips)) continue;
+            const double time = estimate(form, &q, n, cus) * (strips > 1 ? 1.02 : 1.0);
+            if (time < form.time) {
+               form.time = time;
+               form.strips = strips;
+            } else if (strips > form.strips + 1) {
+               break;
+            }
+         }
+         if (form.strips > 0 && form.time < best.time) best = form;
+      }
+      return best;
    }
 
    // All phases of a stride of 2 x 2 by one workgroup: the layer as a single phase whose patch is what the four read. False where

@@ -80,6 +80,36 @@ def test_conv_in_three_parts(ops, kept, shape):
             assert "k_conv_f32_split" not in names or float(err.norm()) <= 3e-7 * float(ref.norm()), i
 
 
+# Layers of stride 2 in slots of eight channels: an odd number of chunks in a slot (9, 25, 49), an even one; one slot, several, the last one in part
+EIGHTS = [
+    (33, 128, 99, 99, 128, 3, 3, (2, 2), (1, 1, 1, 1), (1, 1), 1), (60, 48, 37, 37, 112, 3, 3, (2, 2), (1, 1, 1, 1), (1, 1), 1),
+    (46, 61, 40, 64, 27, 5, 5, (2, 2), (2, 2, 2, 2), (1, 1), 1), (48, 81, 144, 11, 190, 7, 7, (2, 2), (3, 3, 3, 3), (1, 1), 1),
+    (64, 120, 64, 60, 128, 4, 4, (2, 2), (1, 1, 2, 1), (1, 1), 1), (40, 96, 33, 50, 96, 5, 5, (2, 1), (2, 2, 2, 2), (1, 1), 2),
+    (224, 8, 57, 57, 48, 5, 5, (2, 2), (2, 2, 2, 2), (1, 1), 1), (30, 40, 60, 60, 64, 5, 5, (2, 2), (3, 2, 2, 3), (1, 2), 1)]
+
+
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("shape", EIGHTS)
+def test_strided_layers_in_slots_of_eight(ops, kept, shape, large):
+    """Bounds as above; operands of 2^60, whose sums are formed again in fp32, a rounding for each product."""
+    n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
+    g = torch.Generator(device="cuda").manual_seed(n + c + oc)
+    big, products = 2.0 ** 60 if large else 1.0, c // groups * kh * kw
+    x = torch.randn(n, c, h, w, device="cuda", generator=g) * big
+    wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * products ** -0.5 * big
+    zero = torch.zeros(oc, device="cuda")
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: ops.conv2d_f32(x, wt, None, pads, s, d, groups, ctx=kept))
+    assert "k_conv_f32_split" in names, names
+    for i in sorted({0, n // 2, n - 1}):
+        ref = reference(x[i:i + 1], wt, zero, s, pads, d, groups)
+        err = y[i:i + 1].cpu().double() - ref
+        if large:
+            assert bool((err.abs() <= products ** 0.5 * 2.0 ** -24 * reference(x[i:i + 1].abs(), wt.abs(), zero, s, pads, d, groups)).all()), i
+        else:
+            assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())) and float(err.norm()) <= 3e-7 * float(ref.norm()), i
+
+
 @pytest.mark.parametrize("n,c,h,w,oc,k,s", [(64, 128, 28, 28, 64, 4, 2), (30, 143, 32, 34, 181, 4, 2), (30, 64, 26, 15, 93, 4, 2),
                                             (60, 87, 19, 21, 40, 3, 2), (64, 120, 20, 20, 90, 3, 1)])
 def test_transposed_conv_in_three_parts(ops, kept, n, c, h, w, oc, k, s):
