@@ -1,13 +1,13 @@
 // fp32 NCHW convolutions whose outputs are sums of at most nine products (one channel under a 3x3 kernel, up to nine channels under a 1x1), on
 // the vector unit: k_conv_f32_short.
 //
-// A sum this short is a few matrix instructions between the tables, operand loads, waits and stores of a tile. Here a lane owns two
-// pixels, 64 apart in the row of all images' pixels, and keeps the K inputs of each in registers; the weights of an output channel are
+// A sum this short is a few matrix instructions between the tables, operand loads, waits and stores of a tile. Here a lane owns two or
+// four pixels, 64 apart in the row of all images' pixels, and keeps the K inputs of each in registers; the weights of an output channel are
 // uniform, scalar loads; neighbouring lanes load and store neighbouring dwords, whatever the width of a row, and a channel is a
 // uniform offset. (Four neighbouring pixels per lane and 16-byte stores: every load of a window touched 16 lines for 64 lanes,
 // 256x1x40x40 -> 32, 3x3 27.6 us.)
 //
-// Bound: the stores (3.7 TB/s at 229x1x50x50 -> 170). us against k_conv_f32_any: 256x1x40x40 -> 32, 3x3 25.9 -> 19.1; 229x1x50x50 -> 170,
+// Bound: the stores (3.7 TB/s at 229x1x50x50 -> 170). us against k_conv_f32_any: 256x1x40x40 -> 32, 3x3 25.9 -> 15.0; 229x1x50x50 -> 170,
 // 3x3 134 -> 106; 56x1x189x30 -> 33, 1x1 25.6 -> 10.5; random layers of at most nine products 1.1 to 2.7 times shorter, the same distance
 // from 64 bits (3e-8 to 7e-8). Longer sums are bound by vector instructions, 2 K multiply-adds for 8 bytes: 16x12x129x129 -> 86, 1x1
 // s2 17.7 -> 20.8, 11x16x51x167 -> 66, 1x1 18.6 -> 19.4; they stay.
@@ -19,7 +19,7 @@ using namespace sofie;
 namespace {
 
 constexpr unsigned OUTSIDE = 0x40000000u;      // no descriptor of this file reaches it
-constexpr int MAX_K = 9, PIXELS = 2;
+constexpr int MAX_K = 9;
 
 struct ShortArgs {
    const float *x, *w, *bias;
@@ -34,7 +34,8 @@ struct ShortArgs {
    } tap[MAX_K];
 };
 
-template <int K>
+// THROUGH: stores written through the L2
+template <int K, int PIXELS, bool THROUGH>
 __global__ void __launch_bounds__(256) k_conv_f32_short(ShortArgs g)
 {
    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -72,18 +73,19 @@ __global__ void __launch_bounds__(256) k_conv_f32_short(ShortArgs g)
       for (int j = 0; j < PIXELS; ++j) {
          if (g.bias) s[j] = __fadd_rn(s[j], b);
          if (g.relu) s[j] = s[j] > 0.0f ? s[j] : 0.0f;
-         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s[j]), yrs, (int)at[j], (int)channel, 0);
+         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s[j]), yrs, (int)at[j], (int)channel, THROUGH ? 17 : 0);      // sc0 sc1
       }
       channel += (unsigned)g.plane * 4u;
    }
 }
 
 template <int K>
-int launch(sofie_hip_ctx *ctx, const ShortArgs &g, int k, dim3 grid)
+int launch(sofie_hip_ctx *ctx, const ShortArgs &g, int k, int pixels, bool through, dim3 grid)
 {
    if constexpr (K > 1)
-      if (k < K) return launch<K - 1>(ctx, g, k, grid);
-   hipLaunchKernelGGL(k_conv_f32_short<K>, grid, dim3(256), 0, ctx->stream, g);
+      if (k < K) return launch<K - 1>(ctx, g, k, pixels, through, grid);
+   const auto kern = pixels == 4 ? (through ? k_conv_f32_short<K, 4, true> : k_conv_f32_short<K, 4, false>) : (through ? k_conv_f32_short<K, 2, true> : k_conv_f32_short<K, 2, false>);
+   hipLaunchKernelGGL(kern, grid, dim3(256), 0, ctx->stream, g);
    return check_launch(ctx, "k_conv_f32_short");
 }
 
@@ -104,14 +106,20 @@ int sofie::conv_f32_short(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    const long per = (long)(room / (image > out_image ? image : out_image)), plane = (long)f.OH * f.OW;
    const long n_launch = per < p.N ? per : p.N;
    ShortArgs g{};
-   const long blocks = cdiv((int)(n_launch * plane), 256 * PIXELS);
+   // (weights and addresses are shared by twice the outputs: with both 256x1x40x40 -> 32, 3x3 17.9 -> 15.0 us; four on fewer pixels 58x1x22x22 -> 58, 3x3
+   // 7.4 -> 10.6.) Four pixels per lane where eight channels at a time leave six workgroups for a compute unit, else two
+   const int pixels = cdiv((int)(n_launch * plane), 1024) * p.groups * (long)cdiv(ocg, 8) >= 6l * ctx->num_cus ? 4 : 2;
+   // written through the L2s where a store is whole 64-byte pieces and the end of the kernel would be their write-back: 139x1x9x64 -> 48, 3x3 (15 MB) 9.4 -> 8.8,
+   // 16x1x62x56 -> 34, 1x1 (7.6 MB) 4.9 -> 5.6; planes of other sizes 133x1x130x130 -> 60, 3x3 162 -> 262
+   const bool through = plane % 16 == 0 && out_image * p.N >= ((size_t)14 << 20) && (reinterpret_cast<uintptr_t>(p.y) & 63u) == 0;
+   const long blocks = cdiv((int)(n_launch * plane), 256 * pixels);
    g.ocb = 64;
    while (g.ocb > 8 && blocks * p.groups * cdiv(ocg, g.ocb) < 6l * ctx->num_cus) g.ocb /= 2;
    g.oblocks = cdiv(ocg, g.ocb);
    if ((long)p.groups * g.oblocks > 65535) return SOFIE_HIP_OK;
    // outputs at 4 TB/s; vector instructions of a wavefront, four cycles each: the window's, and per channel its multiply-adds and stores
    const double bytes = 4.0 * plane * p.N * p.OC / 4e6;
-   const double waves = (double)plane * p.N / (64.0 * PIXELS);
+   const double waves = (double)plane * p.N / 128.0;
    const double valu = waves * (p.groups * g.oblocks * (40.0 + 16.0 * k) + p.OC * (2.0 * k + 10.0)) * 4.0 / (4.0 * ctx->num_cus) / 2100.0;
    const double us = 3.0 + (bytes > valu ? bytes + 0.3 * valu : valu + 0.3 * bytes);
    if (us >= other_us) return SOFIE_HIP_OK;
@@ -133,7 +141,7 @@ int sofie::conv_f32_short(sofie_hip_ctx *ctx, const ConvProblem &p, double other
       g.xbytes = (unsigned)(n * image);
       g.ybytes = (unsigned)(n * out_image);
       g.P = (int)(n * plane);
-      if (int rc = launch<MAX_K>(ctx, g, k, dim3((unsigned)cdiv(g.P, 256 * PIXELS), (unsigned)(p.groups * g.oblocks)))) return rc;
+      if (int rc = launch<MAX_K>(ctx, g, k, pixels, through, dim3((unsigned)cdiv(g.P, 256 * pixels), (unsigned)(p.groups * g.oblocks)))) return rc;
    }
    *done = true;
    return SOFIE_HIP_OK;

@@ -36,6 +36,7 @@ CONV = [
     (150, 2, 47, 33, 90, 2, 2, (1, 1), (1, 1, 1, 1), (1, 1), 1),
     (3000, 1, 3, 7, 129, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),       # a wavefront's pixels on many images
     (2, 9, 301, 303, 100, 1, 1, (1, 1), (0, 0, 0, 0), (1, 1), 1),
+    (8, 1, 64, 64, 165, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),        # two pixels per lane (four above), stores through the L2
 ]
 
 
