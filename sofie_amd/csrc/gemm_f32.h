@@ -96,8 +96,10 @@ struct SplitChoice {
    int mi, splits;
    float us;
 };
-// The form with the shortest estimate; us = 1e30 where the kernel does not take the product.
+// The form with the shortest estimate; us = 1e30 where the kernel does not take the product. mi = 8 (gemm_f32_shared_choice): tiles of 128 x 128 whose
+// operands are split once for all wavefronts.
 SplitChoice gemm_f32_split_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, bool one_launch);
+SplitChoice gemm_f32_shared_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz);
 int launch_gemm_f32_split(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, const SplitChoice &c);
 
 }  // namespace sofie

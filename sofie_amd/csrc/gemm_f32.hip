@@ -777,6 +777,11 @@ GeneralChoice general_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, uns
    // (operands as three bf16 numbers on the bf16 matrix instructions: 1500 x 1001 x 1111 29 us, 33 on 32 x 64 tiles)
    const SplitChoice split = gemm_f32_split_choice(ctx, g, nz, one_launch);
    consider(SPLIT, split.mi, 4, split.splits, split.us);
+   // (in place of the fp32 instructions: 5938 x 7616 x 728, both transposed, 605 us, 423; 5776 x 1195 x 400 59, 49)
+   if (best.kernel != SPLIT) {
+      const SplitChoice shared = gemm_f32_shared_choice(ctx, g, nz);
+      consider(SPLIT, shared.mi, 4, shared.splits, shared.us);
+   }
    if (g.K >= 4 && best.us >= 1e30f) consider_direct();
    return best;
 }
@@ -885,7 +890,7 @@ extern "C" int sofie_hip_gemm_f32(sofie_hip_ctx *ctx, int transA, int transB, in
       const int per_cu = cdiv(tiles, ctx->num_cus);
       const TileCost &t = small ? kTileCosts[3] : kTileCosts[5];
       const float us = 2.0f + (per_cu == 1 ? t.alone : (float)per_cu * t.among) * steps;
-      split = us >= 24.0f && gemm_f32_split_choice(ctx, g, 1, true).us < us;
+      split = us >= 24.0f && (gemm_f32_split_choice(ctx, g, 1, true).us < us || gemm_f32_shared_choice(ctx, g, 1).us < us);
    }
    if (dma && !split) {
       constexpr auto kern_nk2 = k_gemm_f32_dma<false, 2>, kern_kn2 = k_gemm_f32_dma<true, 2>;

@@ -306,6 +306,265 @@ __global__ void __launch_bounds__(WAVES * 64, 2) k_gemm_f32_split(GemmF32Args g)
    }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// 64 rows of one operand (KM: columns of it), 32 k at a time: what a lane of a wavefront asks for and makes of it. Eight requests of 16 bytes;
+// four fragments of 16 rows. The lane's k are 4 kg .. + 3 and 16 + 4 kg .. + 3, as above; KM: fragment e is every fourth column.
+template <bool KM>
+struct SplitRows {
+   static constexpr unsigned OUTSIDE = 0x80000000u;
+   const float *base;
+   __amdgpu_buffer_rsrc_t rs;
+   unsigned voff[KM ? 1 : 4], ld4;
+   int ld, K, width, kg4;
+   __device__ __forceinline__ void init(const float *p, int ld_, int first, int count, int K_, int lane)
+   {
+      ld = ld_;
+      ld4 = (unsigned)ld_ * 4u;
+      K = K_;
+      kg4 = 4 * (lane >> 4);
+      // (a group that begins behind the matrix: copies of the last rows, sums that nobody stores)
+      const int r16 = lane & 15, there = count - first;
+      if constexpr (KM) {
+         // the last four columns may begin in front of the group: offsets count from the group's start or one group earlier
+         const int from = first > 0 ? (there >= 4 ? first - 4 : count - 4) : 0;
+         base = p + from;
+         width = count - from;
+         const int c = first + 4 * r16;
+         voff[0] = (unsigned)((c < count - 4 ? c : count - 4) - from) * 4u + (unsigned)kg4 * ld4;
+      } else {
+         const int from = there > 0 ? first : count - 1, rows = there > 0 ? (there < 64 ? there : 64) : 1;
+         base = p + (size_t)from * ld;
+         rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, (int)((unsigned)(rows - 1) * ld4 + (unsigned)K * 4u), 0x00020000);
+#pragma unroll
+         for (int f = 0; f < 4; ++f) voff[f] = (unsigned)(16 * f + r16 < rows ? 16 * f + r16 : rows - 1) * ld4;
+      }
+   }
+   // Rows of k behind K arrive as zeros; four k along a row are moved down to end with K, or outside (trim puts them right).
+   __device__ __forceinline__ void request(v4f (&q)[8], int k0)
+   {
+      if constexpr (KM) {
+         const int rows = K - k0 < CH ? K - k0 : CH;
+         rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + (rows > 0 ? (size_t)k0 * ld : 0)), 0, rows > 0 ? (int)((unsigned)(rows - 1) * ld4 + (unsigned)width * 4u) : 0, 0x00020000);
+#pragma unroll
+         for (int u = 0; u < 8; ++u)
+            q[u] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(voff[0] + (unsigned)((u & 3) + 4 * (u & 4)) * ld4), 0, 0));
+      } else {
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            const int k = k0 + 16 * h + kg4;
+            const unsigned at = k < K - 4 ? (unsigned)k * 4u : k < K ? (unsigned)(K - 4) * 4u : OUTSIDE;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) q[2 * f + h] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(voff[f] + at), 0, 0));
+         }
+      }
+   }
+   __device__ __forceinline__ void trim(v4f (&q)[8], int k0) const
+   {
+      if constexpr (!KM) {
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            const int k = k0 + 16 * h + kg4, over = k < K ? k - (K - 4) : 0;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+               v4f &r = q[2 * f + h];
+               if (over > 0) {
+                  if (over & 1) { r[0] = r[1]; r[1] = r[2]; r[2] = r[3]; }
+                  if (over & 2) { r[0] = r[2]; r[1] = r[3]; }
+               }
+#pragma unroll
+               for (int e = 0; e < 4; ++e) r[e] = k + e < K ? r[e] : 0.0f;
+            }
+         }
+      }
+   }
+   // value e (of eight) of fragment f
+   static __device__ __forceinline__ float value(const v4f (&q)[8], int f, int e) { return KM ? q[e][f] : q[2 * f + (e >> 2)][e & 3]; }
+};
+
+// Tiles of 128 x 128, four wavefronts of 4 x 4 tiles of 16 x 16: an operand of the tile is split once, for all wavefronts, into fragments in LDS (48 KB a
+// chunk of 32 k, read without conflicts as they lie). A wavefront reads the chunk's eight fragments into registers; behind a barrier it multiplies them and
+// meanwhile splits the 64 rows it has requested of the next chunk into the same LDS. Two workgroups share a compute unit: one reads while
+// the other multiplies.
+template <bool A_KM, bool B_KM>
+__global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
+{
+   constexpr int BM = 128, BN = 128;
+   extern __shared__ __align__(16) unsigned char smem_raw[];
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int kg = lane >> 4, r16 = lane & 15, wm = wave >> 1, wn = wave & 1;
+   if (g.n_lead > 0) select_product(g, (long long)blockIdx.z + g.z0);
+   int tm, tn;
+   tile_of(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
+   const int m0 = tm * BM, n0 = tn * BN;
+   int k_begin = 0, k_end = g.K;
+   if (gridDim.y > 1) {      // K in slices: raw sums into the slice's plane of the scratch buffer
+      const int chunks = (g.K + CH - 1) / CH, per = (chunks + (int)gridDim.y - 1) / (int)gridDim.y;
+      k_begin = (int)blockIdx.y * per * CH;
+      k_end = k_begin + per * CH < g.K ? k_begin + per * CH : g.K;
+      g.Y = g.partial + (size_t)blockIdx.y * g.M * g.N;
+      g.ldy = g.N;
+      g.alpha = 1.0f;
+      g.bias_kind = SOFIE_BIAS_NONE;
+      g.relu = 0;
+   }
+   const bool ragged = (g.K & 3) != 0;
+   v4f acc[4][4];
+#pragma unroll
+   for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+   // fragments [A 0 .. 7, B 0 .. 7][h, m, l][lane]
+   v4i *const mine = reinterpret_cast<v4i *>(smem_raw) + wave * 4 * 192 + lane;
+   const v8b *const from_a = reinterpret_cast<const v8b *>(smem_raw) + wm * 4 * 192 + lane, *const from_b = reinterpret_cast<const v8b *>(smem_raw) + (8 + wn * 4) * 192 + lane;
+   auto run = [&](auto rows) {
+      typedef decltype(rows) Rows;
+      v4f q[8];
+      v4i part[3];
+      float r0, r1;
+      // two of a fragment's eight values, a few instructions at a time
+      auto pair = [&](int f, int p, int stage) {
+         switch (stage) {
+         case 0:
+            r0 = __fmul_rn(Rows::value(q, f, 2 * p), 65536.0f);
+            r1 = __fmul_rn(Rows::value(q, f, 2 * p + 1), 65536.0f);
+            part[0][p] = (int)f32x2_to_bf16x2(r0, r1);
+            break;
+         case 1: case 3:
+            r0 -= __uint_as_float((unsigned)part[stage >> 1][p] << 16);
+            r1 -= __uint_as_float((unsigned)part[stage >> 1][p] & 0xffff0000u);
+            break;
+         case 2: case 4: part[stage >> 1][p] = (int)f32x2_to_bf16x2(r0, r1); break;
+         }
+      };
+      auto put = [&](int f) {
+#pragma unroll
+         for (int t = 0; t < 3; ++t) mine[(f * 3 + t) * 64] = part[t];
+      };
+      rows.request(q, k_begin);
+      if (ragged && k_begin + CH > g.K) rows.trim(q, k_begin);
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+#pragma unroll
+         for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int t = 0; t < 5; ++t) pair(f, p, t);
+         put(f);
+      }
+      rows.request(q, k_begin + CH < k_end ? k_begin + CH : g.K);
+      for (int k0 = k_begin; k0 < k_end; k0 += CH) {
+         __syncthreads();
+         v8b a[4][3], b[4][3];
+#pragma unroll
+         for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+               a[i][t] = from_a[(i * 3 + t) * 64];
+               b[i][t] = from_b[(i * 3 + t) * 64];
+            }
+         wait_lds_reads();
+         __builtin_amdgcn_s_barrier();
+         asm volatile("" ::: "memory");
+         const int next = k0 + CH;
+         if (ragged && next < k_end && next + CH > g.K) rows.trim(q, next);
+         __builtin_amdgcn_sched_barrier(0);
+         v4f t, before;
+#pragma unroll
+         for (int n = 0; n < 16; ++n) {
+            const int i = n / 4, j = n % 4;
+            constexpr int A[6] = {0, 2, 1, 1, 0, 0}, B[6] = {2, 0, 1, 0, 1, 0};
+            t = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < 6; ++m) {
+               t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j][B[m]], a[i][A[m]], t, 0, 0, 0);
+               if (m < 5) pair(n / 4, n % 4, m);      // of the next chunk, under this one's matrix instructions
+               __builtin_amdgcn_sched_barrier(0);
+               if (n > 0 && m >= 1 && m < 5) acc[(n - 1) / 4][(n - 1) % 4][m - 1] = __fadd_rn(acc[(n - 1) / 4][(n - 1) % 4][m - 1], before[m - 1]);
+               __builtin_amdgcn_sched_barrier(0);
+            }
+            before = t;
+            if (n % 4 == 3) put(n / 4);
+            if (n == 15) rows.request(q, next + CH < k_end ? next + CH : g.K);
+            __builtin_amdgcn_sched_barrier(0);
+         }
+#pragma unroll
+         for (int e = 0; e < 4; ++e) acc[3][3][e] = __fadd_rn(acc[3][3][e], before[e]);
+      }
+   };
+   if (wave < 2) {
+      SplitRows<A_KM> rows;
+      rows.init(g.A, g.lda, m0 + wave * 64, g.M, g.K, lane);
+      run(rows);
+   } else {
+      SplitRows<B_KM> rows;
+      rows.init(g.B, g.ldb, n0 + (wave - 2) * 64, g.N, g.K, lane);
+      run(rows);
+   }
+
+   // sums that are not finite: again, by this wavefront from the operands as they are
+   v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+   for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+         for (int e = 0; e < 4; ++e) {
+            acc[i][j][e] = __fmul_rn(acc[i][j][e], UNSCALE);
+            none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
+         }
+   const int m1 = m0 + wm * 64, n1 = n0 + wn * 64;
+   if (__builtin_amdgcn_ballot_w64((none[0] + none[1]) + (none[2] + none[3]) != 0.0f) != 0) {
+      SplitRows<A_KM> ra;
+      SplitRows<B_KM> rb;
+      ra.init(g.A, g.lda, m1, g.M, g.K, lane);
+      rb.init(g.B, g.ldb, n1, g.N, g.K, lane);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+         for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+      for (int k0 = k_begin; k0 < k_end; k0 += CH) {
+         v4f qa[8], qb[8];
+         ra.request(qa, k0);
+         rb.request(qb, k0);
+         if (ragged && k0 + CH > g.K) {
+            ra.trim(qa, k0);
+            rb.trim(qb, k0);
+         }
+#pragma unroll
+         for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+               for (int j = 0; j < 4; ++j)
+                  acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(SplitRows<B_KM>::value(qb, j, e), SplitRows<A_KM>::value(qa, i, e), acc[i][j], 0, 0, 0);
+      }
+   }
+   // a quad is four consecutive columns of a row: with B along N element q of the four tiles
+#pragma unroll
+   for (int q = 0; q < 4; ++q) {
+      int n = n1 + (B_KM ? 16 * kg + 4 * q : 16 * q + 4 * kg);
+      if (n >= g.N) continue;
+      if constexpr (B_KM) n = n < g.N - 4 ? n : g.N - 4;
+      const v4f bias = bias_row4(g, n);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+         int m = m1 + (A_KM ? 4 * r16 : 16 * i + r16);
+         if (m >= g.M) continue;
+         if constexpr (A_KM) m = (m < g.M - 4 ? m : g.M - 4) + i;
+         const v4f v = B_KM ? v4f{acc[i][0][q], acc[i][1][q], acc[i][2][q], acc[i][3][q]} : acc[i][q];
+         store4(g, finish4(g, v, bias, m, n), m, n);
+      }
+   }
+}
+
+template <bool A_KM, bool B_KM>
+int launch_shared(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, int splits)
+{
+   constexpr auto kern = k_gemm_f32_split_shared<A_KM, B_KM>;
+   hipLaunchKernelGGL(kern, dim3(cdiv(g.M, 128) * cdiv(g.N, 128), splits, nz), dim3(256), 16 * 3072, ctx->stream, g);
+   return check_launch(ctx, "k_gemm_f32_split_shared");
+}
+
 template <bool A_KM, bool B_KM, int MI>
 int launch(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, int splits)
 {
@@ -341,8 +600,26 @@ SplitChoice sofie::gemm_f32_split_choice(const sofie_hip_ctx *ctx, const GemmF32
    return best;
 }
 
+// Tiles of 128 x 128 in one piece, two workgroups to a compute unit: 1.39 us a chunk of each, 8 us around two of them (alone 1.75 and 5). In place of the fp32
+// instructions alone, whose sums are further off: the eight wavefronts above have eight shorter sums (993 products 8.2e-8 off 64 bits, here 1.2e-7, 2000 9.6e-8
+// and 1.6e-7, fp32 instructions 3e-7 and more), and so they keep what they take, though it is the longer way on large products (4096^3 800
+// us, 710 here; 4000 x 4001 x 1002 268, 194). With slices of K this is slow (1500 x 1001 x 1111 44 us: a prologue for seven chunks).
+SplitChoice sofie::gemm_f32_shared_choice(const sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz)
+{
+   const SplitChoice none = {0, 1, 1e30f};
+   auto offsets_fit = [](bool km, int ld) { return (long long)(km ? 32 : 64) * ld * 4 < (1ll << 30); };
+   if (g.K < 64 || g.M < 4 || g.N < 4 || g.bias_kind == SOFIE_BIAS_FULL || !offsets_fit(!g.transB, g.ldb) || !offsets_fit(g.transA, g.lda)) return none;
+   const int cus = ctx->num_cus, chunks = cdiv(g.K, CH);
+   const long long tiles = (long long)cdiv(g.M, 128) * cdiv(g.N, 128), per_cu = (tiles * nz + cus - 1) / cus;
+   if (tiles >= (1ll << 32) / 256) return none;
+   return {8, 1, per_cu == 1 ? 8.0f + 1.75f * chunks : 3.0f + 8.0f * (float)((per_cu + 1) / 2) + 1.39f * (float)per_cu * chunks};
+}
+
 int sofie::launch_gemm_f32_split(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, const SplitChoice &c)
 {
+   if (c.mi == 8)
+      return g.transA ? (g.transB ? launch_shared<true, false>(ctx, g, nz, c.splits) : launch_shared<true, true>(ctx, g, nz, c.splits))
+                      : (g.transB ? launch_shared<false, false>(ctx, g, nz, c.splits) : launch_shared<false, true>(ctx, g, nz, c.splits));
    if (g.transA) return g.transB ? launch<true, false, 4>(ctx, g, nz, c.splits) : launch<true, true, 4>(ctx, g, nz, c.splits);
    switch (c.mi) {
    case 2: return g.transB ? launch<false, false, 2>(ctx, g, nz, c.splits) : launch<false, true, 2>(ctx, g, nz, c.splits);

@@ -127,3 +127,33 @@ def test_magnitudes_of_all_sizes_keep_their_bits(ops, tA, tB, e, f):
     a, b = (a.t() if tA else a).double().contiguous(), (b.t() if tB else b).double().contiguous()
     assert bool(((y.double() - a @ b).abs() <= 2.0 ** -21 * (a.abs() @ b.abs()) + K * 2.0 ** -149).all())
     ctx.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(2710, 5088, 336), (2711, 5089, 337), (3185, 2559, 726), (5043, 4527, 451)])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_in_three_parts_on_shared_fragments(ops, M, N, K, tA, tB):
+    """Tiles of 128 x 128 whose operands are split once for all wavefronts, whole ones and cut in all directions: bounds as above; an infinity, a NaN and
+    sums that overflow stay where fp32 products put them, and sums next to them keep 2^-24 of each of K products, which add as their square root."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g) * K ** -0.5
+    bias = torch.randn(N, device="cuda", generator=g)
+    stored = lambda x, y: (x.t().contiguous() if tA else x, y.t().contiguous() if tB else y)
+    ctx = ops.Context(0)
+    y, names = product(ctx, *stored(a, b), tA, tB, bias, pad=3)
+    assert names == ["k_gemm_f32_split_shared"], names
+    want = a.double() @ b.double() + bias.double()
+    err = y.double() - want
+    assert float(err.norm()) <= 3e-7 * float(want.norm()) and float(err.abs().max()) <= 1e-6 * float(want.abs().max())
+    a[3, 7], a[M - 1, K - 1], a[200, 0] = float("inf"), float("nan"), 3.4e38
+    b[0, N - 1] = 1000.0
+    y, names = product(ctx, *stored(a, b), tA, tB, None)
+    assert names == ["k_gemm_f32_split_shared"], names
+    rows = [0, 3, 63, 64, 127, 128, 199, 200, M - 5, M - 2, M - 1]
+    ad, bd = a[rows].double(), b.double()
+    ref = ad @ bd
+    ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * float("inf"), ref)
+    got = y[rows].double()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    fin = ref.isfinite()
+    assert bool(((got - ref).abs()[fin] <= (K ** 0.5 * 2.0 ** -24 * (ad.nan_to_num(0.0, 0.0, 0.0).abs() @ bd.abs()))[fin]).all())
+    ctx.close()
