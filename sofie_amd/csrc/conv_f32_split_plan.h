@@ -7,7 +7,8 @@
 // same sizes. us of a call on the host without its launches, every form laid out for up to 16 strips / now / without this kernel (2.7 GHz):
 // 256x64x56x56 -> 128, 3x3 6.4 / 2.4 / 0.7; 1x128x56x56 -> 128, 3x3, which k_conv_f32_any takes, 5.9 / 1.3 / 0.7; transposed 1x111x25x25 -> 192,
 // 4x4 s2, taken by it, too, 26 / 2.8 / 1.2, and 17.6 us a call on the device for 11.0 of the kernel; 300 random layers 1.5 / 0.73 / 0.50 in the
-// mean, 17 / 3.2 / 1.3 at most.
+// mean, 17 / 3.2 / 1.3 at most. Slots of 8 channels add 0.55 to strided layers (2000 random ones, with the transposed), the form with a phase per
+// wavefront 0.53 to transposed ones (2.6 without the bound, with the strips laid out for each form again; 10.3 and 3.6 at most).
 #pragma once
 #include <cmath>
 
@@ -81,6 +82,7 @@ struct SplitPlan {
          wofs[i] = pieces;
          pieces += (size_t)p.groups * octiles * steps[i] * 192;
       }
+      for (Strips &s : strips_seen) s.seen = 0;
    }
 
    // Whether four pixels are stored at once.
@@ -127,7 +129,6 @@ struct SplitPlan {
       static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
       Form best{0, 0, 0, 0, 0, other_us};
       if (pieces * 16 > ((size_t)1 << 29)) return best;
-      for (Strips &s : strips_seen) s.seen = 0;
       for (int k = 0; k < kinds; ++k)
          for (int t = 0; t < 3; ++t) least_cells[t][k] = cells_at_least(p.phase[kind[k]], 64 << t);
       // what may be the shortest first
@@ -215,9 +216,11 @@ struct SplitPlan {
          Form form{f[0], f[1], f[2], 8, 0, 0.0};
          if (least_cells[tile_of(form)][0] > cells_of(form) || least_time(form, n, cus) >= best.time) continue;
          form.time = HUGE_VAL;
+         Strips &s = strips_seen[tile_of(form)];
          for (int strips = 1; strips <= MAX_STRIPS; ++strips) {
-            Panels q;
-            if (!panels(q, 0, form.pixels(), strips) || q.cells > cells_of(form)) continue;
+            if (strips > s.seen) look_at(s, form.pixels(), strips);
+            const Panels &q = s.panels[strips - 1][0];
+            if (s.cells[strips - 1] == 0 || q.cells > cells_of(form)) continue;
             if (table_bytes(8) + 2 * (long)slot_bytes(q.cells, 8) > MAX_LDS || (double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
             if (form.ti == 4 && form.tj == 2 && !quads(q.strips)) continue;
             const double time = estimate(form, &q, n, cus) * (strips > 1 ? 1.02 : 1.0);
@@ -275,21 +278,30 @@ struct SplitPlan {
       one_for_all = true;
       chunks[0] = 4 * most;      // (of the tables of offsets, one for each phase)
       steps[0] = (all + 3) / 4;
+      least_cells[0][0] = cells_at_least(p.phase[0], 64);
+      Strips &s = strips_seen[0];      // (all these forms have tiles of 64)
       for (const auto &f : forms) {
          if (f[0] > 1 && f[0] - 1 >= octiles) continue;      // tiles of nothing
          for (int cs = 16; cs <= 32; cs *= 2) {
             // every wavefront comes to the same barriers: steps end with slots, or all alike
             bool fits = true;
             for (int i = 0; i < 4; ++i) fits = fits && (slots(cs) == 1 || (cs / 8 * apart.chunks[i] >= 4 && (even || cs / 8 * apart.chunks[i] % 4 == 0)));
-            for (int strips = 1; fits && strips <= MAX_STRIPS; ++strips) {
-               Form form{f[0], f[1], TOGETHER, cs, strips, 0.0};
-               Panels q;
+            Form form{f[0], f[1], TOGETHER, cs, 0, 0.0};
+            if (!fits || least_cells[0][0] > cells_of(form) || least_time(form, n, cus) >= best.time) continue;
+            form.time = HUGE_VAL;
+            for (int strips = 1; strips <= MAX_STRIPS; ++strips) {
+               if (strips > s.seen) look_at(s, form.pixels(), strips);
+               const Panels &q = s.panels[strips - 1][0];
                // (strips of a few columns: 192x224x13x13 -> 170, 2x2 s2 on strips of one 141 us, 106 apart)
-               if (!panels(q, 0, form.pixels(), strips) || q.cells > cells_of(form) || (strips > 1 && q.ws < 8)) continue;
+               if (strips > 1 && q.ws < 8) break;
+               if (s.cells[strips - 1] == 0 || q.cells > cells_of(form)) continue;
                if (table_bytes(cs) + (slots(cs) > 1 ? 2 : 1) * (long)slot_bytes(q.cells, cs) > MAX_LDS || (double)n * q.strips * q.PHW > (double)(1 << 30)) continue;
-               form.time = estimate(form, &q, n, cus) * (strips > 1 ? 1.02 : 1.0);
-               if (form.time < best.time) best = form;
+               const double time = estimate(form, &q, n, cus) * (strips > 1 ? 1.02 : 1.0);
+               if (time >= form.time) continue;
+               form.time = time;
+               form.strips = strips;
             }
+            if (form.strips > 0 && form.time < best.time) best = form;
          }
       }
       return best;

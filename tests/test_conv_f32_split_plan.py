@@ -93,3 +93,90 @@ def test_the_choice_of_a_full_search_with_few_estimates(tmp_path):
     layers, taken, estimates, without, most = map(int, out.stdout.split())
     assert layers == 3000 and taken > 1000
     assert estimates <= 6 * layers and most <= 50 and without >= 4 * estimates, out.stdout
+
+
+STRIDES = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "conv_f32_split_plan.h"
+using namespace sofie;
+
+// every form, slot and row of strips; apart: the plan of the four phases, nullptr for slots of eight channels of a strided layer
+static double search(SplitPlan &plan, const SplitPlan *apart, size_t n, double other_us)
+{
+   double best = other_us;
+   for (int ti = 1; ti <= 4; ++ti)
+      for (int tj = 2; tj <= 4; tj += 2)
+         for (int cs = apart ? 16 : 8; cs <= (apart ? 32 : 8); cs *= 2) {
+            SplitPlan::Form form{ti, tj, apart ? SplitPlan::TOGETHER : 2, cs, 0, 0.0};
+            if ((apart && tj == 2) || (!apart && ti == 3 && tj == 2) || (ti > 1 && form.beside() * (ti - 1) >= plan.octiles)) continue;
+            bool fits = true, even = true;
+            for (int i = 0; apart && i < 4; ++i) even = even && apart->chunks[i] == apart->chunks[0];
+            for (int i = 0; apart && i < 4; ++i) {
+               const int chunks = cs / 8 * apart->chunks[i];
+               fits = fits && (plan.slots(cs) == 1 || (chunks >= 4 && (even || chunks % 4 == 0)));
+            }
+            if (!fits || (!apart && plan.chunks[0] < 4)) continue;
+            double least = HUGE_VAL;
+            for (int strips = 1; strips <= 16; ++strips) {
+               SplitPlan::Panels q;
+               if (!plan.panels(q, 0, form.pixels(), strips) || q.cells * (cs / 8) > SplitPlan::items_of(ti, tj, form.wo, false) * SplitPlan::THREADS) continue;
+               if (apart && strips > 1 && q.ws < 8) continue;
+               if (plan.table_bytes(cs) + (apart && plan.slots(cs) == 1 ? 1 : 2) * SplitPlan::slot_bytes(q.cells, cs) > SplitPlan::MAX_LDS) continue;
+               if (!apart && ti == 4 && tj == 2 && !plan.quads(q.strips)) continue;
+               const double time = plan.estimate(form, &q, n, 256) * (strips > 1 ? 1.02 : 1.0);
+               if (time < least) least = time, form.strips = strips;
+               else if (!apart && strips > form.strips + 1) break;
+            }
+            if (least < best) best = least;
+         }
+   return best;
+}
+
+int main()
+{
+   srand(9);
+   auto pick = [](int lo, int hi) { return lo + rand() % (hi - lo + 1); };
+   long layers = 0, taken[2] = {0, 0}, estimates = 0, without = 0;
+   while (layers < 2000) {
+      ConvProblem p{};
+      const int k = pick(2, 5);
+      const bool up = k < 5 && (k != 3 || rand() % 2);      // transposed, 2x2, 3x3 and 4x4 of stride 2, or 3x3 and 5x5 of stride 2
+      const int pad = (k - 1) / 2;
+      p.N = 1 << pick(0, 8), p.C = pick(16, 260), p.OC = pick(8, 260), p.groups = 1;
+      p.H = pick(5, 80), p.W = rand() % 2 ? p.H : pick(5, 100);
+      p.dh = p.dw = 1, p.KH0 = p.KW0 = k, p.transposed = up, p.nphases = up ? 4 : 1, p.sh = p.sw = up ? 1 : 2;
+      p.OH0 = up ? 2 * (p.H - 1) + k - 2 * pad : (p.H + 2 * pad - k) / 2 + 1;
+      p.OW0 = up ? 2 * (p.W - 1) + k - 2 * pad : (p.W + 2 * pad - k) / 2 + 1;
+      if ((double)p.N * p.C * p.H * p.W > (1 << 27) || (double)p.N * p.OC * p.OH0 * p.OW0 > (1 << 27)) continue;
+      for (int i = 0; i < p.nphases; ++i) {
+         const int a = i / 2, b = i % 2, z = k != 2;
+         if (!up) p.phase[i] = {p.OH0, p.OW0, k, k, pad, pad, 0, 1, 0, 1, 0, 1, 0, 1};
+         else p.phase[i] = {(p.OH0 + 1 - a) / 2, (p.OW0 + 1 - b) / 2, k == 4 ? 2 : 1 + z * a, k == 4 ? 2 : 1 + z * b, z * (1 - a), z * (1 - b), 0, 2, 0, 2, a, 2, b, 2};
+      }
+      const double other = 7.5 + rand() % 200;
+      ConvProblem u;
+      if (up && !SplitPlan::together(p, u)) return printf("layer %ld: not together\n", layers), 1;
+      SplitPlan apart(p, false), plan(up ? u : p, false);
+      const SplitPlan::Form form = up ? plan.choose_together(apart, p.N, 256, other) : plan.choose_eights(p.N, 256, other);
+      const long made = plan.evaluated;
+      const double best = search(plan, up ? &apart : nullptr, p.N, other);
+      if (form.time != best) return printf("layer %ld: %.17g, searched %.17g\n", layers, form.time, best), 1;
+      ++layers;
+      taken[up] += form.ti > 0;
+      estimates += made;
+      without += plan.evaluated - made;
+   }
+   printf("%ld %ld %ld %ld\n", taken[0], taken[1], estimates, without);
+}
+"""
+
+
+def test_strided_and_transposed_layers_by_a_full_search(tmp_path):
+    src, exe = tmp_path / "strides.cpp", tmp_path / "strides"
+    src.write_text(STRIDES)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "sofie_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    strided, transposed, estimates, without = map(int, out.stdout.split())
+    assert strided > 200 and transposed > 200 and 2 * estimates <= without, out.stdout
