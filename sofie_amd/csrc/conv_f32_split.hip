@@ -257,17 +257,18 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
    __builtin_amdgcn_sched_barrier(0);
    const int taps = q.KH * q.KW;
    int *const table = reinterpret_cast<int *>(smem_raw) + (TOGETHER ? phase * g.table_ints : 0);
+   const int ring = ROWS ? 2 * q.chunks : q.ring, down = TOGETHER ? q.down : 0, right = TOGETHER ? q.right : 0;
    // offset of every chunk of two slots, or of four (chunks behind K, whose weights are zeros, read what lies in the slot: where there is one, its
    // first chunks)
-   for (int e = TOGETHER ? lane : tid; e < q.ring; e += TOGETHER ? 64 : THREADS) {
-      const int slot = (e >= q.chunks) + (e >= 2 * q.chunks) + (e >= 3 * q.chunks), second = slot & 1, k = e - slot * q.chunks, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
+   for (int e = TOGETHER ? lane : tid; e < ring; e += TOGETHER ? 64 : THREADS) {
+      const int slot = (e >= q.chunks) + (ROWS ? 0 : (e >= 2 * q.chunks) + (e >= 3 * q.chunks)), second = slot & 1, k = e - slot * q.chunks, c8 = fdiv(k, q.dTaps), t = k - c8 * (ROWS ? q.KH : taps), a = ROWS ? t : fdiv(t, q.dKW), b = ROWS ? 0 : t - a * q.KW;
       table[e] = (c8 * q.cells + a * g.dh * q.PW + b * g.dw) * CELL + (g.nslots > 1 ? second * g.slot_bytes : 0);
    }
    int base[TJ];
 #pragma unroll
    for (int j = 0; j < TJ; ++j) {
       const int p = p0 + (wp * TJ + j) * 16 + r16, panel = fdiv(p, q.dPHW), r = p - panel * q.PHW, oy = fdiv(r, q.dWS), c = r - oy * q.ws;
-      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh + q.down - origin) * q.PW + (ROWS ? c : c * g.sw) + q.right) * CELL : 0;
+      base[j] = p < q.P && r < q.full ? ((panel * q.HP + oy * g.sh + down - origin) * q.PW + (ROWS ? c : c * g.sw) + right) * CELL : 0;
    }
    v4f acc[TI][TJ];
 #pragma unroll
@@ -310,7 +311,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
             for (int j = 0; j < TJ; ++j) read_x(j, off);
          }
-         place = place + 4 == q.ring ? 0 : place + 4;
+         place = place + 4 == ring ? 0 : place + 4;
          const int ahead = across ? end - 2 : end - 1;
          fresh = step >= ahead;
          const int off = table[(fresh ? 0 : place) + kg];
@@ -676,10 +677,11 @@ int sofie::conv_f32_split(sofie_hip_ctx *ctx, const ConvProblem &p, double other
    g.ocplane4 = (int)out_image;
    g.plane4 = p.OH0 * p.OW0 * 4;
    g.OW0 = p.OW0;
+   const bool eights = best.cs == 8 && !rows;
    for (size_t n0 = 0; n0 < (size_t)p.N; n0 += per) {
       const size_t n = (size_t)p.N - n0 < per ? (size_t)p.N - n0 : per;
       if (n != per) {
-         best = best.wo == SplitPlan::TOGETHER ? one.choose_together(plan, n, cus, HUGE_VAL) : best.cs == 8 ? plan.choose_eights(n, cus, HUGE_VAL) : plan.choose(n, cus, HUGE_VAL);
+         best = best.wo == SplitPlan::TOGETHER ? one.choose_together(plan, n, cus, HUGE_VAL) : eights ? plan.choose_eights(n, cus, HUGE_VAL) : plan.choose(n, cus, HUGE_VAL);
          prepare();
       }
       g.x = p.x + n0 * (image / 4);

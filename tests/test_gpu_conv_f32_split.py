@@ -157,6 +157,27 @@ def test_phases_of_one_workgroup(ops, kept, shape, large):
             assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())) and float(err.norm()) <= 3e-7 * float(ref.norm()), i
 
 
+@pytest.mark.parametrize("n,c,h,oc,k,s,up", [(300, 1, 96, 100, 7, 1, False), (230, 128, 99, 128, 3, 2, False), (1400, 128, 28, 64, 4, 2, True), (300, 32, 99, 96, 3, 1, False)])
+def test_images_of_more_than_a_launch(ops, kept, n, c, h, oc, k, s, up):
+    """Above 1 GiB of images: full launches and one of the rest, whose form is chosen anew (rows of a kernel as cells, slots of eight channels, all
+    phases by one workgroup, a plain layer); the images on both sides of the line, bound as above."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    pad = (k - 1) // 2
+    x, wt = torch.randn(n, c, h, h, device="cuda", generator=g), torch.randn(*((c, oc) if up else (oc, c)), k, k, device="cuda", generator=g) * (c * k * k) ** -0.5
+    torch.cuda.synchronize()
+    if up:
+        y, names = names_of(kept, lambda: ops.conv_transpose2d_f32(x, wt, None, (pad,) * 4, (s, s), (1, 1), 1, (0, 0), ctx=kept))
+    else:
+        y, names = names_of(kept, lambda: ops.conv2d_f32(x, wt, None, (pad,) * 4, (s, s), (1, 1), 1, ctx=kept))
+    assert names.count("k_conv_f32_split") == 2, names
+    per = ((1 << 30) - (16 << 20)) // (4 * max(x[0].numel(), y[0].numel()))
+    assert per < n < 2 * per
+    f = torch.nn.functional.conv_transpose2d if up else torch.nn.functional.conv2d
+    for i in (0, per - 1, per, n - 1):
+        ref = f(x[i:i + 1].cpu().double(), wt.cpu().double(), None, s, pad)
+        assert float((y[i:i + 1].cpu().double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
+
+
 @pytest.mark.parametrize("shape", CONV + [
     (64, 128, 28, 28, 64, 4, 2), (30, 143, 32, 34, 181, 4, 2), (120, 87, 19, 21, 256, 3, 2), (64, 120, 20, 20, 90, 3, 1)])      # transposed: k, stride
 def test_sums_that_are_repeated_in_every_form(ops, kept, shape):
