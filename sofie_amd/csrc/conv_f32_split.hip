@@ -57,12 +57,9 @@ struct SplitPhase {
    int P, PHW, panels;        // pixels, of a panel; panels (strips of images)
    int ws, strips;            // columns of a strip, strips of an image
    int KH, KW, ph, pw;
-   int down, right;           // where its taps begin in the patch, whose pads are ph and pw (a patch of several phases)
-   int OH;
    int HP, PW, cells;         // rows of a panel's input, cells of a row, of a tile's patch
    int full;                  // pixels of a panel that exist (PHW: up to whole tiles where tiles do not run on into the next panel)
    int chunks;                // of a slot: 8 channels of a tap each
-   int ring;                  // of two slots, or of four (an odd number of chunks): whole steps
    int steps;                 // of four chunks, all of K
    int wofs;                  // first 16-byte piece of the phase's fragments
    int OW;
@@ -70,6 +67,9 @@ struct SplitPhase {
    int th0, ths, tw0, tws;
    int tiles;                 // of a panel, where it is whole tiles and not the only one of its image: strips take turns; else 0
    FastDiv dTiles, dPHW, dWS, dHP, dPW, dStrips, dTaps, dKW, dCells;
+   int ring;                  // chunks of two slots, or of four (an odd number of chunks): whole steps
+   int down, right;           // TOGETHER: where its taps begin in the patch, whose pads are ph and pw
+   int OH;
 };
 
 struct SplitArgs {
@@ -82,10 +82,10 @@ struct SplitArgs {
    int octiles, oblocks;
    int chw4, hw4, ocplane4, plane4, OW0;
    int table_bytes, slot_bytes;      // LDS: table of offsets, two slots
-   int table_ints;            // TOGETHER: from one phase's table to the next one's
    int nphases;
    FastDiv dOB, dPhases;
    SplitPhase phase[MAX_PHASES];
+   int table_ints;            // TOGETHER: from one phase's table to the next one's
 };
 
 enum { PIXELS, QUADS };
