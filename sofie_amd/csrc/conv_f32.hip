@@ -292,6 +292,7 @@ __global__ void __launch_bounds__(256) k_conv2d_f32(ConvArgs g)
 template <int TI, int TJ, bool PHASES = false, int KWT = 0>
 __global__ void __launch_bounds__(256, TI == 1 ? 7 : 3) k_conv2d_f32_dma(ConvArgs gg)
 {
+   if constexpr (PHASES) ask_for_arguments<sizeof(gg)>();
    constexpr int BOC = 2 * TI * 32, BP = 2 * TJ * 32;
    constexpr int NP = SOFIE_CONV_DMA_PATCH / 256;
    constexpr int ROWS_PER_REQUEST = 1024 / BOC;       // weight rows one request of 256 lanes x 16 bytes covers

@@ -88,6 +88,7 @@ enum { PIXELS, QUADS, PAIRS };
 template <int TI, int TJ, int MODE, int STORE>
 __global__ void __launch_bounds__(512, TI * TJ >= 10 || (TI * TJ == 8 && STORE == PAIRS) ? 3 : 4) k_conv_f32_any(AnyArgs g)
 {
+   ask_for_arguments<sizeof(g)>();
    extern __shared__ __align__(16) unsigned char smem_raw[];
    constexpr int NH = STORE == PAIRS ? 2 : 1;
    constexpr bool PAD = MODE == TESTED, LOOK = MODE == LOOKED_UP;

@@ -38,6 +38,7 @@ struct ShortArgs {
 template <int K, int PIXELS, bool THROUGH>
 __global__ void __launch_bounds__(256) k_conv_f32_short(ShortArgs g)
 {
+   ask_for_arguments<sizeof(g)>();
    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
    const int grp = fdiv(blockIdx.y, g.dOB), oc0 = (blockIdx.y - grp * g.oblocks) * g.ocb;
    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.x), 0, (int)g.xbytes, 0x00020000);

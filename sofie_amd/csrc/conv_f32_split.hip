@@ -105,6 +105,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 {
    extern __shared__ __align__(16) unsigned char smem_raw[];
    constexpr bool TOGETHER = WO == SplitPlan::TOGETHER;
+   if constexpr (PHASES || TOGETHER) ask_for_arguments<sizeof(g)>();
    constexpr int BP = 4 / WO * TJ * 16, ITEMS = SplitPlan::items_of(TI, TJ, WO, ROWS);
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int r16 = lane & 15, kg = lane >> 4, wp = wave / WO, wo = TOGETHER ? 0 : wave % WO;

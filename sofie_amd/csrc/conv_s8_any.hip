@@ -300,6 +300,7 @@ __global__ void __launch_bounds__(256) k_qconv_any_weights(const int8_t *w, v4i 
 template <bool WHOLE>
 __global__ void __launch_bounds__(256) k_qconv_any_input(QConvArgs g, v4i *dst, int total, int HP, int WP, int cd, FastDiv dcd, FastDiv dWP, FastDiv dHP)
 {
+   ask_for_arguments<sizeof(g) + 48>();
    const int id = blockIdx.x * 256 + threadIdx.x;
    if (id >= total) return;
    const int p = fdiv(4 * id, dcd), R = fdiv(p, dWP), n = fdiv(R, dHP);
@@ -351,6 +352,7 @@ __global__ void __launch_bounds__(256) k_qconv_any_input(QConvArgs g, v4i *dst, 
 template <bool FLOAT>
 __global__ void __launch_bounds__(256) k_qconv_any_planes(QConvArgs g, unsigned *dst, int pixels, int HP, int WP, int cd, FastDiv dPixels, FastDiv dWP, FastDiv dHP)
 {
+   ask_for_arguments<sizeof(g) + 48>();
    const int id = blockIdx.x * 256 + threadIdx.x, k = fdiv(id, dPixels);
    if (k >= cd) return;
    const int p = id - k * pixels, R = fdiv(p, dWP), n = fdiv(R, dHP), c = p - R * WP - g.pw, r = R - n * HP - g.ph;

@@ -109,6 +109,7 @@ template <bool POOL>
 __global__ void __launch_bounds__(256, 4) k_qconv_first(FirstArgs a)
 {
    extern __shared__ __align__(16) unsigned char smem[];
+   ask_for_arguments<sizeof(a)>();
    const int OCP = a.ocb * 32;                                              // channels padded to blocks of 32
    float *const s_scale = reinterpret_cast<float *>(smem);                  // [OCP]
    int *const s_bias = reinterpret_cast<int *>(s_scale + OCP);              // [OCP]

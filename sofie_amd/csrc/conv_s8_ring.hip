@@ -585,6 +585,7 @@ template <int C16, int WN, bool ROWDMA, bool POOL>
 __global__ void __launch_bounds__(512) k_qconv_ring(QConvRingArgs a)
 {
    extern __shared__ __align__(16) unsigned char smem[];
+   ask_for_arguments<sizeof(a)>();
    qconv_ring_body<C16, WN, ROWDMA, POOL>(a, smem);
 }
 
@@ -598,6 +599,7 @@ __global__ void __launch_bounds__(512) k_qconv_ring(QConvRingArgs a)
 template <int C16A, bool POOLA, int WNB>
 __global__ void __launch_bounds__(512) k_qconv_ring_pair(QConvRingArgs a, QConvRingArgs b)
 {
+   ask_for_arguments<2 * sizeof(a)>();
    extern __shared__ __align__(16) unsigned char smem[];
    qconv_ring_body<C16A, 1, true, POOLA>(a, smem);
    wait_vmcnt<0>();

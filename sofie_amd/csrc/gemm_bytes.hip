@@ -977,6 +977,7 @@ struct CopyOperandsArgs {
 
 __global__ void __launch_bounds__(256) k_copy_operands(CopyOperandsArgs g)
 {
+   ask_for_arguments<sizeof(g)>();
    const int b = blockIdx.x - g.blocks_a;
    if (b < 0 || !g.kn) {
       const bool is_a = b < 0;
@@ -1103,6 +1104,7 @@ __device__ __forceinline__ v4i sum_slices(const int *__restrict__ p, size_t plan
 template <int OUT, bool MANY>
 __global__ void __launch_bounds__(256) k_splitk_finish(GemmArgs g, const int *__restrict__ P, int splits, int ldp)
 {
+   ask_for_arguments<sizeof(g) + 16>();
    const int quads = ldp >> 2;
    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
    if (t >= (size_t)g.M * quads) return;
@@ -1145,6 +1147,7 @@ template <int OUT2, int QUADS, bool MANY>
 __global__ void __launch_bounds__(256) k_splitk_finish_pair(GemmArgs g1, const int *__restrict__ P, int splits, int ldp, GemmArgs g2)
 {
    constexpr int quads = QUADS;
+   ask_for_arguments<2 * sizeof(GemmArgs) + 16>();
    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
    if (t >= (size_t)g1.M * quads) return;
    const int m = (int)(t / quads), c = (int)(t % quads), n = c * 4;

@@ -637,6 +637,7 @@ __global__ void __launch_bounds__(256) k_gemm_f32_skinny(GemmF32Args g, float *p
 // eight slices are in flight together; the additions keep the slices' order.
 __global__ void __launch_bounds__(256) k_gemm_f32_skinny_finish(GemmF32Args g, const float *__restrict__ partial, int splits)
 {
+   ask_for_arguments<sizeof(g)>();
    const int idx = blockIdx.x * 256 + threadIdx.x;
    if (idx >= g.M * g.N) return;
    const int m = idx / g.N, n = idx - m * g.N;
@@ -998,15 +999,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_f32(MlpArgs a)
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int c = lane & 15, kg = lane >> 4;
    const int row0 = blockIdx.x * ROWS;
-   {  // the arguments up to the fourth layer are asked for at once: read where a layer needs them they are a trip to memory each
-      constexpr int LINES = 3;
-      const int *const args = (const int *)__builtin_amdgcn_kernarg_segment_ptr();
-      int line[LINES];
-#pragma unroll
-      for (int i = 0; i < LINES; ++i) line[i] = args[16 * i];
-#pragma unroll
-      for (int i = 0; i < LINES; ++i) asm volatile("" : : "s"(line[i]));
-   }
+   ask_for_arguments<3 * 64>();      // up to the fourth layer
 
    // the next piece whose weights are requested: layer, unit (column tile and part), piece of K; and what its layer's pieces share
    int fl = -1, fu = 0, fp = 0, fK = 0, fN = 0, fsh = 0, funits = 0;
