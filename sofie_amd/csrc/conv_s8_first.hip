@@ -43,9 +43,10 @@ struct FirstArgs {
    FastDiv dper_image, dPW, dHW4, dW4;
    // how the coordinates of a work item move from one loop iteration to the next (the loops advance by a fixed
    // number of items, so no iteration divides): a staging thread moves on by 256 groups of four pixels, a
-   // wavefront by 128 (pooled) output pixels
+   // wavefront by 128 (pooled) output pixels times the workgroups that share these images
    int st_im, st_row, st_col;   // 256 = st_im * (H*W/4) + st_row * (W/4) + st_col
-   int px_im, px_row, px_col;   // 128 = px_im * (PH*PW) + px_row * PW + px_col
+   int px_im, px_row, px_col;
+   int px_step;                 // = px_im * (PH*PW) + px_row * PW + px_col
 };
 
 
@@ -102,7 +103,8 @@ __device__ __forceinline__ unsigned quantize4(v4f v, float scale, float inv, int
    }
 }
 
-template <bool POOL>
+// SHARED: gridDim.y workgroups share the pixels of the same images.
+template <bool POOL, bool SHARED>
 // Four workgroups per CU (at most 128 registers): the loop is a chain of dependent vector instructions per group of
 // pixels, and a fourth wavefront per SIMD fills the gaps the other three leave (25.4 us instead of 30.8 us for 4096
 // images of 40x40 with 32 channels and pooling; five workgroups need 102 registers and lose more than they gain).
@@ -256,7 +258,8 @@ __global__ void __launch_bounds__(256, 4) k_qconv_first(FirstArgs a)
       // The wavefront's pixels move on by 128 per iteration; image, row and column of a lane's pixel follow by
       // additions, and the output offset is linear in the pixel's number (the images of a workgroup are stored
       // back to back).
-      int q = wave * 32 + l32;
+      const int g0 = (SHARED ? blockIdx.y * 4 : 0) + wave, step = SHARED ? a.px_step : 128;
+      int q = g0 * 32 + l32;
       int im = fdiv(q, a.dper_image);
       int py, px;
       {
@@ -265,10 +268,10 @@ __global__ void __launch_bounds__(256, 4) k_qconv_first(FirstArgs a)
          px = rem - py * a.PW;
       }
       unsigned yoff = (unsigned)q * (unsigned)a.OC + (unsigned)half * 16u;
-      const unsigned ystep = 128u * (unsigned)a.OC;
+      const unsigned ystep = (unsigned)step * (unsigned)a.OC;
       int8_t *const ybase = a.y + (size_t)n0 * per_image * a.OC;
       const int half_rows = (int)__umul24(2 * half, a.stride);
-      for (int g = wave; g < groups; g += 4) {
+      for (int g = g0; g < groups; g += step >> 5) {
          const bool valid = q < total;
          const int col = (POOL ? 2 * px : px) + 2;
          const int cell = (int)__umul24(im, a.img_bytes) + (int)__umul24(POOL ? 2 * py : py, a.stride) + (col & ~3);
@@ -285,7 +288,7 @@ __global__ void __launch_bounds__(256, 4) k_qconv_first(FirstArgs a)
             pix[0] = pack64(window(base, sh), window(base + a.stride, sh));
          }
          int8_t *out = ybase + yoff;
-         q += 128;
+         q += step;
          yoff += ystep;
          px += a.px_col; py += a.px_row; im += a.px_im;
          if (px >= a.PW) { px -= a.PW; py += 1; }
@@ -383,12 +386,6 @@ int qconv_first_layer(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
       a.st_row = (256 % HW4) / W4;
       a.st_col = (256 % HW4) % W4;
    }
-   {
-      const int per_image = g.PH * g.PW;
-      a.px_im = 128 / per_image;
-      a.px_row = (128 % per_image) / g.PW;
-      a.px_col = (128 % per_image) % g.PW;
-   }
    a.dper_image = make_fastdiv((unsigned)(g.PH * g.PW));
    a.dPW = make_fastdiv((unsigned)g.PW);
    // Images per workgroup: four workgroups share a CU, and the kernel is as slow as the busiest CU, so the
@@ -407,9 +404,22 @@ int qconv_first_layer(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
    if (best == 0) return SOFIE_HIP_OK;
    a.images = best;
    const size_t lds = fixed + (size_t)a.images * a.img_bytes;
-   const dim3 grid((unsigned)((g.N + a.images - 1) / a.images)), block(256);
-   if (pool) hipLaunchKernelGGL(k_qconv_first<true>, grid, block, lds, ctx->stream, a);
-   else hipLaunchKernelGGL(k_qconv_first<false>, grid, block, lds, ctx->stream, a);
+   // Few images: as many workgroups as compute units, several to the same images, each with all of them in LDS and every parts-th row of
+   // four groups of pixels. us without / with: 8x1x112x112 -> 64 63.1 / 9.6, 1x1x180x180 -> 16 pooled 39.7 / 14.2, 128x1x28x28 -> 16 pooled
+   // 4.9 / 4.5, the int8 classifier's five launches on 1 image 22.2 / 21.3, 64 26.8 / 25.5; on two workgroups
+   // per compute unit 200 images 31.9 / 31.7, on four 32.6 and 256 32.4 / 33.8 (each of them reads and converts all of the image).
+   const int blocks = (g.N + a.images - 1) / a.images, per_image = g.PH * g.PW;
+   const int rows = (int)(((long)a.images * per_image + 127) / 128);
+   int parts = (ctx->num_cus > 0 ? ctx->num_cus : 256) / blocks;
+   parts = parts < 1 ? 1 : parts > rows ? rows : parts;
+   a.px_step = 128 * parts;
+   a.px_im = a.px_step / per_image;
+   a.px_row = (a.px_step % per_image) / g.PW;
+   a.px_col = (a.px_step % per_image) % g.PW;
+   const dim3 grid((unsigned)blocks, (unsigned)parts), block(256);
+   auto start = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, lds, ctx->stream, a); };
+   if (pool) start(parts == 1 ? k_qconv_first<true, false> : k_qconv_first<true, true>);
+   else start(parts == 1 ? k_qconv_first<false, false> : k_qconv_first<false, true>);
    *done = true;
    return check_launch(ctx, "k_qconv_first");
 }

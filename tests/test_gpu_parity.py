@@ -848,6 +848,27 @@ def test_first_layer_kernel(ops, cfg):
             assert np.array_equal(yp.transpose(0, 3, 1, 2), pooled)
 
 
+@pytest.mark.parametrize("n,h,w,oc", [(1, 180, 160, 16), (100, 40, 40, 32), (128, 9, 12, 16), (129, 9, 12, 16), (300, 16, 16, 64), (85, 23, 31, 48), (1, 2, 3, 16)])
+def test_first_layer_images_shared_by_workgroups(ops, n, h, w, oc):
+    """Up to half as many images as compute units: workgroups share an image, all of it once, in parts of 128 pixels, one part behind the last whole
+    round; beyond, a workgroup to each. From bytes, pooled with scales of both signs, and from floats: the oracle's bytes."""
+    from sofie_amd import lib as L
+    r = rng(700 + n + h)
+    x = r.integers(-128, 128, (n, 1, h, w)).astype(np.int8)
+    wt = r.integers(-127, 128, (oc, 1, 3, 3)).astype(np.int8)
+    scale = (r.uniform(20, 60, oc) / (73.3 * 73.3 * 3)).astype(np.float32)
+    scale[::3] *= -1
+    bias = r.integers(-3000, 3000, oc).astype(np.int32)
+    ref = oracle.qconv2d_s8(x, wt, scale, bias, (1, 1), (1, 1), 1, 5, -3, False)
+    y = ops.qconv2d_s8(x, wt, scale, bias, (1, 1), (1, 1), 1, 5, -3, False, y_layout=L.LAYOUT_NHWC)
+    assert np.array_equal(y.transpose(0, 3, 1, 2), ref)
+    yp = ops.qconv2d_pool_s8(x, wt, scale, bias, (1, 1), (1, 1), 1, 5, -3, False, y_layout=L.LAYOUT_NHWC)
+    assert np.array_equal(yp.transpose(0, 3, 1, 2), oracle.maxpool2d(ref, (2, 2), (2, 2)))
+    xf = (x.astype(np.float32) - 5.0) * np.float32(0.125)
+    yf = ops.quantize_qconv2d_s8(xf, np.float32(0.125), 5, wt, scale, bias, (1, 1), (1, 1), 1, -3, False, None, (2, 2), y_layout=L.LAYOUT_NHWC)
+    assert np.array_equal(yf.transpose(0, 3, 1, 2), ref)
+
+
 @pytest.mark.parametrize("cfg", [
     dict(N=5, C=1, H=40, W=40, OC=32, k=(3, 3), p=(1, 1), pool=(2, 2)),    # first-layer kernel, dword fill
     dict(N=3, C=1, H=9, W=7, OC=16, k=(3, 3), p=(1, 1), pool=None),        # first-layer kernel, byte fill
