@@ -625,7 +625,10 @@ struct RingPlan {
 };
 
 // Fills `plan` if the kernel takes the problem (*done).
-static int plan_ring(sofie_hip_ctx *ctx, const QConvArgs &g, RingPlan &out, bool *done)
+static int blocks_together(const QConvArgs &g) { return g.OC % 128 == 0 ? 2 : 1; }
+
+// WN: blocks of 64 output channels per workgroup
+static int plan_ring(sofie_hip_ctx *ctx, const QConvArgs &g, int WN, RingPlan &out, bool *done)
 {
    *done = false;
    if (g.xf) return SOFIE_HIP_OK;
@@ -645,7 +648,6 @@ static int plan_ring(sofie_hip_ctx *ctx, const QConvArgs &g, RingPlan &out, bool
    if (mtot >= (1ll << 31) - 1024 || (long long)g.N * HP >= (1ll << 31) - 4096) return SOFIE_HIP_OK;
    const size_t xbytes = (size_t)g.N * g.H * g.W * g.C;
    if (xbytes >= ((size_t)1 << 31)) return SOFIE_HIP_OK;
-   const int WN = g.OC % 128 == 0 ? 2 : 1;
    const int OCT = WN * 64;
    const int C16 = g.C / 16;
    QConvRingArgs a{};
@@ -722,7 +724,17 @@ static int plan_ring(sofie_hip_ctx *ctx, const QConvArgs &g, RingPlan &out, bool
 int qconv_ring(sofie_hip_ctx *ctx, const QConvArgs &g, bool *done)
 {
    RingPlan plan;
-   if (int rc = plan_ring(ctx, g, plan, done)) return rc;
+   *done = false;
+   // Few pixels: 64 channels per workgroup also where there are 128, as long as every unit of pixels and block of channels is a workgroup of its
+   // own: half of the weights come into its LDS in front of the first product. us, 128 / 64: 4x64x28x28 -> 128 5.3 / 5.0, 4x32x28x28 -> 128
+   // pooled 5.4 / 5.1, 8x32x12x12 -> 256 4.4 / 4.2, 2x32x56x56 -> 128 4.3 / 4.2.
+   const int wn = blocks_together(g);
+   const bool pooled = g.pool_kh != 0;
+   const long long units = ((long long)g.N * (pooled ? g.PH : g.OH) * (pooled ? g.PW : g.OW) + (pooled ? 31 : 63)) / (pooled ? 32 : 64);
+   if (wn == 2 && units * (g.OC / 64) <= ctx->num_cus)
+      if (int rc = plan_ring(ctx, g, 1, plan, done)) return rc;
+   if (!*done)
+      if (int rc = plan_ring(ctx, g, wn, plan, done)) return rc;
    if (!*done) return SOFIE_HIP_OK;
    const QConvRingArgs &a = plan.a;
    const size_t lds = plan.lds;
@@ -768,9 +780,9 @@ int qconv_ring_pair(sofie_hip_ctx *ctx, const QConvArgs &g1, const QConvArgs &g2
    if (g2.x != static_cast<const int8_t *>(g1.y) || g1.N != g2.N || g2.pool_kh != 0) return SOFIE_HIP_OK;
    RingPlan p1, p2;
    bool ok1 = false, ok2 = false;
-   if (int rc = plan_ring(ctx, g1, p1, &ok1)) return rc;
+   if (int rc = plan_ring(ctx, g1, blocks_together(g1), p1, &ok1)) return rc;
    if (!ok1) return SOFIE_HIP_OK;
-   if (int rc = plan_ring(ctx, g2, p2, &ok2)) return rc;
+   if (int rc = plan_ring(ctx, g2, blocks_together(g2), p2, &ok2)) return rc;
    if (!ok2) return SOFIE_HIP_OK;
    if (!p1.pool || p1.WN != 1 || p1.nob != 1 || !p1.row || p2.C16 != 4 || p2.nob != 1 || !p2.row || p1.grid != p2.grid) return SOFIE_HIP_OK;
    // the same whole images per workgroup in both layers

@@ -848,6 +848,26 @@ def test_first_layer_kernel(ops, cfg):
             assert np.array_equal(yp.transpose(0, 3, 1, 2), pooled)
 
 
+@pytest.mark.parametrize("n,c,h,w,oc,pool", [(8, 64, 32, 32, 128, None), (9, 64, 32, 32, 128, None), (4, 32, 28, 28, 128, (2, 2)), (24, 32, 28, 28, 128, (2, 2)),
+                                               (3, 64, 9, 13, 256, None), (1, 32, 56, 60, 384, None), (5, 64, 6, 62, 128, (2, 2))])
+def test_ring_blocks_of_channels_by_pixels(ops, n, c, h, w, oc, pool):
+    """64 output channels per workgroup where pixels are few, 128 beyond, on both sides of the line: the oracle's bytes, scales of both signs."""
+    from sofie_amd import lib as L
+    r = rng(800 + n + c + oc)
+    x = r.integers(-128, 128, (n, c, h, w)).astype(np.int8)
+    wt = r.integers(-127, 128, (oc, c, 3, 3)).astype(np.int8)
+    scale = (r.uniform(20, 60, oc) / (73.3 * 73.3 * np.sqrt(9 * c))).astype(np.float32)
+    scale[::3] *= -1
+    bias = r.integers(-3000, 3000, oc).astype(np.int32)
+    ref = oracle.qconv2d_s8(x, wt, scale, bias, (1, 1), (1, 1), 1, 5, -3, False)
+    if pool:
+        ref = oracle.maxpool2d(ref, pool, pool)
+    xh, wh = np.ascontiguousarray(x.transpose(0, 2, 3, 1)), np.ascontiguousarray(wt.transpose(0, 2, 3, 1))
+    call = ops.qconv2d_pool_s8 if pool else ops.qconv2d_s8
+    y = call(xh, wh, scale, bias, (1, 1), (1, 1), 1, 5, -3, False, x_layout=L.LAYOUT_NHWC, y_layout=L.LAYOUT_NHWC, w_layout=L.LAYOUT_NHWC)
+    assert np.array_equal(y.transpose(0, 3, 1, 2), ref)
+
+
 @pytest.mark.parametrize("n,h,w,oc", [(1, 180, 160, 16), (100, 40, 40, 32), (128, 9, 12, 16), (129, 9, 12, 16), (300, 16, 16, 64), (85, 23, 31, 48), (1, 2, 3, 16)])
 def test_first_layer_images_shared_by_workgroups(ops, n, h, w, oc):
     """Up to half as many images as compute units: workgroups share an image, all of it once, in parts of 128 pixels, one part behind the last whole
