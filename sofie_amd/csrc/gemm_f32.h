@@ -89,6 +89,15 @@ __device__ __forceinline__ void store4(const GemmF32Args &g, v4f v, int m, int n
    for (int e = 0; e < 3; ++e)
       if (n + e < g.N) o[e] = v[e];
 }
+// The last four columns of all, of which those in front of `first` are stored by whoever's sums of them may have been formed in another way.
+__device__ __forceinline__ void store4_from(const GemmF32Args &g, v4f v, int m, int n, int first)
+{
+   if (n >= first) return store4(g, v, m, n);
+   float *o = g.Y + (size_t)m * g.ldy + n;
+#pragma unroll
+   for (int e = 1; e < 4; ++e)
+      if (n + e >= first) o[e] = v[e];
+}
 
 // k_gemm_f32_split (gemm_f32_split.hip): the product on the bf16 matrix instructions, operands as three bf16 numbers, 16 mi rows x 64
 // columns per workgroup, K in `splits` slices (above one: raw sums into g.partial, for k_gemm_f32_skinny_finish).

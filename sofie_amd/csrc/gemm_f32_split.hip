@@ -9,7 +9,7 @@
 //     the four belongs to tile e of four: a tile is every fourth column, and nothing is transposed.
 // Both give lane group kg the same eight k of a chunk, in the same order.
 // Rows and columns behind the matrix are copies of the last ones (of the last four, where four are loaded at once: the same sums,
-// stored twice).
+// stored twice, but not those of the tile before: a wavefront that repeats its sums, below, has other last bits than one that does not).
 //
 // Bound: vector instructions (eleven for two numbers to split, four a tile to add) beside the matrix instructions, which
 // run under them only in part: 1.3 us a chunk of 64 rows and SIMD, 0.64 of it matrix instructions. Relative error against 64 bits 7e-8 to
@@ -275,7 +275,10 @@ __global__ void __launch_bounds__(WAVES * 64, 2) k_gemm_f32_split(GemmF32Args g)
    for (int s = 0; s < MINE; ++s) {
       const int at = s * 512 + tid, ln = at & 63, t = at >> 6, i = t / NJ, q = t % NJ, r = ln & 15, c = B_KM ? 16 * (ln >> 4) + 4 * q : 16 * q + 4 * (ln >> 4);
       m[s] = A_KM ? m0 + (i / 4 * 16 + r) * 4 : m0 + i * 16 + r;
-      if constexpr (A_KM) m[s] = m[s] >= g.M ? g.M : (m[s] < g.M - 4 ? m[s] : g.M - 4) + i % 4;
+      if constexpr (A_KM) {
+         m[s] = m[s] >= g.M ? g.M : (m[s] < g.M - 4 ? m[s] : g.M - 4) + i % 4;
+         if (m[s] < m0) m[s] = g.M;      // the tile before's
+      }
       n[s] = n0 + c;
       if constexpr (B_KM) n[s] = n[s] >= g.N ? g.N : n[s] < g.N - 4 ? n[s] : g.N - 4;
       bias[s] = bias_row4(g, n[s]);
@@ -302,7 +305,7 @@ __global__ void __launch_bounds__(WAVES * 64, 2) k_gemm_f32_split(GemmF32Args g)
       for (int w = 1; w < 4; ++w)
 #pragma unroll
          for (int e = 0; e < 4; ++e) sum[e] = __fadd_rn(sum[e], red[w * V + s * 512 + tid][e]);
-      if (m[s] < g.M && n[s] < g.N) store4(g, finish4(g, sum, bias[s], m[s], n[s]), m[s], n[s]);
+      if (m[s] < g.M && n[s] < g.N) store4_from(g, finish4(g, sum, bias[s], m[s], n[s]), m[s], n[s], n0);
    }
 }
 
@@ -539,7 +542,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
                   acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(SplitRows<B_KM>::value(qb, j, e), SplitRows<A_KM>::value(qa, i, e), acc[i][j], 0, 0, 0);
       }
    }
-   // a quad is four consecutive columns of a row: with B along N element q of the four tiles
+   // a quad is four consecutive columns of a row: with B along N element q of the four tiles. (Rows and columns in front of this wavefront's are another one's)
 #pragma unroll
    for (int q = 0; q < 4; ++q) {
       int n = n1 + (B_KM ? 16 * kg + 4 * q : 16 * q + 4 * kg);
@@ -551,8 +554,9 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
          int m = m1 + (A_KM ? 4 * r16 : 16 * i + r16);
          if (m >= g.M) continue;
          if constexpr (A_KM) m = (m < g.M - 4 ? m : g.M - 4) + i;
+         if (A_KM && m < m1) continue;
          const v4f v = B_KM ? v4f{acc[i][0][q], acc[i][1][q], acc[i][2][q], acc[i][3][q]} : acc[i][q];
-         store4(g, finish4(g, v, bias, m, n), m, n);
+         store4_from(g, finish4(g, v, bias, m, n), m, n, n1);
       }
    }
 }

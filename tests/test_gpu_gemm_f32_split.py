@@ -157,3 +157,31 @@ def test_gemm_in_three_parts_on_shared_fragments(ops, M, N, K, tA, tB):
     fin = ref.isfinite()
     assert bool(((got - ref).abs()[fin] <= (K ** 0.5 * 2.0 ** -24 * (ad.nan_to_num(0.0, 0.0, 0.0).abs() @ bd.abs()))[fin]).all())
     ctx.close()
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(1441, 1089, 1538, "k_gemm_f32_split"), (1537, 1025, 2049, "k_gemm_f32_split"), (65, 6210, 1105, "k_gemm_f32_split"),
+                                          (2753, 5121, 336, "k_gemm_f32_split_shared"), (2689, 5186, 337, "k_gemm_f32_split_shared")])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_an_infinity_in_the_last_tile_changes_no_bit_of_the_others(ops, M, N, K, kernel, tA, tB):
+    """One or two columns (rows) in the last tile, and an infinity in the last one alone: its wavefront forms its sums again with fp32 instructions,
+    those of the columns (rows) in front of its first, which it loads in fours with its own, among them. The tile before keeps what it has summed."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g)
+    stored = lambda x, y: (x.t().contiguous() if tA else x, y.t().contiguous() if tB else y)
+    ctx = ops.Context(0)
+    y, names = product(ctx, *stored(a, b), tA, tB, None)
+    assert names == [kernel], names
+    for last in ("column", "row"):
+        ai, bi = a.clone(), b.clone()
+        if last == "column":
+            bi[K // 2, N - 1] = float("inf")
+        else:
+            ai[M - 1, K // 2] = float("inf")
+        for _ in range(3):
+            yi, names = product(ctx, *stored(ai, bi), tA, tB, None)
+            assert names == [kernel], names
+            if last == "column":
+                assert torch.equal(yi[:, :N // 64 * 64], y[:, :N // 64 * 64]) and not bool(yi[:, N - 1].isfinite().any())
+            else:
+                assert torch.equal(yi[:M // 64 * 64 if tA else M // 128 * 128], y[:M // 64 * 64 if tA else M // 128 * 128]) and not bool(yi[M - 1].isfinite().any())
+    ctx.close()
