@@ -385,10 +385,10 @@ private:
          // picked is 2.2 % behind the best of these forms in the mean): each wavefront takes in weights of its own.
          const double uneven = l.one_for_all ? 1.25 : q0.KH * q0.KW != q1.KH * q1.KW ? 1.4 : 1.0;
          const double us = std::sqrt(std::sqrt(w2 * w2 + b2 * b2)) / 2100.0 * uneven + 3.0;
-         // (Under the device's power limit the form with the fewest requests for weights per matrix instruction comes out ahead of what is
-         // estimated: 256x64x56x56 -> 128, 3x3 604 us on 128 channels x 64 pixels, 568 on 128 x 128. Of 50 random layers of 15 GFLOP
-         // and more none changes by more than 1.3 %, what two runs of one side differ by.)
-         return pieces == 16 && us > 150.0 && !l.one_for_all ? 150.0 + 0.93 * (us - 150.0) : us;
+         // (128 channels x 64 pixels ask for twice the weights per matrix instruction: over 221 layers of 15 to 700 us on which forms are close, each form timed, this
+         // one takes 1.085 times what is estimated, 128 x 128 1.045 times, at every size. Of 84 other layers whose form changes by the 1.03, 25 of them above
+         // 150 us, 0.975 times the time in the mean, 5 longer by more than 2 %, 1.043 at most. With 1.04 12x50x88x65 -> 194, 3x3 s2 35.4 -> 45.5.)
+         return f.ti == 4 && f.tj == 2 ? 1.03 * us : us;
       }
    };
 

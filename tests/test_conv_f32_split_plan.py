@@ -180,3 +180,43 @@ def test_strided_and_transposed_layers_by_a_full_search(tmp_path):
     assert out.returncode == 0, out.stdout
     strided, transposed, estimates, without = map(int, out.stdout.split())
     assert strided > 200 and transposed > 200 and 2 * estimates <= without, out.stdout
+
+
+LINEAR = r"""
+#include <cstdio>
+#include "conv_f32_split_plan.h"
+using namespace sofie;
+
+// images of one tile of every form, all channels in one block
+int main()
+{
+   static const int forms[][3] = {{2, 4, 2}, {2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 4, 2}, {1, 2, 2}};
+   for (const auto &f : forms) {
+      ConvProblem p{};
+      const int w = f[1] == 4 ? 16 : 8;
+      p.N = 1, p.C = 16, p.OC = 32 * f[0], p.groups = 1, p.H = 8, p.W = w, p.dh = p.dw = p.sh = p.sw = 1, p.KH0 = p.KW0 = 3, p.nphases = 1, p.OH0 = 8, p.OW0 = w;
+      p.phase[0] = {8, w, 3, 3, 1, 1, 0, 1, 0, 1, 0, 1, 0, 1};
+      SplitPlan plan(p, false);
+      const SplitPlan::Form form{f[0], f[1], f[2], 16, 1, 0.0};
+      SplitPlan::Panels q;
+      if (!plan.panels(q, 0, form.pixels(), 1)) return printf("no panels\n"), 1;
+      const int round = 256 * 12;      // two, three or four workgroups to a compute unit
+      const double one = plan.estimate(form, &q, round, 256), two = plan.estimate(form, &q, 2 * round, 256) - one;
+      for (int k = 3; k <= 64; ++k) {
+         const double time = plan.estimate(form, &q, (size_t)k * round, 256);
+         if (std::fabs(time - one - (k - 1) * two) > 1e-9 * time) return printf("%d%d%d: %d rounds %.6f us, one %.6f, another %.6f\n", f[0], f[1], f[2], k, time, one, two), 1;
+      }
+      printf("%.3f ", one);
+   }
+}
+"""
+
+
+def test_estimates_grow_with_whole_rounds(tmp_path):
+    """As many workgroups again take as long again, whatever the form and from whichever time on: no form is preferred from a certain time on."""
+    src, exe = tmp_path / "linear.cpp", tmp_path / "linear"
+    src.write_text(LINEAR)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "sofie_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    assert len(out.stdout.split()) == 7
