@@ -399,17 +399,6 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
    int tm, tn;
    tile_of(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
    const int m0 = tm * BM, n0 = tn * BN;
-   int k_begin = 0, k_end = g.K;
-   if (gridDim.y > 1) {      // K in slices: raw sums into the slice's plane of the scratch buffer
-      const int chunks = (g.K + CH - 1) / CH, per = (chunks + (int)gridDim.y - 1) / (int)gridDim.y;
-      k_begin = (int)blockIdx.y * per * CH;
-      k_end = k_begin + per * CH < g.K ? k_begin + per * CH : g.K;
-      g.Y = g.partial + (size_t)blockIdx.y * g.M * g.N;
-      g.ldy = g.N;
-      g.alpha = 1.0f;
-      g.bias_kind = SOFIE_BIAS_NONE;
-      g.relu = 0;
-   }
    const bool ragged = (g.K & 3) != 0;
    v4f acc[4][4];
 #pragma unroll
@@ -443,8 +432,8 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
 #pragma unroll
          for (int t = 0; t < 3; ++t) mine[(f * 3 + t) * 64] = part[t];
       };
-      rows.request(q, k_begin);
-      if (ragged && k_begin + CH > g.K) rows.trim(q, k_begin);
+      rows.request(q, 0);
+      if (ragged && CH > g.K) rows.trim(q, 0);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
 #pragma unroll
@@ -453,8 +442,8 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
             for (int t = 0; t < 5; ++t) pair(f, p, t);
          put(f);
       }
-      rows.request(q, k_begin + CH < k_end ? k_begin + CH : g.K);
-      for (int k0 = k_begin; k0 < k_end; k0 += CH) {
+      rows.request(q, CH);
+      for (int k0 = 0; k0 < g.K; k0 += CH) {
          __syncthreads();
          v8b a[4][3], b[4][3];
 #pragma unroll
@@ -468,7 +457,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
          __builtin_amdgcn_s_barrier();
          asm volatile("" ::: "memory");
          const int next = k0 + CH;
-         if (ragged && next < k_end && next + CH > g.K) rows.trim(q, next);
+         if (ragged && next < g.K && next + CH > g.K) rows.trim(q, next);
          __builtin_amdgcn_sched_barrier(0);
          v4f t, before;
 #pragma unroll
@@ -486,7 +475,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
             }
             before = t;
             if (n % 4 == 3) put(n / 4);
-            if (n == 15) rows.request(q, next + CH < k_end ? next + CH : g.K);
+            if (n == 15) rows.request(q, next + CH);
             __builtin_amdgcn_sched_barrier(0);
          }
 #pragma unroll
@@ -525,7 +514,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
 #pragma unroll
          for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-      for (int k0 = k_begin; k0 < k_end; k0 += CH) {
+      for (int k0 = 0; k0 < g.K; k0 += CH) {
          v4f qa[8], qb[8];
          ra.request(qa, k0);
          rb.request(qb, k0);
@@ -562,10 +551,10 @@ __global__ void __launch_bounds__(256, 2) k_gemm_f32_split_shared(GemmF32Args g)
 }
 
 template <bool A_KM, bool B_KM>
-int launch_shared(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, int splits)
+int launch_shared(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz)
 {
    constexpr auto kern = k_gemm_f32_split_shared<A_KM, B_KM>;
-   hipLaunchKernelGGL(kern, dim3(cdiv(g.M, 128) * cdiv(g.N, 128), splits, nz), dim3(256), 16 * 3072, ctx->stream, g);
+   hipLaunchKernelGGL(kern, dim3(cdiv(g.M, 128) * cdiv(g.N, 128), 1, nz), dim3(256), 16 * 3072, ctx->stream, g);
    return check_launch(ctx, "k_gemm_f32_split_shared");
 }
 
@@ -622,8 +611,8 @@ SplitChoice sofie::gemm_f32_shared_choice(const sofie_hip_ctx *ctx, const GemmF3
 int sofie::launch_gemm_f32_split(sofie_hip_ctx *ctx, const GemmF32Args &g, unsigned nz, const SplitChoice &c)
 {
    if (c.mi == 8)
-      return g.transA ? (g.transB ? launch_shared<true, false>(ctx, g, nz, c.splits) : launch_shared<true, true>(ctx, g, nz, c.splits))
-                      : (g.transB ? launch_shared<false, false>(ctx, g, nz, c.splits) : launch_shared<false, true>(ctx, g, nz, c.splits));
+      return g.transA ? (g.transB ? launch_shared<true, false>(ctx, g, nz) : launch_shared<true, true>(ctx, g, nz))
+                      : (g.transB ? launch_shared<false, false>(ctx, g, nz) : launch_shared<false, true>(ctx, g, nz));
    if (g.transA) return g.transB ? launch<true, false, 4>(ctx, g, nz, c.splits) : launch<true, true, 4>(ctx, g, nz, c.splits);
    switch (c.mi) {
    case 2: return g.transB ? launch<false, false, 2>(ctx, g, nz, c.splits) : launch<false, true, 2>(ctx, g, nz, c.splits);
