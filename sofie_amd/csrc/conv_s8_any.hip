@@ -553,7 +553,9 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    // in vain behind a short K), sums and conversions. A fit to 457 random layers of 16 to 256 channels with kept weights, a third of them
    // pooled, on which the forms differ: what it picks is 1.7 % behind the best of ten forms in the mean and 1.14 times faster than
    // a rule by tiles alone with eight wavefronts in every dealt form (16x48x35x29 -> 80, 3x3 s2 6.2 -> 4.1 us; 14792 pooled pixels -> 48
-   // on 7 K-steps 26.9 -> 6.3; 14x14x512 -> 512, 3x3 9.2 -> 6.3).
+   // on 7 K-steps 26.9 -> 6.3; 14x14x512 -> 512, 3x3 9.2 -> 6.3). Pooled and in place, with the bounds of four windows to look up, requests behind
+   // the first ones take longer than in the fit where nothing else runs meanwhile: 14 of 384 layers with fewer tiles than half of the compute units go from four
+   // wavefronts to eight by it, all of them faster, 1.05 to 1.15 times (38x64x8x8 -> 69, 7x7 9.2 -> 8.0, 72x192x13x13 -> 9, 3x3 7.45 -> 6.75).
    struct Few {
       int mb, nb, nw, wk, d;
    };
@@ -565,7 +567,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       if (q.nb > p.nt) continue;      // tiles of nothing
       const float workgroups = (float)cdiv(a.M, q.nw / q.wk * (pool ? 1 : q.mb) * 16) * (float)cdiv(p.nt, q.nb), per_cu = workgroups > (float)cus ? workgroups / (float)cus : 1.0f;
       const int steps = cdiv(p.S, q.wk), mbs = pool ? 4 : q.mb, pieces = mbs * q.nb;
-      const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? 0.353f + 0.153f * (float)(steps - q.d) / (float)q.d : 0.0f);
+      const float behind = pool && bounds && q.wk > 1 && workgroups <= (float)cus ? 0.553f : 0.153f;
+      const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? 0.353f + behind * (float)(steps - q.d) / (float)q.d : 0.0f);
       const float work = (float)q.nw * (0.0379f + ((float)steps + 0.211f * (float)q.d) * (0.0126f * (float)mbs + 0.0059f * (float)q.nb)) +
                          (0.022f * (float)(q.nw / q.wk) + (q.wk > 1 ? 0.0086f * (float)q.nw : 0.0f)) * (float)pieces;
       if (waits + per_cu * work < least) {

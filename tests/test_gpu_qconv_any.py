@@ -42,6 +42,7 @@ SHAPES = [
     (3, 16, 90, 70, 17, 1, 1, (1, 1), (0, 0)),      # one K-step that is a quarter full, no bounds
     (9, 1, 140, 130, 8, 5, 5, (1, 1), (2, 2)),      # one channel
     (20, 5, 62, 61, 9, 2, 3, (1, 2), (0, 1)),       # K of 30 bytes, uneven kernel, stride and pads
+    (6, 64, 9, 8, 37, 7, 7, (1, 1), (3, 3)),        # pooled in place, few tiles: K dealt to eight wavefronts
 ]
 
 
