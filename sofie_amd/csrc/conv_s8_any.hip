@@ -522,7 +522,10 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    } while (0)
    // The form, by the number of workgroups it gives and by what the LDS holds.
    //   A, B  64 pixels x up to 64 channels per wavefront, weights in LDS, as many workgroups as are resident at once walk over the
-   //         tiles: for a tile per compute unit and more, with 16 KB of weights and more from half of that. A: four wavefronts, two or three
+   //         tiles: for a tile per compute unit and more, with 16 KB of weights and more from half of that (unpooled ones from six K-steps on:
+   //         3x32x96x152 -> 188, 3x3 s2 on five 6.8 us in C, 7.95 here). Not where the LDS holds one tile of channels of several, each of which would
+   //         read all of the input: C, D or E take 0.39 to 1.04 times as long there, 0.64 in the mean of 17 (46x128x8x8 -> 252, 7x7 pooled 23.0 us, 32.4
+   //         here). A: four wavefronts, two or three
    //         workgroups in a compute unit; B: eight wavefronts, one workgroup, from four rounds of tiles and, with more than 75 KB of
    //         weights, from two on. Both timed on 220 layers: B takes 0.87 to 0.92 times A's time from four rounds on, 1.02 to 1.13 with
    //         two to four, 0.96 to 1.02 below; C, D or E 1.07 to 1.2 times A's from half a round on 16 KB of weights.
@@ -534,7 +537,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    while (nb > 1 && (size_t)nb * p.S * 1024 > (size_t)144 * 1024) nb = even(nb - 1);
    const size_t wlds = (size_t)nb * p.S * 1024;
    const long long big_tiles = (long long)cdiv(a.M, 4 * mb * 16) * cdiv(p.nt, nb);
-   if ((big_tiles >= cus || (2 * big_tiles >= cus && wlds >= (size_t)16 * 1024)) && wlds <= (size_t)144 * 1024) {
+   const bool half = 2 * big_tiles >= cus && wlds >= (size_t)16 * 1024 && (pool || p.S >= 6);
+   if ((big_tiles >= cus || half) && wlds <= (size_t)144 * 1024 && (nb > 1 || even(4) == 1)) {
       if (big_tiles < 2 * cus || (big_tiles < 4 * cus && wlds + tab_bytes <= (size_t)75 * 1024)) {
          const int resident = (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024)) > 3 ? 3 : (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024));
          if (nb == 1) SOFIE_ANY(4, 4, 1, 4, 1, 4, true, wlds, resident);

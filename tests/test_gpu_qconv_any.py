@@ -37,7 +37,9 @@ SHAPES = [
     (24, 48, 40, 40, 30, 3, 3, (1, 1), (1, 1)),     # large tiles in place, two channel tiles
     (20, 20, 41, 39, 40, 3, 3, (1, 1), (0, 1)),     # large tiles, three channel tiles
     (20, 64, 41, 39, 61, 5, 5, (1, 1), (2, 2)),     # large tiles, more weights than a third of the LDS
-    (9, 128, 33, 33, 100, 7, 7, (1, 1), (3, 3)),    # weights of one channel tile are all that fits the LDS
+    (9, 128, 33, 33, 100, 7, 7, (1, 1), (3, 3)),    # weights of one channel tile of seven are all that would fit the LDS
+    (84, 128, 20, 20, 16, 7, 7, (1, 1), (3, 3)),    # those of one channel tile, which is all there is
+    (13, 32, 48, 60, 188, 3, 3, (1, 1), (1, 1)),    # half a round of large tiles, five K-steps
     # the short sums above once more with the pixels from which on they are this kernel's
     (3, 16, 90, 70, 17, 1, 1, (1, 1), (0, 0)),      # one K-step that is a quarter full, no bounds
     (9, 1, 140, 130, 8, 5, 5, (1, 1), (2, 2)),      # one channel
