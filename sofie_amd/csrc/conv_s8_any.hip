@@ -525,10 +525,11 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    //         tiles: for a tile per compute unit and more, with 16 KB of weights and more from half of that (unpooled ones from six K-steps on:
    //         3x32x96x152 -> 188, 3x3 s2 on five 6.8 us in C, 7.95 here). Not where the LDS holds one tile of channels of several, each of which would
    //         read all of the input: C, D or E take 0.39 to 1.04 times as long there, 0.64 in the mean of 17 (46x128x8x8 -> 252, 7x7 pooled 23.0 us, 32.4
-   //         here). A: four wavefronts, two or three
-   //         workgroups in a compute unit; B: eight wavefronts, one workgroup, from four rounds of tiles and, with more than 75 KB of
-   //         weights, from two on. Both timed on 220 layers: B takes 0.87 to 0.92 times A's time from four rounds on, 1.02 to 1.13 with
-   //         two to four, 0.96 to 1.02 below; C, D or E 1.07 to 1.2 times A's from half a round on 16 KB of weights.
+   //         here). A: four wavefronts, up to three workgroups in a compute unit; B: eight wavefronts, one workgroup, from four rounds of tiles on
+   //         with up to 75 KB of weights: 0.94 times A's time in the mean of 161 layers (three and four tiles of channels 0.91, of which A holds two
+   //         wavefronts to a SIMD as well), with more weights 1.095 over 17, with two to four rounds 1.05 over 90. Four K-steps and fewer of an unpooled copy
+   //         stay in A, whose third wavefront to a SIMD covers the trips to memory: B 1.034 times as long over 60, 0.91 to 1.14 (192x3x181x192 -> 25, 5x5
+   //         122 us in A, 139 in B).
    //   C, D, E  weights from memory, below.
    // Channels per workgroup: up to four tiles of 16, as few idle ones as possible.
    auto even = [&](int most) { return cdiv(p.nt, cdiv(p.nt, most)); };
@@ -539,7 +540,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    const long long big_tiles = (long long)cdiv(a.M, 4 * mb * 16) * cdiv(p.nt, nb);
    const bool half = 2 * big_tiles >= cus && wlds >= (size_t)16 * 1024 && (pool || p.S >= 6);
    if ((big_tiles >= cus || half) && wlds <= (size_t)144 * 1024 && (nb > 1 || even(4) == 1)) {
-      if (big_tiles < 2 * cus || (big_tiles < 4 * cus && wlds + tab_bytes <= (size_t)75 * 1024)) {
+      const bool few_steps = p.copy && !pool && nb <= 2 && p.S <= 4;
+      if (big_tiles < 4 * cus || wlds + tab_bytes > (size_t)75 * 1024 || few_steps) {
          const int resident = (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024)) > 3 ? 3 : (int)((size_t)156 * 1024 / (wlds + tab_bytes + 1024));
          if (nb == 1) SOFIE_ANY(4, 4, 1, 4, 1, 4, true, wlds, resident);
          if (nb == 2) SOFIE_ANY(4, 4, 2, 4, 1, 4, true, wlds, resident);
