@@ -523,7 +523,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    // The form, by the number of workgroups it gives and by what the LDS holds.
    //   A, B  64 pixels x up to 64 channels per wavefront, weights in LDS, as many workgroups as are resident at once walk over the
    //         tiles: for a tile per compute unit and more, with 16 KB of weights and more from half of that (unpooled ones from six K-steps on:
-   //         3x32x96x152 -> 188, 3x3 s2 on five 6.8 us in C, 7.95 here). Not where the LDS holds one tile of channels of several, each of which would
+   //         3x32x96x152 -> 188, 3x3 s2 on five 6.8 us in C, 7.95 here; and where the LDS holds as many tiles of channels as a wavefront: else C, D or E
+   //         0.80 to 1.26 times as long over seven, 56x155x13x13 -> 120, 5x5 pooled 17.4 in D, 22.9 here). Not where the LDS holds one tile of channels of several, each of which would
    //         read all of the input: C, D or E take 0.39 to 1.04 times as long there, 0.64 in the mean of 17 (46x128x8x8 -> 252, 7x7 pooled 23.0 us, 32.4
    //         here). A: four wavefronts, up to three workgroups in a compute unit; B: eight wavefronts, one workgroup, from four rounds of tiles on
    //         with up to 75 KB of weights: 0.94 times A's time in the mean of 161 layers (three and four tiles of channels 0.91, of which A holds two
@@ -538,7 +539,7 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    while (nb > 1 && (size_t)nb * p.S * 1024 > (size_t)144 * 1024) nb = even(nb - 1);
    const size_t wlds = (size_t)nb * p.S * 1024;
    const long long big_tiles = (long long)cdiv(a.M, 4 * mb * 16) * cdiv(p.nt, nb);
-   const bool half = 2 * big_tiles >= cus && wlds >= (size_t)16 * 1024 && (pool || p.S >= 6);
+   const bool half = 2 * big_tiles >= cus && wlds >= (size_t)16 * 1024 && nb == even(4) && (pool || p.S >= 6);
    if ((big_tiles >= cus || half) && wlds <= (size_t)144 * 1024 && (nb > 1 || even(4) == 1)) {
       const bool few_steps = p.copy && !pool && nb <= 2 && p.S <= 4;
       if (big_tiles < 4 * cus || wlds + tab_bytes > (size_t)75 * 1024 || few_steps) {
@@ -561,7 +562,8 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
    // a rule by tiles alone with eight wavefronts in every dealt form (16x48x35x29 -> 80, 3x3 s2 6.2 -> 4.1 us; 14792 pooled pixels -> 48
    // on 7 K-steps 26.9 -> 6.3; 14x14x512 -> 512, 3x3 9.2 -> 6.3). Pooled and in place, with the bounds of four windows to look up, requests behind
    // the first ones take longer than in the fit where nothing else runs meanwhile: 14 of 384 layers with fewer tiles than half of the compute units go from four
-   // wavefronts to eight by it, all of them faster, 1.05 to 1.15 times (38x64x8x8 -> 69, 7x7 9.2 -> 8.0, 72x192x13x13 -> 9, 3x3 7.45 -> 6.75).
+   // wavefronts to eight by it, all of them faster, 1.05 to 1.15 times (38x64x8x8 -> 69, 7x7 9.2 -> 8.0, 72x192x13x13 -> 9, 3x3 7.45 -> 6.75; with five steps
+   // for each of four 4x128x8x8 -> 48, 3x3 6.2 -> 5.7).
    struct Few {
       int mb, nb, nw, wk, d;
    };
@@ -573,8 +575,9 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       if (q.nb > p.nt) continue;      // tiles of nothing
       const float workgroups = (float)cdiv(a.M, q.nw / q.wk * (pool ? 1 : q.mb) * 16) * (float)cdiv(p.nt, q.nb), per_cu = workgroups > (float)cus ? workgroups / (float)cus : 1.0f;
       const int steps = cdiv(p.S, q.wk), mbs = pool ? 4 : q.mb, pieces = mbs * q.nb;
-      const float behind = pool && bounds && q.wk > 1 && workgroups <= (float)cus ? 0.553f : 0.153f;
-      const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? 0.353f + behind * (float)(steps - q.d) / (float)q.d : 0.0f);
+      const bool looked_up = pool && bounds && q.wk > 1 && workgroups <= (float)cus;
+      const float first = looked_up ? 0.753f : 0.353f, others = looked_up ? 0.503f : 0.153f;
+      const float waits = 2.681f + (q.wk > 1 ? 0.068f : 0.0f) + (steps > q.d ? first + others * (float)(steps - q.d) / (float)q.d : 0.0f);
       const float work = (float)q.nw * (0.0379f + ((float)steps + 0.211f * (float)q.d) * (0.0126f * (float)mbs + 0.0059f * (float)q.nb)) +
                          (0.022f * (float)(q.nw / q.wk) + (q.wk > 1 ? 0.0086f * (float)q.nw : 0.0f)) * (float)pieces;
       if (waits + per_cu * work < least) {
