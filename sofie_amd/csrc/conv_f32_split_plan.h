@@ -203,8 +203,8 @@ struct SplitPlan {
       return s.time();
    }
 
-   // The best form with slots of 8 channels, below other_us: strided layers, whose patches are too large for more (16x16x... pixels under a stride of 2
-   // read 33x33 cells).
+   // The best form with slots of 8 channels, below other_us: strided layers, whose patches are too large for more (8x8 pixels under a 3x3
+   // kernel of stride 2 read 17x17 cells, of 16 channels more than the 256 that the threads of a workgroup carry).
    Form choose_eights(size_t n, int cus, double other_us)
    {
       static const int forms[][3] = {{2, 2, 2}, {4, 4, 2}, {3, 4, 2}, {4, 2, 2}, {1, 2, 2}, {2, 4, 2}, {1, 4, 2}};

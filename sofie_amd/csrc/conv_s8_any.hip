@@ -6,8 +6,8 @@
 //   * in place (BOUNDS): channels-last, C a multiple of 16, 16-byte aligned. A chunk lies inside one tap; a chunk outside
 //     the image is replaced by the zero-point.
 //   * a copy in scratch memory, [N][H + pads][W + pads][Cp], Cp = C rounded up to whole dwords, pads filled with the
-//     zero-point: written by k_qconv_any_input from channels-last or channel-plane int8 or from the float tensor that
-//     QuantizeLinear would read. One kernel row of a window is then KW * Cp contiguous bytes, which are cut into chunks
+//     zero-point: written by k_qconv_any_input from channels-last int8, by k_qconv_any_planes from channel planes, int8 or the float
+//     tensor that QuantizeLinear would read. One kernel row of a window is then KW * Cp contiguous bytes, which are cut into chunks
 //     together (a 7x7 kernel on 3 channels: 14 chunks instead of 49), and no tap needs a bounds check.
 // The weights are copied fragment by fragment ([16 channels][K-step][lane][16 bytes], zeros behind the last channel and the
 // last tap), so that what an operand reads behind a row or a pixel is multiplied by 0 and a fragment is 1 KB in one piece.
@@ -53,9 +53,9 @@ constexpr unsigned OUTSIDE = 0x80000000u;
 // MB x NB tiles of 16 pixels x 16 channels per wavefront; NW wavefronts, groups of WK of them share their pixels and deal
 // the K-steps among themselves; D fragments of every pixel tile in flight. POOL: the four pixel tiles are the positions of
 // a 2x2 window with stride 2. BLDS: the weights of the workgroup's channels stay in LDS while it walks over its tiles.
-// (Two wavefronts to a SIMD said so: left to itself the compiler took more than 256 registers with the accumulators for four wavefronts on four tiles
-// of channels, one to a SIMD: 121x16x32x32 -> 128, 5x5 27.9 -> 21 us, 16x70x59x31 -> 97, 3x3 pooled 27.7 -> 12. Three on up to two tiles of channels: 1.2
-// times longer with two.)
+// (At least two wavefronts to a SIMD where weights are in LDS: left to itself the compiler took more than 256 registers with the accumulators for four
+// wavefronts on four tiles of channels, one to a SIMD: 121x16x32x32 -> 128, 5x5 27.9 -> 21 us, 16x70x59x31 -> 97, 3x3 pooled 27.7 -> 12. One tile of channels takes 120
+// to 180 registers, two tiles 160 to 186, so that two to four wavefronts share a SIMD, three and four tiles 189 to 256, two.)
 template <int MB, int NB, int NW, int WK, int D, bool BOUNDS, bool POOL, bool BLDS>
 __global__ void __launch_bounds__(NW * 64, BLDS ? 2 : 1) k_qconv_any(AnyArgs a)
 {
@@ -474,7 +474,7 @@ int qconv_any(sofie_hip_ctx *ctx, const QConvArgs &g, int8_t *scratch, bool *don
       else if (!g.x_nhwc) hipLaunchKernelGGL(k_qconv_any_planes<false>, grid, block, 0, ctx->stream, g, dst, pixels, p.HP, p.WP, cd, dPixels, dWP, dHP);
       else if (cd % 4 == 0) hipLaunchKernelGGL(k_qconv_any_input<true>, grid, block, 0, ctx->stream, g, dst4, total, p.HP, p.WP, cd, dcd, dWP, dHP);
       else hipLaunchKernelGGL(k_qconv_any_input<false>, grid, block, 0, ctx->stream, g, dst4, total, p.HP, p.WP, cd, dcd, dWP, dHP);
-      if (int rc = check_launch(ctx, "k_qconv_any_input")) return rc;
+      if (int rc = check_launch(ctx, g.xf || !g.x_nhwc ? "k_qconv_any_planes" : "k_qconv_any_input")) return rc;
    }
    AnyArgs a{};
    a.x = p.copy ? xs : g.x;

@@ -624,10 +624,9 @@ struct RingPlan {
    int image_px;             // (pooled) pixels of one image
 };
 
-// Fills `plan` if the kernel takes the problem (*done).
 static int blocks_together(const QConvArgs &g) { return g.OC % 128 == 0 ? 2 : 1; }
 
-// WN: blocks of 64 output channels per workgroup
+// Fills `out` if the kernel takes the problem (*done). WN: blocks of 64 output channels per workgroup
 static int plan_ring(sofie_hip_ctx *ctx, const QConvArgs &g, int WN, RingPlan &out, bool *done)
 {
    *done = false;
