@@ -80,7 +80,7 @@ def test_conv_in_three_parts(ops, kept, shape):
             assert "k_conv_f32_split" not in names or float(err.norm()) <= 3e-7 * float(ref.norm()), i
 
 
-# Layers of stride 2 in slots of eight channels: an odd number of chunks in a slot (9, 25, 49), an even one; one slot, several, the last one in part
+# Layers of stride 2 in slots of eight channels (tests/test_conv_f32_split_plan.py: where the kernel takes them, it is in these): an odd number of chunks in a slot (9, 25, 49), an even one; one slot, several, the last one in part
 EIGHTS = [
     (33, 128, 99, 99, 128, 3, 3, (2, 2), (1, 1, 1, 1), (1, 1), 1), (60, 48, 37, 37, 112, 3, 3, (2, 2), (1, 1, 1, 1), (1, 1), 1),
     (46, 61, 40, 64, 27, 5, 5, (2, 2), (2, 2, 2, 2), (1, 1), 1), (48, 81, 144, 11, 190, 7, 7, (2, 2), (3, 3, 3, 3), (1, 1), 1),
@@ -124,16 +124,21 @@ def test_transposed_conv_in_three_parts(ops, kept, n, c, h, w, oc, k, s):
         assert float((y[i:i + 1].cpu().double() - ref).abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())), i
 
 
-# N, C, H, W, OC, k, (pad, right and bottom pad less), groups: all four phases by one workgroup; 16-byte stores where W is whole fours and the output
+# N, C, H, W, OC, k, (pad, right and bottom pad), groups: all four phases by one workgroup (as above, by its choice); 16-byte stores where W is whole fours and the output
 # twice as wide; phases of equal and of unequal length and extent; one slot and several, the last one in part; blocks of 16 to 64 channels
 TOGETHER = [
-    (64, 128, 28, 28, 64, 4, (1, 1), 1), (48, 54, 31, 29, 64, 4, (1, 1), 1), (40, 33, 24, 20, 48, 4, (0, 0), 1), (128, 32, 24, 24, 17, 2, (0, 0), 1),
+    (64, 128, 28, 28, 64, 4, (1, 1), 1), (48, 54, 31, 29, 40, 4, (1, 1), 1), (60, 33, 24, 20, 48, 4, (0, 0), 1), (128, 32, 24, 24, 17, 2, (0, 0), 1),
     (30, 70, 31, 33, 60, 2, (0, 0), 1), (60, 46, 24, 23, 64, 3, (1, 0), 1), (60, 46, 20, 24, 70, 3, (1, 1), 1), (24, 40, 23, 26, 96, 5, (2, 1), 1),
-    (30, 96, 20, 20, 128, 4, (1, 1), 2), (200, 24, 9, 8, 130, 3, (1, 0), 1), (16, 20, 70, 72, 16, 6, (2, 2), 1)]
+    (200, 24, 9, 8, 130, 3, (1, 0), 1), (16, 20, 70, 72, 16, 6, (2, 2), 1),
+    (40, 96, 28, 28, 64, 4, (1, 1), 2), (40, 96, 24, 27, 32, 4, (1, 1), 2), (60, 92, 27, 28, 66, 3, (1, 0), 2), (40, 92, 27, 25, 34, 3, (1, 0), 2)]      # groups, 16 and 4 bytes
+
+
+# phases of a workgroup each, or not, by a little
+APART = [(48, 54, 31, 29, 64, 4, (1, 1), 1), (40, 33, 24, 20, 48, 4, (0, 0), 1), (30, 96, 20, 20, 128, 4, (1, 1), 2)]
 
 
 @pytest.mark.parametrize("large", [False, True])
-@pytest.mark.parametrize("shape", TOGETHER)
+@pytest.mark.parametrize("shape", TOGETHER + APART)
 def test_phases_of_one_workgroup(ops, kept, shape, large):
     """Bounds as above: 1e-5 of the largest output and 3e-7 in the 2-norm; operands of 2^60, whose sums are formed again in fp32, a rounding for each
     product."""
@@ -155,6 +160,48 @@ def test_phases_of_one_workgroup(ops, kept, shape, large):
             assert bool((err.abs() <= (c * k * k) ** 0.5 * 2.0 ** -24 * conv(xi.abs(), wi.abs())).all()), i
         else:
             assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())) and float(err.norm()) <= 3e-7 * float(ref.norm()), i
+
+
+@pytest.mark.parametrize("shape,up", [(s, False) for s in EIGHTS[:3] + EIGHTS[5:6]] + [(s, True) for s in TOGETHER[:7] + TOGETHER[10:]])
+def test_bias_and_relu_of_strided_and_transposed_layers(ops, kept, shape, up):
+    """A bias for every channel, in 16-byte and in 4-byte stores, in the exchange between two phases and behind sums that are formed again; ReLU; bounds
+    as above. One image has an infinity, which meets its own window alone: NaN or an infinity there, the rest as without it."""
+    if up:
+        n, c, h, w, oc, k, (before, behind), groups = shape
+        g = torch.Generator(device="cuda").manual_seed(n + oc)
+        wt = torch.randn(c, oc // groups, k, k, device="cuda", generator=g) * (c // groups * k * k / 4) ** -0.5
+        call = lambda x, relu: ops.conv_transpose2d_f32(x, wt, bias, (before, before, behind, behind), (2, 2), (1, 1), groups, (0, 0), relu=relu, ctx=kept)
+    else:
+        n, c, h, w, oc, kh, kw, s, pads, d, groups = shape
+        g = torch.Generator(device="cuda").manual_seed(n + oc)
+        wt = torch.randn(oc, c // groups, kh, kw, device="cuda", generator=g) * (c // groups * kh * kw) ** -0.5
+        call = lambda x, relu: ops.conv2d_f32(x, wt, bias, pads, s, d, groups, relu=relu, ctx=kept)
+    x, bias = torch.randn(n, c, h, w, device="cuda", generator=g), torch.randn(oc, device="cuda", generator=g)
+    torch.cuda.synchronize()
+    y, names = names_of(kept, lambda: call(x, True))
+    plain, _ = names_of(kept, lambda: call(x, False))
+    assert names[-1] == "k_conv_f32_split", names
+    assert torch.equal(y, plain.clamp(min=0)) and bool((plain < 0).any())
+    H, W = y.shape[2:]
+    for i in sorted({0, n // 2, n - 1}):
+        xi = x[i:i + 1].cpu().double()
+        if up:
+            ref = torch.nn.functional.conv_transpose2d(xi, wt.cpu().double(), None, 2, 0, 0, groups)[:, :, before:before + H, before:before + W] + bias.cpu().double().view(1, -1, 1, 1)
+        else:
+            ref = reference(x[i:i + 1], wt, bias, s, pads, d, groups)
+        err = plain[i:i + 1].cpu().double() - ref
+        assert float(err.abs().max()) <= 1e-5 * max(1.0, float(ref.abs().max())) and float(err.norm()) <= 3e-7 * float(ref.norm()), i
+    x[n // 2, 0, h // 2, w // 2] = float("inf")
+    torch.cuda.synchronize()
+    z, names = names_of(kept, lambda: call(x, False))
+    assert names[-1] == "k_conv_f32_split", names
+    bad = ~z[n // 2].isfinite()
+    assert bool(bad.any()) and not bool((~z.isfinite()).sum() != bad.sum())
+    rows, cols = bad.any(0).any(1).nonzero(), bad.any(0).any(0).nonzero()
+    size = (k, k) if up else ((kh - 1) // s[0] + 1, (kw - 1) // s[1] + 1)
+    assert int(rows.max() - rows.min()) < max(size[0], 1) * (1 if up else d[0]) + 1 and int(cols.max() - cols.min()) < max(size[1], 1) * (1 if up else d[1]) + 1
+    keep = z.isfinite()
+    assert float((z[keep] - plain[keep]).abs().max()) <= 2e-5 * max(1.0, float(plain.abs().max()))      # (the two sums' bounds together)
 
 
 @pytest.mark.parametrize("n,c,h,oc,k,s,up", [(300, 1, 96, 100, 7, 1, False), (230, 128, 99, 128, 3, 2, False), (1400, 128, 28, 64, 4, 2, True), (300, 32, 99, 96, 3, 1, False)])
