@@ -354,9 +354,11 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 
    // (what was requested behind the last step is let in here: the compiler would wait for it between stores, and so for stores)
    __builtin_amdgcn_s_waitcnt(0);
-   // sums that are not finite: again, with fp32 instructions on the operands as they were given. 256x64x56x56 -> 128, 3x3, 0.6 ms: 0.16 ms more
-   // with one infinity, 0.46 with one in every image, 6 to 8 with an infinite weight or one infinity in a hundred cells (every tile repeated);
-   // 16x3x224x224 -> 64, 7x7 s2, 33 us: 0.13, 0.42 and 0.44 ms more
+   // sums that are not finite: again, tile by tile of 16 x 16, with fp32 instructions on the operands as they were given. One gathers 0.35 us for every four
+   // products of a sum. us without one, with one infinity in x, one in every image, all sums above 2^95: 256x64x56x56 -> 128, 3x3 581 / 644 / 1190 / 13000;
+   // 33x128x99x99 -> 128, 3x3 s2 171 / 550 / 624 / 4340 (1950 / 2050 / 5000 with all of a wavefront's tiles); 48x80x144x11 -> 192, 7x7 s2 171 / 1650 / 1760 / 4670;
+   // transposed 64x128x28x28 -> 64, 4x4 s2 89 / 452 / 523 / 1890 (890 / 970 / 1830); 60x46x24x23 -> 64, 3x3 s2 31 / 92 / 104 / 336. The branch
+   // lies behind the kernel: in front of the stores each of its instructions cost the others (two steps at a time 1.16 times longer at 13 us).
    v4f none = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
    for (int i = 0; i < TI; ++i)
@@ -365,14 +367,14 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
          for (int e = 0; e < 4; ++e) none[e] = fmaf(acc[i][j][e], 0.0f, none[e]);
    const float any = (none[0] + none[1]) + (none[2] + none[3]);
-   float factor = UNSCALE;
+   unsigned again_of = 0;      // the tiles whose sums were formed again, a bit each
    int p1 = p0;      // (so that nothing of the pixels' places is kept in registers through the loop)
    asm volatile("" : "+s"(p1));
-   if (__builtin_amdgcn_ballot_w64(any != 0.0f) != 0) {
+   if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0.0f) != 0, 0)) {
       // (the arguments once more, from memory, and one tile after the other: in registers through the loop, for this branch, they cost 3 %
       // of every call and up to 13 with few channels. 32 channels x 128 pixels read the weights' alone again: with all of them the
       // compiler spills fragments in the loop.)
-      constexpr bool ALL = TI * TJ != 4 || WO == 1 || TI == 2;
+      constexpr bool ALL = (TI * TJ != 4 || WO == 1 || TI == 2);
       auto again = __builtin_amdgcn_kernarg_segment_ptr();
       asm volatile("" : "+s"(again));
       const SplitArgs &late = *(const SplitArgs *)again, &h = ALL ? late : g;
@@ -380,23 +382,42 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
       const int ftaps = f.KH * f.KW;
       const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(h.x), 0, (int)h.xbytes, 0x00020000);
       const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(late.w0), 0, (int)OUTSIDE, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+         for (int j = 0; j < TJ; ++j) {
+            float z = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z = fmaf(acc[i][j][e], 0.0f, z);
+            if (__builtin_amdgcn_ballot_w64(z != 0.0f) != 0) again_of |= 1u << (i * TJ + j);
+         }
+      const int total = (h.icg + 3) / 4 * ftaps;
 #pragma unroll 1
-      for (int tile = 0; tile < TI * TJ; ++tile) {
+      for (unsigned left = again_of; left != 0; left &= left - 1) {
+         const int tile = __builtin_ctz(left);
          const int p = p1 + (wp * TJ + tile % TJ) * 16 + r16, panel = fdiv(p, f.dPHW), r = p - panel * f.PHW, oy = fdiv(r, f.dWS), n = fdiv(panel, f.dStrips);
          const int iy0 = oy * h.sh + f.down - f.ph, ix0 = ((panel - n * f.strips) * f.ws + r - oy * f.ws) * h.sw + f.right - f.pw;
          const int oc = (tile0 + tile / TJ) * 16 + r16;
          v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+         int c = kg, t = 0;
+         // (requests of two steps leave together)
 #pragma unroll 1
-         for (int c0 = 0; c0 < h.icg; c0 += 4) {
-            const int c = c0 + kg;
-#pragma unroll 1
-            for (int t = 0; t < ftaps; ++t) {
+         for (int step = 0; step < total; step += 2) {
+            float xv[2], wv[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
                const int a = fdiv(t, f.dKW), b = t - a * f.KW, iy = iy0 + a * h.dh, ix = ix0 + b * h.dw;
                const bool in = p < f.P && r < f.full && c < h.icg && (unsigned)iy < (unsigned)h.H && (unsigned)ix < (unsigned)h.W;
-               const float xv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * h.chw4 + (iy * h.W + ix) * 4 + (grp * h.icg + c) * h.hw4) : OUTSIDE), 0, 0));
-               const float wv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ors, (int)(c < h.icg && oc < h.ocg ? 4u * weight_at(late, weights, grp, oc, c, a, b, ROWS) : OUTSIDE), 0, 0));
-               sum = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wv, sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv, sum, 0, 0, 0);
+               xv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, (int)(in ? (unsigned)(n * h.chw4 + (iy * h.W + ix) * 4 + (grp * h.icg + c) * h.hw4) : OUTSIDE), 0, 0));
+               wv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ors, (int)(c < h.icg && oc < h.ocg ? 4u * weight_at(late, weights, grp, oc, c, a, b, ROWS) : OUTSIDE), 0, 0));
+               if (++t == ftaps) {
+                  t = 0;
+                  c += 4;
+               }
             }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+               if (step + u < total) sum = STORE == QUADS ? __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u], wv[u], sum, 0, 0, 0) : __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u], xv[u], sum, 0, 0, 0);
          }
 #pragma unroll
          for (int i = 0; i < TI; ++i)
@@ -405,13 +426,12 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
                for (int e = 0; e < 4; ++e) acc[i][j][e] = tile == i * TJ + j ? sum[e] : acc[i][j][e];
       }
-      factor = 1.0f;
    }
 
    const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(g.y, 0, (int)g.ybytes, 0x00020000);
    const rsrc_t yrs4 = make_rsrc(g.y, g.ybytes);
-   auto finish = [&](float v, float b) {
-      v = __fmul_rn(v, factor);
+   auto finish = [&](float v, float b, int tile) {
+      v = __fmul_rn(v, again_of >> tile & 1 ? 1.0f : UNSCALE);
       if (g.bias) v = __fadd_rn(v, b);
       return g.relu ? (v > 0.0f ? v : 0.0f) : v;
    };
@@ -426,7 +446,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
 #pragma unroll
          for (int j = 0; j < TJ; ++j) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][j][e] = finish(acc[i][j][e], bias[i][0]);
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = finish(acc[i][j][e], bias[i][0], i * TJ + j);
             swap[((wave * TI + i) * TJ + j) * 64 + lane] = odd ? v2f{acc[i][j][0], acc[i][j][1]} : v2f{acc[i][j][2], acc[i][j][3]};
          }
       __syncthreads();
@@ -455,7 +475,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
                v = q.ox0 != 0 ? v4f{o[0], v[2], o[1], v[3]} : v4f{v[0], o[0], v[1], o[1]};
             } else {
 #pragma unroll
-               for (int e = 0; e < 4; ++e) v[e] = finish(v[e], bias[i][0]);
+               for (int e = 0; e < 4; ++e) v[e] = finish(v[e], bias[i][0], i * TJ + j);
             }
             store16_buf(yrs4, v, there ? at_pixel + (unsigned)(r16 * g.plane4) : OUTSIDE, (unsigned)(grp * g.ocg + oc) * (unsigned)g.plane4);
          } else {
@@ -463,7 +483,7 @@ __global__ void __launch_bounds__(THREADS, SplitPlan::resident_of(TI, TJ, WO)) k
             for (int e = 0; e < 4; ++e) {
                if (oc + e >= g.ocg) continue;
                const bool there = pixel && oc + 4 * kg + e < g.ocg;
-               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, finish(v[e], bias[i][STORE == QUADS ? 0 : e])), yrs, (int)(there ? at_pixel + (unsigned)(kg * 4 * g.plane4) : OUTSIDE),
+               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, finish(v[e], bias[i][STORE == QUADS ? 0 : e], i * TJ + j)), yrs, (int)(there ? at_pixel + (unsigned)(kg * 4 * g.plane4) : OUTSIDE),
                                                      (int)((unsigned)(grp * g.ocg + oc + e) * (unsigned)g.plane4), 0);
             }
          }

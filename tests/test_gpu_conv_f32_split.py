@@ -336,3 +336,35 @@ def test_whole_numbers_are_exact(ops, kept):
     y, names = names_of(kept, lambda: ops.conv2d_f32(x, w, None, (1, 1), ctx=kept))
     assert names[-1] == "k_conv_f32_split"
     assert torch.equal(y.cpu(), torch.nn.functional.conv2d(x.cpu(), w.cpu(), None, 1, 1))
+
+
+@pytest.mark.parametrize("kind", ["cell of a strided layer", "cell of a transposed layer", "weight"])
+def test_sums_are_formed_again_in_their_tiles_alone(ops, kept, kind):
+    """An infinity in a cell that few windows hold, or in one weight: tiles of 16 pixels x 16 channels without a sum that is not finite keep every bit."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    up, s = kind == "cell of a transposed layer", 2 if kind == "cell of a strided layer" else 1
+    n, c, h, w, oc, k = (64, 128, 28, 28, 64, 4) if up else EIGHTS[0][:6] if s == 2 else CONV[0][:6]
+    x, wt = torch.randn(n, c, h, w, device="cuda", generator=g), torch.randn(*((c, oc) if up else (oc, c)), k, k, device="cuda", generator=g) * (c * k * k) ** -0.5
+    torch.cuda.synchronize()
+    if up:
+        call = lambda ctx: ops.conv_transpose2d_f32(x, wt, None, (1, 1, 1, 1), (2, 2), (1, 1), 1, (0, 0), ctx=ctx)
+    else:
+        call = lambda ctx: ops.conv2d_f32(x, wt, None, (1, 1, 1, 1), (s, s), (1, 1), 1, ctx=ctx)
+    y, names = names_of(kept, lambda: call(kept))
+    assert names[-1] == "k_conv_f32_split"
+    if kind == "weight":
+        wt[70, 3, 1, 1] = float("inf")
+    else:
+        x[5, 2, 10, 12] = float("inf")
+    torch.cuda.synchronize()
+    other = ops.Context(0)      # (keeps no weights of the call before)
+    other.check(other.lib.sofie_hip_constant_weights(other.h, 1))
+    z, names = names_of(other, lambda: call(other))
+    assert names[-1] == "k_conv_f32_split"
+    differs, bad = z != y, ~z.isfinite()
+    if kind == "weight":
+        assert bool(bad[:, 70].all()) and not bool(differs[:, :64].any() or differs[:, 80:].any()) and not bool(bad[:, 71:].any())
+    else:
+        pixels = bad.any(1).sum()
+        assert int(pixels) == (16 if up else 1) and int(differs.any(1).sum()) <= 16 * int(pixels) and not bool(differs[:5].any() or differs[6:].any())
+    other.close()
