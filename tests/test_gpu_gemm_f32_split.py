@@ -17,7 +17,7 @@ def ops():
     return o
 
 
-def product(ctx, a, b, tA, tB, bias, alpha=1.0, beta=1.0, relu=False, pad=0):
+def product(ctx, a, b, tA, tB, bias, alpha=1.0, beta=1.0, relu=False, pad=0, kind=L.BIAS_ROW):
     """The call through the C ABI, rows of all operands `pad` floats further apart than they are long; the result and the kernels' names."""
     M, N, K = (a.shape[1] if tA else a.shape[0]), (b.shape[0] if tB else b.shape[1]), (a.shape[0] if tA else a.shape[1])
 
@@ -32,7 +32,7 @@ def product(ctx, a, b, tA, tB, bias, alpha=1.0, beta=1.0, relu=False, pad=0):
     buf, n = C.create_string_buffer(4096), C.c_int(-1)
     ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
     ctx.check(ctx.lib.sofie_hip_gemm_f32(ctx.h, tA, tB, M, N, K, alpha, a.data_ptr(), a.shape[1], b.data_ptr(), b.shape[1], beta if bias is not None else 0.0,
-                                         bias.data_ptr() if bias is not None else None, L.BIAS_ROW if bias is not None else L.BIAS_NONE,
+                                         bias.data_ptr() if bias is not None else None, kind if bias is not None else L.BIAS_NONE,
                                          y[1].data_ptr(), N + pad, L.ACT_RELU if relu else L.ACT_NONE))
     ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(n)))
     ctx.sync()
@@ -184,4 +184,63 @@ def test_an_infinity_in_the_last_tile_changes_no_bit_of_the_others(ops, M, N, K,
                 assert torch.equal(yi[:, :N // 64 * 64], y[:, :N // 64 * 64]) and not bool(yi[:, N - 1].isfinite().any())
             else:
                 assert torch.equal(yi[:M // 64 * 64 if tA else M // 128 * 128], y[:M // 64 * 64 if tA else M // 128 * 128]) and not bool(yi[M - 1].isfinite().any())
+    ctx.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(2711, 5089, 337), (5043, 4527, 451)])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("kind", [L.BIAS_NONE, L.BIAS_ROW, L.BIAS_COL])
+def test_scale_bias_and_relu_on_shared_fragments(ops, M, N, K, tA, tB, kind):
+    g = torch.Generator(device="cuda").manual_seed(M + kind)
+    a, b = torch.randn(M, K, device="cuda", generator=g), torch.randn(K, N, device="cuda", generator=g) * K ** -0.5
+    bias = None if kind == L.BIAS_NONE else torch.randn(N if kind == L.BIAS_ROW else M, device="cuda", generator=g)
+    stored = (a.t().contiguous() if tA else a, b.t().contiguous() if tB else b)
+    ctx = ops.Context(0)
+    y, names = product(ctx, *stored, tA, tB, bias, alpha=-0.5, beta=2.0, relu=True, pad=3, kind=kind)
+    assert names == ["k_gemm_f32_split_shared"], names
+    want = -0.5 * (a.double() @ b.double())
+    if bias is not None:
+        want += 2.0 * (bias.double() if kind == L.BIAS_ROW else bias.double()[:, None])
+    want = want.clamp(min=0)
+    err = y.double() - want
+    assert float(err.norm()) <= 3e-7 * float(want.norm()) and float(err.abs().max()) <= 1e-6 * float(want.abs().max())
+    ctx.close()
+
+
+# leading dimensions of A and of B (1: one matrix for all), M, N, K: 512 tiles of 128 x 128, the last ones cut
+@pytest.mark.parametrize("la,lb,M,N,K", [((2,), (2,), 2041, 2047, 330), ((2, 4), (1, 4), 1021, 1019, 451), ((4, 1), (1, 2), 1021, 1019, 330), ((1,), (4,), 2045, 1017, 451)])
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_stacks_on_shared_fragments(ops, la, lb, M, N, K, tA, tB, relu):
+    """Stacked products, broadcast ones among them, each against float64; an infinity in one product's last row changes no other product."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, b = torch.randn(*la, M, K, device="cuda", generator=g), torch.randn(*lb, K, N, device="cuda", generator=g) * K ** -0.5
+    lead = torch.broadcast_shapes(la, lb)
+    n, strides = len(lead), lambda l, mat: [0 if l[i] == 1 else mat * int(torch.tensor(l[i + 1:]).prod()) for i in range(len(l))]
+    ctx = ops.Context(0)
+
+    def stacked(a, b):
+        a, b = a.transpose(-1, -2).contiguous() if tA else a, b.transpose(-1, -2).contiguous() if tB else b
+        y = torch.full((*lead, M, N), 77.0, device="cuda")
+        torch.cuda.synchronize()
+        buf, m = C.create_string_buffer(4096), C.c_int(-1)
+        ctx.check(ctx.lib.sofie_hip_trace_begin(ctx.h))
+        ctx.check(ctx.lib.sofie_hip_gemm_f32_stacked(ctx.h, tA, tB, M, N, K, -0.5, a.data_ptr(), a.shape[-1], b.data_ptr(), b.shape[-1], y.data_ptr(), N, n,
+                                                     (C.c_int * n)(*lead), (C.c_longlong * n)(*strides(la, M * K)), (C.c_longlong * n)(*strides(lb, K * N)),
+                                                     L.ACT_RELU if relu else L.ACT_NONE))
+        ctx.check(ctx.lib.sofie_hip_trace_end(ctx.h, buf, 4096, C.byref(m)))
+        ctx.sync()
+        assert [line.split()[0] for line in buf.value.decode().splitlines()] == ["k_gemm_f32_split_shared"]
+        return y.reshape(-1, M, N)
+    y = stacked(a, b)
+    af, bf = a.expand(*lead, M, K).reshape(-1, M, K), b.expand(*lead, K, N).reshape(-1, K, N)
+    for i in range(y.shape[0]):
+        want = -0.5 * (af[i].double() @ bf[i].double())
+        want = want.clamp(min=0) if relu else want
+        err = y[i].double() - want
+        assert float(err.norm()) <= 3e-7 * float(want.norm()) and float(err.abs().max()) <= 1e-6 * float(want.abs().max()), i
+    if la == lead:
+        a[(-1,) * len(la) + (M - 1, K - 1)] = float("inf")
+        z = stacked(a, b)
+        assert torch.equal(z[:-1], y[:-1]) and torch.equal(z[-1, :M // 128 * 128 - 128], y[-1, :M // 128 * 128 - 128]) and not bool(z[-1, M - 1].isfinite().all())
     ctx.close()
