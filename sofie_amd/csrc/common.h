@@ -135,8 +135,8 @@ __device__ __forceinline__ int fdiv(int x, FastDiv f)
 // Every line of a kernel's arguments (BYTES of them, 64 each) is asked for at once: the compiler reads them where they are first needed, each a trip to
 // memory of its own while the launch is new to the chip. For kernels with three lines and more, or behind a copy in one call. us, in turn with
 // the same code without it: int8 classifier of 64 images (five launches) 27.9 -> 26.6, of 1 23.4 -> 22.4, float classifier of 1 31.3 -> 30.2; fp32 convolutions of
-// 4 to 9 us (k_conv_f32_any, ten lines) 1.04 to 1.11 times shorter, transposed ones 1.026 in the mean over 45, 0.97 the worst (127x4x6x6 -> 71,
-// 3x3 s2 11.7 -> 12.0); int8 convolutions with a copy in front 1.00 to 1.13. Not in kernels of two lines (k_gemm_bytes_direct, k_gemm_f32_direct: 0.95 to
+// 4 to 9 us (k_conv_f32_any, ten lines) 1.04 to 1.11 times shorter, transposed ones 1.026 in the mean over 45 and, with the rest of its changes, 1.036 over 47 others, of which
+// four are longer (3x152x27x27 -> 17, 2x2 s2 8.15 -> 8.44, 127x4x6x6 -> 71, 3x3 s2 11.6 -> 11.85); int8 convolutions with a copy in front 1.00 to 1.13. Not in kernels of two lines (k_gemm_bytes_direct, k_gemm_f32_direct: 0.95 to
 // 1.01), nor in k_qconv_any (0.94 to 1.02), k_conv_f32_split of one phase (0.99 to 1.01), k_conv2d_f32_dma of one (0.93 to 1.0).
 template <int BYTES>
 __device__ __forceinline__ void ask_for_arguments()
